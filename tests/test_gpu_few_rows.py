@@ -1,0 +1,38 @@
+"""Products of a few rows with a transposed weight, against sums in 64 bits."""
+import numpy as np
+import pytest
+
+from webdnn_amd import hostops as H
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("n,k", [(2, 128), (3, 131), (7, 1023), (1000, 2048), (4099, 516), (8192, 128), (4096, 130)])
+def test_few_rows(ctx, m, n, k):
+    rng = np.random.default_rng(m * 100003 + n * 101 + k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    got = H.gemm(ctx, ctx.move_tensor(a), ctx.move_tensor(b), ctx.move_tensor(bias), 0.5, 2.0, 0, 1, epilogue="relu").get_data()
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    want = np.maximum(0.5 * (a64 @ b64.T) + 2.0 * bias, 0.0)
+    # a chain of at most k roundings of half an ulp of the sum of magnitudes, then alpha, beta and the bias
+    bound = (k + 4) * 2.0 ** -24 * (0.5 * (np.abs(a64) @ np.abs(b64.T)) + 2.0 * np.abs(bias))
+    assert got.shape == want.shape and (np.abs(got - want) <= bound).all()
+
+
+def test_few_rows_agree_with_the_other_form_and_keep_inf_and_nan(ctx):
+    rng = np.random.default_rng(5)
+    a, b = rng.standard_normal((3, 700)).astype(np.float32), rng.standard_normal((37, 700)).astype(np.float32)
+    a[1, 3], b[5, 699], b[36, 0] = np.inf, np.nan, -np.inf
+    ta, tb = ctx.move_tensor(a), ctx.move_tensor(b)
+    got = H.gemm(ctx, ta, tb, None, 1.0, 1.0, 0, 1).get_data()
+    ctx.set_option("gemm_wavesplit", 0)
+    try:
+        other = H.gemm(ctx, ta, tb, None, 1.0, 1.0, 0, 1).get_data()
+    finally:
+        ctx.set_option("gemm_wavesplit", 1)
+    assert (np.isnan(got) == np.isnan(other)).all() and (np.isinf(got) == np.isinf(other)).all()
+    fin = np.isfinite(other)
+    assert (got[~fin & ~np.isnan(got)] == other[~fin & ~np.isnan(other)]).all()
+    np.testing.assert_allclose(got[fin], other[fin], rtol=0, atol=700 * 2.0 ** -23 * 700)

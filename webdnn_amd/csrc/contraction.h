@@ -1725,6 +1725,8 @@ extern bool g_static_scratch;  // set for the duration of a wdh_gemm_static call
 // what launch_planned decided for the most recent launch (wdh_last_plan)
 struct LastPlan { int bm, bn, split, form; long long full, tail; };
 extern LastPlan g_last_plan;
+constexpr int GEMM_ROWS_MAX = 4;  // rows gemm_rows_kernel keeps sums for
+int launch_gemm_rows(const Params &p, int batch, bool vec);
 extern int g_stream_spin;
 extern unsigned *g_stream_error_dev;
 float *static_scratch();     // device address of the static workspace on the current device, or null

@@ -309,6 +309,16 @@ static bool wavesplit_suits(int batch, int m, int n, int k) {
          (blocks32 * 2 >= wdh::compute_units() || k <= 512);
 }
 
+// Whether a product (both operands k-contiguous) is one for gemm_rows_kernel: so few rows that reading the weight
+// is all there is to it.  At four rows it takes 16.4 us where gemm_wavesplit_kernel
+// takes 29.7 (n = k = 4096), 6.0 against 20.1 (n 1000), 47 against 61 (n = k = 8192) and 3.1 against 3.7 (n = k = 256);
+// each row costs registers and a load of its own, so more of them belong to the matrix cores.  A group's products
+// (wdh_linear_group) have weights that are not k-contiguous, or leave in one launch.
+static bool gemm_rows_suits(int m, int n, int k) {
+  return g_wavesplit && g_forced_tile < 0 && g_forced_split < 0 && m <= GEMM_ROWS_MAX && k >= 128 && n >= 2 &&
+         !g_group.collecting;
+}
+
 extern "C" int wdh_set_option(const char *name, int value) {
   if (!name) return fail(WDH_EINVAL, "wdh_set_option: name is NULL");
   if (strcmp(name, "contraction_tile") == 0) {
@@ -530,6 +540,8 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
     p.c_bytes = ok ? (int)c_bytes : 0;
     set_wide(p, false);
   }
+  // A few rows against a transposed weight: a pass over the weight (gemm_rows.hip)
+  if (useA_kc && useB_kc && gemm_rows_suits(m, n, k)) return launch_gemm_rows(p, batch, vec);
   // Few result tiles and a K worth cutting: one launch with K cut across the wavefronts of a
   // workgroup (gemm_wavesplit_kernel) instead of chunks in a workspace and a reduce pass
   if (useA_kc && p.fast && wavesplit_suits(batch, m, n, k)) {
