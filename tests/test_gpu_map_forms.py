@@ -1,7 +1,9 @@
-"""Reductions over an inner axis on the GPU, against sums in 64 bits."""
+"""Reductions over an inner axis, squares and Sigmoid on the GPU, where they take forms of their own."""
 import numpy as np
 import pytest
 
+from oracle import ref
+from util import ulp_diff
 from webdnn_amd import hostops as H
 
 pytestmark = pytest.mark.gpu
@@ -16,3 +18,32 @@ def test_mean_over_an_inner_axis(ctx, shape, axis):
     # sums in double whatever their order: one rounding to fp32, and a sum's double error under cancellation
     slack = shape[axis] * 2.0 ** -52 * np.abs(x.astype(np.float64)).mean(axis)
     assert (np.abs(got - want) <= 2.0 ** -24 * np.abs(want) * 1.0001 + slack).all()
+
+
+def test_square_is_the_rounded_double_product(ctx):
+    rng = np.random.default_rng(9)
+    x = np.concatenate([rng.standard_normal(4099) * 10.0 ** rng.integers(-30, 19, 4099),
+                        [0.0, -0.0, np.inf, -np.inf, np.nan, 1e-45, 3e38]]).astype(np.float32)
+    with np.errstate(over="ignore", under="ignore"):
+        want = (x.astype(np.float64) * x.astype(np.float64)).astype(np.float32)
+    two = ctx.move_tensor(np.array([2.0], np.float32))
+    got = H.binary(ctx, "Pow", ctx.move_tensor(x), two).get_data()
+    assert (got.view(np.uint32) == want.view(np.uint32))[~np.isnan(want)].all() and np.isnan(got[np.isnan(want)]).all()
+    mixed = np.where(np.arange(x.size) % 3 == 0, 2.0, 3.0).astype(np.float32)
+    got = H.binary(ctx, "Pow", ctx.move_tensor(x), ctx.move_tensor(mixed)).get_data()
+    assert (got.view(np.uint32) == want.view(np.uint32))[~np.isnan(want) & (mixed == 2.0)].all()
+
+
+def test_sigmoid_over_the_whole_range(ctx):
+    x = np.concatenate([np.linspace(-60, 60, 200003), [-12.0, 40.0, np.nextafter(np.float32(-12), np.float32(-13)), 1e30, -1e30,
+                                                       np.inf, -np.inf, np.nan, 0.0]]).astype(np.float32)
+    got = H.unary(ctx, "Sigmoid", ctx.move_tensor(x)).get_data()
+    want = ref.unary("Sigmoid", x)
+    assert np.isnan(got[np.isnan(x)]).all()
+    # down to -12 the reference's cancelled sum is right to 2^-53 / sigmoid(-12), under 2^-35: only a value that lies
+    # that close to a rounding boundary may land one ulp away
+    near = x >= -12
+    assert ulp_diff(got[near], want[near]).max() <= 1
+    # below, both sides form tanh + 1, whose last place is 2^-53 (a double tanh is right to two of them)
+    far = x < -12
+    assert (np.abs(got[far].astype(np.float64) - want[far]) <= 2.0 ** -51 + 2.0 ** -23 * want[far]).all()

@@ -45,6 +45,10 @@ __device__ __forceinline__ float apply_f(float l, float r) {
   if (OP == WDH_BIN_SUB) return l - r;
   if (OP == WDH_BIN_MUL) return l * r;
   if (OP == WDH_BIN_DIV) return l / r;
+  // x^2 (a written-out variance): the square of an fp32 number is exact in double, so one fp32 product rounds it
+  // the same, and a wavefront whose exponents are all 2 skips pow's few hundred instructions
+  // ([8, 95, 126, 192] to the power of a scalar 2: 119.7 -> 31.3 us, 4.6 TB/s)
+  if (r == 2.0f) return l * l;
   return (float)pow((double)l, (double)r);
 }
 
@@ -321,10 +325,19 @@ __device__ __forceinline__ float relu_js(float v) {
   return v <= 0.0f ? 0.0f : v;
 }
 
+// (tanh(v/2) + 1) / 2 as the reference writes it.  Where the sum does not cancel, 1 / (1 + e^-v) is the same number
+// within a few double ulps and needs a quarter of the instructions (double tanh alone takes a wavefront longer than
+// its loads and stores); further out the written form's own rounding shows in fp32 and is kept
+// ([8, 192, 95, 126]: 94.9 -> 35.9 us).
+__device__ __forceinline__ double sigmoid_d(double v) {
+  if (v >= -12.0 && v <= 40.0) return 1.0 / (1.0 + exp(-v));
+  return (tanh(v / 2.0) + 1.0) / 2.0;
+}
+
 template <int OP>
 __device__ __forceinline__ float unary_f(float v) {
   if (OP == WDH_UN_RELU) return relu_js(v);
-  if (OP == WDH_UN_SIGMOID) return (float)((tanh((double)v / 2.0) + 1.0) / 2.0);
+  if (OP == WDH_UN_SIGMOID) return (float)sigmoid_d((double)v);
   if (OP == WDH_UN_SQRT) return (float)sqrt((double)v);
   if (OP == WDH_UN_EXP) return (float)exp((double)v);
   if (OP == WDH_UN_TANH) return (float)tanh((double)v);
