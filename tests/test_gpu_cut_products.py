@@ -1,0 +1,37 @@
+"""Products cut along K whose chunk sums a second kernel adds, against sums in 64 bits."""
+import numpy as np
+import pytest
+
+from webdnn_amd import hostops as H
+
+pytestmark = pytest.mark.gpu
+
+
+def within(got, a, b, extra):
+    """A chain of at most k roundings of half an ulp of the sum of magnitudes, and three more for the epilogue."""
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    want = a @ b + extra
+    bound = (a.shape[-1] + 4) * 2.0 ** -24 * (np.abs(a) @ np.abs(b) + np.abs(extra))
+    return (np.abs(got - np.maximum(want, 0.0)) <= bound).all()
+
+
+# chunk counts below, at and above the eight requested at a time; planes whose quads are whole and ragged; groups
+@pytest.mark.parametrize("split", [2, 7, 8, 9, 17])
+@pytest.mark.parametrize("c,cout,h,w,group", [(320, 24, 8, 8, 1), (320, 70, 7, 7, 1), (640, 12, 6, 10, 2), (320, 5, 1, 3, 1)])
+def test_cut_conv_with_residual(ctx, split, c, cout, h, w, group):
+    rng = np.random.default_rng(split * 1000 + c + h)
+    x = rng.standard_normal((3, c, h, w)).astype(np.float32)
+    wt, bias = rng.standard_normal((cout, c // group, 1, 1)).astype(np.float32), rng.standard_normal(cout).astype(np.float32)
+    r = rng.standard_normal((3, cout, h, w)).astype(np.float32)
+    ctx.set_option("split_k", split)
+    try:
+        got = H.conv(ctx, ctx.move_tensor(x), ctx.move_tensor(wt), ctx.move_tensor(bias), None, group, None, [0] * 4, [1, 1],
+                     epilogue="relu", residual=ctx.move_tensor(r)).get_data()
+    finally:
+        ctx.set_option("split_k", -1)
+    cg, og = c // group, cout // group
+    for i in range(3):
+        for g in range(group):
+            o = slice(g * og, (g + 1) * og)
+            extra = bias[o, None].astype(np.float64) + r[i, o].reshape(og, -1)
+            assert within(got[i, o].reshape(og, -1), wt[o, :, 0, 0], x[i, g * cg:(g + 1) * cg].reshape(cg, -1), extra)
