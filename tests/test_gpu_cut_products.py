@@ -15,6 +15,19 @@ def within(got, a, b, extra):
     return (np.abs(got - np.maximum(want, 0.0)) <= bound).all()
 
 
+# around the line between one workgroup a block and cut tiles, whole and ragged
+@pytest.mark.parametrize("m,n,k", [(384, 768, 3072), (257, 1025, 2560), (288, 928, 2559), (500, 514, 4099), (256, 1024, 2560), (33, 4127, 5000)])
+def test_long_k_with_residual(ctx, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    bias, r = rng.standard_normal(n).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    ta, tb, tbias, tr = (ctx.move_tensor(v) for v in (a, b, bias, r))
+    got = H.matmul(ctx, ta, tb, tbias, tr, "relu").get_data()
+    assert within(got, a, b, bias.astype(np.float64) + r)
+    got = H.gemm(ctx, ta, ctx.move_tensor(np.ascontiguousarray(b.T)), tbias, 1.0, 1.0, 0, 1, epilogue="relu").get_data()
+    assert within(got, a, b, bias.astype(np.float64))
+
+
 # chunk counts below, at and above the eight requested at a time; planes whose quads are whole and ragged; groups
 @pytest.mark.parametrize("split", [2, 7, 8, 9, 17])
 @pytest.mark.parametrize("c,cout,h,w,group", [(320, 24, 8, 8, 1), (320, 70, 7, 7, 1), (640, 12, 6, 10, 2), (320, 5, 1, 3, 1)])

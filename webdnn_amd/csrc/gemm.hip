@@ -319,6 +319,17 @@ static bool gemm_rows_suits(int m, int n, int k) {
          !g_group.collecting;
 }
 
+// Of the products gemm_wavesplit_kernel could take, those that the ordinary tiles, cut along K, do faster: a block of
+// 32x32 results is one workgroup's whole K, so with a few more blocks than CUs some CUs work twice as long, and once the
+// launch is bound by its products that shows.  Both sides (us; B n-contiguous, B k-contiguous): 384x768x3072 38.0 / 48.6
+// against 28.1 / 28.4 as tiles, 500x1024x4096 49.5 / 65.4 against 45.2 / 45.0, 700x512x2048 27.0 / 34.3 against 26.1 /
+// 25.7, 1000x1024x1024 30.3 / 37.0 against 30.2 / 29.8; below the line 500x1024x1024 16.2 / 20.3 against 21.6 / 21.7,
+// and with fewer blocks than CUs 850x256x2048 17.8 / 20.1 against 19.4 / 20.0.
+static bool tiles_beat_wavesplit(int batch, int m, int n, int k) {
+  const long long blocks32 = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch, cus = wdh::compute_units();
+  return blocks32 > cus && blocks32 * k >= 2560 * cus;
+}
+
 extern "C" int wdh_set_option(const char *name, int value) {
   if (!name) return fail(WDH_EINVAL, "wdh_set_option: name is NULL");
   if (strcmp(name, "contraction_tile") == 0) {
@@ -545,6 +556,11 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
   // Few result tiles and a K worth cutting: one launch with K cut across the wavefronts of a
   // workgroup (gemm_wavesplit_kernel) instead of chunks in a workspace and a reduce pass
   if (useA_kc && p.fast && wavesplit_suits(batch, m, n, k)) {
+    if (!g_group.collecting && !g_static_scratch && tiles_beat_wavesplit(batch, m, n, k)) {
+      // (the chunks' sums need a workspace, which this kernel does without: it serves when there is none left)
+      const int rc = launch_gemm_a_kc(useB_kc, p, batch, vec);
+      if (rc != WDH_ENOMEM) return rc;
+    }
     const long long blocks32 = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch;
     if (useB_kc || (long long)(k - 1) * p.sB0 * 4 < 0x7fffffffLL) {
       p.tiles_m = (m + 31) / 32;
