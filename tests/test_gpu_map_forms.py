@@ -47,3 +47,13 @@ def test_sigmoid_over_the_whole_range(ctx):
     # below, both sides form tanh + 1, whose last place is 2^-53 (a double tanh is right to two of them)
     far = x < -12
     assert (np.abs(got[far].astype(np.float64) - want[far]) <= 2.0 ** -51 + 2.0 ** -23 * want[far]).all()
+
+
+@pytest.mark.parametrize("rows,length", [(1, 65), (5, 256), (4095, 256), (4096, 256), (4097, 255), (5003, 65), (4099, 68), (9001, 257),
+                                         (3, 260), (7, 1024), (6, 4099), (2, 100004)])
+def test_row_means(ctx, rows, length):
+    x = np.random.default_rng(rows + length).standard_normal((rows, length)).astype(np.float32)
+    got = H.reduce_mean(ctx, ctx.move_tensor(x), [-1], 0).get_data()
+    want = x.astype(np.float64).mean(1)
+    slack = length * 2.0 ** -52 * np.abs(x.astype(np.float64)).mean(1)
+    assert (np.abs(got - want) <= 2.0 ** -24 * np.abs(want) * 1.0001 + slack).all()
