@@ -1,0 +1,15 @@
+"""Downloads in pieces."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def test_downloads_of_many_pieces(ctx):
+    """Sizes around the pieces that downloads and uploads travel in, with more pieces than are in flight."""
+    for n in (1, (1 << 18) - 1, 1 << 18, (1 << 18) + 1, 5 * (1 << 18) + 3, 9 * (1 << 18)):
+        x = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+        t = ctx.move_tensor(x)
+        assert (t.get_data() == x).all()
+        t.set_data(-x)
+        assert (t.get_data() == -x).all()

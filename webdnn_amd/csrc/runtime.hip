@@ -24,6 +24,8 @@ constexpr size_t kStagingBytes = 32u << 20;  // per pinned buffer, two of them
 // own, so that the host's copy of piece i+1 into pinned memory overlaps the DMA of piece i.
 constexpr size_t kUploadPiece = 4u << 20;
 constexpr int kUploadSlots = (int)(2 * kStagingBytes / kUploadPiece);
+constexpr size_t kReadPiece = 1u << 20;      // downloads: length of a piece, in the first staging buffer,
+constexpr size_t kReadAhead = 4;             // and pieces in flight
 constexpr size_t kSmallGranule = 512;        // allocation rounding below 1 MiB
 constexpr size_t kLargeGranule = 1u << 20;   // and above
 
@@ -76,8 +78,7 @@ struct Runtime {
   uint64_t limit = 0;  // "memory_limit_mib": the pool asks the driver for no more than this (0 = no limit)
   // pinned staging, ping-pong
   void *stage[2] = {nullptr, nullptr};
-  hipEvent_t stage_done[2] = {nullptr, nullptr};   // downloads: one event per buffer
-  hipEvent_t up_done[kUploadSlots] = {};            // uploads: one event per piece
+  hipEvent_t up_done[kUploadSlots] = {};            // uploads and downloads: one event per piece
   bool up_busy[kUploadSlots] = {};
   int up_next = 0;
   // timing events, created lazily
@@ -257,8 +258,6 @@ static int init_device(int device) {
     if (hipHostMalloc(&g.stage[i], kStagingBytes, hipHostMallocDefault) !=
         hipSuccess)
       return fail(WDH_ENOMEM, "wdh_init: pinned staging allocation failed");
-    WDH_HIP_CHECK(
-        hipEventCreateWithFlags(&g.stage_done[i], hipEventDisableTiming));
   }
   for (int i = 0; i < kUploadSlots; i++) {
     WDH_HIP_CHECK(hipEventCreateWithFlags(&g.up_done[i], hipEventDisableTiming));
@@ -324,9 +323,7 @@ static void release_everything() {
   g.in_use = g.cached = g.reserved = g.peak = 0;
   for (int i = 0; i < 2; i++) {
     if (g.stage[i]) (void)hipHostFree(g.stage[i]);
-    if (g.stage_done[i]) (void)hipEventDestroy(g.stage_done[i]);
     g.stage[i] = nullptr;
-    g.stage_done[i] = nullptr;
   }
   for (int i = 0; i < kUploadSlots; i++) {
     if (g.up_done[i]) (void)hipEventDestroy(g.up_done[i]);
@@ -671,34 +668,24 @@ int wdh_read(wdh_buf h, size_t src_offset, void *dst, size_t bytes) {
   // staging buffers may still carry an in-flight upload
   if (int rc = wait_for_uploads()) return rc;
   char *d = (char *)dst;
-  size_t issued = 0, copied = 0;
-  size_t chunk_of[2] = {0, 0};
-  int which = 0;
-  // ping-pong: the D2H of chunk i+1 overlaps the host memcpy of chunk i
-  if (bytes) {
-    chunk_of[0] = bytes < kStagingBytes ? bytes : kStagingBytes;
-    WDH_HIP_CHECK(hipMemcpyAsync(g.stage[0], src + src_offset, chunk_of[0],
-                                 hipMemcpyDeviceToHost, g.stream));
-    WDH_HIP_CHECK(hipEventRecord(g.stage_done[0], g.stream));
-    issued = chunk_of[0];
-  } else {
-    WDH_HIP_CHECK(hipStreamSynchronize(g.stream));
-  }
-  while (copied < bytes) {
-    int next = which ^ 1;
-    if (issued < bytes) {
-      chunk_of[next] =
-          bytes - issued < kStagingBytes ? bytes - issued : kStagingBytes;
-      WDH_HIP_CHECK(hipMemcpyAsync(g.stage[next], src + src_offset + issued,
-                                   chunk_of[next], hipMemcpyDeviceToHost,
+  // Short pieces through the staging memory of the uploads, all free by now, kReadAhead of them in flight: a piece is
+  // copied out of pinned memory while the next ones arrive, and a slot is asked for again only after that.
+  // (12.6 MB, the results of an [8, 512, 768] block: the whole host-to-host pass 1476 -> 1296 us; one piece of up to
+  // 32 MB, as before, leaves the copy into cold user memory no transfer to overlap with.)
+  if (!bytes) WDH_HIP_CHECK(hipStreamSynchronize(g.stream));
+  auto length = [&](size_t at) { return bytes - at < kReadPiece ? bytes - at : kReadPiece; };
+  auto read_slot = [](int slot) { return (char *)g.stage[0] + slot * kReadPiece; };
+  size_t issued = 0;
+  for (size_t copied = 0; copied < bytes; copied += kReadPiece) {
+    for (; issued < bytes && issued < copied + kReadAhead * kReadPiece; issued += kReadPiece) {
+      const int slot = (int)(issued / kReadPiece % kReadAhead);
+      WDH_HIP_CHECK(hipMemcpyAsync(read_slot(slot), src + src_offset + issued, length(issued), hipMemcpyDeviceToHost,
                                    g.stream));
-      WDH_HIP_CHECK(hipEventRecord(g.stage_done[next], g.stream));
-      issued += chunk_of[next];
+      WDH_HIP_CHECK(hipEventRecord(g.up_done[slot], g.stream));
     }
-    WDH_HIP_CHECK(hipEventSynchronize(g.stage_done[which]));
-    memcpy(d + copied, g.stage[which], chunk_of[which]);
-    copied += chunk_of[which];
-    which = next;
+    const int slot = (int)(copied / kReadPiece % kReadAhead);
+    WDH_HIP_CHECK(hipEventSynchronize(g.up_done[slot]));
+    memcpy(d + copied, read_slot(slot), length(copied));
   }
   g.lane_dirty[g.lane] = false;     // (the stream has drained up to the data just read)
   return wdh::contraction_check();
