@@ -2,6 +2,7 @@
 import numpy as np
 import pytest
 
+from webdnn_amd import capi
 from webdnn_amd import hostops as H
 
 pytestmark = pytest.mark.gpu
@@ -26,6 +27,25 @@ def test_long_k_with_residual(ctx, m, n, k):
     assert within(got, a, b, bias.astype(np.float64) + r)
     got = H.gemm(ctx, ta, ctx.move_tensor(np.ascontiguousarray(b.T)), tbias, 1.0, 1.0, 0, 1, epilogue="relu").get_data()
     assert within(got, a, b, bias.astype(np.float64))
+
+
+def test_no_room_for_the_chunk_sums(ctx):
+    """Without memory for the workspace of cut tiles the product runs in one launch, and no error stays behind."""
+    rng = np.random.default_rng(3)
+    a, b = rng.standard_normal((384, 3072)).astype(np.float32), rng.standard_normal((3072, 768)).astype(np.float32)
+    ta, tb, mine = ctx.move_tensor(a), ctx.move_tensor(b), ctx.empty_tensor([384, 768])
+    H.matmul(ctx, ta, tb).dispose()
+    assert ctx.last_plan()["split"] > 1 and ctx.last_plan()["tile"] == "64x64"
+    ctx.sync()
+    capi.call("wdh_trim", 0)
+    ctx.set_option("memory_limit_mib", 1)
+    try:
+        mine.dispose()  # (the one block the pool has: the result takes it, and no other fits)
+        y = H.matmul(ctx, ta, tb, epilogue="relu")
+        assert ctx.last_plan()["tile"] == "32x32" and capi.last_error() == ""
+    finally:
+        ctx.set_option("memory_limit_mib", 0)
+    assert within(y.get_data(), a, b, np.zeros(768))
 
 
 # chunk counts below, at and above the eight requested at a time; planes whose quads are whole and ragged; groups

@@ -560,6 +560,7 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
       // (the chunks' sums need a workspace, which this kernel does without: it serves when there is none left)
       const int rc = launch_gemm_a_kc(useB_kc, p, batch, vec);
       if (rc != WDH_ENOMEM) return rc;
+      wdh::clear_error();  // (nothing failed for the caller)
     }
     const long long blocks32 = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch;
     if (useB_kc || (long long)(k - 1) * p.sB0 * 4 < 0x7fffffffLL) {
