@@ -160,7 +160,8 @@ int wdh_set_option(const char *name, int value);
                                    * batched product (tile and split are the product's) */
 #define WDH_FORM_CONV3X3_WINOGRAD4 10 /* ... as F(4x4, 3x3)                              */
 #define WDH_FORM_CONV_DEPTHWISE 11 /* one input channel per group: no product, a pass over memory
-                                   * (tile_m and tile_n are a thread's rows and columns)   */
+                                   * (tile_m and tile_n are a thread's rows and columns,
+                                   * whole_tiles the threads with work)         */
 int wdh_last_plan(int *tile_m, int *tile_n, int64_t *whole_tiles,
                   int64_t *split_tiles, int *split, int *form);
 

@@ -9,39 +9,47 @@ from webdnn_amd import hostops as H
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # n, c, multiplier, h, w, kernel, pads, strides, dilations
-    (2, 16, 1, 9, 9, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1]),        # rows of 9: ragged column tiles
-    (1, 3, 1, 1, 1, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1]),         # a single cell, every other tap in the padding
-    (3, 5, 1, 7, 7, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1]),         # planes packed into wavefronts
-    (16, 64, 1, 36, 40, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1]),     # whole 16-byte tiles
-    (8, 320, 1, 32, 48, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1]),     # four rows a thread
-    (8, 320, 1, 66, 95, (3, 3), [1, 1, 1, 1], [2, 2], [1, 1]),     # two rows a thread, stride 2, odd rows
-    (2, 8, 1, 11, 14, (3, 3), [0, 1, 1, 0], [2, 2], [1, 1]),       # unequal pads
-    (2, 8, 1, 12, 13, (3, 3), [3, 1, 2, 3], [1, 1], [1, 1]),       # whole rows in the padding
-    (2, 6, 1, 15, 18, (5, 5), [2, 2, 2, 2], [1, 1], [1, 1]),
-    (4, 160, 1, 48, 50, (5, 5), [2, 2, 2, 2], [1, 1], [1, 1]),     # four rows a thread, 5x5
-    (2, 6, 1, 15, 18, (5, 5), [2, 2, 2, 2], [2, 2], [1, 1]),
-    (4, 330, 1, 48, 49, (5, 5), [2, 2, 2, 2], [2, 2], [1, 1]),
-    (2, 4, 3, 10, 11, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1]),       # three output channels per input channel
-    (2, 3, 16, 14, 9, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1]),       # as many as this form takes
-    (2, 4, 1, 10, 11, (3, 3), [2, 2, 2, 2], [1, 1], [2, 2]),       # dilation: the general kernel
-    (2, 4, 2, 10, 11, (7, 2), [3, 0, 3, 1], [2, 3], [1, 1]),
+    # n, c, multiplier, h, w, kernel, pads, strides, dilations, rows x columns of a thread
+    (2, 16, 1, 9, 9, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1], "1x4"),        # rows of 9: ragged column tiles
+    (1, 3, 1, 1, 1, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1], "1x4"),         # a single cell, every other tap in the padding
+    (3, 5, 1, 7, 7, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1], "1x4"),         # planes packed into wavefronts
+    (16, 64, 1, 36, 40, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1], "1x4"),     # whole 16-byte tiles
+    (8, 320, 1, 32, 48, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1], "1x4"),     # the last size before four rows a thread
+    (8, 352, 1, 32, 48, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1], "4x4"),
+    (8, 360, 1, 33, 46, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1], "4x4"),     # three of the last four rows and two of four columns empty
+    (8, 320, 1, 66, 95, (3, 3), [1, 1, 1, 1], [2, 2], [1, 1], "2x4"),     # stride 2, odd rows
+    (2, 8, 1, 11, 14, (3, 3), [0, 1, 1, 0], [2, 2], [1, 1], "1x4"),       # unequal pads
+    (2, 8, 1, 12, 13, (3, 3), [3, 1, 2, 3], [1, 1], [1, 1], "1x4"),       # whole rows in the padding
+    (2, 6, 1, 15, 18, (5, 5), [2, 2, 2, 2], [1, 1], [1, 1], "1x4"),
+    (4, 160, 1, 48, 50, (5, 5), [2, 2, 2, 2], [1, 1], [1, 1], "1x4"),
+    (4, 424, 1, 48, 50, (5, 5), [2, 2, 2, 2], [1, 1], [1, 1], "4x4"),     # four rows a thread, 5x5
+    (4, 424, 1, 46, 49, (5, 5), [2, 2, 2, 2], [1, 1], [1, 1], "4x4"),     # two of the last four rows and three of four columns empty
+    (2, 6, 1, 15, 18, (5, 5), [2, 2, 2, 2], [2, 2], [1, 1], "1x4"),
+    (4, 330, 1, 48, 49, (5, 5), [2, 2, 2, 2], [2, 2], [1, 1], "1x4"),
+    (8, 392, 1, 48, 49, (5, 5), [2, 2, 2, 2], [2, 2], [1, 1], "2x4"),     # two rows a thread
+    (8, 392, 1, 46, 49, (5, 5), [2, 2, 2, 2], [2, 2], [1, 1], "2x4"),     # and one of the last two empty
+    (2, 4, 3, 10, 11, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1], "1x4"),       # three output channels per input channel
+    (2, 3, 16, 14, 9, (3, 3), [1, 1, 1, 1], [1, 1], [1, 1], "1x4"),       # as many as this form takes
+    (2, 4, 1, 10, 11, (3, 3), [2, 2, 2, 2], [1, 1], [2, 2], "1x1"),       # dilation: the general kernel
+    (2, 4, 2, 10, 11, (7, 2), [3, 0, 3, 1], [2, 3], [1, 1], "1x1"),
 ]
 
 
 @pytest.mark.parametrize("case", CASES)
 def test_depthwise_conv(ctx, case):
-    n, c, mult, h, w, (kh, kw), pads, strides, dil = case
+    n, c, mult, h, w, (kh, kw), pads, strides, dil, tile = case
     rng = np.random.default_rng(1000 * c + 10 * h + w)
     X = rng.standard_normal((n, c, h, w)).astype(np.float32)
     W = rng.standard_normal((c * mult, 1, kh, kw)).astype(np.float32)
     B = rng.standard_normal(c * mult).astype(np.float32)
     tx, tw, tb = ctx.move_tensor(X), ctx.move_tensor(W), ctx.move_tensor(B)
     got = H.conv(ctx, tx, tw, tb, dil, c, None, pads, strides).get_data()
-    assert ctx.last_plan()["form"] == "conv, depthwise"
     want = ref.conv(X, W, B, dil, c, None, pads, strides)
     # a chain of kh*kw fp32 products and the bias: each of at most 2^-24 of the sum of magnitudes so far
     bound = (kh * kw + 2) * 2.0 ** -24 * ref.conv(np.abs(X), np.abs(W), np.abs(B), dil, c, None, pads, strides)
+    plan, (rows, cols) = ctx.last_plan(), map(int, tile.split("x"))
+    assert plan["form"] == "conv, depthwise" and plan["tile"] == tile, plan
+    assert plan["whole_tiles"] == n * c * mult * -(-want.shape[2] // rows) * -(-want.shape[3] // cols)
     assert got.shape == want.shape
     assert np.all(np.abs(got.astype(np.float64) - want) <= bound)
     R = rng.standard_normal(want.shape).astype(np.float32)

@@ -51,11 +51,13 @@ bool conv_patch_applies(int c, int cout, int kh, int kw, int sh, int sw, int dh,
 int conv_patch_launch(const float *X, const float *W, const float *Bias, const float *R, float *Y, int n,
                       int h, int w, int oh, int ow, int pt, int pl, int relu);
 
-// Depthwise convolutions (depthwise.hip): whether a geometry qualifies, and the launch.
+// Depthwise convolutions (depthwise.hip): whether a geometry qualifies, and the launch, which says how many rows and
+// columns a thread has and how many threads have work.
+struct DepthwisePlan { int rows, cols; long long threads; };
 bool depthwise_applies(int n, int cout, int c_in_g, int cout_g, int group, int oh, int ow);
 int depthwise_launch(const float *X, const float *W, const float *Bias, const float *R, float *Y, int n, int c, int h,
                      int w, int cout, int kh, int kw, int pt, int pl, int sh, int sw, int dh, int dw, int oh, int ow,
-                     int relu);
+                     int relu, DepthwisePlan &plan);
 
 // The transforms of the minimal-filtering forms of a 3x3 stride-1 conv (winograd.hip), r = 2 for F(2x2, 3x3)
 // (16 positions) or 4 for F(4x4, 3x3) (36 positions): filters -> U [positions][cout][c], input ->

@@ -172,7 +172,7 @@ bool depthwise_applies(int n, int cout, int c_in_g, int cout_g, int group, int o
 
 int depthwise_launch(const float *X, const float *W, const float *Bias, const float *R, float *Y, int n, int c, int h,
                      int w, int cout, int kh, int kw, int pt, int pl, int sh, int sw, int dh, int dw, int oh, int ow,
-                     int relu) {
+                     int relu, DepthwisePlan &plan) {
   DwParams p = {};
   p.X = X; p.W = W; p.Bias = Bias; p.R = R; p.Y = Y;
   p.h = h; p.w = w; p.oh = oh; p.ow = ow; p.cout = cout; p.mult = cout / c;
@@ -190,6 +190,7 @@ int depthwise_launch(const float *X, const float *W, const float *Bias, const fl
   const bool tile = kh == kw && sh == sw && dh == 1 && dw == 1 && pl == (kw - 1) / 2 && (kh == 3 || kh == 5) && sh <= 2;
   if (!tile) {
     tiled(1, 1);
+    plan = {1, 1, planes * p.tiles};
     hipLaunchKernelGGL(depthwise_any_kernel, dim3((p.total + 255u) / 256u), dim3(256), 0, wdh::stream(), p);
     WDH_LAUNCH_CHECK();
     return WDH_OK;
@@ -199,6 +200,7 @@ int depthwise_launch(const float *X, const float *W, const float *Bias, const fl
   const int rows = sh == 1 ? 4 : 2;
   const bool tall = planes * ((ow + 3) / 4) * ((oh + rows - 1) / rows) >= 4LL * 64 * 4 * compute_units();
   tiled(tall ? rows : 1, 4);
+  plan = {tall ? rows : 1, 4, planes * p.tiles};
   if (kh == 3 && sh == 1) tall ? start<3, 1, 4>(p) : start<3, 1, 1>(p);
   else if (kh == 3) tall ? start<3, 2, 2>(p) : start<3, 2, 1>(p);
   else if (sh == 1) tall ? start<5, 1, 4>(p) : start<5, 1, 1>(p);

@@ -832,9 +832,11 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
 
   if (g_descriptors && g_forced_tile < 0 && g_forced_split < 0 &&
       wdh::depthwise_applies(n, cout, c_in_g, cout_g, group, oh, ow)) {
-    g_last_plan = {1, 4, 1, WDH_FORM_CONV_DEPTHWISE, (long long)n * cout * oh * ow, 0};
-    return wdh::depthwise_launch(p.B, p.A, p.C, p.R, p.Y, n, c, h, w, cout, kh, kw, pt, pl, sh, sw, dh, dw, oh, ow,
-                                 epilogue == WDH_EPI_RELU);
+    wdh::DepthwisePlan plan = {};
+    const int rc = wdh::depthwise_launch(p.B, p.A, p.C, p.R, p.Y, n, c, h, w, cout, kh, kw, pt, pl, sh, sw, dh, dw, oh, ow,
+                                         epilogue == WDH_EPI_RELU, plan);
+    g_last_plan = {plan.rows, plan.cols, 1, WDH_FORM_CONV_DEPTHWISE, plan.threads, 0};
+    return rc;
   }
   if (g_stem && g_descriptors && wdh::conv_patch_applies(c, cout, kh, kw, sh, sw, dh, dw, group, h, w, pt, pl, oh, ow)) {
     const long long tiles = (long long)n * ((oh + 7) / 8) * ((ow + 15) / 16);
