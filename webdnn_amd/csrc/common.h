@@ -51,10 +51,12 @@ bool conv_patch_applies(int c, int cout, int kh, int kw, int sh, int sw, int dh,
 int conv_patch_launch(const float *X, const float *W, const float *Bias, const float *R, float *Y, int n,
                       int h, int w, int oh, int ow, int pt, int pl, int relu);
 
-// Depthwise convolutions (depthwise.hip): whether a geometry qualifies, and the launch, which says how many rows and
-// columns a thread has and how many threads have work.
+// Depthwise convolutions (depthwise.hip): whether a geometry is possible, whether it is the faster form, and the launch,
+// which says how many rows and columns a thread has and how many threads have work.
 struct DepthwisePlan { int rows, cols; long long threads; };
-bool depthwise_applies(int n, int cout, int c_in_g, int cout_g, int group, int oh, int ow);
+bool depthwise_fits(int n, int cout, int c_in_g, int cout_g, int group, int oh, int ow);
+bool depthwise_applies(int n, int cout, int c_in_g, int cout_g, int group, int kh, int kw, int pl, int sh, int sw, int dh,
+                       int dw, int oh, int ow);
 int depthwise_launch(const float *X, const float *W, const float *Bias, const float *R, float *Y, int n, int c, int h,
                      int w, int cout, int kh, int kw, int pt, int pl, int sh, int sw, int dh, int dw, int oh, int ow,
                      int relu, DepthwisePlan &plan);

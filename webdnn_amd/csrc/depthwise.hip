@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256) void depthwise_tile_kernel(DwParams p) {
   }
 }
 
-// Any other kernel size, stride, padding or dilation: a thread per output, taps from the vector L1.
+// Any other kernel size, stride, padding or dilation, and small launches: a thread per output, taps from the vector L1.
 __global__ __launch_bounds__(256) void depthwise_any_kernel(DwParams p) {
   const unsigned id = blockIdx.x * 256u + threadIdx.x;
   if (id >= p.total) return;
@@ -162,12 +162,61 @@ void start(const DwParams &p) {
 
 namespace wdh {
 
-bool depthwise_applies(int n, int cout, int c_in_g, int cout_g, int group, int oh, int ow) {
-  // The thread numbering is 32-bit.  Many output channels per input channel are a product again: 64 channels
-  // @56x56, batch 8, take 11.0 / 13.6 / 23.8 / 42.4 us here with 2 / 4 / 8 / 16 outputs each and 85 / 86 / 88 / 93
-  // as 64-row tiles, which cost the same up to 64 outputs; past 16 the two meet.
-  return c_in_g == 1 && cout_g <= 16 && (long long)n * cout * oh * ow <= 0x7fffffffLL - 256 &&
-         (long long)n * group < 0x7fffffffLL;
+// The geometries depthwise_tile_kernel is built for.
+static bool tile_geometry(int kh, int kw, int pl, int sh, int sw, int dh, int dw) {
+  return kh == kw && sh == sw && dh == 1 && dw == 1 && pl == (kw - 1) / 2 && (kh == 3 || kh == 5) && sh <= 2;
+}
+// Rows whose last tile is ragged take both paths of the tile kernel, load by load.  Up to 512 outputs a CU that
+// latency is all of the time, and a thread per output is done sooner (us, tile against cell kernel, 7x7 planes): 3x3
+// 4.7 / 3.9, stride 2 5.6 / 4.0, 5x5 6.7 / 5.3, stride 2 8.2 / 5.4; from twice as many outputs on the tiles are ahead.
+static bool tile_suits(long long outputs, int ow) { return ow % 4 == 0 || outputs > 512LL * compute_units(); }
+// Several rows per thread read the shared input rows once; below four threads per lane of the chip it pays more to
+// have every SIMD busy (us, one row a thread against several): 3x3 32 @112x112 batch 4 / 8 / 16 / 32 6.9 / 11.8 / 20.0 /
+// 36.5 against 7.6 / 10.6 / 14.3 / 26.4, 5x5 16.2 / 26.2 / 46.6 / 85.6 against 11.8 / 17.4 / 29.8 / 55.2; 3x3 stride 2
+// gains or loses 5 %; 3x3 512 @14x14, where every fourth row of the tiles is empty, batch 64 25.2 against 34.8.
+static bool several_rows(long long planes, int sh, int oh, int ow) {
+  const int rows = sh == 1 ? 4 : 2;
+  return planes * ((ow + 3) / 4) * ((oh + rows - 1) / rows) >= 4LL * 64 * 4 * compute_units();
+}
+
+bool depthwise_fits(int n, int cout, int c_in_g, int cout_g, int group, int oh, int ow) {
+  // (the thread numbering is 32-bit)
+  return c_in_g == 1 && cout_g <= 16 && (long long)n * cout * oh * ow <= 0x7fffffffLL - 256 && (long long)n * group < 0x7fffffffLL;
+}
+
+// Whether the pass over memory beats the gathered matrix tiles, by an estimate of both (us), fitted to a sweep of 6900
+// geometries: 1x1 to 31x31 taps, planes of 1 to 112x112, 1 to 1024 channels of 1 to 16 outputs, batch 1 to 64.  Both
+// sides measured there, it takes the pass where that is 4 to 7 % slower in 18 of them, and leaves 246 to the tiles that
+// the pass would do in 0.7 to 0.96 of the time (two in 0.54), sixteen outputs a channel or planes of a few cells mostly.
+bool depthwise_applies(int n, int cout, int c_in_g, int cout_g, int group, int kh, int kw, int pl, int sh, int sw, int dh,
+                       int dw, int oh, int ow) {
+  if (!depthwise_fits(n, cout, c_in_g, cout_g, group, oh, ow)) return false;
+  const double chip = compute_units() / 256.0, taps = (double)kh * kw;
+  const double planes = (double)n * group, outputs = (double)n * cout * oh * ow;
+  auto larger = [](double a, double b) { return a > b ? a : b; };
+  // The tiles compute 64 rows for a group's one to sixteen, whatever their number, and cut long sums along the taps.
+  const double tiles = (double)group * (double)(((long long)n * oh * ow + 63) / 64) / 256.0 / chip;
+  const double matrix_us = 4.0 + larger(1.0 + (taps < 41.0 ? 0.12 * taps : 5.0), tiles * (0.7 + 0.022 * taps + (taps > 31.0 && taps < 64.0 ? 0.35 : 0.0)));
+  // Here a tap costs every output: 3x3 dilated, 64 channels @56x56, batch 8, of 2 / 4 / 8 / 16 outputs each 26 / 45 / 81 /
+  // 143 us against 85 / 87 / 87 / 91 as tiles.
+  if (tile_geometry(kh, kw, pl, sh, sw, dh, dw) && tile_suits((long long)n * cout * oh * ow, ow)) {
+    // [5x5][stride 2][ragged rows] ([several rows a thread]): the least time, and 10^6 outputs per us
+    static const double least[2][2][2] = {{{3.9, 4.7}, {3.8, 5.6}}, {{5.3, 6.7}, {5.1, 8.2}}};
+    static const double rate[2][2][2][2] = {{{{0.5, 0.5}, {0.5, 0.5}}, {{0.35, 0.35}, {0.15, 0.17}}},
+                                            {{{0.18, 0.4}, {0.15, 0.4}}, {{0.16, 0.17}, {0.08, 0.115}}}};
+    const int i = kh == 5, j = sh == 2, r = ow % 4 != 0;
+    return larger(least[i][j][r], 2.3 + outputs / (rate[i][j][r][several_rows((long long)n * cout, sh, oh, ow)] * 1e6 * chip)) < matrix_us;
+  }
+  // The cell kernel: a thread's taps are one chain (a 28x28 kernel over a 28x28 plane 185 us against 30), and
+  // neighbouring threads that read different planes fetch a line each.
+  const int plane = oh * ow < 16 ? oh * ow : 16;
+  if (plane < 4)
+    return 2.3 + 0.16 * taps + planes * taps / ((taps > 9.0 ? 0.17e6 : 1e6) * chip) +
+           outputs * taps / ((taps > 25.0 ? 0.4e6 : 1.2e6) * chip) < matrix_us;
+  const double tap_rate = plane < 9 ? (taps > 100.0 ? 0.6e6 : 1.2e6)
+                          : ow >= 32 || oh * ow % 16 == 0 ? (taps > 25.0 ? 2.3e6 : 1.8e6)
+                          : ow >= 16 ? 1.8e6 : taps > 81.0 ? 1.05e6 : 1.25e6;
+  return 2.3 + larger((plane < 9 ? 0.13 : taps > 49.0 ? 0.098 : 0.11) * taps, outputs / chip * larger(taps / tap_rate, 1.0 / (taps > 1.0 ? 0.2e6 : 0.3e6))) < matrix_us;
 }
 
 int depthwise_launch(const float *X, const float *W, const float *Bias, const float *R, float *Y, int n, int c, int h,
@@ -187,18 +236,15 @@ int depthwise_launch(const float *X, const float *W, const float *Bias, const fl
     p.fd_tiles = make_fastdiv(p.tiles);
     p.total = (unsigned)(planes * p.tiles);
   };
-  const bool tile = kh == kw && sh == sw && dh == 1 && dw == 1 && pl == (kw - 1) / 2 && (kh == 3 || kh == 5) && sh <= 2;
-  if (!tile) {
+  if (!tile_geometry(kh, kw, pl, sh, sw, dh, dw) || !tile_suits(planes * oh * ow, ow)) {
     tiled(1, 1);
     plan = {1, 1, planes * p.tiles};
     hipLaunchKernelGGL(depthwise_any_kernel, dim3((p.total + 255u) / 256u), dim3(256), 0, wdh::stream(), p);
     WDH_LAUNCH_CHECK();
     return WDH_OK;
   }
-  // Several rows per thread read the shared input rows once; below four threads per lane of the chip
-  // it pays more to have every SIMD busy.
   const int rows = sh == 1 ? 4 : 2;
-  const bool tall = planes * ((ow + 3) / 4) * ((oh + rows - 1) / rows) >= 4LL * 64 * 4 * compute_units();
+  const bool tall = several_rows(planes, sh, oh, ow);
   tiled(tall ? rows : 1, 4);
   plan = {tall ? rows : 1, 4, planes * p.tiles};
   if (kh == 3 && sh == 1) tall ? start<3, 1, 4>(p) : start<3, 1, 1>(p);

@@ -830,14 +830,16 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   p.cv.fd_ohw = make_fastdiv((long long)oh * ow);
   p.cv.fd_plane = make_fastdiv((long long)h * w);
 
-  if (g_descriptors && g_forced_tile < 0 && g_forced_split < 0 &&
-      wdh::depthwise_applies(n, cout, c_in_g, cout_g, group, oh, ow)) {
+  const bool may_depthwise = g_descriptors && g_forced_tile < 0 && g_forced_split < 0;
+  auto depthwise = [&]() {
     wdh::DepthwisePlan plan = {};
     const int rc = wdh::depthwise_launch(p.B, p.A, p.C, p.R, p.Y, n, c, h, w, cout, kh, kw, pt, pl, sh, sw, dh, dw, oh, ow,
                                          epilogue == WDH_EPI_RELU, plan);
     g_last_plan = {plan.rows, plan.cols, 1, WDH_FORM_CONV_DEPTHWISE, plan.threads, 0};
     return rc;
-  }
+  };
+  if (may_depthwise && wdh::depthwise_applies(n, cout, c_in_g, cout_g, group, kh, kw, pl, sh, sw, dh, dw, oh, ow))
+    return depthwise();
   if (g_stem && g_descriptors && wdh::conv_patch_applies(c, cout, kh, kw, sh, sw, dh, dw, group, h, w, pt, pl, oh, ow)) {
     const long long tiles = (long long)n * ((oh + 7) / 8) * ((ow + 15) / 16);
     g_last_plan = {64, 128, 1, WDH_FORM_CONV_STEM, tiles, 0};
@@ -994,7 +996,8 @@ direct_forms:
   auto it = g_ktabs.find(key);
   if (it == g_ktabs.end()) {
     if (wdh::capturing()) {
-      // building the table takes a synchronous copy
+      // building the table takes a synchronous copy; the depthwise form needs none
+      if (may_depthwise && wdh::depthwise_fits(n, cout, c_in_g, cout_g, group, oh, ow)) return depthwise();
       wdh::poison_capture();
       return fail(WDH_ESTATE, "wdh_conv2d: first use of this geometry; run it once before capturing a graph");
     }
