@@ -21,6 +21,21 @@ def test_few_rows(ctx, m, n, k):
     assert got.shape == want.shape and (np.abs(got - want) <= bound).all()
 
 
+# K long enough for the loop with four steps in flight, with nothing, less than a wavefront and more of it left over;
+# by itself (n from about 4096 on) and shared by the wavefronts of a workgroup
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+@pytest.mark.parametrize("n,k", [(4099, 1024), (4096, 1028), (4097, 2052), (4096, 2040), (8192, 1000), (1000, 4096), (11, 4100), (1000, 8188), (10, 12292), (4096, 4097)])
+def test_few_rows_of_a_long_k(ctx, m, n, k):
+    rng = np.random.default_rng(m * 100003 + n * 101 + k)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
+    got = H.gemm(ctx, ctx.move_tensor(a), ctx.move_tensor(b), None, 1.0, 1.0, 0, 1).get_data()
+    plan = ctx.last_plan()
+    assert plan["tile"] == "%dx2" % m and plan["split"] == (1 if n >= 4096 else 4), plan
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    bound = (k + 4) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64.T))
+    assert (np.abs(got - a64 @ b64.T) <= bound).all()
+
+
 def test_few_rows_agree_with_the_other_form_and_keep_inf_and_nan(ctx):
     rng = np.random.default_rng(5)
     a, b = rng.standard_normal((3, 700)).astype(np.float32), rng.standard_normal((37, 700)).astype(np.float32)
