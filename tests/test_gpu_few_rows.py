@@ -2,6 +2,7 @@
 import numpy as np
 import pytest
 
+from webdnn_amd import capi
 from webdnn_amd import hostops as H
 
 pytestmark = pytest.mark.gpu
@@ -34,6 +35,22 @@ def test_few_rows_of_a_long_k(ctx, m, n, k):
     a64, b64 = a.astype(np.float64), b.astype(np.float64)
     bound = (k + 4) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64.T))
     assert (np.abs(got - a64 @ b64.T) <= bound).all()
+
+
+# more rows than one and a short K: where the matrix cores' form was measured faster it serves
+@pytest.mark.parametrize("batch,m,n,k,few", [(1, 1, 3000, 128, True), (1, 4, 3000, 128, False), (1, 3, 3000, 384, False), (1, 4, 910, 256, True),
+                                            (1, 4, 911, 256, False), (1, 4, 1000, 257, True), (1, 2, 16384, 191, False), (1, 2, 16384, 192, True), (1, 4, 8192, 512, True),
+                                            (1, 4, 8192, 508, False), (1, 4, 8192, 449, False), (1, 4, 8192, 451, True), (4, 4, 577, 192, False), (32, 3, 200, 255, False), (32, 4, 577, 320, True),
+                                            (300, 4, 64, 192, False), (300, 2, 64, 128, False), (300, 2, 200, 128, True), (300, 4, 16, 128, True), (256, 4, 16, 128, False), (4096, 1, 2, 128, True)])
+def test_which_form_few_rows_take(ctx, batch, m, n, k, few):
+    rng = np.random.default_rng(batch + n + k)
+    a, b = rng.standard_normal((batch, m, k), dtype=np.float32), rng.standard_normal((batch, n, k), dtype=np.float32)
+    ta, tb, y = ctx.move_tensor(a), ctx.move_tensor(b), ctx.empty_tensor([batch, m, n])
+    capi.call("wdh_gemm", ta.handle, tb.handle, 0, y.handle, batch, m, n, k, m * k, k, 1, n * k, 1, k, 0, 0, 1.0, 1.0, 0, 0)
+    assert (ctx.last_plan()["tile"] == "%dx2" % m) == few, ctx.last_plan()
+    a64, b64 = a.astype(np.float64), b.astype(np.float64).transpose(0, 2, 1)
+    bound = (k + 4) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64))
+    assert (np.abs(y.get_data() - a64 @ b64) <= bound).all()
 
 
 def test_few_rows_agree_with_the_other_form_and_keep_inf_and_nan(ctx):

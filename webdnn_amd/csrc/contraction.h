@@ -1764,6 +1764,8 @@ extern bool g_static_scratch;  // set for the duration of a wdh_gemm_static call
 struct LastPlan { int bm, bn, split, form; long long full, tail; };
 extern LastPlan g_last_plan;
 constexpr int GEMM_ROWS_MAX = 4;  // rows gemm_rows_kernel keeps sums for
+long long gemm_rows_waves(int n, int batch);
+bool gemm_rows_share_k(long long waves);
 int launch_gemm_rows(const Params &p, int batch, bool vec);
 extern int g_stream_spin;
 extern unsigned *g_stream_error_dev;

@@ -310,13 +310,28 @@ static bool wavesplit_suits(int batch, int m, int n, int k) {
 }
 
 // Whether a product (both operands k-contiguous) is one for gemm_rows_kernel: so few rows that reading the weight
-// is all there is to it.  At four rows it takes 16.4 us where gemm_wavesplit_kernel
-// takes 29.7 (n = k = 4096), 6.0 against 20.1 (n 1000), 47 against 61 (n = k = 8192) and 3.1 against 3.7 (n = k = 256);
-// each row costs registers and a load of its own, so more of them belong to the matrix cores.  A group's products
-// (wdh_linear_group) have weights that are not k-contiguous, or leave in one launch.
-static bool gemm_rows_suits(int m, int n, int k) {
-  return g_wavesplit && g_forced_tile < 0 && g_forced_split < 0 && m <= GEMM_ROWS_MAX && k >= 128 && n >= 2 &&
-         !g_group.collecting;
+// is all there is to it.  At four rows it takes 13.6 us where gemm_wavesplit_kernel takes 24.0 (n = k = 4096),
+// 6.0 against 20.0 (n 1000), 22.9 against 29.3 (n 8192, k 4096) and 3.2 against 3.7 (n = k = 256); each row costs
+// registers and a load of its own, so more of them belong to the matrix cores.  With one row it is ahead from k = 128 on.
+// With more and a short K it is not: a weight's row no longer fills the loads, and every row adds a tree over the
+// lanes.  The lines are those of a sweep of n 2 to 30000, k 128 to 12289 and batches of 2 to 4000 (us, this kernel
+// against the other at two, three and four rows): where the wavefronts share K and there are many columns n 3000, k 128
+// 3.8 / 4.5 / 5.3 against 3.0, k 384 3.7 / 4.7 / 5.5 against 4.7; not shared, n 16384 k 128 4.9 / 5.8 / 6.8 against
+// 4.5, k 256 5.3 / 6.0 / 7.1 against 5.7, k 384 6.6 / 7.1 / 8.0 against 7.5; in batches, which leave the other kernel
+// ragged blocks, 300 of n 200, k 192 12.3 / 16.0 / 20.3 against 22.3, and 1024 of n 2, k 256 4.2 / 4.7 / 5.1 against 21.
+// Rows that are not 16-byte aligned slow the other kernel more than this one (n 1000, k 257 3.2 / 3.3 / 3.5 against 4.5).
+// Of 4400 products 6 are slower than without this kernel, by 4 to 6 %.
+// A group's products (wdh_linear_group) have weights that are not k-contiguous, or leave in one launch.
+static bool gemm_rows_suits(int batch, int m, int n, int k, bool vec) {
+  if (!g_wavesplit || g_forced_tile >= 0 || g_forced_split >= 0 || m > GEMM_ROWS_MAX || k < 128 || n < 2 || g_group.collecting)
+    return false;
+  if (m == 1) return true;
+  // (a batch of a few columns each leaves the other kernel a block per entry that is mostly padding)
+  if (n <= 16 && batch > wdh::compute_units()) return true;
+  const long long waves = gemm_rows_waves(n, batch);
+  if (gemm_rows_share_k(waves)) return (!vec || k >= 48 * m) && (vec ? 36 : 24) * m * waves <= (long long)k * k;
+  static const int least[4][3] = {{192, 320, 512}, {257, 320, 450}, {192, 256, 384}, {128, 192, 320}};  // [.][rows - 2]
+  return k >= least[batch == 1 ? (vec ? 0 : 1) : (vec && n % 32 == 0) || waves < 32LL * wdh::compute_units() ? 2 : 3][m - 2];
 }
 
 // Of the products gemm_wavesplit_kernel could take, those that the ordinary tiles, cut along K, do faster: a block of
@@ -552,7 +567,7 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
     set_wide(p, false);
   }
   // A few rows against a transposed weight: a pass over the weight (gemm_rows.hip)
-  if (useA_kc && useB_kc && gemm_rows_suits(m, n, k)) return launch_gemm_rows(p, batch, vec);
+  if (useA_kc && useB_kc && gemm_rows_suits(batch, m, n, k, vec)) return launch_gemm_rows(p, batch, vec);
   // Few result tiles and a K worth cutting: one launch with K cut across the wavefronts of a
   // workgroup (gemm_wavesplit_kernel) instead of chunks in a workspace and a reduce pass
   if (useA_kc && p.fast && wavesplit_suits(batch, m, n, k)) {

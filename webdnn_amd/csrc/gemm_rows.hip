@@ -121,10 +121,14 @@ void start(const Params &p, int batch, bool vec, bool share) {
 }  // namespace
 
 namespace wdhc {
+long long gemm_rows_waves(int n, int batch) { return ((long long)n + ROWS_COLS - 1) / ROWS_COLS * batch; }
+// Fewer than eight wavefronts a CU leave too few loads in flight: the four of a workgroup then share K.
+bool gemm_rows_share_k(long long waves) { return waves < 8LL * wdh::compute_units(); }
+
 // A and B k-contiguous, 1 <= m <= GEMM_ROWS_MAX; vec: bases and strides keep 16-byte alignment.
 int launch_gemm_rows(const Params &p, int batch, bool vec) {
-  const long long waves = ((long long)p.n + ROWS_COLS - 1) / ROWS_COLS * batch;
-  const bool share = waves < 8LL * wdh::compute_units();
+  const long long waves = gemm_rows_waves(p.n, batch);
+  const bool share = gemm_rows_share_k(waves);
   switch (p.m) {
     case 1: start<1>(p, batch, vec, share); break;
     case 2: start<2>(p, batch, vec, share); break;
