@@ -29,6 +29,19 @@ def test_long_k_with_residual(ctx, m, n, k):
     assert within(got, a, b, bias.astype(np.float64))
 
 
+# which form serves on either side of each line, B n-contiguous and k-contiguous
+@pytest.mark.parametrize("m,n,k,plain,transposed", [(384, 768, 3072, True, True), (500, 1024, 2048, False, True), (500, 1024, 2000, False, False),
+                                                   (500, 1024, 2560, True, True), (800, 640, 3072, False, True), (530, 1024, 1280, False, True),
+                                                   (530, 1024, 1536, True, True), (700, 1024, 1000, False, False), (1000, 1024, 768, False, True),
+                                                   (1000, 1024, 1280, True, True), (384, 768, 2303, True, True), (256, 1024, 4096, False, False)])
+def test_which_form_long_products_take(ctx, m, n, k, plain, transposed):
+    a, b = ctx.empty_tensor([m, k]), ctx.empty_tensor([n, k])
+    H.gemm(ctx, a, b.alias([k, n])).dispose()
+    assert (ctx.last_plan()["tile"] == "64x64") == plain, ctx.last_plan()
+    H.gemm(ctx, a, b, trans_b=1).dispose()
+    assert (ctx.last_plan()["tile"] == "64x64") == transposed, ctx.last_plan()
+
+
 def test_no_room_for_the_chunk_sums(ctx):
     """Without memory for the workspace of cut tiles the product runs in one launch, and no error stays behind."""
     rng = np.random.default_rng(3)

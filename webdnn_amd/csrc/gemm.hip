@@ -336,13 +336,26 @@ static bool gemm_rows_suits(int batch, int m, int n, int k, bool vec) {
 
 // Of the products gemm_wavesplit_kernel could take, those that the ordinary tiles, cut along K, do faster: a block of
 // 32x32 results is one workgroup's whole K, so with a few more blocks than CUs some CUs work twice as long, and once the
-// launch is bound by its products that shows.  Both sides (us; B n-contiguous, B k-contiguous): 384x768x3072 38.0 / 48.6
-// against 28.1 / 28.4 as tiles, 500x1024x4096 49.5 / 65.4 against 45.2 / 45.0, 700x512x2048 27.0 / 34.3 against 26.1 /
-// 25.7, 1000x1024x1024 30.3 / 37.0 against 30.2 / 29.8; below the line 500x1024x1024 16.2 / 20.3 against 21.6 / 21.7,
-// and with fewer blocks than CUs 850x256x2048 17.8 / 20.1 against 19.4 / 20.0.
-static bool tiles_beat_wavesplit(int batch, int m, int n, int k) {
+// launch is bound by its products that shows.  The lines are those of a sweep of 868 products (257 to 1024 columns, 250 to
+// 1000 rows, k 512 to 4096; us, that kernel against tiles):
+//   B n-contiguous: 384x768x3072 36.1 / 28.1, 350x768x2560 29.2 / 25.6; 500x1024x2048 (two blocks a CU, no CU idle) 25.7 /
+//   28.5, x2560 31.6 / 31.6; beyond two blocks a CU 530x1024x1280 23.6 / 24.1, x1536 27.5 / 25.7, 700x1024x1024 25.4 /
+//   24.5, x1000 21.6 / 24.0, 1000x1024x1280 33.2 / 31.9; 800x640x3072 37.2 / 39.9: cut in two, more tiles than half the
+//   CUs no longer fit side by side.
+//   B k-contiguous: its rows of 4 KB steps meet in the same memory channels, and unaligned ones are read in single
+//   floats, by that kernel's loads more than by the tiles': 500x1024x1536 25.8 / 25.0, 1000x1024x1024 34.4 / 28.2,
+//   700x1024x1023 45.2 / 38.8; other rows 480x1024x2000 26.6 / 28.8, 700x1024x1000 22.3 / 24.5, 1000x1024x768 27.2 / 24.8.
+// With no more blocks than CUs there is nothing to gain (850x256x2048 17.8 / 19.4).
+static bool tiles_beat_wavesplit(int batch, int m, int n, int k, bool b_kc, bool vec) {
   const long long blocks32 = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch, cus = wdh::compute_units();
-  return blocks32 > cus && blocks32 * k >= 2560 * cus;
+  const long long tiles64 = (long long)((m + 63) / 64) * ((n + 63) / 64) * batch;
+  if (blocks32 <= cus || blocks32 * k < 2560 * cus) return false;
+  if (b_kc && (!vec || k % 1024 == 0)) return true;
+  if (blocks32 <= 2 * cus)
+    return b_kc ? k >= 2560 || blocks32 * 5 <= 8 * cus
+                : tiles64 * 2 <= cus && (k >= 2560 || (!vec && blocks32 * 5 <= 8 * cus));
+  if (b_kc) return k >= 1024 || blocks32 > 3 * cus;
+  return k >= (blocks32 * 2 <= 5 * cus ? 1536 : 1200);
 }
 
 extern "C" int wdh_set_option(const char *name, int value) {
@@ -571,7 +584,7 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
   // Few result tiles and a K worth cutting: one launch with K cut across the wavefronts of a
   // workgroup (gemm_wavesplit_kernel) instead of chunks in a workspace and a reduce pass
   if (useA_kc && p.fast && wavesplit_suits(batch, m, n, k)) {
-    if (!g_group.collecting && !g_static_scratch && tiles_beat_wavesplit(batch, m, n, k)) {
+    if (!g_group.collecting && !g_static_scratch && tiles_beat_wavesplit(batch, m, n, k, useB_kc, vec)) {
       // (the chunks' sums need a workspace, which this kernel does without: it serves when there is none left)
       const int rc = launch_gemm_a_kc(useB_kc, p, batch, vec);
       if (rc != WDH_ENOMEM) return rc;
