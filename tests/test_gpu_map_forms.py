@@ -4,13 +4,14 @@ import pytest
 
 from oracle import ref
 from util import ulp_diff
+from webdnn_amd import capi
 from webdnn_amd import hostops as H
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("shape,axis", [((3, 31, 5), 1), ((2, 32, 7), 1), ((2, 500, 17), 1), ((1, 33, 16), 1), ((40, 129, 500), 1),
-                                        ((300, 63, 255), 1), ((4, 5, 70000), 1), ((1, 71, 66000), 1)])
+                                        ((300, 63, 255), 1), ((7, 1, 11), 1), ((3, 7, 300), 1), ((3, 8, 300), 1), ((3, 9, 300), 1), ((4, 5, 70000), 1), ((1, 71, 66000), 1)])
 def test_mean_over_an_inner_axis(ctx, shape, axis):
     x = np.random.default_rng(sum(shape)).standard_normal(shape).astype(np.float32)
     got = H.reduce_mean(ctx, ctx.move_tensor(x), [axis], 0).get_data()
@@ -57,3 +58,15 @@ def test_row_means(ctx, rows, length):
     want = x.astype(np.float64).mean(1)
     slack = length * 2.0 ** -52 * np.abs(x.astype(np.float64)).mean(1)
     assert (np.abs(got - want) <= 2.0 ** -24 * np.abs(want) * 1.0001 + slack).all()
+
+
+# one pass of a mean over several axes: rows of any length, as few and as many pieces a lane as each form requests ahead
+@pytest.mark.parametrize("rows,length", [(4100, 3), (4100, 16), (4100, 18), (4100, 33), (4100, 60), (4100, 64), (10240, 255), (10239, 255), (5, 2), (5, 63),
+                                         (5, 65), (5, 129), (5, 257), (9, 513), (9, 512), (9, 1028)])
+def test_row_sums_with_another_divisor(ctx, rows, length):
+    x = np.random.default_rng(rows + length).standard_normal((rows, length)).astype(np.float32)
+    tx, y = ctx.move_tensor(x), ctx.empty_tensor([rows])
+    capi.call("wdh_reduce_axis", tx.handle, y.handle, rows, length, 1, 7 * length)
+    want = x.astype(np.float64).sum(1) / (7 * length)
+    slack = 2.0 ** -52 * np.abs(x.astype(np.float64)).sum(1) / 7
+    assert (np.abs(y.get_data() - want) <= 2.0 ** -24 * np.abs(want) * 1.0001 + slack).all()

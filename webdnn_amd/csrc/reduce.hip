@@ -335,10 +335,10 @@ __global__ __launch_bounds__(64 * SMALL_ROW_WAVES) void mean_rows_small(
 // lanes for the many short rows of a last-axis mean, so that a wavefront's loads cover four rows and the tree has
 // four steps instead of six.  Rows of 192, 95 760 of them (73.5 MB, 6.3 TB/s): 26 us with a
 // wavefront a row and 4-byte loads before, 11.7 now.
-template <int LANES, bool VEC>
+template <int LANES, bool VEC, int AHEAD>
 __global__ __launch_bounds__(64 * WAVES_PER_BLOCK) void sum_rows_lanes(
     const float *__restrict__ X, float *__restrict__ Y, long long outer, int len, double divisor) {
-  constexpr int PER_BLOCK = 64 * WAVES_PER_BLOCK / LANES, AHEAD = VEC ? 4 : 8;
+  constexpr int PER_BLOCK = 64 * WAVES_PER_BLOCK / LANES;
   const int lane = threadIdx.x % LANES;
   const long long row = (long long)blockIdx.x * PER_BLOCK + threadIdx.x / LANES;
   const bool live = row < outer;
@@ -376,16 +376,23 @@ __global__ __launch_bounds__(64 * WAVES_PER_BLOCK) void sum_rows_lanes(
 // elements j, j + PARTS, ..., and their sums are added in that order.  PARTS = 1 adds in index order.
 // The four of an element-wise chain over [8, 192, 95, 126] (two maps to per-row sums, a map to 193 536 columns and
 // those to 1536 results): 31.6 us on average before; 13.8 now with one thread a result, 7.8 with four, 4.7 with sixteen.
-template <int PARTS>
+// Sums of fewer than eight have nothing to request ahead, and the instructions around it show (12.4 M sums of two 35.5 us
+// with them, 34.1 without): AHEAD = 1.
+template <int PARTS, int AHEAD = 8>
 __global__ __launch_bounds__(256) void sum_axis_kernel(const float *__restrict__ X,
                                                        float *__restrict__ Y, long long outer,
                                                        int red, long long inner, double divisor) {
-  constexpr int COLS = 256 / PARTS, AHEAD = 8;
+  constexpr int COLS = 256 / PARTS;
   const int col = threadIdx.x % COLS, part = threadIdx.x / COLS;
   const long long idx = (long long)blockIdx.x * COLS + col;
   const bool live = idx < outer * inner;
+  if (PARTS == 1 && !live) return;  // (with several parts every thread meets at the barrier)
   double s = 0.0;
-  if (live) {
+  if (AHEAD == 1) {
+    const long long o = idx / inner, i = idx - o * inner;
+    const float *x = X + o * red * inner + i;
+    for (int r = 0; r < red; r++) s += (double)x[(long long)r * inner];
+  } else if (live) {
     const long long o = idx / inner, i = idx - o * inner;
     const float *x = X + o * red * inner + i;
     long long r = part;
@@ -414,7 +421,9 @@ __global__ __launch_bounds__(256) void sum_axis_kernel(const float *__restrict__
 void launch_sum_axis(const float *X, float *Y, long long outer, int red, long long inner, double divisor) {
   const long long results = outer * inner, fill = 256LL * wdh::compute_units();
   auto blocks = [&](int cols) { return dim3((unsigned)((results + cols - 1) / cols)); };
-  if (results >= fill || red < 32)
+  if (red < 8)
+    hipLaunchKernelGGL((sum_axis_kernel<1, 1>), blocks(256), dim3(256), 0, wdh::stream(), X, Y, outer, red, inner, divisor);
+  else if (results >= fill || red < 32)
     hipLaunchKernelGGL(sum_axis_kernel<1>, blocks(256), dim3(256), 0, wdh::stream(), X, Y, outer, red, inner, divisor);
   else if (results * 4 >= fill)
     hipLaunchKernelGGL(sum_axis_kernel<4>, blocks(64), dim3(256), 0, wdh::stream(), X, Y, outer, red, inner, divisor);
@@ -426,16 +435,30 @@ unsigned row_blocks(long long outer) {
   return (unsigned)((outer + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK);
 }
 
-// Sixteen lanes a row where a row fits in four 16-byte pieces a lane and there are enough rows for every CU.
-void launch_sum_rows(const float *X, float *Y, long long outer, int len, double divisor) {
-  const bool vec = len % 4 == 0 && ((uintptr_t)X & 15) == 0, part = len <= 256 && outer >= 16LL * wdh::compute_units();
-  const int per_block = part ? 4 * WAVES_PER_BLOCK : WAVES_PER_BLOCK;
-  const dim3 grid((unsigned)((outer + per_block - 1) / per_block)), block(64 * WAVES_PER_BLOCK);
+// Pieces requested ahead: as many as a lane has, since those beyond the row are added as zeros.
+template <int LANES, bool VEC>
+void start_sum_rows(const float *X, float *Y, long long outer, int len, double divisor) {
+  constexpr int PER_BLOCK = 64 * WAVES_PER_BLOCK / LANES;
+  const dim3 grid((unsigned)((outer + PER_BLOCK - 1) / PER_BLOCK)), block(64 * WAVES_PER_BLOCK);
+  const long long pieces = ((long long)(VEC ? len / 4 : len) + LANES - 1) / LANES;
   hipStream_t st = wdh::stream();
-  if (part && vec) hipLaunchKernelGGL((sum_rows_lanes<16, true>), grid, block, 0, st, X, Y, outer, len, divisor);
-  else if (part) hipLaunchKernelGGL((sum_rows_lanes<16, false>), grid, block, 0, st, X, Y, outer, len, divisor);
-  else if (vec) hipLaunchKernelGGL((sum_rows_lanes<64, true>), grid, block, 0, st, X, Y, outer, len, divisor);
-  else hipLaunchKernelGGL((sum_rows_lanes<64, false>), grid, block, 0, st, X, Y, outer, len, divisor);
+  if (pieces <= 1) hipLaunchKernelGGL((sum_rows_lanes<LANES, VEC, 1>), grid, block, 0, st, X, Y, outer, len, divisor);
+  else if (pieces <= 2) hipLaunchKernelGGL((sum_rows_lanes<LANES, VEC, 2>), grid, block, 0, st, X, Y, outer, len, divisor);
+  else if (VEC || pieces <= 4) hipLaunchKernelGGL((sum_rows_lanes<LANES, VEC, 4>), grid, block, 0, st, X, Y, outer, len, divisor);
+  else hipLaunchKernelGGL((sum_rows_lanes<LANES, VEC, 8>), grid, block, 0, st, X, Y, outer, len, divisor);
+}
+
+// Sixteen lanes a row where a row fits in four 16-byte pieces a lane and there are enough rows for every CU.  Rows that
+// are read in single floats have up to sixteen a lane then, two rounds of loads: from 128 on they need more rows for it
+// (us, 64 lanes a row against sixteen, rows of 255: 4096 of them 3.9 / 4.2, 6000 4.0 / 4.4, 8192 4.3 / 4.4, and from
+// 12000 on sixteen are ahead).
+void launch_sum_rows(const float *X, float *Y, long long outer, int len, double divisor) {
+  const bool vec = len % 4 == 0 && ((uintptr_t)X & 15) == 0;
+  const bool part = len <= 256 && outer >= (vec || len <= 128 ? 16LL : 40LL) * wdh::compute_units();
+  if (part && vec) start_sum_rows<16, true>(X, Y, outer, len, divisor);
+  else if (part) start_sum_rows<16, false>(X, Y, outer, len, divisor);
+  else if (vec) start_sum_rows<64, true>(X, Y, outer, len, divisor);
+  else start_sum_rows<64, false>(X, Y, outer, len, divisor);
 }
 
 int check_rows(const char *fn, long long outer, int len) {
