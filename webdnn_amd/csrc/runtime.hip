@@ -24,8 +24,9 @@ constexpr size_t kStagingBytes = 32u << 20;  // per pinned buffer, two of them
 // own, so that the host's copy of piece i+1 into pinned memory overlaps the DMA of piece i.
 constexpr size_t kUploadPiece = 4u << 20;
 constexpr int kUploadSlots = (int)(2 * kStagingBytes / kUploadPiece);
-constexpr size_t kReadPiece = 1u << 20;      // downloads: length of a piece, in the first staging buffer,
+constexpr size_t kReadPiece = 1u << 20;      // downloads: the least length of a piece, in the first staging buffer,
 constexpr size_t kReadAhead = 4;             // and pieces in flight
+constexpr size_t kReadPieceMax = kStagingBytes / kReadAhead;
 constexpr size_t kSmallGranule = 512;        // allocation rounding below 1 MiB
 constexpr size_t kLargeGranule = 1u << 20;   // and above
 
@@ -671,19 +672,23 @@ int wdh_read(wdh_buf h, size_t src_offset, void *dst, size_t bytes) {
   // Short pieces through the staging memory of the uploads, all free by now, kReadAhead of them in flight: a piece is
   // copied out of pinned memory while the next ones arrive, and a slot is asked for again only after that.
   // (12.6 MB, the results of an [8, 512, 768] block: the whole host-to-host pass 1476 -> 1296 us; one piece of up to
-  // 32 MB, as before, leaves the copy into cold user memory no transfer to overlap with.)
+  // 32 MB, as before, leaves the copy into cold user memory no transfer to overlap with.)  Beyond 64 pieces they grow:
+  // each costs a few microseconds of calls beside its copy (512 MB 19.3 ms in pieces of 32 MB, 20.5 in 512 of 1 MiB, 19.0 in
+  // 64 of 8 MiB; 128 MB 5.3, 5.0 and 4.9).
   if (!bytes) WDH_HIP_CHECK(hipStreamSynchronize(g.stream));
-  auto length = [&](size_t at) { return bytes - at < kReadPiece ? bytes - at : kReadPiece; };
-  auto read_slot = [](int slot) { return (char *)g.stage[0] + slot * kReadPiece; };
+  size_t piece = kReadPiece;
+  while (piece < kReadPieceMax && bytes / piece > 64) piece *= 2;
+  auto length = [&](size_t at) { return bytes - at < piece ? bytes - at : piece; };
+  auto read_slot = [&](int slot) { return (char *)g.stage[0] + slot * piece; };
   size_t issued = 0;
-  for (size_t copied = 0; copied < bytes; copied += kReadPiece) {
-    for (; issued < bytes && issued < copied + kReadAhead * kReadPiece; issued += kReadPiece) {
-      const int slot = (int)(issued / kReadPiece % kReadAhead);
+  for (size_t copied = 0; copied < bytes; copied += piece) {
+    for (; issued < bytes && issued < copied + kReadAhead * piece; issued += piece) {
+      const int slot = (int)(issued / piece % kReadAhead);
       WDH_HIP_CHECK(hipMemcpyAsync(read_slot(slot), src + src_offset + issued, length(issued), hipMemcpyDeviceToHost,
                                    g.stream));
       WDH_HIP_CHECK(hipEventRecord(g.up_done[slot], g.stream));
     }
-    const int slot = (int)(copied / kReadPiece % kReadAhead);
+    const int slot = (int)(copied / piece % kReadAhead);
     WDH_HIP_CHECK(hipEventSynchronize(g.up_done[slot]));
     memcpy(d + copied, read_slot(slot), length(copied));
   }
