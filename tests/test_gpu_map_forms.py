@@ -42,7 +42,9 @@ def test_sigmoid_over_the_whole_range(ctx):
     want = ref.unary("Sigmoid", x)
     assert np.isnan(got[np.isnan(x)]).all()
     # down to -12 the reference's cancelled sum is right to 2^-53 / sigmoid(-12), under 2^-35: only a value that lies
-    # that close to a rounding boundary may land one ulp away
+    # that close to a rounding boundary may land one ulp away from it, or from the value itself
+    true = 1.0 / (1.0 + np.exp(-x[x >= -12].astype(np.float64)))
+    assert ulp_diff(got[x >= -12], true.astype(np.float32)).max() <= 1
     near = x >= -12
     assert ulp_diff(got[near], want[near]).max() <= 1
     # below, both sides form tanh + 1, whose last place is 2^-53 (a double tanh is right to two of them)

@@ -325,13 +325,16 @@ __device__ __forceinline__ float relu_js(float v) {
   return v <= 0.0f ? 0.0f : v;
 }
 
-// (tanh(v/2) + 1) / 2 as the reference writes it.  Where the sum does not cancel, 1 / (1 + e^-v) is the same number
-// within a few double ulps and needs a quarter of the instructions (double tanh alone takes a wavefront longer than
-// its loads and stores); further out the written form's own rounding shows in fp32 and is kept
-// ([8, 192, 95, 126]: 94.9 -> 35.9 us).
+// (tanh(v/2) + 1) / 2 as the reference writes it, without tanh: with a = e^-|v| it is q = 1 / (1 + a), or a / (1 + a)
+// below zero, to a few double ulps, where the sum does not cancel.  Further down the sum's rounding shows in fp32: tanh
+// is 2q - 1 rounded to the places it has next to -1, so that adding and taking away the 1 gives the same multiple of
+// 2^-53.  Down to -12 that rounding is left out: a double tanh is right to two of those last places, so that the written
+// form is off by up to 2^-53 / sigmoid(v), under 2^-35 of the result, and an fp32 result can differ by one ulp where it
+// lies that close to a rounding boundary.  One exponential and one division whatever the value ([8, 192, 95, 126]: 94.9 us
+// as written; with tanh below -12 only 35.9, but 109 to 118 where such values are among them).
 __device__ __forceinline__ double sigmoid_d(double v) {
-  if (v >= -12.0 && v <= 40.0) return 1.0 / (1.0 + exp(-v));
-  return (tanh(v / 2.0) + 1.0) / 2.0;
+  const double a = exp(-fabs(v)), q = (v < 0.0 ? a : 1.0) / (1.0 + a);
+  return v < -12.0 ? ((2.0 * q - 1.0) + 1.0) / 2.0 : q;
 }
 
 template <int OP>
