@@ -52,6 +52,27 @@ __device__ __forceinline__ float apply_f(float l, float r) {
   return (float)pow((double)l, (double)r);
 }
 
+// Four at a time, powers with one branch for the four, or none where the caller has asked already (ASK): those of another
+// exponent than 2 then run side by side (1 M elements to the power of 3 12.2 us, 14.3 with a branch each and 11.9 with
+// none, when squares took pow too).
+__device__ __forceinline__ bool all_twos(f32x4 b) { return b.x == 2.0f && b.y == 2.0f && b.z == 2.0f && b.w == 2.0f; }
+template <int OP, bool ASK = true>
+__device__ __forceinline__ f32x4 apply_f4(f32x4 a, f32x4 b) {
+  f32x4 v;
+  if (OP == WDH_BIN_POW) {
+    if (ASK && all_twos(b)) return a * a;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const float y = (float)pow((double)a[e], (double)b[e]);
+      v[e] = b[e] == 2.0f ? a[e] * a[e] : y;
+    }
+    return v;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e++) v[e] = apply_f<OP>(a[e], b[e]);
+  return v;
+}
+
 template <int OP>
 __device__ __forceinline__ int apply_i(int l, int r) {
   double a = (double)l, b = (double)r;
@@ -76,12 +97,7 @@ __global__ __launch_bounds__(256) void binary_dense_f32(const float *__restrict_
   const f32x4 *R4 = reinterpret_cast<const f32x4 *>(R);
   f32x4 *Y4 = reinterpret_cast<f32x4 *>(Y);
   for (long long v = i; v < nvec; v += stride) {
-    f32x4 a = L4[v], b = R4[v], y;
-    y.x = apply_f<OP>(a.x, b.x);
-    y.y = apply_f<OP>(a.y, b.y);
-    y.z = apply_f<OP>(a.z, b.z);
-    y.w = apply_f<OP>(a.w, b.w);
-    Y4[v] = y;
+    Y4[v] = apply_f4<OP>(L4[v], R4[v]);
   }
   const long long tail = (nvec << 2) + i;
   if (i < (total & 3)) Y[tail] = apply_f<OP>(L[tail], R[tail]);
@@ -128,12 +144,7 @@ __global__ __launch_bounds__(256) void binary_plane(BinaryParams p, wdh::PlaneWa
     for (int k = 0; k < 4; k++) {
       if (ok[k]) {
         const unsigned x = q.x0 + k * q.dx, y = q.y0 + k * q.dy;
-        f32x4 v;
-        v.x = apply_f<OP>(a[k].x, b[k].x);
-        v.y = apply_f<OP>(a[k].y, b[k].y);
-        v.z = apply_f<OP>(a[k].z, b[k].z);
-        v.w = apply_f<OP>(a[k].w, b[k].w);
-        *reinterpret_cast<f32x4 *>((float *)Y + ((row0 + y) * inner + x) * 4) = v;
+        *reinterpret_cast<f32x4 *>((float *)Y + ((row0 + y) * inner + x) * 4) = apply_f4<OP>(a[k], b[k]);
       }
     }
   } else {
@@ -184,6 +195,7 @@ __global__ __launch_bounds__(256) void binary_flat(BinaryParams p, wdh::FlatWalk
   typedef typename std::conditional<UNIT == 4, f32x4, T>::type V;
   for (unsigned u0 = q.begin + threadIdx.x; u0 < q.end; u0 += 1024) {
     V a[4], b[4];
+    bool squares = OP == WDH_BIN_POW && UNIT == 4;  // ([100, 768] to powers of 3 by column: 31.7 us, 33.5 with a branch an item)
 #pragma unroll
     for (int k = 0; k < 4; k++) {
       const unsigned u = u0 + 256 * k;
@@ -196,29 +208,27 @@ __global__ __launch_bounds__(256) void binary_flat(BinaryParams p, wdh::FlatWalk
           else { const float s = *l; a[k] = f32x4{s, s, s, s}; }
           if (sr1) b[k] = *reinterpret_cast<const f32x4 *>(r);
           else { const float s = *r; b[k] = f32x4{s, s, s, s}; }
+          squares = squares && all_twos(b[k]);
         } else {
           a[k] = *l;
           b[k] = *r;
         }
       }
     }
+    auto store = [&](auto value) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const unsigned u = u0 + 256 * k;
-      if (u < q.end) {
-        if constexpr (UNIT == 4) {
-          f32x4 v;
-          v.x = apply_f<OP>(a[k].x, b[k].x);
-          v.y = apply_f<OP>(a[k].y, b[k].y);
-          v.z = apply_f<OP>(a[k].z, b[k].z);
-          v.w = apply_f<OP>(a[k].w, b[k].w);
-          *reinterpret_cast<f32x4 *>(Y + (long long)u * 4) = v;
-        } else if constexpr (__is_same(T, float)) {
-          Y[u] = apply_f<OP>(a[k], b[k]);
-        } else {
-          Y[u] = apply_i<OP>(a[k], b[k]);
-        }
+      for (int k = 0; k < 4; k++) {
+        const unsigned u = u0 + 256 * k;
+        if (u < q.end) *reinterpret_cast<V *>(Y + (long long)u * UNIT) = value(k);
       }
+    };
+    if constexpr (UNIT == 4) {
+      if (squares) store([&](int k) { return a[k] * a[k]; });
+      else store([&](int k) { return apply_f4<OP, false>(a[k], b[k]); });
+    } else if constexpr (__is_same(T, float)) {
+      store([&](int k) { return apply_f<OP>(a[k], b[k]); });
+    } else {
+      store([&](int k) { return apply_i<OP>(a[k], b[k]); });
     }
   }
 }
