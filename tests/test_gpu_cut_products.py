@@ -61,10 +61,12 @@ def test_no_room_for_the_chunk_sums(ctx):
     assert within(y.get_data(), a, b, np.zeros(768))
 
 
-# chunk counts below, at and above the eight requested at a time; planes whose quads are whole and ragged; groups
-@pytest.mark.parametrize("split", [2, 7, 8, 9, 17])
-@pytest.mark.parametrize("c,cout,h,w,group", [(320, 24, 8, 8, 1), (320, 70, 7, 7, 1), (640, 12, 6, 10, 2), (320, 5, 1, 3, 1)])
-def test_cut_conv_with_residual(ctx, split, c, cout, h, w, group):
+# chunk counts below, at and above the eight requested at a time and twice that, two slabs of 16 channels a chunk; planes
+# whose quads are whole and ragged; groups
+@pytest.mark.parametrize("split", [2, 7, 8, 9, 16, 17])
+@pytest.mark.parametrize("cout,h,w,group", [(24, 8, 8, 1), (70, 7, 7, 1), (12, 6, 10, 2), (5, 1, 3, 1)])
+def test_cut_conv_with_residual(ctx, split, cout, h, w, group):
+    c = 32 * split * group
     rng = np.random.default_rng(split * 1000 + c + h)
     x = rng.standard_normal((3, c, h, w)).astype(np.float32)
     wt, bias = rng.standard_normal((cout, c // group, 1, 1)).astype(np.float32), rng.standard_normal(cout).astype(np.float32)
@@ -73,8 +75,10 @@ def test_cut_conv_with_residual(ctx, split, c, cout, h, w, group):
     try:
         got = H.conv(ctx, ctx.move_tensor(x), ctx.move_tensor(wt), ctx.move_tensor(bias), None, group, None, [0] * 4, [1, 1],
                      epilogue="relu", residual=ctx.move_tensor(r)).get_data()
+        plan = ctx.last_plan()
     finally:
         ctx.set_option("split_k", -1)
+    assert plan["split"] == split and plan["split_tiles"] > 0, plan
     cg, og = c // group, cout // group
     for i in range(3):
         for g in range(group):
