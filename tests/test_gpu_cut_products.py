@@ -30,16 +30,38 @@ def test_long_k_with_residual(ctx, m, n, k):
 
 
 # which form serves on either side of each line, B n-contiguous and k-contiguous
-@pytest.mark.parametrize("m,n,k,plain,transposed", [(384, 768, 3072, True, True), (500, 1024, 2048, False, True), (500, 1024, 2000, False, False),
-                                                   (500, 1024, 2560, True, True), (800, 640, 3072, False, True), (530, 1024, 1280, False, True),
-                                                   (530, 1024, 1536, True, True), (700, 1024, 1000, False, False), (1000, 1024, 768, False, True),
-                                                   (1000, 1024, 1280, True, True), (384, 768, 2303, True, True), (256, 1024, 4096, False, False)])
+@pytest.mark.parametrize("m,n,k,plain,transposed", [(384, 768, 3072, True, True), (384, 768, 2816, True, True), (384, 768, 2815, True, True),
+                                                   (384, 768, 2812, False, True), (384, 1024, 2047, True, True), (384, 1024, 2000, False, False),
+                                                   (500, 1024, 2048, False, False), (500, 1024, 2560, False, True), (500, 1024, 4096, True, True),
+                                                   (500, 1024, 4092, False, True), (530, 1024, 2304, True, True), (530, 1024, 2300, False, True),
+                                                   (530, 1024, 2044, False, False), (700, 1024, 1023, False, True), (1000, 768, 3072, True, True),
+                                                   (1000, 768, 3068, False, True), (1000, 1024, 4096, False, True), (256, 1024, 4096, False, False)])
 def test_which_form_long_products_take(ctx, m, n, k, plain, transposed):
     a, b = ctx.empty_tensor([m, k]), ctx.empty_tensor([n, k])
     H.gemm(ctx, a, b.alias([k, n])).dispose()
     assert (ctx.last_plan()["tile"] == "64x64") == plain, ctx.last_plan()
     H.gemm(ctx, a, b, trans_b=1).dispose()
     assert (ctx.last_plan()["tile"] == "64x64") == transposed, ctx.last_plan()
+
+
+@pytest.mark.parametrize("m,n,k", [(384, 768, 3072), (530, 1024, 2304), (700, 1024, 4100)])
+@pytest.mark.parametrize("transposed", [0, 1])
+def test_cut_tiles_round_no_more_than_sixteen_chains(ctx, m, n, k, transposed):
+    """A result is the sum of sixteen chains of one rounding a product, as in the one-launch form that the tiles stand in for."""
+    rng = np.random.default_rng(m + k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    got = H.gemm(ctx, ctx.move_tensor(a), ctx.move_tensor(np.ascontiguousarray(b.T) if transposed else b), trans_b=transposed).get_data()
+    assert ctx.last_plan()["tile"] == "64x64" and ctx.last_plan()["split"] == 16, ctx.last_plan()
+    a64, b64 = a[:64].astype(np.float64), b[:, :128].astype(np.float64)
+    chunk = -(-(-(-k // 16)) // 16) * 16
+    want, chains = a64 @ b64, np.zeros((64, 128), np.float32)
+    for first in range(0, k, chunk):
+        acc = np.zeros((64, 128), np.float32)
+        for i in range(first, min(first + chunk, k)):
+            acc = (acc + np.outer(a64[:, i], b64[i])).astype(np.float32)
+        chains += acc
+    # the same roundings in another order: over 8192 results the two norms differ by a few per cent
+    assert np.linalg.norm(got[:64, :128] - want) <= 1.1 * np.linalg.norm(chains - want)
 
 
 def test_no_room_for_the_chunk_sums(ctx):

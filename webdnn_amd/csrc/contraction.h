@@ -1756,6 +1756,7 @@ const int kTileN[] = {128, 256, 128, 64, 64};
 
 // ---- state and planning shared by the translation units (defined in gemm.hip) -------------
 extern int g_forced_tile;    // >= 0: overrides the tile choice (tuning hook)
+extern int g_chunks_hint;    // >= 2: chunks that every tile of the next product is cut into, set likewise
 extern int g_tile_hint;      // >= 0: tile for the next Gemm / MatMul launch, set by a caller inside the library
 extern int g_forced_split;   // >= 1: overrides the split-K heuristic
 extern int g_last_form;

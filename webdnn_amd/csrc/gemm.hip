@@ -117,6 +117,7 @@ TileId pick_tile(int m, int n, int nz) {
 }
 int g_forced_tile = -1;   // >= 0: overrides pick_tile (tuning hook)
 int g_tile_hint = -1;     // >= 0: the caller inside the library knows the tile for its next product
+int g_chunks_hint = -1;   // >= 2: the caller inside the library knows how often its next product is to be cut
 int g_forced_split = -1;  // >= 1: overrides the split-K heuristic
 int g_descriptors = 1;    // 0: every operand is treated as if it spanned 2 GiB or more
 // what launch_planned decided for the most recent launch (wdh_last_plan)
@@ -183,9 +184,10 @@ WorkPlan plan_work(long long tiles, int k, int bm, int bn, bool gather, int kgra
     r.full = tiles - r.tail;
     return r;
   };
-  if (g_forced_split >= 1) {
-    // tuning / test hook: every tile is split this many ways
-    const int s = g_forced_split < slabs ? g_forced_split : (slabs > 0 ? slabs : 1);
+  if (g_forced_split >= 1 || g_chunks_hint > 1) {
+    // tuning / test hook, or a caller that asks for it: every tile is split this many ways
+    const int want = g_forced_split >= 1 ? g_forced_split : g_chunks_hint;
+    const int s = want < slabs ? want : (slabs > 0 ? slabs : 1);
     return s > 1 ? with_split(tiles, s) : w;
   }
   if (slabs * per16 < 8) return w;
@@ -336,26 +338,26 @@ static bool gemm_rows_suits(int batch, int m, int n, int k, bool vec) {
 
 // Of the products gemm_wavesplit_kernel could take, those that the ordinary tiles, cut along K, do faster: a block of
 // 32x32 results is one workgroup's whole K, so with a few more blocks than CUs some CUs work twice as long, and once the
-// launch is bound by its products that shows.  The lines are those of a sweep of 868 products (257 to 1024 columns, 250 to
-// 1000 rows, k 512 to 4096; us, that kernel against tiles):
-//   B n-contiguous: 384x768x3072 36.1 / 28.1, 350x768x2560 29.2 / 25.6; 500x1024x2048 (two blocks a CU, no CU idle) 25.7 /
-//   28.5, x2560 31.6 / 31.6; beyond two blocks a CU 530x1024x1280 23.6 / 24.1, x1536 27.5 / 25.7, 700x1024x1024 25.4 /
-//   24.5, x1000 21.6 / 24.0, 1000x1024x1280 33.2 / 31.9; 800x640x3072 37.2 / 39.9: cut in two, more tiles than half the
-//   CUs no longer fit side by side.
-//   B k-contiguous: its rows of 4 KB steps meet in the same memory channels, and unaligned ones are read in single
-//   floats, by that kernel's loads more than by the tiles': 500x1024x1536 25.8 / 25.0, 1000x1024x1024 34.4 / 28.2,
-//   700x1024x1023 45.2 / 38.8; other rows 480x1024x2000 26.6 / 28.8, 700x1024x1000 22.3 / 24.5, 1000x1024x768 27.2 / 24.8.
+// launch is bound by its products that shows.  The tiles are cut where that kernel's wavefronts cut K, so that a result is
+// the sum of as many chains of the same length (2-norm error against 64 bits, 384x768x3072 2.6e-7 both ways; in the 3 to
+// 10 chunks that launch_planned would take 3.2e-7, and 1000x1024x1280 3.7e-7 for 1.8e-7).
+// The lines are those of a sweep of 1100 products (257 to 1024 columns, 250 to 1000 rows, k 512 to 8192; us, that kernel
+// against tiles):
+//   B n-contiguous: 384x768x3072 37.7 / 31.6, x2560 31.0 / 30.3; 500x1024x3072 (two blocks a CU, no CU idle) 36.1 / 38.4,
+//   x4096 46.5 / 44.9; beyond two blocks a CU 530x1024x2560 42.8 / 39.2, x2048 34.5 / 35.1,
+//   1000x768x3072 61.8 / 53.0, 1000x1024x3072 67.9 / 71.6.
+//   B k-contiguous, whose rows that kernel reads in 64-byte pieces: 384x768x3072 46.7 / 32.0, 500x1024x2560 40.1 / 36.0,
+//   x2048 33.3 / 33.6, 384x1024x2000 26.2 / 30.5, 700x1024x1536 36.1 / 35.0, 1000x768x1536 36.9 / 37.6; rows that are not
+//   16-byte aligned cost it more (384x1024x2047 61.6 / 41.7, 700x1024x1023 44.9 / 38.6).
 // With no more blocks than CUs there is nothing to gain (850x256x2048 17.8 / 19.4).
 static bool tiles_beat_wavesplit(int batch, int m, int n, int k, bool b_kc, bool vec) {
   const long long blocks32 = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch, cus = wdh::compute_units();
-  const long long tiles64 = (long long)((m + 63) / 64) * ((n + 63) / 64) * batch;
   if (blocks32 <= cus || blocks32 * k < 2560 * cus) return false;
-  if (b_kc && (!vec || k % 1024 == 0)) return true;
-  if (blocks32 <= 2 * cus)
-    return b_kc ? k >= 2560 || blocks32 * 5 <= 8 * cus
-                : tiles64 * 2 <= cus && (k >= 2560 || (!vec && blocks32 * 5 <= 8 * cus));
-  if (b_kc) return k >= 1024 || blocks32 > 3 * cus;
-  return k >= (blocks32 * 2 <= 5 * cus ? 1536 : 1200);
+  const double per_cu = (double)blocks32 / (double)cus;
+  const bool few = per_cu <= 1.6, over = per_cu > 2.0;
+  if (b_kc) return !vec || k >= 2560 || (k >= 2048 && (few || over));
+  return k >= (few ? 2816 : !over ? 4096 : per_cu <= 2.6 ? 2304 : per_cu <= 3.3 ? 3072 : 6000) ||
+         (!vec && (few || (over && per_cu <= 2.6)) && k >= 2000);
 }
 
 extern "C" int wdh_set_option(const char *name, int value) {
@@ -586,7 +588,9 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
   if (useA_kc && p.fast && wavesplit_suits(batch, m, n, k)) {
     if (!g_group.collecting && !g_static_scratch && tiles_beat_wavesplit(batch, m, n, k, useB_kc, vec)) {
       // (the chunks' sums need a workspace, which this kernel does without: it serves when there is none left)
+      g_chunks_hint = WS_WAVES;
       const int rc = launch_gemm_a_kc(useB_kc, p, batch, vec);
+      g_chunks_hint = -1;
       if (rc != WDH_ENOMEM) return rc;
       wdh::clear_error();  // (nothing failed for the caller)
     }
