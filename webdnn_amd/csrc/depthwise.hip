@@ -138,16 +138,20 @@ __global__ __launch_bounds__(256) void depthwise_any_kernel(DwParams p) {
   const int in_plane = img * (p.cout / p.mult) + (p.mult == 1 ? oc : fdiv(oc, p.fd_mult));
   const float *x = p.X + (long long)in_plane * p.h * p.w;
   const float *w = p.W + (long long)oc * p.kh * p.kw;
+  // (a sum a row of the kernel, since rounding errors grow with the length of a chain: 31x31, 128 channels @28x28, 2-norm
+  // error against 64 bits 1.3e-7, 4.15e-7 as one chain and 4.08e-7 as matrix tiles cut in two along the taps)
   float acc = 0.0f;
   for (int ky = 0; ky < p.kh; ky++) {
     const int iy = oy * p.sh - p.pt + ky * p.dh;
     const bool row_in = (unsigned)iy < (unsigned)p.h;
+    float row = 0.0f;
     for (int kx = 0; kx < p.kw; kx++) {
       const int ix = ox * p.sw - p.pl + kx * p.dw;
       const bool in = row_in && (unsigned)ix < (unsigned)p.w;
       const float t = x[in ? (long long)iy * p.w + ix : 0];
-      acc = __builtin_fmaf(in ? t : 0.0f, w[ky * p.kw + kx], acc);
+      row = __builtin_fmaf(in ? t : 0.0f, w[ky * p.kw + kx], row);
     }
+    acc += row;
   }
   const long long off = (long long)plane * p.oh * p.ow + cell;
   p.Y[off] = finish(p, acc, p.Bias ? p.Bias[oc] : 0.0f, p.R ? p.R + off : nullptr);
