@@ -96,7 +96,8 @@ int wdh_device_info(char *name, int name_cap, int *compute_units,
  *   "memory_limit_mib"  0 (default) = no limit, or the most device memory, in MiB, that the buffer pool
  *                       asks the driver for: an allocation beyond it first gives cached blocks back, then
  *                       fails with WDH_ENOMEM.  Workspaces are subject to it: a conv that cannot get
- *                       the tensors of its minimal-filtering form takes a direct form instead.
+ *                       the tensors of its minimal-filtering form takes a direct form instead, a long
+ *                       product without room for its chunk sums runs in one launch.
  *   "conv_stem"         1 (default) = a 7x7, stride-2, undilated convolution from 3 to 64
  *                       channels (the stem of an image network) runs in a kernel that keeps
  *                       all weights and a tile's input patch in LDS; 0 = it gathers taps
@@ -144,6 +145,8 @@ int wdh_set_option(const char *name, int value);
  * and of tiles cut along K, chunks per cut tile (1 = none), and which form of the
  * kernel ran: WDH_FORM_* below.  A launch scheduled as a stream of K slabs ("stream_k")
  * reports split = 0, all its tiles as whole_tiles and its workgroup count as split_tiles.
+ * A Gemm of a few rows reports a wavefront's rows and columns as its tile, and as split how
+ * many wavefronts share K.
  * Any pointer may be NULL. */
 #define WDH_FORM_GEMM_KC 0        /* B k-contiguous (transB)                    */
 #define WDH_FORM_GEMM_MC 1        /* B n-contiguous                             */
