@@ -1,0 +1,160 @@
+"""Products on the bf16 matrix cores (operands split into three bfloat16 parts) against sums in 64 bits and against the fp32
+instruction."""
+import numpy as np
+import pytest
+
+from webdnn_amd import hostops as H
+
+pytestmark = pytest.mark.gpu
+
+TILES = {3: "128x128", 4: "64x128", 5: "128x64", 6: "64x64", 7: "256x128"}
+
+
+@pytest.fixture
+def split(ctx):
+    yield lambda value: ctx.set_option("split_products", value)
+    for name, value in (("split_products", 1), ("split_k", -1), ("conv3x3_winograd", 1), ("conv1x1_stride2_in_place", 1)):
+        ctx.set_option(name, value)
+
+
+def product(ctx, a, b, transposed, bias=None, r=None, epilogue=None):
+    tb = ctx.move_tensor(np.ascontiguousarray(b.T) if transposed else b)
+    if r is not None:
+        return H.matmul(ctx, ctx.move_tensor(a), tb, ctx.move_tensor(bias), ctx.move_tensor(r), epilogue).get_data()
+    return H.gemm(ctx, ctx.move_tensor(a), tb, None if bias is None else ctx.move_tensor(bias), trans_b=int(transposed), epilogue=epilogue).get_data()
+
+
+def within(got, want, magnitudes, k):
+    """A chain of at most k roundings of half an ulp of the sum of magnitudes, and a few more for the two sums and the epilogue."""
+    return (np.abs(got - want) <= (k + 8) * 2.0 ** -24 * magnitudes + 1e-37).all()
+
+
+# one slab, a ragged last one, two to five slabs (the loop's prologue and tail), edges of every tile in both directions
+@pytest.mark.parametrize("mode", sorted(TILES))
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("m,n,k", [(64, 64, 16), (1, 4, 20), (65, 132, 32), (128, 128, 48), (129, 68, 64), (257, 260, 76), (256, 256, 80), (63, 516, 644)])
+def test_tiles_and_edges(ctx, split, mode, transposed, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    bias, r = rng.standard_normal(n).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    split(mode)
+    ctx.set_option("gemm_wavesplit", 0)  # (and one row goes to the kernel of few rows otherwise)
+    try:
+        got = product(ctx, a, b, transposed, bias, None if transposed else r, "relu")
+    finally:
+        ctx.set_option("gemm_wavesplit", 1)
+    assert ctx.last_plan()["tile"] == TILES[mode], ctx.last_plan()
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    extra = bias + (0.0 if transposed else r)
+    assert within(got, np.maximum(a @ b + extra, 0), np.abs(a) @ np.abs(b) + np.abs(extra), k)
+
+
+@pytest.mark.parametrize("mode", sorted(TILES))
+@pytest.mark.parametrize("chunks", [2, 5, 16])
+def test_cut_along_k(ctx, split, mode, chunks):
+    rng = np.random.default_rng(chunks)
+    a, b = rng.standard_normal((150, 1044)).astype(np.float32), rng.standard_normal((1044, 200)).astype(np.float32)
+    split(mode)
+    ctx.set_option("split_k", chunks)
+    got = product(ctx, a, b, False)
+    assert ctx.last_plan()["tile"] == TILES[mode] and ctx.last_plan()["split"] > 1, ctx.last_plan()
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    assert within(got, a @ b, np.abs(a) @ np.abs(b), 1044)
+
+
+@pytest.mark.parametrize("k", [64, 512, 2048])
+@pytest.mark.parametrize("positive", [False, True])
+def test_errors_are_no_larger_than_the_fp32_instructions(ctx, split, k, positive):
+    """2-norms against 64 bits over 512 x 512 results, uncut; and no drift to one side, which would add up over layers."""
+    rng = np.random.default_rng(k)
+    a, b = rng.standard_normal((512, k)).astype(np.float32), (rng.standard_normal((k, 512)) * 0.03).astype(np.float32)
+    if positive:
+        a, b = np.abs(a), np.abs(b)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    err, drift = {}, 0.0
+    ctx.set_option("gemm_wavesplit", 0)
+    try:
+        for mode in (0, 6):
+            split(mode)
+            ctx.set_option("split_k", 1)
+            got = product(ctx, a, b, True)
+            err[mode] = np.linalg.norm(got - want) / np.linalg.norm(want)
+            drift = float(np.sum((got - want) * np.sign(want)) / np.sum(np.abs(want)))
+    finally:
+        ctx.set_option("gemm_wavesplit", 1)
+    assert err[6] <= err[0], err
+    assert abs(drift) <= 2.0 ** -26, drift
+
+
+@pytest.mark.parametrize("mode", [3, 6])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_values_the_split_cannot_hold(ctx, split, mode, transposed):
+    """Inf and NaN, the largest floats, sums that overflow, subnormals: as with the fp32 instruction."""
+    rng = np.random.default_rng(11)
+    a, b = rng.standard_normal((200, 100)).astype(np.float32), rng.standard_normal((100, 260)).astype(np.float32)
+    a[3, 7], a[70, 99], a[130, 0] = np.inf, np.nan, -np.inf
+    b[50, 5], b[99, 250] = np.inf, -np.inf
+    a[5, :], b[:, 9] = 0, 0
+    a[5, 2], b[2, 9] = np.finfo(np.float32).max, 1.0
+    a[199, :], a[199, :2] = 0, 3e38  # (two products: the order of a longer sum would decide where it overflows)
+    a[64, :] *= np.float32(1e-38)
+    a[65, :] *= np.float32(1e-42)
+    a[66, :] *= np.float32(1e-25)
+    out = {}
+    ctx.set_option("gemm_wavesplit", 0)
+    try:
+        for value in (0, mode):
+            split(value)
+            out[value] = product(ctx, a, b, transposed)
+    finally:
+        ctx.set_option("gemm_wavesplit", 1)
+    assert ctx.last_plan()["tile"] == TILES[mode]
+    want, got = out[0], out[mode]
+    assert (np.isnan(want) == np.isnan(got)).all()
+    assert (np.isposinf(want) == np.isposinf(got)).all() and (np.isneginf(want) == np.isneginf(got)).all()
+    finite = np.isfinite(want)
+    with np.errstate(all="ignore"):
+        magnitudes = np.nan_to_num(np.abs(a.astype(np.float64)), posinf=0) @ np.nan_to_num(np.abs(b.astype(np.float64)), posinf=0)
+    assert (np.abs(got.astype(np.float64) - want)[finite] <= (108 * 2.0 ** -23 * magnitudes + 2e-45 * 100)[finite]).all()
+
+
+CONVS = [
+    # n, cin, h, w, cout, kernel, stride, pad, dilation, group
+    (3, 32, 8, 10, 70, 1, 1, 0, 1, 1),       # in place, pairs of pixels
+    (2, 36, 7, 7, 64, 1, 1, 0, 1, 1),        # odd planes: a pixel at a time
+    (5, 128, 9, 11, 130, 1, 2, 0, 1, 1),
+    (2, 96, 13, 8, 40, 1, 3, 0, 1, 2),       # groups, a stride of 3
+    (2, 64, 12, 12, 64, 1, 2, 0, 1, 1),      # even rows, stride 2
+    (2, 16, 9, 14, 64, 3, 1, 1, 1, 1),
+    (3, 64, 15, 11, 130, 3, 2, 1, 1, 1),
+    (2, 24, 17, 19, 40, 5, 2, 2, 1, 2),      # 25 taps, ragged K, groups
+    (2, 16, 20, 21, 24, 7, 1, 3, 1, 1),      # 49 taps
+    (2, 20, 16, 16, 66, 3, 1, 2, 2, 1),      # dilated
+]
+
+
+@pytest.mark.parametrize("mode", [3, 4, 5, 6])
+@pytest.mark.parametrize("shape", CONVS)
+def test_convs(ctx, split, mode, shape):
+    n, cin, h, w, cout, kernel, stride, pad, dil, group = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal((n, cin, h, w)).astype(np.float32)
+    wt, bias = rng.standard_normal((cout, cin // group, kernel, kernel)).astype(np.float32), rng.standard_normal(cout).astype(np.float32)
+    ctx.set_option("conv3x3_winograd", 0)
+    out = {}
+    for value in (0, mode):
+        split(value)
+        y = H.conv(ctx, ctx.move_tensor(x), ctx.move_tensor(wt), ctx.move_tensor(bias), [dil, dil], group, None, [pad] * 4, [stride, stride],
+                   epilogue="relu")
+        out[value], plan = y.get_data(), ctx.last_plan()
+    assert plan["tile"] == TILES[mode], plan
+    y = H.conv(ctx, ctx.move_tensor(np.abs(x)), ctx.move_tensor(np.abs(wt)), ctx.move_tensor(np.abs(bias)), [dil, dil], group, None, [pad] * 4,
+               [stride, stride])
+    k = cin // group * kernel * kernel
+    assert (np.abs(out[0].astype(np.float64) - out[mode]) <= 2 * (k + 8) * 2.0 ** -24 * y.get_data()).all()
+    x[0, 1, h // 2, w // 2], x[n - 1, 0, 0, 0] = np.inf, np.nan   # what a padded tap must not touch stays clean
+    for value in (0, mode):
+        split(value)
+        out[value] = H.conv(ctx, ctx.move_tensor(x), ctx.move_tensor(wt), ctx.move_tensor(bias), [dil, dil], group, None, [pad] * 4,
+                            [stride, stride]).get_data()
+    assert (np.isnan(out[0]) == np.isnan(out[mode])).all() and (np.isinf(out[0]) == np.isinf(out[mode])).all()

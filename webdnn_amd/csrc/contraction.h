@@ -126,7 +126,9 @@ constexpr int MC_PAD = 8;    // MC tile row stride = extent + 8 (floats)
 // even number of pixels: two neighbouring output pixels are elements 0 and 2 of four consecutive
 // input floats, so a thread's four pixels arrive as two 16-byte pieces (each with its own offset:
 // the two pairs may lie in different rows) of which every other element is kept.
-enum BMode { B_KC = 0, B_MC = 1, B_IM2COL32 = 2, B_IM2COL64 = 3, B_IM2COL_BIG = 4, B_PIXELS = 5, B_PIXELS_S2 = 8 };
+enum BMode { B_KC = 0, B_MC = 1, B_IM2COL32 = 2, B_IM2COL64 = 3, B_IM2COL_BIG = 4, B_PIXELS = 5, B_PIXELS_S2 = 8,
+             // split_product.h only: any 1x1 unpadded conv, each pixel with an offset of its own
+             B_PIXELS_ANY = 9 };
 
 struct ConvGeom {
   int c_in_g;        // input channels per group
@@ -1790,11 +1792,12 @@ int stream_width(long long tiles, int slabs, int kgran, const WorkPlan &w, int t
 // max_wgs_per_cu: how many workgroups of this kernel a CU holds (its launch bounds).
 // (max_wgs_per_cu = 0: this kernel has no stream form.)
 template <int BM, int BN, typename Start>
-int launch_planned(Params &p, int nz, bool conv, int kgran, int max_wgs_per_cu, Start start) {
+int launch_planned(Params &p, int nz, bool conv, int kgran, int max_wgs_per_cu, Start start,
+                   const WorkPlan *plan = nullptr) {
   p.tiles_m = (p.m + BM - 1) / BM;
   p.tiles_n = (p.n + BN - 1) / BN;
   const long long tiles = (long long)p.tiles_m * p.tiles_n * nz;
-  const WorkPlan w = plan_work(tiles, p.k, BM, BN, conv, kgran);
+  const WorkPlan w = plan ? *plan : plan_work(tiles, p.k, BM, BN, conv, kgran);
   p.nz = nz;
   p.fd_tiles_per_z = make_fastdiv((long long)p.tiles_m * p.tiles_n);
   p.fd_group = make_fastdiv((long long)TILE_GROUP * p.tiles_n);
@@ -1942,5 +1945,14 @@ int launch_gemm_a_mc(bool b_kc, Params &p, int nz, bool vec);     // contraction
 int launch_conv_gather(int mode, Params &p, int nz, bool vec);    // contraction_conv_gather.hip
 int launch_conv_pixels(Params &p, int nz, bool vec, bool stride2);  // contraction_conv_pixels.hip
 int launch_conv3x3(int tile, Params &p, int nz, int vecw);        // contraction_conv3x3.hip
+// The same products on the bf16 matrix cores (split_product.h); A k-contiguous, descriptors, 16-byte pieces, k % 4 == 0.
+enum SplitTile { S128x128 = 0, S64x128 = 1, S128x64 = 2, S64x64 = 3, S256x128 = 4 };
+struct SplitPlan {
+  int tile;       // SplitTile, or -1: not a product for them
+  WorkPlan work;
+  double us;      // estimate
+};
+int launch_split_gemm(bool b_kc, const SplitPlan &s, Params &p, int nz);    // split_gemm.hip
+int launch_split_conv(int mode, const SplitPlan &s, Params &p, int nz);     // split_conv.hip
 
 }  // namespace wdhc

@@ -116,6 +116,7 @@ TileId pick_tile(int m, int n, int nz) {
   return tiles128 >= 2LL * wdh::compute_units() && filled >= 0.8 ? T128x128 : T64x64;
 }
 int g_forced_tile = -1;   // >= 0: overrides pick_tile (tuning hook)
+bool g_fp32_hint = false;  // the caller inside the library wants the fp32 instruction for its next product
 int g_tile_hint = -1;     // >= 0: the caller inside the library knows the tile for its next product
 int g_chunks_hint = -1;   // >= 2: the caller inside the library knows how often its next product is to be cut
 int g_forced_split = -1;  // >= 1: overrides the split-K heuristic
@@ -139,6 +140,7 @@ int g_stem = 1;           // 0: the 7x7 stride-2 stem conv gathers its taps like
 int g_pixels_s2 = 1;      // 0: 1x1 convs with a column stride of 2 gather their taps like any other geometry
 int g_winograd4_channels = 0;  // when not 0: "conv3x3_winograd" 1 takes F(4x4, 3x3) from this many input and output channels on
 int g_winograd = 1;       // 3x3 stride-1 convs by minimal filtering: 0 never, 1 = F(2x2, 3x3) where it wins, 2 / 3 = F(2x2, 3x3) / F(4x4, 3x3) wherever legal
+int g_split = 1;          // products on the bf16 matrix cores (split_product.h): 0 never, 1 where they are faster, 2 wherever legal, 3 + t: that with tile t
 int g_wide_stores = 1;    // 0: whole tiles store one element per lane and instruction
 int g_stream = 1;         // launches scheduled as streams of K slabs: 0 never, 1 where the plan below gains, 2 wherever legal
 int g_stream_wgs = 4;     // workgroups per CU of a stream launch (at most what the kernel's resources allow)
@@ -360,6 +362,119 @@ static bool tiles_beat_wavesplit(int batch, int m, int n, int k, bool b_kc, bool
          (!vec && (few || (over && per_cu <= 2.6)) && k >= 2000);
 }
 
+// How a product on the bf16 matrix cores is laid out: the tile and the cut along K with the least estimated time.
+// The model (us): a CU works through its workgroups' slabs of 16 k at `slab` each, a workgroup alone on a CU at `solo`;
+// `fixed` is a launch with one empty workgroup a CU (prologue, epilogue); a cut adds the pass over the partial sums, which
+// are written and read once.  Fitted to 21 products of 33x4096x4096 to 4096x4096x4096 on every tile in 1 to 12 cuts and to
+// 40 convs (the form it picks takes at most 11 % longer than the best one).
+enum SplitSource { SPLIT_GEMM, SPLIT_PIXELS, SPLIT_TAPS };  // where B comes from: a matrix, X in place, gathered taps
+static SplitPlan search_split(int nz, int m, int n, int k, SplitSource source, bool large_tiles) {
+  struct Model { int bm, bn; double slab, solo, fixed; };
+  static const Model models[3][5] = {
+      {{128, 128, 0.63, 0.56, 9.5}, {64, 128, 0.37, 0.39, 6.5}, {128, 64, 0.37, 0.39, 6.5}, {64, 64, 0.21, 0.29, 5.2}, {256, 128, 1.20, 0.95, 10.0}},
+      {{128, 128, 0.63, 0.60, 9.5}, {64, 128, 0.38, 0.42, 6.5}, {128, 64, 0.37, 0.42, 6.5}, {64, 64, 0.21, 0.36, 5.2}, {0, 0, 0, 0, 0}},
+      // (gathered taps: two more vector instructions an element, and a slab's loads wait for its part of the tap table)
+      {{128, 128, 0.66, 0.80, 9.5}, {64, 128, 0.43, 0.60, 6.5}, {128, 64, 0.39, 0.50, 6.5}, {64, 64, 0.24, 0.36, 5.2}, {0, 0, 0, 0, 0}}};
+  const long long cus = wdh::compute_units();
+  const int slabs = (k + BK - 1) / BK;
+  SplitPlan best = {-1, {}, 1e30};
+  for (int t = 0; t <= S256x128; t++) {
+    const Model &mo = models[source][t];
+    if (mo.bm == 0 || (large_tiles && t == S64x64) || (g_split >= 3 && t != g_split - 3)) continue;
+    const long long tiles = (long long)((m + mo.bm - 1) / mo.bm) * ((n + mo.bn - 1) / mo.bn) * nz;
+    const int most = g_forced_split >= 1 ? (g_forced_split < slabs ? g_forced_split : slabs)
+                                         : slabs / 4 < 32 ? slabs / 4 : 32;  // at least 64 elements of K per chunk
+    for (int s = 1; s == 1 || s <= most; s++) {
+      if (g_forced_split >= 1 && s != most) continue;
+      const int per = (slabs + s - 1) / s;
+      const int chunks = (slabs + per - 1) / per;
+      if (chunks != s && g_forced_split < 1) continue;
+      // the whole launch cut s ways, or only the tiles beyond the last full round
+      for (int part = 0; part < (s > 1 && g_forced_split < 1 ? 2 : 1); part++) {
+        const long long tail = s == 1 ? 0 : part ? tiles % cus : tiles;
+        if (part && (tail == 0 || tail == tiles)) continue;
+        const long long whole = tiles - tail;
+        const long long rounds = s == 1 ? (tiles + cus - 1) / cus : whole / cus, cut_rounds = (tail * s + cus - 1) / cus;
+        double us = mo.fixed + (rounds + cut_rounds == 1 ? (rounds ? slabs : per) * mo.solo
+                                                          : rounds * slabs * mo.slab + cut_rounds * per * mo.slab);
+        us += 0.3 * (mo.fixed - 3.5) * (double)(rounds + cut_rounds - 1);
+        if (s > 1) us += 3.0 + 2.0 * (double)tail * s * mo.bm * mo.bn * 4.0 / 7.0e6;
+        if (us < best.us) {
+          best.tile = t;
+          best.us = us;
+          best.work = {whole, tail, chunks, per * BK};
+        }
+      }
+    }
+  }
+  return best;
+}
+// (the search takes a few microseconds on the host, so the plans of the last sizes are kept)
+static SplitPlan plan_split(int nz, int m, int n, int k, SplitSource source, bool large_tiles = false) {
+  struct Kept { int cus, nz, m, n, k, source, large_tiles; SplitPlan plan; };
+  static thread_local Kept kept[256] = {};
+  if (g_split != 1 || g_forced_split >= 1) return search_split(nz, m, n, k, source, large_tiles);
+  const int cus = wdh::compute_units();
+  unsigned h = (unsigned)nz;
+  for (int v : {m, n, k, (int)source, (int)large_tiles}) h = (h ^ (unsigned)v) * 0x9e3779b1u;
+  Kept &e = kept[h >> 24];
+  if (e.cus != cus || e.nz != nz || e.m != m || e.n != n || e.k != k || e.source != (int)source || e.large_tiles != (int)large_tiles)
+    e = {cus, nz, m, n, k, (int)source, (int)large_tiles, search_split(nz, m, n, k, source, large_tiles)};
+  return e.plan;
+}
+// Whether a Gemm / MatMul that may go to them does, and how.
+// Where gemm_wavesplit_kernel could serve, whose time is its blocks' rounds over the CUs: long products that go to cut
+// 64x64 tiles anyway (tiles_beat_wavesplit) take them here, in as many chunks (384x768x3072 31.6 us with the fp32
+// instruction, 27.5 here); the others wider tiles if those are estimated faster (us, that kernel / this: 1024x1024x1024 31 / 25.5,
+// 597x941x1108 28.8 / 22, 174x2128x2380 39.7 / 26.4; but 950x530x808 17.5 / 18.0, 356x514x1160 12.6 / 14.4, 1000x512x512 11.0 / 13.7).
+// Against ordinary tiles 590x2960x72 9.2 / 8.5, 880x93x1532 14.5 / 13.0, 2431x641x360 20.5 / 16.8, 4096x3072x768 143 / 107;
+// with little to multiply a longer prologue shows: 183x232x624 8.9 / 9.5, 249x1188x56 7.1 / 7.5.
+static SplitPlan split_gemm_plan(int batch, int m, int n, int k, bool b_kc) {
+  if (g_split > 1) return plan_split(batch, m, n, k, SPLIT_GEMM);
+  SplitPlan none = {-1, {}, 0.0};
+  if (wavesplit_suits(batch, m, n, k)) {
+    if (g_group.collecting) return none;
+    if (tiles_beat_wavesplit(batch, m, n, k, b_kc, true)) {
+      const int slabs = (k + BK - 1) / BK, per = (slabs + WS_WAVES - 1) / WS_WAVES;
+      return {S64x64, {0, (long long)((m + 63) / 64) * ((n + 63) / 64) * batch, (slabs + per - 1) / per, per * BK}, 0.0};
+    }
+    const long long blocks32 = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch, cus = wdh::compute_units();
+    const SplitPlan s = plan_split(batch, m, n, k, SPLIT_GEMM, true);
+    return s.us < 0.9 * (3.0 + 0.0078 * (double)((blocks32 + cus - 1) / cus) * k) ? s : none;
+  }
+  return (double)batch * m * n * k >= 1e8 ? plan_split(batch, m, n, k, SPLIT_GEMM) : none;
+}
+// Whether a conv of a batch does.  A single image stays with the fp32 instruction: its launches are short of tiles (ResNet-50's
+// 50 of them take 3 to 10 us each, mostly latency), and its results stay bit for bit what they were.  K below 96 leaves
+// nothing to gain from faster products (128 images 64 -> 256 on 56x56 173 us / 190, 16 images 32 -> 64 on 112x112 18.4 / 20).
+// Gathered taps cost vector instructions, which pay where whole tiles of output channels share them: 64 -> 64 on 56x56,
+// 32 images 73 / 66, 256 -> 256 on 28x28 stride 2 82 / 63; 108 -> 94 39 / 44, 400 -> 32 14.4 / 16.3.
+static bool split_conv_suits(int images, int m, int k, SplitSource source) {
+  return false;  // (convs stay with the fp32 instruction)
+  if (images < 2 || k < 96) return false;
+  return source == SPLIT_PIXELS || (m >= 64 && m * 10 >= (m + 63) / 64 * 64 * 9);
+}
+// Whether the fp32 form of a conv that reads X in place would run as a stream of K slabs (64x64 tiles; see stream_width).
+static bool conv_streams(const Params &p, int group) {
+  const long long tiles = (long long)((p.m + 63) / 64) * ((p.n + 63) / 64) * group;
+  const WorkPlan w = plan_work(tiles, p.k, 64, 64, true);
+  return !(p.m >= 256 && p.k >= 2048) && stream_width(tiles, (p.k + BK - 1) / BK, BK, w, 64 * 64, stream_blocks(64, 64)) > 0;
+}
+// Launches a plan; without room for the sums of cut tiles the product runs uncut.
+template <typename Launch>
+static int run_split(SplitPlan s, Launch launch) {
+  const int rc = launch(s);
+  if (rc != WDH_ENOMEM || s.work.tail == 0) return rc;
+  wdh::clear_error();  // (nothing failed for the caller)
+  s.work = {s.work.full + s.work.tail, 0, 1, 0};
+  return launch(s);
+}
+// Whether the bf16 matrix cores may serve a product at all.
+static bool split_legal(const Params &p, bool vec) {
+  if (!g_split || g_fp32_hint || g_stream == 2 || !p.fast || !vec || p.k % 4 != 0 || p.k < BK || g_static_scratch) return false;
+  return g_split > 1 || (g_forced_tile < 0 && g_forced_split < 0);
+}
+
 extern "C" int wdh_set_option(const char *name, int value) {
   if (!name) return fail(WDH_EINVAL, "wdh_set_option: name is NULL");
   if (strcmp(name, "contraction_tile") == 0) {
@@ -391,6 +506,11 @@ extern "C" int wdh_set_option(const char *name, int value) {
     if (value != 0 && value != 1)
       return fail(WDH_EINVAL, "wdh_set_option: wide_stores %d (use 0 or 1)", value);
     g_wide_stores = value;
+    return WDH_OK;
+  }
+  if (strcmp(name, "split_products") == 0) {
+    if (value < 0 || value > 3 + S256x128) return fail(WDH_EINVAL, "wdh_set_option: split_products %d (use 0..%d)", value, 3 + S256x128);
+    g_split = value;
     return WDH_OK;
   }
   if (strcmp(name, "conv_stem") == 0) {
@@ -583,6 +703,15 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
   }
   // A few rows against a transposed weight: a pass over the weight (gemm_rows.hip)
   if (useA_kc && useB_kc && gemm_rows_suits(batch, m, n, k, vec)) return launch_gemm_rows(p, batch, vec);
+  // Enough to multiply: the bf16 matrix cores (split_product.h)
+  if (useA_kc && split_legal(p, vec)) {
+    if (const SplitPlan s = split_gemm_plan(batch, m, n, k, useB_kc); s.tile >= 0) {
+      auto launch = [&](const SplitPlan &q) { return launch_split_gemm(useB_kc, q, p, batch); };
+      const int rc = wavesplit_suits(batch, m, n, k) ? launch(s) : run_split(s, launch);
+      if (rc != WDH_ENOMEM) return rc;
+      wdh::clear_error();  // (no room for the sums of cut tiles: gemm_wavesplit_kernel needs none)
+    }
+  }
   // Few result tiles and a K worth cutting: one launch with K cut across the wavefronts of a
   // workgroup (gemm_wavesplit_kernel) instead of chunks in a workspace and a reduce pass
   if (useA_kc && p.fast && wavesplit_suits(batch, m, n, k)) {
@@ -885,6 +1014,13 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   const long long w_bytes = (long long)cout_g * kdim * 4;
   const bool small = g_descriptors && x_bytes < 0x7fffffffLL && w_bytes < 0x7fffffffLL;
   const bool vec = aligned16(p.A) && kdim % 4 == 0 && ((long long)cout_g * kdim) % 4 == 0;
+  // the bf16 matrix cores (split_product.h) by gathering taps
+  auto split_possible = [&](int images, int rows, int depth) {
+    Params q = {};
+    q.k = depth;
+    q.fast = small ? 1 : 0;
+    return split_legal(q, vec) && (g_split > 1 || split_conv_suits(images, rows, depth, SPLIT_TAPS));
+  };
   // 1x1, stride 1, no padding: X is the B matrix as it lies (B_PIXELS), provided every K slab
   // is whole and four consecutive pixels never straddle two images.  The last tile may hang
   // over the end of the pixels: its surplus columns read the next k row or, past the last
@@ -913,8 +1049,21 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
     p.y_bytes = g_descriptors && out_bytes < 0x7fffffffULL ? (int)out_bytes : 0;
     p.c_bytes = cout * 4;
     set_wide(p, true);
+    // (what the plan schedules as a stream of K slabs stays one)
+    g_last_form = in_place_s2 ? B_PIXELS_S2 : B_PIXELS;
+    if (split_legal(p, true) && !(g_split == 1 && conv_streams(p, group)))
+      if (const SplitPlan s = plan_split(group, p.m, p.n, p.k, SPLIT_PIXELS);
+          s.tile >= 0 && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS)))
+        return run_split(s, [&](const SplitPlan &q) { return launch_split_conv(in_place_s2 ? B_PIXELS_ANY : B_PIXELS, q, p, group); });
     return launch_conv_pixels(p, group, true, in_place_s2);
   }
+  const int mode = !small || ntaps > 63 ? B_IM2COL_BIG : (ntaps > 31 ? B_IM2COL64 : B_IM2COL32);
+  KtabKey key;
+  memset(&key, 0, sizeof(key));
+  key.c_in_g = c_in_g; key.kh = kh; key.kw = kw; key.dh = dh; key.dw = dw;
+  key.h = h; key.w = w; key.mode = mode;
+  // (while a graph is being recorded the gathered forms serve only geometries whose tap table is there already)
+  const bool gather_split = mode != B_IM2COL_BIG && (!wdh::capturing() || g_ktabs.count(key)) && split_possible(n, cout_g, (int)kdim);
   // 3x3, stride 1, no dilation, one group, many channels: minimal filtering -- filters and input patches
   // are transformed, the positions of the transform domain (16 for F(2x2, 3x3), 36 for F(4x4, 3x3)) are
   // one batched product M[xi] = U[xi] [cout, c] x V[xi] [c, tiles] with 4/9 or 1/4 of the direct form's
@@ -922,13 +1071,20 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   // g_winograd: 0 never; 1 = F(2x2, 3x3) from 128 channels on (F(4x4, 3x3) from g_winograd4_channels on, when
   // that is set: faster from 64 channels on, but its rounding errors are about ten times the direct form's,
   // which a 50-layer network's logits show); 2 / 3 = F(2x2, 3x3) / F(4x4, 3x3) wherever legal.
+  // (transform-domain tensors that outgrow the 256 MB last-level cache cost more than the multiplications saved once the
+  // direct form runs on the bf16 matrix cores: 128 images 128 -> 128 on 28x28, V and M 206 MB each, 254 us against 193;
+  // 256 -> 256 on 14x14, 103 MB each, 149 against 194)
+  bool wino_memory = true;  // there was room for the transform-domain tensors, if they were wanted
+  auto wino_outgrown = [&]() {
+    return g_winograd == 1 && gather_split && 64LL * (c + cout) * wdh::wino_tiles(2, n, oh, ow) > (256LL << 20);
+  };
   const int wino_min = c < cout ? c : cout;
   int wino_r = 0;
   if (g_winograd == 2) wino_r = 2;
   else if (g_winograd == 3) wino_r = 4;
   else if (g_winograd == 1) wino_r = g_winograd4_channels && wino_min >= g_winograd4_channels ? 4 : wino_min >= 128 ? 2 : 0;
   if (wino_r && kh == 3 && kw == 3 && sh == 1 && sw == 1 && dh == 1 && dw == 1 && group == 1 && c % BK == 0 &&
-      g_forced_tile < 0 && g_forced_split < 0) {
+      g_forced_tile < 0 && g_forced_split < 0 && !(wino_r == 2 && wino_outgrown())) {
     const int r = wino_r, positions = (r + 2) * (r + 2);
     const long long tiles = wdh::wino_pitch(wdh::wino_tiles(r, n, oh, ow));  // (row length of V and M)
     const size_t u_bytes = (size_t)positions * cout * c * 4, v_bytes = (size_t)positions * c * tiles * 4,
@@ -962,6 +1118,7 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
         if (hV) (void)wdh_free(hV);
         if (hM) (void)wdh_free(hM);
         wdh::clear_error();
+        wino_memory = false;
         goto direct_forms;
       }
       {
@@ -974,9 +1131,11 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
         // every 3x3 layer shape of ResNet-50 and DETR, 35 against 44 us where the general choice
         // takes 128x128)
         g_tile_hint = T64x64;
+        g_fp32_hint = true;
         rc = wdh_gemm(hU, hV, 0, hM, positions, cout, (int)tiles, c, (int64_t)cout * c, c, 1, (int64_t)c * tiles, tiles, 1,
                       0, 0, 1.0f, 1.0f, WDH_EPI_NONE, 0);
         g_tile_hint = -1;
+        g_fp32_hint = false;
       }
       if (rc == WDH_OK) {
         g_last_plan.form = r == 2 ? WDH_FORM_CONV3X3_WINOGRAD : WDH_FORM_CONV3X3_WINOGRAD4;
@@ -994,7 +1153,8 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
 direct_forms:
   // 3x3, stride 1, no dilation, input channels in blocks of 8: taps read from an input
   // tile staged in LDS (conv3x3_halo_kernel)
-  if (g_halo && small && kh == 3 && kw == 3 && sh == 1 && sw == 1 && dh == 1 && dw == 1 &&
+  // (a batch's with enough output channels gather their taps for the bf16 matrix cores instead: split_conv_suits)
+  if (g_halo && !(gather_split && wino_memory) && small && kh == 3 && kw == 3 && sh == 1 && sw == 1 && dh == 1 && dw == 1 &&
       c_in_g % HALO_CB == 0 && aligned16(p.A)) {
     const int vecw = (w % 4 == 0 && aligned16(p.B)) ? 4 : ((w % 2 == 0 && ((uintptr_t)p.B & 7) == 0) ? 2 : 1);
     p.cv.h = h; p.cv.w = w; p.cv.oh = oh; p.cv.ow = ow; p.cv.pt = pt; p.cv.pl = pl;
@@ -1020,11 +1180,29 @@ direct_forms:
       return launch_conv3x3(tile, p, group, vecw);
     }
   }
-  const int mode = !small || ntaps > 63 ? B_IM2COL_BIG : (ntaps > 31 ? B_IM2COL64 : B_IM2COL32);
-  KtabKey key;
-  memset(&key, 0, sizeof(key));
-  key.c_in_g = c_in_g; key.kh = kh; key.kw = kw; key.dh = dh; key.dw = dw;
-  key.h = h; key.w = w; key.mode = mode;
+  // any other unpadded 1x1 conv of a batch: each pixel of X is read where it lies, whatever the strides and the plane
+  if (small && vec && ntaps == 1 && pt == 0 && pl == 0 && pb == 0 && pr == 0) {
+    p.m = cout_g; p.n = (int)npix; p.k = (int)kdim;
+    p.fast = 1;
+    if (split_legal(p, true) && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS))) {
+      p.sAb = (long long)cout_g * kdim; p.sA0 = kdim; p.sA1 = 1;
+      p.sBb = (long long)c_in_g * plane; p.sB0 = plane; p.sB1 = 1;
+      p.alpha = 1.0f; p.beta = 1.0f; p.epilogue = epilogue;
+      p.cv.c_in_g = c_in_g; p.cv.h = h; p.cv.w = w; p.cv.oh = oh; p.cv.ow = ow;
+      p.cv.sh = sh; p.cv.sw = sw;
+      p.cv.kh = p.cv.kw = p.cv.dh = p.cv.dw = 1;
+      p.cv.c_total = c; p.cv.cout_total = cout; p.cv.cout_g = cout_g;
+      p.cv.ntaps = 1; p.cv.npix = npix;
+      p.a_bytes = (int)w_bytes;
+      p.b_bytes = (int)x_bytes;
+      p.y_bytes = g_descriptors && out_bytes < 0x7fffffffULL ? (int)out_bytes : 0;
+      p.c_bytes = cout * 4;
+      set_wide(p, true);
+      g_last_form = WDH_FORM_CONV_GATHER32;  // (the form it stands in for)
+      return run_split(plan_split(group, p.m, p.n, p.k, SPLIT_PIXELS),
+                       [&](const SplitPlan &q) { return launch_split_conv(B_PIXELS_ANY, q, p, group); });
+    }
+  }
   auto it = g_ktabs.find(key);
   if (it == g_ktabs.end()) {
     if (wdh::capturing()) {
@@ -1079,5 +1257,8 @@ direct_forms:
   p.y_bytes = g_descriptors && out_bytes < 0x7fffffffULL ? (int)out_bytes : 0;
   p.c_bytes = cout * 4;
   set_wide(p, true);
+  if (gather_split)
+    if (const SplitPlan s = plan_split(group, p.m, p.n, p.k, SPLIT_TAPS); s.tile >= 0)
+      return run_split(s, [&](const SplitPlan &q) { return launch_split_conv(mode, q, p, group); });
   return launch_conv_gather(mode, p, group, vec);
 }

@@ -1,0 +1,399 @@
+// Products of fp32 operands on the bf16 matrix cores, without giving up fp32 accuracy.
+//
+// A float is the exact sum of three bfloat16 values: h = x rounded to the nearest one, m = x - h rounded likewise, and
+// l = x - h - m (both subtractions are exact, and what is left fits eight bits).  Of the nine products of two such sums
+// the three below 2^-25 of the whole (m*l, l*m, l*l) are left out; the other six go through
+// v_mfma_f32_32x32x16_bf16, which multiplies sixteen times as many pairs a cycle as v_mfma_f32_32x32x2_f32 and adds in
+// fp32.  Rounding to nearest matters: with the upper sixteen bits instead the parts share a sign, what is left out too, and
+// every product is 3e-8 too small, which fifty layers add up (ResNet-50's logits 2.4e-3 off where 1e-3 is allowed; 6e-4 now).
+// The matrix core adds a product to a far larger sum less exactly than a fused multiply-add does, so the leading
+// products h*h and the five small ones are summed apart and meet once at the end: a chain has K/16 (small ones:
+// 5K/16) additions where the fp32 instruction makes K/2.  Errors against 64 bits (2-norm, normally distributed operands, fp32
+// instruction / this): K 64 14.5e-8 / 5.0e-8, 256 28.7e-8 / 8.9e-8, 1024 5.8e-7 / 1.9e-7, 4096 11.5e-7 / 4.0e-7; positive
+// operands 12.2e-8 / 5.2e-8 to 9.8e-7 / 3.5e-7, no drift to either side (below 1e-8).
+//
+// Bound: power.  A loop of nothing but these instructions runs at 1550 to 1800 TFLOP/s, which is 260 to 300 of fp32
+// products (the fp32 instruction's own limit is 157); at 4096^3 the matrix cores are busy 79 % of the cycles and the clock
+// falls to 1.5 GHz.  What a slab adds to the products is the split (11 vector instructions per pair of elements) and
+// LDS traffic (6 bytes an element), so an operand is split once, on its way from registers to LDS, not by every
+// wavefront that multiplies it.  The split and the LDS stores of the next slab are placed between the matrix
+// instructions of this one (sched_group_barrier): 195 -> 209 TFLOP/s, because the wavefronts of a SIMD else meet the same phase
+// at the same time.  Measured at 4096^3 (TFLOP/s; fp32 instruction 146): 64x64 tiles 159, 64x128 and 128x64 181, 128x128 209,
+// 256x128 210 to 222.  Tried without gain: fragments of the next slab read ahead (204), loads two to eight slabs ahead (204), small
+// products in two or three chains; LDS planes without the 64 bytes between their halves (a third more LDS cycles, 198).
+//
+// What the split cannot hold is done again with the fp32 instruction, a whole tile (or chunk) at a time:
+//   * an Inf or NaN operand leaves NaN in x - h and therefore in every sum it enters; so does a sum that overflows;
+//   * elements below 2^-110 lose bits of l below 2^-133.  Only a sum of such elements shows that, and it is tiny:
+//     a tile that holds a nonzero sum below 2^-100 is done again.
+// Both show in the sums themselves, so the loop carries no test.
+#pragma once
+#include "contraction.h"
+
+namespace wdhc {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+// Two elements -> their three parts, packed (the first in the lower sixteen bits).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+struct SplitPair { unsigned h, m, l; };
+__device__ __forceinline__ unsigned nearest_pair(float x0, float x1) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x0, x1}, bf16x2));
+}
+__device__ __forceinline__ SplitPair split_pair(float x0, float x1) {
+  const unsigned h = nearest_pair(x0, x1);
+  const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
+  const unsigned m = nearest_pair(r0, r1);
+  const float s0 = r0 - __uint_as_float(m << 16), s1 = r1 - __uint_as_float(m & 0xffff0000u);
+  return SplitPair{h, m, nearest_pair(s0, s1)};
+}
+
+// Workgroups a CU holds: the accumulators are two per result, so 128x128 tiles take 64 + 64 registers of
+// accumulators and two of them fit; 256x128 is the same wavefront with eight of them in one workgroup.
+constexpr int split_blocks(int bm, int bn) { return bm * bn >= 128 * 128 ? 2 : (bm * bn > 64 * 64 ? 3 : 4); }
+
+// LDS: three planes (h, m, l) per operand, each [k / 8][row or column][8 bf16], so that a fragment of a 32x16 block
+// is one 16-byte read per lane, 32 lanes side by side.
+template <int BM, int BN, int WM, int WN, int BMODE>
+__global__ __launch_bounds__(WM * WN * 64, split_blocks(BM, BN)) void split_kernel(Params p) {
+  constexpr int THREADS = WM * WN * 64;
+  constexpr bool IM2COL = BMODE == B_IM2COL32 || BMODE == B_IM2COL64;
+  constexpr bool PIX_ANY = BMODE == B_PIXELS_ANY;
+  constexpr bool PIXELS = BMODE == B_PIXELS || PIX_ANY;
+  constexpr bool CONV = IM2COL || PIXELS;
+  constexpr bool B_IS_KC = BMODE == B_KC;
+  constexpr bool B_COLUMNS = !B_IS_KC && !IM2COL;  // B contiguous along its columns
+  constexpr int MT = BM / (WM * 32), NT = BN / (WN * 32);
+  // (bytes; the 64 between the halves of a plane keep the 8-byte stores of 16 lanes, four k of each of eight rows, on
+  // different banks)
+  constexpr int HALF_A = BM * 16 + 64, HALF_B = BN * 16 + 64, PLANE_A = 2 * HALF_A, PLANE_B = 2 * HALF_B;
+  constexpr int BUF = 3 * (PLANE_A + PLANE_B);
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2][BUF];
+  static_assert(2 * BUF >= WM * WN * STAGE_FLOATS * 4, "epilogue staging");
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int wm = wave / WN, wn = wave % WN;
+  const int li = lane & 31, half = lane >> 5;
+  const int wrow = wm * (MT * 32), wcol = wn * (NT * 32);
+
+  const TileWork tw = decode_work(p);
+  const int bz = tw.bz, row0 = tw.tm * BM, col0 = tw.tn * BN;
+  const int kbeg = tw.whole ? 0 : tw.chunk * p.kchunk;
+  const int kend = tw.whole ? p.k : (kbeg + p.kchunk < p.k ? kbeg + p.kchunk : p.k);
+  const float *const A = p.A + (long long)bz * p.sAb;
+  const float *const B = CONV ? p.B + (long long)bz * p.cv.c_in_g * p.cv.h * p.cv.w : p.B + (long long)bz * p.sBb;
+  const int lda = (int)p.sA0, ldb = (int)(B_IS_KC ? p.sB1 : p.sB0);
+
+  // ---- fetch plans: one byte offset per piece, every address term folded in -------------------------
+  // k-contiguous: thread t takes k 4*(t%4)..+3 of rows t/4 + i*THREADS/4.
+  constexpr int RPP = THREADS / 4, NA = BM / RPP;
+  static_assert(NA >= 1 && BM % RPP == 0, "rows per pass");
+  const int kq = tid & 3;
+  int voff_a[NA];
+#pragma unroll
+  for (int i = 0; i < NA; i++) {
+    int r = row0 + (tid >> 2) + i * RPP;
+    r = r < p.m ? r : p.m - 1;  // rows and columns past the edge feed only sums that are never stored
+    voff_a[i] = (r * lda + kq * 4) * 4;
+  }
+  const rsrc_t rsrc_a = make_rsrc(A, p.a_bytes);
+
+  // column-contiguous: a piece is four k of CPP neighbouring columns.  Neighbouring lanes take the lower and the
+  // upper four k of one plane row, so that their 8-byte LDS stores lie side by side.
+  constexpr int CPP = BN * 4 / THREADS;  // columns per thread (1 or 2)
+  constexpr int NB = B_IS_KC ? BN / RPP : 1;
+  constexpr int G = THREADS / BN > 0 ? THREADS / BN : 1, L = BK / G;  // im2col: L consecutive k of one pixel
+  static_assert(!B_COLUMNS || CPP == 1 || CPP == 2, "column pieces");
+  static_assert(!IM2COL || (L == 4 || L == 8), "im2col pieces");
+  const int bkq = B_COLUMNS ? (tid & 1) | ((tid / (2 * (BN / CPP))) << 1) : 0;
+  const int bcol = B_COLUMNS ? ((tid >> 1) % (BN / CPP)) * CPP : 0;
+  int voff_b[B_IS_KC ? NB : CPP];
+  PixelFast pf = {0, 0xffffffffu, 0xffffffffu};
+  const int bias = IM2COL ? p.cv.pt * p.cv.w + p.cv.pl : 0;  // makes every corner offset >= 0
+  const int kgroup0 = IM2COL ? __builtin_amdgcn_readfirstlane(tid / BN) * L : 0;
+  // element offset of a column of B at k = 0 (conv: of a pixel of the group's first channel; im2col: of the
+  // receptive field's corner, plus `bias`)
+  auto column = [&](int col) -> int {
+    if (!CONV) return col;
+    const unsigned P = (unsigned)col < (unsigned)p.n ? (unsigned)col : (unsigned)p.n - 1u;
+    const unsigned plane = (unsigned)(p.cv.h * p.cv.w), ohw = (unsigned)(p.cv.oh * p.cv.ow);
+    const unsigned img = (unsigned)fdiv((int)P, p.cv.fd_ohw), q = P - img * ohw;
+    const unsigned oy = (unsigned)fdiv((int)q, p.cv.fd_ow), ox = q - oy * (unsigned)p.cv.ow;
+    return (int)(img * (unsigned)p.cv.c_total * plane) + ((int)oy * p.cv.sh - (IM2COL ? p.cv.pt : 0)) * p.cv.w +
+           (int)ox * p.cv.sw - (IM2COL ? p.cv.pl : 0) + bias;
+  };
+  auto padding = [&](int col, PixelFast &f) {  // which taps of this pixel lie in the padding
+    f.pad_lo = f.pad_hi = 0xffffffffu;
+    if (col >= p.n) return;
+    const unsigned ohw = (unsigned)(p.cv.oh * p.cv.ow);
+    const unsigned q = (unsigned)col - (unsigned)fdiv(col, p.cv.fd_ohw) * ohw;
+    const int oy = fdiv((int)q, p.cv.fd_ow), ox = (int)q - oy * p.cv.ow;
+    unsigned long long inside = 0;
+    int t = 0;
+    for (int ky = 0; ky < p.cv.kh; ky++) {
+      const bool row_in = (unsigned)(oy * p.cv.sh - p.cv.pt + ky * p.cv.dh) < (unsigned)p.cv.h;
+      for (int kx = 0; kx < p.cv.kw; kx++, t++)
+        if (row_in && (unsigned)(ox * p.cv.sw - p.cv.pl + kx * p.cv.dw) < (unsigned)p.cv.w) inside |= 1ull << t;
+    }
+    f.pad_lo = ~(unsigned)inside;
+    f.pad_hi = ~(unsigned)(inside >> 32);
+  };
+  if (B_IS_KC) {
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      int c = col0 + (tid >> 2) + i * RPP;
+      c = c < p.n ? c : p.n - 1;
+      voff_b[i] = (c * ldb + kq * 4) * 4;
+    }
+  } else if (IM2COL) {
+    const int col = col0 + tid % BN;
+    pf.valid = column(col) * 4;
+    padding(col, pf);
+  } else {
+#pragma unroll
+    for (int i = 0; i < CPP; i++) voff_b[i] = (bkq * 4 * ldb + column(col0 + bcol + i)) * 4;
+  }
+  const int b_window = CONV ? p.b_bytes - (int)((long long)bz * p.cv.c_in_g * p.cv.h * p.cv.w * 4) : p.b_bytes;
+  const rsrc_t rsrc_b = make_rsrc(B - bias, b_window);
+
+  struct Slab {
+    f32x4 a[NA];
+    f32x4 b[B_IS_KC ? NB : (IM2COL ? L / 4 : CPP)];  // four consecutive k each
+  };
+  // im2col: the tap table's entries of the slab to be fetched next (scalar loads, a slab ahead of their use)
+  struct { int2 e[IM2COL ? L : 1]; } taps;
+  const int ktab_last = IM2COL ? (p.k + BK - 1) / BK * BK - BK : 0;
+  auto read_taps = [&](int k0) {
+    if (!IM2COL) return;
+    k0 = k0 < ktab_last ? k0 : ktab_last;
+#pragma unroll
+    for (int i = 0; i < (IM2COL ? L : 1); i++) taps.e[i] = p.cv.ktab[k0 + kgroup0 + i];
+  };
+  // last: the slab may reach past kend (a multiple of four): pieces beyond it read as zeros
+  auto fetch = [&](int k0, Slab &s, bool last) {
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+      s.a[i] = buf_load4(rsrc_a, last && k0 + kq * 4 >= kend ? BUF_OOB : voff_a[i], k0 * 4);
+    if (B_IS_KC) {
+#pragma unroll
+      for (int i = 0; i < NB; i++)
+        s.b[i] = buf_load4(rsrc_b, last && k0 + kq * 4 >= kend ? BUF_OOB : voff_b[i], k0 * 4);
+    } else if (IM2COL) {
+#pragma unroll
+      for (int i = 0; i < L; i++) {
+        const int2 e = taps.e[i];
+        const unsigned word = (BMODE == B_IM2COL64 && (e.y & 32)) ? pf.pad_hi : pf.pad_lo;
+        const int pad = __builtin_amdgcn_sbfe((int)word, (unsigned)e.y & 31u, 1u);
+        s.b[i >> 2][i & 3] = buf_load(rsrc_b, (pad & BUF_OOB) | pf.valid, e.x);
+      }
+      read_taps(k0 + BK);
+    } else {
+      const bool out = last && k0 + bkq * 4 >= kend;
+      const int voff = out ? BUF_OOB : voff_b[0];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int soff = (k0 + e) * ldb * 4;
+        if (CPP == 1) {
+          s.b[0][e] = buf_load(rsrc_b, voff, soff);
+        } else if (PIX_ANY) {
+          s.b[0][e] = buf_load(rsrc_b, voff, soff);
+          s.b[CPP - 1][e] = buf_load(rsrc_b, out ? BUF_OOB : voff_b[CPP - 1], soff);
+        } else {
+          const f32x2 v = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc_b, voff, soff, 0));
+          s.b[0][e] = v.x;
+          s.b[CPP - 1][e] = v.y;
+        }
+      }
+    }
+  };
+  auto put4 = [&](unsigned char *cell, int plane, f32x4 v) {
+    const SplitPair lo = split_pair(v.x, v.y), hi = split_pair(v.z, v.w);
+    *reinterpret_cast<u32x2 *>(cell) = u32x2{lo.h, hi.h};
+    *reinterpret_cast<u32x2 *>(cell + plane) = u32x2{lo.m, hi.m};
+    *reinterpret_cast<u32x2 *>(cell + 2 * plane) = u32x2{lo.l, hi.l};
+  };
+  auto put = [&](unsigned char *buf, const Slab &s) {
+    unsigned char *const b = buf + 3 * PLANE_A;
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+      put4(buf + (kq >> 1) * HALF_A + ((tid >> 2) + i * RPP) * 16 + (kq & 1) * 8, PLANE_A, s.a[i]);
+    if (B_IS_KC) {
+#pragma unroll
+      for (int i = 0; i < NB; i++)
+        put4(b + (kq >> 1) * HALF_B + ((tid >> 2) + i * RPP) * 16 + (kq & 1) * 8, PLANE_B, s.b[i]);
+    } else if (IM2COL) {
+#pragma unroll
+      for (int i = 0; i < L / 4; i++) {
+        const int q = (kgroup0 >> 2) + i;
+        put4(b + (q >> 1) * HALF_B + (tid % BN) * 16 + (q & 1) * 8, PLANE_B, s.b[i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < CPP; i++) put4(b + (bkq >> 1) * HALF_B + (bcol + i) * 16 + (bkq & 1) * 8, PLANE_B, s.b[i]);
+    }
+  };
+
+  f32x16 acc[MT][NT], small[MT][NT];
+#pragma unroll
+  for (int a = 0; a < MT; a++)
+#pragma unroll
+    for (int b = 0; b < NT; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[a][b][r] = small[a][b][r] = 0.0f;
+
+  auto compute = [&](const unsigned char *buf) {
+    const unsigned char *const fa = buf + half * HALF_A + (wrow + li) * 16;
+    const unsigned char *const fb = buf + 3 * PLANE_A + half * HALF_B + (wcol + li) * 16;
+    bf16x8 a[MT][3], b[NT][3];
+#pragma unroll
+    for (int pl = 0; pl < 3; pl++) {
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) a[mt][pl] = *reinterpret_cast<const bf16x8 *>(fa + pl * PLANE_A + mt * 512);
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++) b[nt][pl] = *reinterpret_cast<const bf16x8 *>(fb + pl * PLANE_B + nt * 512);
+    }
+    auto products = [&](int i, int j, f32x16 (&sum)[MT][NT]) {
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+          sum[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mt][i], b[nt][j], sum[mt][nt], 0, 0, 0);
+    };
+    products(0, 0, acc);
+    products(0, 1, small);
+    products(1, 0, small);
+    products(1, 1, small);
+    products(0, 2, small);
+    products(2, 0, small);
+  };
+
+  // Slab s+2 is requested, slab s+1 split and stored to the other LDS buffer, slab s multiplied: one barrier a slab.
+  const int nslabs = (kend - kbeg + BK - 1) / BK, nfull = (kend - kbeg) / BK;
+  Slab next;
+  read_taps(kbeg);
+  fetch(kbeg, next, true);
+  put(lds[0], next);
+  if (nslabs > 1) fetch(kbeg + BK, next, true);
+  __syncthreads();
+  auto step = [&](int s, int cur) {
+    const Slab now = next;
+    fetch(kbeg + (s + 2) * BK, next, false);
+    __builtin_amdgcn_s_setprio(1);
+    compute(lds[cur]);
+    put(lds[cur ^ 1], now);
+    // fragment reads, requests, then products with the split and the stores in between
+    constexpr int PIECES = NA + (B_IS_KC ? NB : (IM2COL ? L / 4 : CPP));
+    constexpr int PRODUCTS = MT * NT * 6, VALU = PIECES * 22 + (IM2COL ? 2 * L : 0), STORES = PIECES * 3;
+    constexpr int LOADS = NA + (B_IS_KC ? NB : (IM2COL ? L : PIX_ANY ? 4 * CPP : 4));
+    __builtin_amdgcn_sched_group_barrier(0x100, (MT + NT) * 3, 0);
+    __builtin_amdgcn_sched_group_barrier(0x20, LOADS, 0);
+#pragma unroll
+    for (int i = 0; i < PRODUCTS; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x2, (VALU + PRODUCTS - 1) / PRODUCTS, 0);
+      if ((i + 1) * STORES / PRODUCTS > i * STORES / PRODUCTS) __builtin_amdgcn_sched_group_barrier(0x200, (STORES + PRODUCTS - 1) / PRODUCTS, 0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __syncthreads();
+  };
+  int s = 0;
+  for (; s + 3 < nfull; s += 2) {
+    step(s, 0);
+    step(s + 1, 1);
+  }
+  for (; s < nslabs; s++) {
+    const Slab now = next;
+    if (s + 2 < nslabs) fetch(kbeg + (s + 2) * BK, next, true);
+    compute(lds[s & 1]);
+    if (s + 1 < nslabs) put(lds[(s & 1) ^ 1], now);
+    __syncthreads();
+  }
+
+  // ---- the two sums meet; is there anything the split could not hold? ------------------------------------
+  // (bits of |sum| doubled: zero is fine, so is 2^-100 up to the largest float)
+  unsigned most = 0, least = 0xffffffffu;
+#pragma unroll
+  for (int a = 0; a < MT; a++)
+#pragma unroll
+    for (int b = 0; b < NT; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        acc[a][b][r] += small[a][b][r];
+        const unsigned u = __float_as_uint(acc[a][b][r]) << 1;
+        most = u > most ? u : most;
+        least = u - 1u < least ? u - 1u : least;
+      }
+  const bool odd = most >= 0xff000000u || least < ((127u - 100u) << 24) - 1u;
+  if (__syncthreads_or(odd)) {
+    // Operands straight from memory, one element a lane and k; never the common case.
+    const float *pa[MT];
+    int cb[NT];
+    PixelFast pb[NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      const int r = row0 + wrow + mt * 32 + li;
+      pa[mt] = A + (long long)(r < p.m ? r : p.m - 1) * lda;
+    }
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+      int c = col0 + wcol + nt * 32 + li;
+      if (IM2COL) padding(c, pb[nt]);
+      c = c < p.n ? c : p.n - 1;
+      cb[nt] = B_IS_KC ? c * ldb : column(c) - bias;
+    }
+#pragma unroll
+    for (int a = 0; a < MT; a++)
+#pragma unroll
+      for (int b = 0; b < NT; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
+    for (int k0 = kbeg; k0 < kend; k0 += 2) {
+      const int k = k0 + half;
+      const bool in = k < kend;
+      float ea[MT], eb[NT];
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) ea[mt] = in ? pa[mt][k] : 0.0f;
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++) {
+        if (IM2COL) {
+          const int2 e = p.cv.ktab[in ? k : kbeg];
+          const unsigned word = (BMODE == B_IM2COL64 && (e.y & 32)) ? pb[nt].pad_hi : pb[nt].pad_lo;
+          eb[nt] = in && !((word >> (e.y & 31)) & 1u) ? B[cb[nt] + (e.x >> 2)] : 0.0f;
+        } else {
+          eb[nt] = in ? B[B_IS_KC ? (long long)cb[nt] + k : (long long)k * ldb + cb[nt]] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(ea[mt], eb[nt], acc[mt][nt], 0, 0, 0);
+    }
+  }
+  finish_tile<BM, BN, WM, WN, CONV>(p, acc, tw.whole, tw.lin, tw.chunk, bz, row0, col0,
+                                    reinterpret_cast<float *>(&lds[0][0]) + wave * STAGE_FLOATS);
+}
+
+template <int BM, int BN, int WM, int WN, int BMODE>
+int launch_split_tile(Params &p, int nz, const WorkPlan &w) {
+  if (BMODE != B_PIXELS_ANY) g_last_form = BMODE;  // (otherwise the caller says which conv it is)
+  return launch_planned<BM, BN>(p, nz, BMODE >= B_IM2COL32, BK, 0, [&](dim3 grid, bool) {
+    hipLaunchKernelGGL((split_kernel<BM, BN, WM, WN, BMODE>), grid, dim3(WM * WN * 64), 0, wdh::stream(), p);
+  }, &w);
+}
+template <int BMODE>
+int launch_split(const SplitPlan &s, Params &p, int nz) {
+  switch (s.tile) {
+    case S256x128:
+      if constexpr (BMODE == B_KC || BMODE == B_MC) return launch_split_tile<256, 128, 4, 2, BMODE>(p, nz, s.work);
+      [[fallthrough]];  // (not planned for convs)
+    case S128x128: return launch_split_tile<128, 128, 2, 2, BMODE>(p, nz, s.work);
+    case S64x128: return launch_split_tile<64, 128, 2, 2, BMODE>(p, nz, s.work);
+    case S128x64: return launch_split_tile<128, 64, 2, 2, BMODE>(p, nz, s.work);
+    default: return launch_split_tile<64, 64, 2, 2, BMODE>(p, nz, s.work);
+  }
+}
+
+}  // namespace wdhc
