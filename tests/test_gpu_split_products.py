@@ -158,3 +158,38 @@ def test_convs(ctx, split, mode, shape):
         out[value] = H.conv(ctx, ctx.move_tensor(x), ctx.move_tensor(wt), ctx.move_tensor(bias), [dil, dil], group, None, [pad] * 4,
                             [stride, stride]).get_data()
     assert (np.isnan(out[0]) == np.isnan(out[mode])).all() and (np.isinf(out[0]) == np.isinf(out[mode])).all()
+
+
+def test_one_image_keeps_its_bits(ctx, split):
+    """A single image stays with the fp32 instruction; the same image in a batch agrees with it as sums in another order do."""
+    rng = np.random.default_rng(4)
+    x = rng.standard_normal((2, 256, 28, 28)).astype(np.float32)
+    for cout, kernel in ((128, 1), (256, 3)):
+        wt = ctx.move_tensor((rng.standard_normal((cout, 256, kernel, kernel)) * 0.03).astype(np.float32))
+        out = {}
+        for value in (0, 1):
+            split(value)
+            out[value] = H.conv(ctx, ctx.move_tensor(x[:1]), wt, pads=[kernel // 2] * 4).get_data()
+        assert (out[0] == out[1]).all()
+        both = H.conv(ctx, ctx.move_tensor(x), wt, pads=[kernel // 2] * 4).get_data()
+        assert np.abs(both[:1] - out[0]).max() <= 1e-5 * np.abs(out[0]).max()
+
+
+def test_a_geometry_first_met_while_recording(ctx, split):
+    """The gathered form needs a tap table, which cannot be built then: the form that reads an LDS tile serves."""
+    rng = np.random.default_rng(6)
+    x, wt = ctx.move_tensor(rng.standard_normal((2, 64, 20, 24)).astype(np.float32)), ctx.move_tensor(rng.standard_normal((64, 64, 3, 3)).astype(np.float32))
+    ctx.sync()
+    ctx.graph_begin()
+    y = H.conv(ctx, x, wt, pads=[1] * 4)
+    form = ctx.last_plan()["form"]
+    graph = ctx.graph_end()
+    assert form == "conv 3x3, LDS tile", form
+    for _ in range(3):
+        ctx.graph_launch(graph)
+        got = y.get_data()
+        want = H.conv(ctx, x, wt, pads=[1] * 4)
+        assert ctx.last_plan()["form"] == "conv, gathered taps", ctx.last_plan()
+        assert np.abs(got - want.get_data()).max() <= 1e-5 * np.abs(got).max()
+        want.dispose()
+    ctx.graph_destroy(graph)

@@ -450,7 +450,6 @@ static SplitPlan split_gemm_plan(int batch, int m, int n, int k, bool b_kc) {
 // Gathered taps cost vector instructions, which pay where whole tiles of output channels share them: 64 -> 64 on 56x56,
 // 32 images 73 / 66, 256 -> 256 on 28x28 stride 2 82 / 63; 108 -> 94 39 / 44, 400 -> 32 14.4 / 16.3.
 static bool split_conv_suits(int images, int m, int k, SplitSource source) {
-  return false;  // (convs stay with the fp32 instruction)
   if (images < 2 || k < 96) return false;
   return source == SPLIT_PIXELS || (m >= 64 && m * 10 >= (m + 63) / 64 * 64 * 9);
 }
@@ -1131,7 +1130,7 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
         // every 3x3 layer shape of ResNet-50 and DETR, 35 against 44 us where the general choice
         // takes 128x128)
         g_tile_hint = T64x64;
-        g_fp32_hint = true;
+        g_fp32_hint = n < 2;  // (split_conv_suits)
         rc = wdh_gemm(hU, hV, 0, hM, positions, cout, (int)tiles, c, (int64_t)cout * c, c, 1, (int64_t)c * tiles, tiles, 1,
                       0, 0, 1.0f, 1.0f, WDH_EPI_NONE, 0);
         g_tile_hint = -1;
