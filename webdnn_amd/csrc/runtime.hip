@@ -15,12 +15,16 @@
 #include <utility>
 #include <vector>
 
+#if defined(__SSE2__) && !defined(__HIP_DEVICE_COMPILE__)
+#include <emmintrin.h>
+#endif
+
 #include "common.h"
 
 namespace {
 
 constexpr size_t kStagingBytes = 32u << 20;  // per pinned buffer, two of them
-// Uploads go through the staging buffers in pieces of kUploadPiece, each with an event of its
+// Uploads go through the staging buffers in pieces of up to kUploadPiece, each with an event of its
 // own, so that the host's copy of piece i+1 into pinned memory overlaps the DMA of piece i.
 constexpr size_t kUploadPiece = 4u << 20;
 constexpr int kUploadSlots = (int)(2 * kStagingBytes / kUploadPiece);
@@ -482,6 +486,36 @@ int wdh_free(wdh_buf h) {
     }                                                                             \
   } while (0)
 
+// The host's copies between the caller's memory and pinned memory, which bound a transfer once DMA and copy overlap (DMA
+// 55 GB/s).  From a megabyte on the stores go past the caches: a plain copy reads every line of its target first, and the
+// data is on its way elsewhere (12.6 MB into pinned memory 221 to 468 us / 166, out of it behind a DMA 374 to 492 / 278 to 314;
+// 512 KB 9 to 21 / 16 to 23).
+static void copy_through(void *to, const void *from, size_t bytes, size_t whole) {
+#if defined(__SSE2__) && !defined(__HIP_DEVICE_COMPILE__)
+  if (whole >= (1u << 20)) {
+    char *d = (char *)to;
+    const char *s = (const char *)from;
+    const size_t head = (64 - ((uintptr_t)d & 63)) & 63;
+    if (bytes > head + 64) {
+      memcpy(d, s, head);
+      size_t i = head;
+      for (; i + 64 <= bytes; i += 64) {
+        const __m128i a = _mm_loadu_si128((const __m128i *)(s + i)), b = _mm_loadu_si128((const __m128i *)(s + i + 16)),
+                      c = _mm_loadu_si128((const __m128i *)(s + i + 32)), e = _mm_loadu_si128((const __m128i *)(s + i + 48));
+        _mm_stream_si128((__m128i *)(d + i), a);
+        _mm_stream_si128((__m128i *)(d + i + 16), b);
+        _mm_stream_si128((__m128i *)(d + i + 32), c);
+        _mm_stream_si128((__m128i *)(d + i + 48), e);
+      }
+      memcpy(d + i, s + i, bytes - i);
+      _mm_sfence();  // (before anybody, the DMA engine among them, is told that the data is there)
+      return;
+    }
+  }
+#endif
+  memcpy(to, from, bytes);
+}
+
 // Blocks until no upload piece is still on its way out of the staging buffers.
 static int wait_for_uploads() {
   for (int i = 0; i < kUploadSlots; i++)
@@ -489,6 +523,7 @@ static int wait_for_uploads() {
       WDH_HIP_CHECK(hipEventSynchronize(g.up_done[i]));
       g.up_busy[i] = false;
     }
+  g.up_next = 0;  // (the next upload finds staging memory that is still in the host's caches)
   return WDH_OK;
 }
 
@@ -636,8 +671,11 @@ int wdh_write(wdh_buf h, size_t dst_offset, const void *src, size_t bytes) {
   wdh::conv_forget_weights(h);
   const char *s = (const char *)src;
   size_t done = 0;
+  // (a short first piece lets the DMA begin early; beyond it each piece costs a gap of about ten microseconds between transfers)
+  size_t grow = bytes <= (2u << 20) ? kUploadPiece : 1u << 20;
   while (done < bytes) {
-    const size_t chunk = bytes - done < kUploadPiece ? bytes - done : kUploadPiece;
+    const size_t chunk = bytes - done < grow ? bytes - done : grow;
+    if (grow < kUploadPiece) grow *= 2;
     const int slot = g.up_next;
     g.up_next = (g.up_next + 1) % kUploadSlots;
     if (g.up_busy[slot]) {
@@ -646,7 +684,7 @@ int wdh_write(wdh_buf h, size_t dst_offset, const void *src, size_t bytes) {
     }
     const size_t per_buffer = kStagingBytes / kUploadPiece;
     char *piece = (char *)g.stage[slot / per_buffer] + (slot % per_buffer) * kUploadPiece;
-    memcpy(piece, s + done, chunk);
+    copy_through(piece, s + done, chunk, bytes);
     WDH_HIP_CHECK(hipMemcpyAsync(dst + dst_offset + done, piece, chunk, hipMemcpyHostToDevice, g.stream));
     WDH_HIP_CHECK(hipEventRecord(g.up_done[slot], g.stream));
     g.up_busy[slot] = true;
@@ -671,12 +709,13 @@ int wdh_read(wdh_buf h, size_t src_offset, void *dst, size_t bytes) {
   char *d = (char *)dst;
   // Short pieces through the staging memory of the uploads, all free by now, kReadAhead of them in flight: a piece is
   // copied out of pinned memory while the next ones arrive, and a slot is asked for again only after that.
-  // (12.6 MB, the results of an [8, 512, 768] block: the whole host-to-host pass 1476 -> 1296 us; one piece of up to
-  // 32 MB, as before, leaves the copy into cold user memory no transfer to overlap with.)  Beyond 64 pieces they grow:
+  // (12.6 MB, the results of an [8, 512, 768] block: one piece of up to 32 MB leaves the copy into cold user memory no
+  // transfer to overlap with.)  From 8 MiB on pieces of 2 MiB, whose gaps between transfers count less: the whole
+  // host-to-host pass of that block 954 us in pieces of 1 MiB, 924 of 2, 963 of 4.  Beyond 64 pieces they grow:
   // each costs a few microseconds of calls beside its copy (512 MB 19.3 ms in pieces of 32 MB, 20.5 in 512 of 1 MiB, 19.0 in
   // 64 of 8 MiB; 128 MB 5.3, 5.0 and 4.9).
   if (!bytes) WDH_HIP_CHECK(hipStreamSynchronize(g.stream));
-  size_t piece = kReadPiece;
+  size_t piece = bytes >= 8 * kReadPiece ? 2 * kReadPiece : kReadPiece;
   while (piece < kReadPieceMax && bytes / piece > 64) piece *= 2;
   auto length = [&](size_t at) { return bytes - at < piece ? bytes - at : piece; };
   auto read_slot = [&](int slot) { return (char *)g.stage[0] + slot * piece; };
@@ -690,7 +729,7 @@ int wdh_read(wdh_buf h, size_t src_offset, void *dst, size_t bytes) {
     }
     const int slot = (int)(copied / piece % kReadAhead);
     WDH_HIP_CHECK(hipEventSynchronize(g.up_done[slot]));
-    memcpy(d + copied, read_slot(slot), length(copied));
+    copy_through(d + copied, read_slot(slot), length(copied), bytes);
   }
   g.lane_dirty[g.lane] = false;     // (the stream has drained up to the data just read)
   return wdh::contraction_check();
