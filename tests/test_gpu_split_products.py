@@ -178,7 +178,7 @@ def test_one_image_keeps_its_bits(ctx, split):
 def test_a_geometry_first_met_while_recording(ctx, split):
     """The gathered form needs a tap table, which cannot be built then: the form that reads an LDS tile serves."""
     rng = np.random.default_rng(6)
-    x, wt = ctx.move_tensor(rng.standard_normal((2, 64, 20, 24)).astype(np.float32)), ctx.move_tensor(rng.standard_normal((64, 64, 3, 3)).astype(np.float32))
+    x, wt = ctx.move_tensor(rng.standard_normal((2, 72, 20, 24)).astype(np.float32)), ctx.move_tensor(rng.standard_normal((64, 72, 3, 3)).astype(np.float32))
     ctx.sync()
     ctx.graph_begin()
     y = H.conv(ctx, x, wt, pads=[1] * 4)
@@ -193,3 +193,71 @@ def test_a_geometry_first_met_while_recording(ctx, split):
         assert np.abs(got - want.get_data()).max() <= 1e-5 * np.abs(got).max()
         want.dispose()
     ctx.graph_destroy(graph)
+
+
+ROWS = [
+    # n, c, h, w, cout, pads: ragged tiles and channels, tiles over several images, unequal and wide pads, wide rows
+    (2, 16, 8, 9, 64, [1, 1, 1, 1]),
+    (3, 64, 15, 13, 70, [1, 1, 1, 1]),
+    (9, 48, 5, 5, 130, [1, 1, 1, 1]),
+    (2, 32, 11, 7, 64, [0, 0, 0, 0]),
+    (3, 80, 10, 12, 128, [2, 0, 1, 2]),
+    (2, 32, 6, 78, 64, [1, 1, 1, 1]),
+    (20, 16, 3, 3, 64, [1, 1, 1, 1]),
+]
+
+
+@pytest.mark.parametrize("mode,chunks", [(3, 1), (4, 1), (4, 2), (2, -1)])
+@pytest.mark.parametrize("shape", ROWS)
+def test_rows_of_3x3_convs(ctx, split, mode, chunks, shape):
+    """Input rows in LDS, weights laid out in parts; kept per buffer when the caller vouches for them, until it is written to."""
+    n, c, h, w, cout, pads = shape
+    rng = np.random.default_rng(sum(shape[:5]))
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt, bias = rng.standard_normal((cout, c, 3, 3)).astype(np.float32), rng.standard_normal(cout).astype(np.float32)
+    tx, tw, tb = (ctx.move_tensor(v) for v in (x, wt, bias))
+    ctx.set_option("conv3x3_winograd", 0)
+    split(0)
+    plain = H.conv(ctx, tx, tw, tb, pads=pads)
+    r = rng.standard_normal(plain.dims).astype(np.float32)
+    tr = ctx.move_tensor(r)
+    want = np.maximum(plain.get_data().astype(np.float64) + r, 0)
+    bound = 2 * (9 * c + 8) * 2.0 ** -24 * (H.conv(ctx, *(ctx.move_tensor(np.abs(v)) for v in (x, wt, bias)), pads=pads).get_data() + np.abs(r))
+    split(mode)
+    ctx.set_option("split_k", chunks)
+    for constant in (False, True, True):
+        got = H.conv(ctx, tx, tw, tb, pads=pads, epilogue="relu", residual=tr, constant_weights=constant)
+        plan = ctx.last_plan()
+        assert plan["form"] == "conv 3x3, LDS tile" and plan["tile"] in ("128x128", "64x128"), plan
+        assert (np.abs(got.get_data() - want) <= bound).all()
+    tw.set_data(2 * wt)
+    again = H.conv(ctx, tx, tw, None, pads=pads, constant_weights=True).get_data()
+    assert (np.abs(again - 2 * (plain.get_data().astype(np.float64) - bias.reshape(1, -1, 1, 1))) <= 4 * bound + 1e-5).all()
+    x[0, c - 1, h // 2, w // 2], x[n - 1, 0, 0, 0] = np.inf, np.nan
+    tx.set_data(x)
+    out = {}
+    for value in (0, mode):
+        split(value)
+        out[value] = H.conv(ctx, tx, tw, tb, pads=pads).get_data()
+    assert (np.isnan(out[0]) == np.isnan(out[mode])).all() and (np.isinf(out[0]) == np.isinf(out[mode])).all()
+
+
+def test_rows_while_recording(ctx, split):
+    """Weights laid out while a graph is recorded belong to it; those kept from before are used by it."""
+    rng = np.random.default_rng(8)
+    x, wt = ctx.move_tensor(rng.standard_normal((4, 64, 20, 24)).astype(np.float32)), ctx.move_tensor(rng.standard_normal((64, 64, 3, 3)).astype(np.float32))
+    want = H.conv(ctx, x, wt, pads=[1] * 4).get_data()
+    for warm in (False, True):
+        if warm:
+            H.conv(ctx, x, wt, pads=[1] * 4, constant_weights=True).dispose()
+        ctx.sync()
+        ctx.graph_begin()
+        y = H.conv(ctx, x, wt, pads=[1] * 4, constant_weights=True)
+        graph = ctx.graph_end()
+        for _ in range(3):
+            ctx.graph_launch(graph)
+            assert (y.get_data() == want).all()
+            other = H.conv(ctx, x, wt, pads=[1] * 4)
+            assert (other.get_data() == want).all()
+            other.dispose()
+        ctx.graph_destroy(graph)

@@ -1954,5 +1954,10 @@ struct SplitPlan {
 };
 int launch_split_gemm(bool b_kc, const SplitPlan &s, Params &p, int nz);    // split_gemm.hip
 int launch_split_conv(int mode, const SplitPlan &s, Params &p, int nz);     // split_conv.hip
+// 3x3 convs of a batch read straight from the input (conv3x3_split.hip); `packed`: what pack3x3_launch made of the weights
+bool conv3x3_split_fits(ConvGeom &cv, int bn, int images, int pr);
+size_t packed3x3_bytes(int cout, int c);
+int pack3x3_launch(const float *W, void *P, int cout, int c);
+int launch_conv3x3_split(Params &p, const SplitPlan &s, const void *packed);
 
 }  // namespace wdhc

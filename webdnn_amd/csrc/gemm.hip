@@ -367,26 +367,28 @@ static bool tiles_beat_wavesplit(int batch, int m, int n, int k, bool b_kc, bool
 // `fixed` is a launch with one empty workgroup a CU (prologue, epilogue); a cut adds the pass over the partial sums, which
 // are written and read once.  Fitted to 21 products of 33x4096x4096 to 4096x4096x4096 on every tile in 1 to 12 cuts and to
 // 40 convs (the form it picks takes at most 11 % longer than the best one).
-enum SplitSource { SPLIT_GEMM, SPLIT_PIXELS, SPLIT_TAPS };  // where B comes from: a matrix, X in place, gathered taps
+enum SplitSource { SPLIT_GEMM, SPLIT_PIXELS, SPLIT_TAPS, SPLIT_ROWS };  // where B comes from: a matrix, X in place, gathered taps, rows of X in LDS
 static SplitPlan search_split(int nz, int m, int n, int k, SplitSource source, bool large_tiles) {
   struct Model { int bm, bn; double slab, solo, fixed; };
-  static const Model models[3][5] = {
+  static const Model models[4][5] = {
       {{128, 128, 0.63, 0.56, 9.5}, {64, 128, 0.37, 0.39, 6.5}, {128, 64, 0.37, 0.39, 6.5}, {64, 64, 0.21, 0.29, 5.2}, {256, 128, 1.20, 0.95, 10.0}},
       {{128, 128, 0.63, 0.60, 9.5}, {64, 128, 0.38, 0.42, 6.5}, {128, 64, 0.37, 0.42, 6.5}, {64, 64, 0.21, 0.36, 5.2}, {0, 0, 0, 0, 0}},
       // (gathered taps: two more vector instructions an element, and a slab's loads wait for its part of the tap table)
-      {{128, 128, 0.66, 0.80, 9.5}, {64, 128, 0.43, 0.60, 6.5}, {128, 64, 0.39, 0.50, 6.5}, {64, 64, 0.24, 0.36, 5.2}, {0, 0, 0, 0, 0}}};
+      {{128, 128, 0.66, 0.80, 9.5}, {64, 128, 0.43, 0.60, 6.5}, {128, 64, 0.39, 0.50, 6.5}, {64, 64, 0.24, 0.36, 5.2}, {0, 0, 0, 0, 0}},
+      {{128, 128, 0.66, 0.62, 11.0}, {64, 128, 0.35, 0.40, 8.0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}}};
   const long long cus = wdh::compute_units();
+  const int unit = source == SPLIT_ROWS ? 9 : 1;  // a chunk is a whole number of these, in slabs
   const int slabs = (k + BK - 1) / BK;
   SplitPlan best = {-1, {}, 1e30};
   for (int t = 0; t <= S256x128; t++) {
     const Model &mo = models[source][t];
     if (mo.bm == 0 || (large_tiles && t == S64x64) || (g_split >= 3 && t != g_split - 3)) continue;
     const long long tiles = (long long)((m + mo.bm - 1) / mo.bm) * ((n + mo.bn - 1) / mo.bn) * nz;
-    const int most = g_forced_split >= 1 ? (g_forced_split < slabs ? g_forced_split : slabs)
+    const int most = g_forced_split >= 1 && slabs > 0 ? (g_forced_split < slabs ? g_forced_split : slabs)
                                          : slabs / 4 < 32 ? slabs / 4 : 32;  // at least 64 elements of K per chunk
     for (int s = 1; s == 1 || s <= most; s++) {
       if (g_forced_split >= 1 && s != most) continue;
-      const int per = (slabs + s - 1) / s;
+      const int per = ((slabs + s - 1) / s + unit - 1) / unit * unit;
       const int chunks = (slabs + per - 1) / per;
       if (chunks != s && g_forced_split < 1) continue;
       // the whole launch cut s ways, or only the tiles beyond the last full round
@@ -1070,20 +1072,30 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   // g_winograd: 0 never; 1 = F(2x2, 3x3) from 128 channels on (F(4x4, 3x3) from g_winograd4_channels on, when
   // that is set: faster from 64 channels on, but its rounding errors are about ten times the direct form's,
   // which a 50-layer network's logits show); 2 / 3 = F(2x2, 3x3) / F(4x4, 3x3) wherever legal.
-  // (transform-domain tensors that outgrow the 256 MB last-level cache cost more than the multiplications saved once the
-  // direct form runs on the bf16 matrix cores: 128 images 128 -> 128 on 28x28, V and M 206 MB each, 254 us against 193;
-  // 256 -> 256 on 14x14, 103 MB each, 149 against 194)
-  bool wino_memory = true;  // there was room for the transform-domain tensors, if they were wanted
-  auto wino_outgrown = [&]() {
-    return g_winograd == 1 && gather_split && 64LL * (c + cout) * wdh::wino_tiles(2, n, oh, ow) > (256LL << 20);
-  };
   const int wino_min = c < cout ? c : cout;
+  auto rows_possible = [&]() {
+    if (!(g_halo && kh == 3 && kw == 3 && sh == 1 && sw == 1 && dh == 1 && dw == 1 && group == 1 && c % 16 == 0)) return false;
+    if (!split_possible(n, cout, (int)kdim) || packed3x3_bytes(cout, c) >= 0x7fffffffULL || g_split > 4) return false;
+    p.cv.h = h; p.cv.w = w; p.cv.oh = oh; p.cv.ow = ow; p.cv.pt = pt; p.cv.pl = pl;
+    return conv3x3_split_fits(p.cv, 128, n, pr);
+  };
+  const bool rows_split = rows_possible();
+  bool wino_memory = true;  // there was room for the transform-domain tensors, if they were wanted
+  // Where the direct forms on the bf16 matrix cores are the faster ones after all: below 256 channels rows read straight from X
+  // do not pay for transforms (us, transforms / rows: 32 images 128 -> 128 on 28x28 61 / 52, 12 on 34x39 45 / 36, 5 on 24x32 21 / 18;
+  // small planes stay: 20 us either way), and transform-domain tensors that outgrow the 256 MB last-level cache
+  // cost more than the multiplications saved (128 images of it, V and M 206 MB each, 254 / 150).  From 256 channels on the
+  // multiplications count: 32 images 256 -> 256 on 14x14 46 / 61, 512 -> 512 on 7x7 47 / 61.
+  auto direct_suits = [&]() {
+    if (g_winograd != 1 || !(gather_split || rows_split)) return false;
+    return (rows_split && wino_min < 256 && npix >= 3500) || 64LL * (c + cout) * wdh::wino_tiles(2, n, oh, ow) > (256LL << 20);
+  };
   int wino_r = 0;
   if (g_winograd == 2) wino_r = 2;
   else if (g_winograd == 3) wino_r = 4;
   else if (g_winograd == 1) wino_r = g_winograd4_channels && wino_min >= g_winograd4_channels ? 4 : wino_min >= 128 ? 2 : 0;
   if (wino_r && kh == 3 && kw == 3 && sh == 1 && sw == 1 && dh == 1 && dw == 1 && group == 1 && c % BK == 0 &&
-      g_forced_tile < 0 && g_forced_split < 0 && !(wino_r == 2 && wino_outgrown())) {
+      g_forced_tile < 0 && g_forced_split < 0 && !(wino_r == 2 && direct_suits())) {
     const int r = wino_r, positions = (r + 2) * (r + 2);
     const long long tiles = wdh::wino_pitch(wdh::wino_tiles(r, n, oh, ow));  // (row length of V and M)
     const size_t u_bytes = (size_t)positions * cout * c * 4, v_bytes = (size_t)positions * c * tiles * 4,
@@ -1150,6 +1162,47 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
     }
   }
 direct_forms:
+  // 3x3, stride 1 of a batch: rows of X in LDS, split once, against weights that are laid out in parts (conv3x3_split.hip)
+  if (rows_split) {
+    wdh_buf hP = 0;
+    bool kept = false, ready = false;
+    if (flags & WDH_CONV_CONSTANT_WEIGHTS) {
+      auto it = g_filters.find(hW);
+      if (it != g_filters.end() && it->second.cout == cout && it->second.c == c && it->second.r == 0) {
+        hP = it->second.u;
+        kept = ready = true;
+      } else if (!wdh::capturing()) {
+        wdh::conv_forget_weights(hW);
+        hP = wdh_alloc(packed3x3_bytes(cout, c));
+        if (hP) {
+          g_filters[hW] = FilterEntry{hP, cout, c, 0};
+          kept = true;
+        }
+      }
+    }
+    if (!hP) hP = wdh_alloc(packed3x3_bytes(cout, c));
+    if (hP) {
+      p.m = cout_g; p.n = (int)npix; p.k = (int)kdim;
+      p.sAb = 0; p.sA0 = kdim; p.sA1 = 1;
+      p.alpha = 1.0f; p.beta = 1.0f; p.epilogue = epilogue;
+      p.cv.c_in_g = c; p.cv.sh = p.cv.sw = p.cv.dh = p.cv.dw = 1; p.cv.kh = p.cv.kw = 3;
+      p.cv.c_total = c; p.cv.cout_total = cout; p.cv.cout_g = cout;
+      p.cv.ntaps = 9; p.cv.npix = npix;
+      p.fast = 1;
+      p.b_bytes = (int)((long long)n * c * h * w * 4);
+      p.y_bytes = g_descriptors && out_bytes < 0x7fffffffULL ? (int)out_bytes : 0;
+      p.c_bytes = cout * 4;
+      set_wide(p, true);
+      void *const packed = wdh::resolve(hP, nullptr);
+      int rc = ready ? WDH_OK : pack3x3_launch(p.A, packed, cout, c);
+      if (rc == WDH_OK)
+        rc = run_split(plan_split(1, p.m, p.n, p.k, SPLIT_ROWS), [&](const SplitPlan &q) { return launch_conv3x3_split(p, q, packed); });
+      if (rc != WDH_OK && kept && !ready) wdh::conv_forget_weights(hW);  // (may not have been filled)
+      if (!kept) (void)wdh_free(hP);
+      return rc;
+    }
+    wdh::clear_error();  // (no room for them: the forms below need none)
+  }
   // 3x3, stride 1, no dilation, input channels in blocks of 8: taps read from an input
   // tile staged in LDS (conv3x3_halo_kernel)
   // (a batch's with enough output channels gather their taps for the bf16 matrix cores instead: split_conv_suits)

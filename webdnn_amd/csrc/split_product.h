@@ -49,6 +49,12 @@ __device__ __forceinline__ SplitPair split_pair(float x0, float x1) {
   return SplitPair{h, m, nearest_pair(s0, s1)};
 }
 
+// Whether a tile holds a sum that the split cannot vouch for, from the largest and the least (zeros aside) of the doubled
+// bits of its sums: not finite, or nonzero below 2^-100.
+__device__ __forceinline__ bool split_fails(unsigned most, unsigned least) {
+  return most >= 0xff000000u || least < ((127u - 100u) << 24) - 1u;
+}
+
 // Workgroups a CU holds: the accumulators are two per result, so 128x128 tiles take 64 + 64 registers of
 // accumulators and two of them fit; 256x128 is the same wavefront with eight of them in one workgroup.
 constexpr int split_blocks(int bm, int bn) { return bm * bn >= 128 * 128 ? 2 : (bm * bn > 64 * 64 ? 3 : 4); }
@@ -325,8 +331,7 @@ __global__ __launch_bounds__(WM * WN * 64, split_blocks(BM, BN)) void split_kern
         most = u > most ? u : most;
         least = u - 1u < least ? u - 1u : least;
       }
-  const bool odd = most >= 0xff000000u || least < ((127u - 100u) << 24) - 1u;
-  if (__syncthreads_or(odd)) {
+  if (__syncthreads_or(split_fails(most, least))) {
     // Operands straight from memory, one element a lane and k; never the common case.
     const float *pa[MT];
     int cb[NT];
