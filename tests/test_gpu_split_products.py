@@ -7,7 +7,7 @@ from webdnn_amd import hostops as H
 
 pytestmark = pytest.mark.gpu
 
-TILES = {3: "128x128", 4: "64x128", 5: "128x64", 6: "64x64", 7: "256x128"}
+TILES = {3: "128x128", 4: "64x128", 5: "128x64", 6: "64x64", 7: "256x128", 8: "64x64", 9: "64x64"}
 
 
 @pytest.fixture
@@ -86,7 +86,7 @@ def test_errors_are_no_larger_than_the_fp32_instructions(ctx, split, k, positive
     assert abs(drift) <= 2.0 ** -26, drift
 
 
-@pytest.mark.parametrize("mode", [3, 6])
+@pytest.mark.parametrize("mode", [3, 6, 8, 9])
 @pytest.mark.parametrize("transposed", [False, True])
 def test_values_the_split_cannot_hold(ctx, split, mode, transposed):
     """Inf and NaN, the largest floats, sums that overflow, subnormals: as with the fp32 instruction."""
@@ -133,7 +133,7 @@ CONVS = [
 ]
 
 
-@pytest.mark.parametrize("mode", [3, 4, 5, 6])
+@pytest.mark.parametrize("mode", [3, 4, 5, 6, 8, 9])
 @pytest.mark.parametrize("shape", CONVS)
 def test_convs(ctx, split, mode, shape):
     n, cin, h, w, cout, kernel, stride, pad, dil, group = shape
@@ -261,3 +261,24 @@ def test_rows_while_recording(ctx, split):
             assert (other.get_data() == want).all()
             other.dispose()
         ctx.graph_destroy(graph)
+
+
+def test_groups_that_fill_the_chip(ctx, split):
+    """The projections of an attention block as one launch of 64x64 tiles; ragged rows and columns, one weight k-contiguous by shape."""
+    rng = np.random.default_rng(9)
+    for t, d, n in ((384, 768, 768), (509, 512, 516), (256, 768, 772)):
+        x = rng.standard_normal((t, d)).astype(np.float32)
+        x[t - 1, 5] = np.inf if n == 772 else 1.0
+        ws = [(rng.standard_normal((d, n)).astype(np.float32), rng.standard_normal(n).astype(np.float32)) for _ in range(3)]
+        tx = ctx.move_tensor(x)
+        args = [(tx, ctx.move_tensor(w), ctx.move_tensor(b)) for w, b in ws]
+        out = {}
+        for value in (0, 1):
+            split(value)
+            out[value] = [y.get_data() for y in H.linear_group(ctx, args)]
+            assert ctx.last_plan()["tile"] == ("64x64" if value else "32x32"), ctx.last_plan()
+        rows = slice(0, t - 1)
+        for (w, b), y0, y1 in zip(ws, out[0], out[1]):
+            a64, w64 = x[rows].astype(np.float64), w.astype(np.float64)
+            assert within(y1[rows], a64 @ w64 + b, np.abs(a64) @ np.abs(w64) + np.abs(b), d)
+            assert (np.isfinite(y0) == np.isfinite(y1)).all()

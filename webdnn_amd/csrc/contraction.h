@@ -243,9 +243,8 @@ struct TileWork {
   bool whole;
   int lin, chunk, bz, tm, tn;
 };
-__device__ __forceinline__ TileWork decode_work(const Params &p) {
+__device__ __forceinline__ TileWork decode_work(const Params &p, int pid) {
   TileWork t;
-  const int pid = blockIdx.x;
   t.whole = pid < p.full_tiles;
   t.chunk = 0;
   if (t.whole) {
@@ -1095,7 +1094,7 @@ __global__ __launch_bounds__(NTHREADS, STREAM ? stream_blocks(BM, BN) : min_bloc
       c.bz = fdiv(c.lin, p.fd_tiles_per_z);
       tile_coords(p, c.lin - c.bz * (p.tiles_m * p.tiles_n), &tm, &tn);
     } else {
-      const TileWork tw = decode_work(p);
+      const TileWork tw = decode_work(p, (int)blockIdx.x);
       c.whole = tw.whole;
       c.first = c.last = true;
       c.tile_begin = 0;
@@ -1413,7 +1412,7 @@ __global__ __launch_bounds__(NTHREADS, halo_blocks(BM, BN)) void conv3x3_halo_ke
       c.kbeg = sg.sbeg * HALO_KB;
       c.kend = sg.send * HALO_KB < p.k ? sg.send * HALO_KB : p.k;
     } else {
-      t = decode_work(p);
+      t = decode_work(p, (int)blockIdx.x);
       c.first = c.last = true;
       c.tile_begin = 0;
       c.kbeg = t.whole ? 0 : t.chunk * p.kchunk;
@@ -1946,13 +1945,15 @@ int launch_conv_gather(int mode, Params &p, int nz, bool vec);    // contraction
 int launch_conv_pixels(Params &p, int nz, bool vec, bool stride2);  // contraction_conv_pixels.hip
 int launch_conv3x3(int tile, Params &p, int nz, int vecw);        // contraction_conv3x3.hip
 // The same products on the bf16 matrix cores (split_product.h); A k-contiguous, descriptors, 16-byte pieces, k % 4 == 0.
-enum SplitTile { S128x128 = 0, S64x128 = 1, S128x64 = 2, S64x64 = 3, S256x128 = 4 };
+enum SplitTile { S128x128 = 0, S64x128 = 1, S128x64 = 2, S64x64 = 3, S256x128 = 4,
+                 S64x64K2 = 5, S64x64K4 = 6 };  // (two, four groups of wavefronts share the K of a tile)
 struct SplitPlan {
   int tile;       // SplitTile, or -1: not a product for them
   WorkPlan work;
   double us;      // estimate
 };
 int launch_split_gemm(bool b_kc, const SplitPlan &s, Params &p, int nz);    // split_gemm.hip
+int launch_split_group(bool b_kc, int count, Params *p);                     // split_gemm.hip: whole 64x64 tiles, batch 1
 int launch_split_conv(int mode, const SplitPlan &s, Params &p, int nz);     // split_conv.hip
 // 3x3 convs of a batch read straight from the input (conv3x3_split.hip); `packed`: what pack3x3_launch made of the weights
 bool conv3x3_split_fits(ConvGeom &cv, int bn, int images, int pr);

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
   const ConvGeom &cv = p.cv;
   const int plane_in = cv.h * cv.w;
 
-  const TileWork tw = decode_work(p);
+  const TileWork tw = decode_work(p, (int)blockIdx.x);
   const int row0 = tw.tm * BM, col0 = tw.tn * BN;
   const int kbeg = tw.whole ? 0 : tw.chunk * p.kchunk;
   const int kend = tw.whole ? p.k : (kbeg + p.kchunk < p.k ? kbeg + p.kchunk : p.k);

@@ -370,19 +370,19 @@ static bool tiles_beat_wavesplit(int batch, int m, int n, int k, bool b_kc, bool
 enum SplitSource { SPLIT_GEMM, SPLIT_PIXELS, SPLIT_TAPS, SPLIT_ROWS };  // where B comes from: a matrix, X in place, gathered taps, rows of X in LDS
 static SplitPlan search_split(int nz, int m, int n, int k, SplitSource source, bool large_tiles) {
   struct Model { int bm, bn; double slab, solo, fixed; };
-  static const Model models[4][5] = {
-      {{128, 128, 0.63, 0.56, 9.5}, {64, 128, 0.37, 0.39, 6.5}, {128, 64, 0.37, 0.39, 6.5}, {64, 64, 0.21, 0.29, 5.2}, {256, 128, 1.20, 0.95, 10.0}},
-      {{128, 128, 0.63, 0.60, 9.5}, {64, 128, 0.38, 0.42, 6.5}, {128, 64, 0.37, 0.42, 6.5}, {64, 64, 0.21, 0.36, 5.2}, {0, 0, 0, 0, 0}},
+  static const Model models[4][7] = {
+      {{128, 128, 0.63, 0.56, 9.5}, {64, 128, 0.37, 0.39, 6.5}, {128, 64, 0.37, 0.39, 6.5}, {64, 64, 0.21, 0.29, 5.2}, {256, 128, 1.20, 0.95, 10.0}, {64, 64, 0.21, 0.20, 5.7}, {64, 64, 0.25, 0.16, 6.2}},
+      {{128, 128, 0.63, 0.60, 9.5}, {64, 128, 0.38, 0.42, 6.5}, {128, 64, 0.37, 0.42, 6.5}, {64, 64, 0.21, 0.36, 5.2}, {0, 0, 0, 0, 0}, {64, 64, 0.21, 0.22, 5.7}, {64, 64, 0.25, 0.18, 6.2}},
       // (gathered taps: two more vector instructions an element, and a slab's loads wait for its part of the tap table)
-      {{128, 128, 0.66, 0.80, 9.5}, {64, 128, 0.43, 0.60, 6.5}, {128, 64, 0.39, 0.50, 6.5}, {64, 64, 0.24, 0.36, 5.2}, {0, 0, 0, 0, 0}},
-      {{128, 128, 0.66, 0.62, 11.0}, {64, 128, 0.35, 0.40, 8.0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}}};
+      {{128, 128, 0.66, 0.80, 9.5}, {64, 128, 0.43, 0.60, 6.5}, {128, 64, 0.39, 0.50, 6.5}, {64, 64, 0.24, 0.36, 5.2}, {0, 0, 0, 0, 0}, {64, 64, 0.24, 0.25, 5.7}, {64, 64, 0.28, 0.20, 6.2}},
+      {{128, 128, 0.66, 0.90, 11.0}, {64, 128, 0.35, 0.40, 8.0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}}};
   const long long cus = wdh::compute_units();
   const int unit = source == SPLIT_ROWS ? 9 : 1;  // a chunk is a whole number of these, in slabs
   const int slabs = (k + BK - 1) / BK;
   SplitPlan best = {-1, {}, 1e30};
-  for (int t = 0; t <= S256x128; t++) {
+  for (int t = 0; t <= S64x64K4; t++) {
     const Model &mo = models[source][t];
-    if (mo.bm == 0 || (large_tiles && t == S64x64) || (g_split >= 3 && t != g_split - 3)) continue;
+    if (mo.bm == 0 || (large_tiles && mo.bm * mo.bn == 64 * 64) || (g_split >= 3 && t != g_split - 3)) continue;
     const long long tiles = (long long)((m + mo.bm - 1) / mo.bm) * ((n + mo.bn - 1) / mo.bn) * nz;
     const int most = g_forced_split >= 1 && slabs > 0 ? (g_forced_split < slabs ? g_forced_split : slabs)
                                          : slabs / 4 < 32 ? slabs / 4 : 32;  // at least 64 elements of K per chunk
@@ -441,8 +441,9 @@ static SplitPlan split_gemm_plan(int batch, int m, int n, int k, bool b_kc) {
       return {S64x64, {0, (long long)((m + 63) / 64) * ((n + 63) / 64) * batch, (slabs + per - 1) / per, per * BK}, 0.0};
     }
     const long long blocks32 = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch, cus = wdh::compute_units();
-    const SplitPlan s = plan_split(batch, m, n, k, SPLIT_GEMM, true);
-    return s.us < 0.9 * (3.0 + 0.0078 * (double)((blocks32 + cus - 1) / cus) * k) ? s : none;
+    // (below the lengths that tiles_beat_wavesplit looks at the tile is free)
+    const SplitPlan s = plan_split(batch, m, n, k, SPLIT_GEMM, k >= 2000);
+    return s.us < 0.85 * (3.0 + 0.0078 * (double)((blocks32 + cus - 1) / cus) * k) ? s : none;
   }
   return (double)batch * m * n * k >= 1e8 ? plan_split(batch, m, n, k, SPLIT_GEMM) : none;
 }
@@ -510,7 +511,7 @@ extern "C" int wdh_set_option(const char *name, int value) {
     return WDH_OK;
   }
   if (strcmp(name, "split_products") == 0) {
-    if (value < 0 || value > 3 + S256x128) return fail(WDH_EINVAL, "wdh_set_option: split_products %d (use 0..%d)", value, 3 + S256x128);
+    if (value < 0 || value > 3 + S64x64K4) return fail(WDH_EINVAL, "wdh_set_option: split_products %d (use 0..%d)", value, 3 + S64x64K4);
     g_split = value;
     return WDH_OK;
   }
@@ -758,8 +759,37 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
 
 namespace {
 // Launches what wdh_linear_group queued: one launch per kernel variant and GROUP_MAX problems.
+// Problems queued for gemm_wavesplit_kernel that together fill the chip with 64x64 tiles, one a CU at most, whose K four
+// groups of wavefronts share (split_product.h): 32x32 blocks read every operand twice as often.  Three of 384x768x768 23.7 us as
+// blocks, 19.1 so; 512x512x512 17.3 / 14.5, 300x1024x1024 29.8 / 23.9, 256x768x768 19.0 / 17.5; 850x256x256 (8.2) and 200x768x768
+// (13.8 / 13.7) stay.
+bool group_splits(int variant) {
+  if (!g_split || g_split > 1 || g_stream == 2 || !(variant & 1)) return false;
+  long long tiles = 0, blocks = 0;
+  int count = 0, k = 0;
+  for (int i = 0; i < g_group.count; i++) {
+    if (g_group.variant[i] != variant) continue;
+    const Params &p = g_group.p[i];
+    if (!split_legal(p, true) || (k && p.k != k)) return false;
+    k = p.k;
+    count++;
+    tiles += (long long)((p.m + 63) / 64) * ((p.n + 63) / 64);
+    blocks += g_group.blocks[i];
+  }
+  const long long cus = wdh::compute_units();
+  return count > 1 && count <= GROUP_MAX && tiles <= cus &&
+         6.2 + 0.16 * ((k + BK - 1) / BK) < 0.9 * (3.0 + 0.0065 * (double)((blocks + cus - 1) / cus) * k);
+}
 int flush_group() {
   for (int variant = 0; variant < 4; variant++) {
+    if (group_splits(variant)) {
+      Params problems[GROUP_MAX];
+      int count = 0;
+      for (int i = 0; i < g_group.count; i++)
+        if (g_group.variant[i] == variant) problems[count++] = g_group.p[i];
+      if (int rc = launch_split_group((variant & 2) != 0, count, problems)) return rc;
+      continue;
+    }
     GroupParams g;
     g.count = 0;
     long long blocks = 0;

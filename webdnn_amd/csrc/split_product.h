@@ -61,9 +61,15 @@ constexpr int split_blocks(int bm, int bn) { return bm * bn >= 128 * 128 ? 2 : (
 
 // LDS: three planes (h, m, l) per operand, each [k / 8][row or column][8 bf16], so that a fragment of a 32x16 block
 // is one 16-byte read per lane, 32 lanes side by side.
-template <int BM, int BN, int WM, int WN, int BMODE>
-__global__ __launch_bounds__(WM * WN * 64, split_blocks(BM, BN)) void split_kernel(Params p) {
-  constexpr int THREADS = WM * WN * 64;
+//
+// KG: groups of WM x WN wavefronts that share the K of a tile, each with LDS of its own; their sums meet in LDS, in
+// order.  A 64x64 tile by itself on a CU keeps one wavefront a SIMD, which issues its 110 instructions a slab one after
+// the other in 0.29 us, where the products alone take 0.08; two groups take 0.20 for a slab, four 0.16.  (us, one / two / four:
+// 384x2304x768 21.2 / 18.0 / 16.8, 1024^3 26.8 / 22.6 / 21.3, 8 images 512 -> 512 on 14x14 16.6 / 14.3 / 13.8; with two tiles a CU
+// there is nothing to gain, 850x2048x256 13.3 / 13.2 / 18.2.)
+template <int BM, int BN, int WM, int WN, int BMODE, int KG>
+__device__ __forceinline__ void split_tile(const Params &p, int pid) {
+  constexpr int THREADS = WM * WN * 64;  // of a group
   constexpr bool IM2COL = BMODE == B_IM2COL32 || BMODE == B_IM2COL64;
   constexpr bool PIX_ANY = BMODE == B_PIXELS_ANY;
   constexpr bool PIXELS = BMODE == B_PIXELS || PIX_ANY;
@@ -75,19 +81,25 @@ __global__ __launch_bounds__(WM * WN * 64, split_blocks(BM, BN)) void split_kern
   // different banks)
   constexpr int HALF_A = BM * 16 + 64, HALF_B = BN * 16 + 64, PLANE_A = 2 * HALF_A, PLANE_B = 2 * HALF_B;
   constexpr int BUF = 3 * (PLANE_A + PLANE_B);
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2][BUF];
+  __shared__ __attribute__((aligned(16))) unsigned char lds_all[KG][2][BUF];
   static_assert(2 * BUF >= WM * WN * STAGE_FLOATS * 4, "epilogue staging");
+  static_assert(KG == 1 || 2 * BUF >= BM * BN * 4, "partial sums");
 
-  const int tid = threadIdx.x;
+  const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / THREADS);
+  unsigned char(*const lds)[BUF] = lds_all[group];
+  const int tid = (int)threadIdx.x - group * THREADS;
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
   const int li = lane & 31, half = lane >> 5;
   const int wrow = wm * (MT * 32), wcol = wn * (NT * 32);
 
-  const TileWork tw = decode_work(p);
+  const TileWork tw = decode_work(p, pid);
   const int bz = tw.bz, row0 = tw.tm * BM, col0 = tw.tn * BN;
-  const int kbeg = tw.whole ? 0 : tw.chunk * p.kchunk;
-  const int kend = tw.whole ? p.k : (kbeg + p.kchunk < p.k ? kbeg + p.kchunk : p.k);
+  const int kfirst = tw.whole ? 0 : tw.chunk * p.kchunk;
+  const int klast = tw.whole ? p.k : (kfirst + p.kchunk < p.k ? kfirst + p.kchunk : p.k);
+  const int kshare = KG == 1 ? klast - kfirst : ((klast - kfirst + BK - 1) / BK + KG - 1) / KG * BK;
+  const int kbeg = kfirst + group * kshare;   // (a group may have less than the others, or nothing: zeros, then)
+  const int kend = KG == 1 || kbeg + kshare < klast ? kbeg + kshare : klast;
   const float *const A = p.A + (long long)bz * p.sAb;
   const float *const B = CONV ? p.B + (long long)bz * p.cv.c_in_g * p.cv.h * p.cv.w : p.B + (long long)bz * p.sBb;
   const int lda = (int)p.sA0, ldb = (int)(B_IS_KC ? p.sB1 : p.sB0);
@@ -276,7 +288,7 @@ __global__ __launch_bounds__(WM * WN * 64, split_blocks(BM, BN)) void split_kern
   };
 
   // Slab s+2 is requested, slab s+1 split and stored to the other LDS buffer, slab s multiplied: one barrier a slab.
-  const int nslabs = (kend - kbeg + BK - 1) / BK, nfull = (kend - kbeg) / BK;
+  const int nslabs = (kshare + BK - 1) / BK, nfull = kend > kbeg ? (kend - kbeg) / BK : 0;
   Slab next;
   read_taps(kbeg);
   fetch(kbeg, next, true);
@@ -305,7 +317,8 @@ __global__ __launch_bounds__(WM * WN * 64, split_blocks(BM, BN)) void split_kern
     __syncthreads();
   };
   int s = 0;
-  for (; s + 3 < nfull; s += 2) {
+  // (every group takes the barriers of the one that has most)
+  for (const int nall = KG == 1 ? nfull : (klast - kfirst - (KG - 1) * kshare) / BK; s + 3 < nall; s += 2) {
     step(s, 0);
     step(s + 1, 1);
   }
@@ -331,7 +344,33 @@ __global__ __launch_bounds__(WM * WN * 64, split_blocks(BM, BN)) void split_kern
         most = u > most ? u : most;
         least = u - 1u < least ? u - 1u : least;
       }
-  if (__syncthreads_or(split_fails(most, least))) {
+  const bool again = __syncthreads_or(split_fails(most, least));
+  if (KG > 1 && !again) {
+    // sums of the groups behind the first, in order; each through its own LDS
+    float *const mine = reinterpret_cast<float *>(&lds[0][0]);
+    if (group > 0) {
+#pragma unroll
+      for (int a = 0; a < MT; a++)
+#pragma unroll
+        for (int b = 0; b < NT; b++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) mine[((a * NT + b) * 16 + r) * THREADS + tid] = acc[a][b][r];
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int g = 1; g < KG; g++) {
+      const float *const other = reinterpret_cast<const float *>(&lds_all[g][0][0]);
+#pragma unroll
+      for (int a = 0; a < MT; a++)
+#pragma unroll
+        for (int b = 0; b < NT; b++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc[a][b][r] += other[((a * NT + b) * 16 + r) * THREADS + tid];
+    }
+  }
+  if (again) {
+    if (group > 0) return;  // (the first group does the whole K again)
     // Operands straight from memory, one element a lane and k; never the common case.
     const float *pa[MT];
     int cb[NT];
@@ -354,16 +393,16 @@ __global__ __launch_bounds__(WM * WN * 64, split_blocks(BM, BN)) void split_kern
       for (int b = 0; b < NT; b++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
-    for (int k0 = kbeg; k0 < kend; k0 += 2) {
+    for (int k0 = kfirst; k0 < klast; k0 += 2) {
       const int k = k0 + half;
-      const bool in = k < kend;
+      const bool in = k < klast;
       float ea[MT], eb[NT];
 #pragma unroll
       for (int mt = 0; mt < MT; mt++) ea[mt] = in ? pa[mt][k] : 0.0f;
 #pragma unroll
       for (int nt = 0; nt < NT; nt++) {
         if (IM2COL) {
-          const int2 e = p.cv.ktab[in ? k : kbeg];
+          const int2 e = p.cv.ktab[in ? k : kfirst];
           const unsigned word = (BMODE == B_IM2COL64 && (e.y & 32)) ? pb[nt].pad_hi : pb[nt].pad_lo;
           eb[nt] = in && !((word >> (e.y & 31)) & 1u) ? B[cb[nt] + (e.x >> 2)] : 0.0f;
         } else {
@@ -381,11 +420,26 @@ __global__ __launch_bounds__(WM * WN * 64, split_blocks(BM, BN)) void split_kern
                                     reinterpret_cast<float *>(&lds[0][0]) + wave * STAGE_FLOATS);
 }
 
-template <int BM, int BN, int WM, int WN, int BMODE>
+template <int BM, int BN, int WM, int WN, int BMODE, int KG>
+__global__ __launch_bounds__(WM * WN * 64 * KG, split_blocks(BM, BN)) void split_kernel(Params p) {
+  split_tile<BM, BN, WM, WN, BMODE, KG>(p, (int)blockIdx.x);
+}
+
+// Several independent products in one launch: the tiles of problem i follow those of problem i - 1.
+template <int BMODE, int KG>
+__global__ __launch_bounds__(256 * KG, split_blocks(64, 64)) void split_group_kernel(GroupParams g) {
+  int i = 0;
+#pragma unroll
+  for (int j = 1; j < GROUP_MAX; j++)
+    if (j < g.count && (int)blockIdx.x >= g.first[j]) i = j;
+  split_tile<64, 64, 2, 2, BMODE, KG>(g.p[i], (int)blockIdx.x - g.first[i]);
+}
+
+template <int BM, int BN, int WM, int WN, int BMODE, int KG = 1>
 int launch_split_tile(Params &p, int nz, const WorkPlan &w) {
   if (BMODE != B_PIXELS_ANY) g_last_form = BMODE;  // (otherwise the caller says which conv it is)
   return launch_planned<BM, BN>(p, nz, BMODE >= B_IM2COL32, BK, 0, [&](dim3 grid, bool) {
-    hipLaunchKernelGGL((split_kernel<BM, BN, WM, WN, BMODE>), grid, dim3(WM * WN * 64), 0, wdh::stream(), p);
+    hipLaunchKernelGGL((split_kernel<BM, BN, WM, WN, BMODE, KG>), grid, dim3(WM * WN * 64 * KG), 0, wdh::stream(), p);
   }, &w);
 }
 template <int BMODE>
@@ -397,6 +451,8 @@ int launch_split(const SplitPlan &s, Params &p, int nz) {
     case S128x128: return launch_split_tile<128, 128, 2, 2, BMODE>(p, nz, s.work);
     case S64x128: return launch_split_tile<64, 128, 2, 2, BMODE>(p, nz, s.work);
     case S128x64: return launch_split_tile<128, 64, 2, 2, BMODE>(p, nz, s.work);
+    case S64x64K2: return launch_split_tile<64, 64, 2, 2, BMODE, 2>(p, nz, s.work);
+    case S64x64K4: return launch_split_tile<64, 64, 2, 2, BMODE, 4>(p, nz, s.work);
     default: return launch_split_tile<64, 64, 2, 2, BMODE>(p, nz, s.work);
   }
 }
