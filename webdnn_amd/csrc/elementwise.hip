@@ -73,6 +73,22 @@ __device__ __forceinline__ f32x4 apply_f4(f32x4 a, f32x4 b) {
   return v;
 }
 
+// A piece of two or four elements; every element of a piece the same value.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+template <int UNIT> struct Piece;
+template <> struct Piece<2> {
+  typedef f32x2 type;
+  static __device__ __forceinline__ type same(float s) { return f32x2{s, s}; }
+};
+template <> struct Piece<4> {
+  typedef f32x4 type;
+  static __device__ __forceinline__ type same(float s) { return f32x4{s, s, s, s}; }
+};
+template <int OP, bool ASK = true>
+__device__ __forceinline__ f32x4 apply_piece(f32x4 a, f32x4 b) { return apply_f4<OP, ASK>(a, b); }
+template <int OP, bool ASK = true>
+__device__ __forceinline__ f32x2 apply_piece(f32x2 a, f32x2 b) { return f32x2{apply_f<OP>(a.x, b.x), apply_f<OP>(a.y, b.y)}; }
+
 template <int OP>
 __device__ __forceinline__ int apply_i(int l, int r) {
   double a = (double)l, b = (double)r;
@@ -124,27 +140,28 @@ __global__ __launch_bounds__(256) void binary_plane(BinaryParams p, wdh::PlaneWa
   const T *L = (const T *)p.L, *R = (const T *)p.R;
   T *Y = (T *)p.Y;
   const long long row0 = (long long)q.outer_linear * second;
-  if (UNIT == 4) {
-    f32x4 a[4], b[4];
+  if constexpr (UNIT > 1) {
+    typedef typename Piece<UNIT>::type V;
+    V a[4], b[4];
     bool ok[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
       const unsigned x = q.x0 + k * q.dx, y = q.y0 + k * q.dy;
       ok[k] = x < inner && y < second;
       if (ok[k]) {
-        const float *l = (const float *)L + bl + (long long)y * sl2 + (long long)x * 4 * sl1;
-        const float *r = (const float *)R + br + (long long)y * sr2 + (long long)x * 4 * sr1;
-        if (sl1) a[k] = *reinterpret_cast<const f32x4 *>(l);
-        else { const float s = *l; a[k] = f32x4{s, s, s, s}; }
-        if (sr1) b[k] = *reinterpret_cast<const f32x4 *>(r);
-        else { const float s = *r; b[k] = f32x4{s, s, s, s}; }
+        const float *l = (const float *)L + bl + (long long)y * sl2 + (long long)x * UNIT * sl1;
+        const float *r = (const float *)R + br + (long long)y * sr2 + (long long)x * UNIT * sr1;
+        if (sl1) a[k] = *reinterpret_cast<const V *>(l);
+        else a[k] = Piece<UNIT>::same(*l);
+        if (sr1) b[k] = *reinterpret_cast<const V *>(r);
+        else b[k] = Piece<UNIT>::same(*r);
       }
     }
 #pragma unroll
     for (int k = 0; k < 4; k++) {
       if (ok[k]) {
         const unsigned x = q.x0 + k * q.dx, y = q.y0 + k * q.dy;
-        *reinterpret_cast<f32x4 *>((float *)Y + ((row0 + y) * inner + x) * 4) = apply_f4<OP>(a[k], b[k]);
+        *reinterpret_cast<V *>((float *)Y + ((row0 + y) * inner + x) * UNIT) = apply_piece<OP>(a[k], b[k]);
       }
     }
   } else {
@@ -192,7 +209,7 @@ __global__ __launch_bounds__(256) void binary_flat(BinaryParams p, wdh::FlatWalk
   const long long sl1 = p.sl[nd - 1] * UNIT, sr1 = p.sr[nd - 1] * UNIT;
   const T *L = (const T *)p.L + bl, *R = (const T *)p.R + br;
   T *Y = (T *)p.Y + (long long)q.outer_linear * f.plane * UNIT;
-  typedef typename std::conditional<UNIT == 4, f32x4, T>::type V;
+  typedef typename std::conditional<UNIT == 4, f32x4, typename std::conditional<UNIT == 2, f32x2, T>::type>::type V;
   for (unsigned u0 = q.begin + threadIdx.x; u0 < q.end; u0 += 1024) {
     V a[4], b[4];
     bool squares = OP == WDH_BIN_POW && UNIT == 4;  // ([100, 768] to powers of 3 by column: 31.7 us, 33.5 with a branch an item)
@@ -203,12 +220,12 @@ __global__ __launch_bounds__(256) void binary_flat(BinaryParams p, wdh::FlatWalk
         const unsigned row = (unsigned)wdh::fdiv((int)u, fd_inner), col = u - row * f.inner;
         const T *l = L + (long long)row * sl2 + (long long)col * sl1;
         const T *r = R + (long long)row * sr2 + (long long)col * sr1;
-        if constexpr (UNIT == 4) {
-          if (sl1) a[k] = *reinterpret_cast<const f32x4 *>(l);
-          else { const float s = *l; a[k] = f32x4{s, s, s, s}; }
-          if (sr1) b[k] = *reinterpret_cast<const f32x4 *>(r);
-          else { const float s = *r; b[k] = f32x4{s, s, s, s}; }
-          squares = squares && all_twos(b[k]);
+        if constexpr (UNIT > 1) {
+          if (sl1) a[k] = *reinterpret_cast<const V *>(l);
+          else a[k] = Piece<UNIT>::same(*l);
+          if (sr1) b[k] = *reinterpret_cast<const V *>(r);
+          else b[k] = Piece<UNIT>::same(*r);
+          if constexpr (UNIT == 4) squares = squares && all_twos(b[k]);
         } else {
           a[k] = *l;
           b[k] = *r;
@@ -225,6 +242,8 @@ __global__ __launch_bounds__(256) void binary_flat(BinaryParams p, wdh::FlatWalk
     if constexpr (UNIT == 4) {
       if (squares) store([&](int k) { return a[k] * a[k]; });
       else store([&](int k) { return apply_f4<OP, false>(a[k], b[k]); });
+    } else if constexpr (UNIT == 2) {
+      store([&](int k) { return apply_piece<OP>(a[k], b[k]); });
     } else if constexpr (__is_same(T, float)) {
       store([&](int k) { return apply_f<OP>(a[k], b[k]); });
     } else {
@@ -278,13 +297,13 @@ BinaryParams for_walk(const BinaryParams &p, const wdh::PlaneWalk &w) {
 }
 
 template <int OP>
-int launch_binary(const BinaryParams &p, int dtype, bool dense, bool vec) {
+int launch_binary(const BinaryParams &p, int dtype, bool dense, int unit) {
   hipStream_t st = wdh::stream();
   const bool small = p.total <= 0xffffffffLL;
   wdh::PlaneWalk w;
   wdh::FlatWalk fw;
-  const bool vec4 = dtype == 0 && vec;
-  const unsigned inner_units = vec4 ? p.shape[p.ndim - 1] / 4 : p.shape[p.ndim - 1];
+  if (dtype != 0) unit = 1;
+  const unsigned inner_units = p.shape[p.ndim - 1] / (unsigned)unit;
   if (dtype == 0 && dense) {
     hipLaunchKernelGGL(binary_dense_f32<OP>, dim3(grid_for((p.total + 3) / 4, 256)),
                        dim3(256), 0, st, (const float *)p.L, (const float *)p.R,
@@ -294,16 +313,21 @@ int launch_binary(const BinaryParams &p, int dtype, bool dense, bool vec) {
              wdh::plan_flat_walk(&fw, p.ndim, p.shape, inner_units)) {
     const dim3 grid(fw.outer * fw.chunks);
     const wdh::FastDiv fd = wdh::make_fastdiv(fw.inner);
-    if (vec4)
+    if (unit == 4)
       hipLaunchKernelGGL((binary_flat<OP, float, 4>), grid, dim3(256), 0, st, p, fw, fd);
+    else if (unit == 2)
+      hipLaunchKernelGGL((binary_flat<OP, float, 2>), grid, dim3(256), 0, st, p, fw, fd);
     else if (dtype == 0)
       hipLaunchKernelGGL((binary_flat<OP, float, 1>), grid, dim3(256), 0, st, p, fw, fd);
     else
       hipLaunchKernelGGL((binary_flat<OP, int, 1>), grid, dim3(256), 0, st, p, fw, fd);
-  } else if (dtype == 0 && vec &&
-             wdh::plan_plane_walk(&w, p.ndim, p.shape, p.shape[p.ndim - 1] / 4)) {
-    hipLaunchKernelGGL((binary_plane<OP, float, 4>), wdh::plane_grid(w), dim3(256), 0, st,
-                       for_walk(p, w), w);
+  } else if (unit > 1 && wdh::plan_plane_walk(&w, p.ndim, p.shape, inner_units)) {
+    if (unit == 4)
+      hipLaunchKernelGGL((binary_plane<OP, float, 4>), wdh::plane_grid(w), dim3(256), 0, st,
+                         for_walk(p, w), w);
+    else
+      hipLaunchKernelGGL((binary_plane<OP, float, 2>), wdh::plane_grid(w), dim3(256), 0, st,
+                         for_walk(p, w), w);
   } else if (wdh::plan_plane_walk(&w, p.ndim, p.shape, p.shape[p.ndim - 1])) {
     if (dtype == 0)
       hipLaunchKernelGGL((binary_plane<OP, float, 1>), wdh::plane_grid(w), dim3(256), 0, st,
@@ -487,21 +511,24 @@ extern "C" int wdh_binary(int op, int dtype, wdh_buf hL, wdh_buf hR, wdh_buf hY,
   // 16-byte accesses: the output always; an operand that steps by 1 along the
   // innermost axis needs an aligned base and outer strides that are multiples
   // of 4; one that does not step there (stride 0) is read with scalar loads
-  auto vec_ok = [&](const void *base, const long long *st) {
+  auto piece_ok = [&](const void *base, const long long *st, int unit) {
     if (st[nd - 1] == 0) return true;
-    if (st[nd - 1] != 1 || ((uintptr_t)base & 15)) return false;
+    if (st[nd - 1] != 1 || ((uintptr_t)base & (4 * unit - 1))) return false;
     for (int d = 0; d + 1 < nd; d++)
-      if (st[d] % 4) return false;
+      if (st[d] % unit) return false;
     return true;
   };
-  const bool vec = ((uintptr_t)p.Y & 15) == 0 && p.shape[nd - 1] % 4 == 0 &&
-                   vec_ok(p.L, p.sl) && vec_ok(p.R, p.sr);
+  // (pieces of two where pieces of four do not fit: a scale by channel over 8 x 192 planes of 95 x 126 29.9 us with single ones, 27.9 with these)
+  int unit = 1;
+  for (int u : {4, 2})
+    if (unit == 1 && ((uintptr_t)p.Y & (4 * u - 1)) == 0 && p.shape[nd - 1] % u == 0 && piece_ok(p.L, p.sl, u) && piece_ok(p.R, p.sr, u))
+      unit = u;
   switch (op) {
-    case WDH_BIN_ADD: return launch_binary<WDH_BIN_ADD>(p, dtype, dense, vec);
-    case WDH_BIN_SUB: return launch_binary<WDH_BIN_SUB>(p, dtype, dense, vec);
-    case WDH_BIN_MUL: return launch_binary<WDH_BIN_MUL>(p, dtype, dense, vec);
-    case WDH_BIN_DIV: return launch_binary<WDH_BIN_DIV>(p, dtype, dense, vec);
-    default: return launch_binary<WDH_BIN_POW>(p, dtype, dense, vec);
+    case WDH_BIN_ADD: return launch_binary<WDH_BIN_ADD>(p, dtype, dense, unit);
+    case WDH_BIN_SUB: return launch_binary<WDH_BIN_SUB>(p, dtype, dense, unit);
+    case WDH_BIN_MUL: return launch_binary<WDH_BIN_MUL>(p, dtype, dense, unit);
+    case WDH_BIN_DIV: return launch_binary<WDH_BIN_DIV>(p, dtype, dense, unit);
+    default: return launch_binary<WDH_BIN_POW>(p, dtype, dense, unit);
   }
 }
 

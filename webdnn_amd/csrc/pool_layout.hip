@@ -82,21 +82,27 @@ struct PoolBand {
   int tx_log2;  // threads along ow = 2^tx_log2 (at most one wavefront)
 };
 
-template <int KH, int KW, bool VEC>
+// Bound: the latency of the copy.  Pieces of four, two or one floats, as the rows are aligned, four of a thread in flight
+// (8 x 192 planes of 95 x 126: 37.2 us with one 4-byte load at a time, 22.1 now).
+template <int KH, int KW, int VECW>
 __global__ __launch_bounds__(256) void maxpool2d_band_kernel(PoolParams p, PoolBand b) {
-  extern __shared__ float band[];
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  extern __shared__ __attribute__((aligned(16))) float band[];
+  typedef float piece __attribute__((ext_vector_type(VECW)));
   const int oy0 = blockIdx.y * b.rows;
   const int iy0 = oy0 * p.sh - p.pt;                // may lie in the top padding
   const int lo = iy0 < 0 ? 0 : iy0;
   const int hi = iy0 + b.in_rows < p.h ? iy0 + b.in_rows : p.h;
   const float *x = p.X + (long long)blockIdx.x * p.h * p.w + (long long)lo * p.w;
   const int count = (hi - lo) * p.w;                // floats of rows lo..hi-1
-  if (VEC) {
-    for (int i = threadIdx.x * 4; i < count; i += 1024)
-      *reinterpret_cast<f32x4 *>(band + i) = *reinterpret_cast<const f32x4 *>(x + i);
-  } else {
-    for (int i = threadIdx.x; i < count; i += 256) band[i] = x[i];
+  constexpr int AHEAD = 4, STEP = 256 * VECW;
+  for (int i = threadIdx.x * VECW; i < count; i += AHEAD * STEP) {
+    piece v[AHEAD];
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++)
+      if (i + k * STEP < count) v[k] = *reinterpret_cast<const piece *>(x + i + k * STEP);
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++)
+      if (i + k * STEP < count) *reinterpret_cast<piece *>(band + i + k * STEP) = v[k];
   }
   __syncthreads();
   const int nrows = p.oh - oy0 < b.rows ? p.oh - oy0 : b.rows;
@@ -408,6 +414,32 @@ __global__ __launch_bounds__(256) void transpose_tiled_wide(TileParams p) {
   }
 }
 
+// Whole runs of `inner` elements per index: a workgroup copies up to 1024 pieces of UNIT elements of one run, a thread four of
+// them, all requested before the first is stored; the index is read once, by the workgroup.
+// (96 of 192 planes of 95 x 126, eight times: 27.8 us an element at a time, with its three 64-bit divisions; 15.6 now.)
+template <int UNIT>
+__global__ __launch_bounds__(256) void gather_rows_kernel(const uint32_t *__restrict__ D, const int *__restrict__ Idx,
+                                                          uint32_t *__restrict__ Y, int axis_len, unsigned units, wdh::FastDiv fd_chunks,
+                                                          wdh::FastDiv fd_idx) {
+  typedef uint32_t piece __attribute__((ext_vector_type(UNIT)));
+  const int row = wdh::fdiv((int)blockIdx.x, fd_chunks), chunk = (int)blockIdx.x - row * fd_chunks.d;
+  const int o = wdh::fdiv(row, fd_idx);
+  int ix = Idx[row - o * fd_idx.d];
+  if (ix < 0) ix += axis_len;
+  // out-of-range indices read element 0 rather than stray memory
+  if (ix < 0 || ix >= axis_len) ix = 0;
+  const piece *const src = reinterpret_cast<const piece *>(D) + ((long long)o * axis_len + ix) * units;
+  piece *const dst = reinterpret_cast<piece *>(Y) + (long long)row * units;
+  const unsigned first = (unsigned)chunk * 1024 + threadIdx.x;
+  piece v[4];
+#pragma unroll
+  for (unsigned k = 0; k < 4; k++)
+    if (first + 256 * k < units) v[k] = src[first + 256 * k];
+#pragma unroll
+  for (unsigned k = 0; k < 4; k++)
+    if (first + 256 * k < units) dst[first + 256 * k] = v[k];
+}
+
 __global__ __launch_bounds__(256) void gather_axis_kernel(
     const uint32_t *__restrict__ D, const int *__restrict__ Idx,
     uint32_t *__restrict__ Y, long long outer, int axis_len, long long inner,
@@ -524,13 +556,14 @@ extern "C" int wdh_maxpool2d(wdh_buf hX, wdh_buf hY, int n, int c, int h, int w,
     const long long bands = (oh + b.rows - 1) / b.rows;
     if (cells >= 256 && in_rows * w <= 8192 && bands <= 65535) {
       b.in_rows = (int)in_rows;
-      const bool vec = w % 4 == 0 && ((long long)h * w) % 4 == 0 && ((uintptr_t)px & 15) == 0;
+      const int vecw = w % 4 == 0 && ((uintptr_t)px & 15) == 0 ? 4 : w % 2 == 0 && ((uintptr_t)px & 7) == 0 ? 2 : 1;
       const dim3 grid((unsigned)planes, (unsigned)bands);
       const size_t lds = (size_t)in_rows * w * 4;
 #define WDH_POOL_BAND(KH, KW)                                                                     \
   do {                                                                                            \
-    if (vec) hipLaunchKernelGGL((maxpool2d_band_kernel<KH, KW, true>), grid, dim3(256), lds, st, p, b); \
-    else hipLaunchKernelGGL((maxpool2d_band_kernel<KH, KW, false>), grid, dim3(256), lds, st, p, b);    \
+    if (vecw == 4) hipLaunchKernelGGL((maxpool2d_band_kernel<KH, KW, 4>), grid, dim3(256), lds, st, p, b);      \
+    else if (vecw == 2) hipLaunchKernelGGL((maxpool2d_band_kernel<KH, KW, 2>), grid, dim3(256), lds, st, p, b); \
+    else hipLaunchKernelGGL((maxpool2d_band_kernel<KH, KW, 1>), grid, dim3(256), lds, st, p, b);                \
   } while (0)
       if (kh == 3 && kw == 3) WDH_POOL_BAND(3, 3);
       else if (kh == 2 && kw == 2) WDH_POOL_BAND(2, 2);
@@ -654,6 +687,21 @@ extern "C" int wdh_gather(wdh_buf hD, wdh_buf hI, wdh_buf hY, int64_t outer,
   if (!wdh::operand(hD, (size_t)outer * axis_len * inner * 4, "wdh_gather: Data", &pd)) return WDH_EINVAL;
   if (!wdh::operand(hI, (size_t)n_idx * 4, "wdh_gather: Indices", &pi)) return WDH_EINVAL;
   if (!wdh::operand(hY, (size_t)total * 4, "wdh_gather: Y", &py)) return WDH_EINVAL;
+  // runs long enough to occupy a wavefront: 16-, 8- or 4-byte pieces as they are aligned
+  const uintptr_t at = (uintptr_t)pd | (uintptr_t)py;
+  const int unit = inner % 4 == 0 && (at & 15) == 0 ? 4 : inner % 2 == 0 && (at & 7) == 0 ? 2 : 1;
+  const long long units = inner / unit, rows = (long long)outer * n_idx, chunks = (units + 1023) / 1024;
+  if (units >= 48 && rows <= 0x7fffffffLL / chunks && units <= 0x7fffffffLL) {
+    const wdh::FastDiv fd_chunks = wdh::make_fastdiv(chunks), fd_idx = wdh::make_fastdiv(n_idx);
+    const dim3 grid((unsigned)(rows * chunks)), block(256);
+    const uint32_t *d = (const uint32_t *)pd;
+    uint32_t *y = (uint32_t *)py;
+    if (unit == 4) hipLaunchKernelGGL(gather_rows_kernel<4>, grid, block, 0, wdh::stream(), d, (const int *)pi, y, axis_len, (unsigned)units, fd_chunks, fd_idx);
+    else if (unit == 2) hipLaunchKernelGGL(gather_rows_kernel<2>, grid, block, 0, wdh::stream(), d, (const int *)pi, y, axis_len, (unsigned)units, fd_chunks, fd_idx);
+    else hipLaunchKernelGGL(gather_rows_kernel<1>, grid, block, 0, wdh::stream(), d, (const int *)pi, y, axis_len, (unsigned)units, fd_chunks, fd_idx);
+    WDH_LAUNCH_CHECK();
+    return WDH_OK;
+  }
   hipLaunchKernelGGL(gather_axis_kernel, dim3(grid_for(total)), dim3(256), 0,
                      wdh::stream(), (const uint32_t *)pd, (const int *)pi,
                      (uint32_t *)py, (long long)outer, axis_len, (long long)inner,
