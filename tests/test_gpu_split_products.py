@@ -263,6 +263,34 @@ def test_rows_while_recording(ctx, split):
         ctx.graph_destroy(graph)
 
 
+def test_recorded_weights_outlive_another_size(ctx, split):
+    """One weight, two sizes of input that take two forms: what a recorded run reads stays while the other size runs."""
+    rng = np.random.default_rng(10)
+    wt = ctx.move_tensor(rng.standard_normal((128, 128, 3, 3)).astype(np.float32))
+    large, small = (ctx.move_tensor(rng.standard_normal((n, 128, s, s)).astype(np.float32)) for n, s in ((4, 32), (2, 10)))
+    run = lambda x: H.conv(ctx, x, wt, pads=[1] * 4, constant_weights=True)
+    want, forms = [], []
+    for x in (large, small):
+        want.append(H.conv(ctx, x, wt, pads=[1] * 4).get_data())
+        forms.append(ctx.last_plan()["form"])
+    assert forms[0] != forms[1], forms
+    for recorded, other, a, b in ((large, small, *want), (small, large, *want[::-1])):
+        run(recorded).dispose()
+        ctx.sync()
+        ctx.graph_begin()
+        y = run(recorded)
+        graph = ctx.graph_end()
+        for _ in range(3):
+            z = run(other)
+            # (blocks that went back to the pool are written over)
+            junk = [ctx.move_tensor(np.full(elements, 7.0, np.float32)) for elements in (221184, 262144) * 4]
+            ctx.graph_launch(graph)
+            assert (y.get_data() == a).all() and (z.get_data() == b).all()
+            for t in junk + [z]:
+                t.dispose()
+        ctx.graph_destroy(graph)
+
+
 def test_groups_that_fill_the_chip(ctx, split):
     """The projections of an attention block as one launch of 64x64 tiles; ragged rows and columns, one weight k-contiguous by shape."""
     rng = np.random.default_rng(9)

@@ -55,6 +55,7 @@
 #include <string.h>
 
 #include <map>
+#include <tuple>
 #include <vector>
 
 #include "contraction.h"
@@ -865,13 +866,35 @@ struct KtabVal {
 
 std::map<KtabKey, KtabVal> g_ktabs;
 
-// Transformed filters (U of the F(2x2, 3x3) form) of weight buffers whose owner promised not to
-// write to them (WDH_CONV_CONSTANT_WEIGHTS): weight handle -> a pool block that holds U.
-struct FilterEntry {
-  wdh_buf u;
-  int cout, c, r;  // r: 2 or 4, the form the filters were transformed for
+// What was made of weight buffers whose owner promised not to write to them (WDH_CONV_CONSTANT_WEIGHTS): filters transformed
+// for F(2x2, 3x3) or F(4x4, 3x3), or laid out in bfloat16 parts -> a pool block that holds them.  The form goes by the size of
+// the input, and one set of weights serves several sizes: each form has a block of its own, which stays until the weights
+// go, because recorded graphs read it.
+struct FilterKey {
+  wdh_buf weights;
+  int form, cout, c;  // form: 2 or 4 = transformed for that output patch, 0 = in parts (conv3x3_split.hip)
+  bool operator<(const FilterKey &o) const {
+    return std::tie(weights, form, cout, c) < std::tie(o.weights, o.form, o.cout, o.c);
+  }
 };
-std::map<wdh_buf, FilterEntry> g_filters;
+std::map<FilterKey, wdh_buf> g_filters;
+// The block for `key`, from before (ready) or newly allocated (to be filled, or dropped); 0: to be had for this call only.
+wdh_buf kept_filters(const FilterKey &key, size_t bytes, bool *ready) {
+  auto it = g_filters.find(key);
+  *ready = it != g_filters.end();
+  if (*ready) return it->second;
+  if (wdh::capturing()) return 0;  // (a block allocated while a graph is being recorded belongs to that graph)
+  const wdh_buf u = wdh_alloc(bytes);
+  if (u) g_filters[key] = u;
+  return u;
+}
+void drop_filters(const FilterKey &key) {
+  auto it = g_filters.find(key);
+  if (it == g_filters.end()) return;
+  const wdh_buf u = it->second;
+  g_filters.erase(it);  // first: wdh_free comes back to conv_forget_weights for `u`
+  (void)wdh_free(u);
+}
 
 }  // namespace
 
@@ -887,12 +910,9 @@ void release_conv_tables() {
 // any synchronisation without a copy.
 // The buffer behind `h` is about to be freed or written to: data derived from it is stale.
 void conv_forget_weights(wdh_buf h) {
-  if (g_filters.empty()) return;
-  auto it = g_filters.find(h);
-  if (it == g_filters.end()) return;
-  const wdh_buf u = it->second.u;
-  g_filters.erase(it);  // first: wdh_free comes back here for `u`
-  (void)wdh_free(u);
+  for (auto it = g_filters.lower_bound(FilterKey{h, 0, 0, 0}); it != g_filters.end() && it->first.weights == h;
+       it = g_filters.lower_bound(FilterKey{h, 0, 0, 0}))
+    drop_filters(FilterKey(it->first));
 }
 
 int init_contraction(int device) {
@@ -1132,30 +1152,17 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
                  m_bytes = (size_t)positions * cout * tiles * 4;
     if (tiles < 0x7fffffffLL && v_bytes < ((size_t)1 << 33) && m_bytes < ((size_t)1 << 33)) {
       // the transformed filters: kept from call to call when the caller vouches for the weights
-      // (a block allocated while a graph is being recorded belongs to that graph, so nothing is kept then)
-      wdh_buf hU = 0;
-      bool u_kept = false, u_ready = false;
-      if (flags & WDH_CONV_CONSTANT_WEIGHTS) {
-        auto it = g_filters.find(hW);
-        if (it != g_filters.end() && it->second.cout == cout && it->second.c == c && it->second.r == r) {
-          hU = it->second.u;
-          u_kept = u_ready = true;
-        } else if (!wdh::capturing()) {
-          wdh::conv_forget_weights(hW);
-          hU = wdh_alloc(u_bytes);
-          if (hU) {
-            g_filters[hW] = FilterEntry{hU, cout, c, r};
-            u_kept = true;
-          }
-        }
-      }
+      const FilterKey key = {hW, r, cout, c};
+      bool u_ready = false;
+      wdh_buf hU = flags & WDH_CONV_CONSTANT_WEIGHTS ? kept_filters(key, u_bytes, &u_ready) : 0;
+      const bool u_kept = hU != 0;
       if (!hU) hU = wdh_alloc(u_bytes);
       const wdh_buf hV = wdh_alloc(v_bytes), hM = wdh_alloc(m_bytes);
       int rc = WDH_OK;
       if (!(hU && hV && hM)) {
         // no room for the transform-domain tensors: the direct forms below need none
         if (hU && !u_kept) (void)wdh_free(hU);
-        if (u_kept && !u_ready) wdh::conv_forget_weights(hW);  // (registered above, never filled)
+        if (u_kept && !u_ready) drop_filters(key);  // (registered above, never filled)
         if (hV) (void)wdh_free(hV);
         if (hM) (void)wdh_free(hM);
         wdh::clear_error();
@@ -1184,7 +1191,7 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
                                      epilogue == WDH_EPI_RELU);
       }
       // (the blocks go back to the pool at once: whoever gets them next is ordered behind these kernels)
-      if (rc != WDH_OK && u_kept && !u_ready) wdh::conv_forget_weights(hW);  // (may not have been filled)
+      if (rc != WDH_OK && u_kept && !u_ready) drop_filters(key);  // (may not have been filled)
       if (hU && !u_kept) (void)wdh_free(hU);
       if (hV) (void)wdh_free(hV);
       if (hM) (void)wdh_free(hM);
@@ -1194,22 +1201,10 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
 direct_forms:
   // 3x3, stride 1 of a batch: rows of X in LDS, split once, against weights that are laid out in parts (conv3x3_split.hip)
   if (rows_split) {
-    wdh_buf hP = 0;
-    bool kept = false, ready = false;
-    if (flags & WDH_CONV_CONSTANT_WEIGHTS) {
-      auto it = g_filters.find(hW);
-      if (it != g_filters.end() && it->second.cout == cout && it->second.c == c && it->second.r == 0) {
-        hP = it->second.u;
-        kept = ready = true;
-      } else if (!wdh::capturing()) {
-        wdh::conv_forget_weights(hW);
-        hP = wdh_alloc(packed3x3_bytes(cout, c));
-        if (hP) {
-          g_filters[hW] = FilterEntry{hP, cout, c, 0};
-          kept = true;
-        }
-      }
-    }
+    const FilterKey filters = {hW, 0, cout, c};
+    bool ready = false;
+    wdh_buf hP = flags & WDH_CONV_CONSTANT_WEIGHTS ? kept_filters(filters, packed3x3_bytes(cout, c), &ready) : 0;
+    const bool kept = hP != 0;
     if (!hP) hP = wdh_alloc(packed3x3_bytes(cout, c));
     if (hP) {
       p.m = cout_g; p.n = (int)npix; p.k = (int)kdim;
@@ -1227,7 +1222,7 @@ direct_forms:
       int rc = ready ? WDH_OK : pack3x3_launch(p.A, packed, cout, c);
       if (rc == WDH_OK)
         rc = run_split(plan_split(1, p.m, p.n, p.k, SPLIT_ROWS), [&](const SplitPlan &q) { return launch_conv3x3_split(p, q, packed); });
-      if (rc != WDH_OK && kept && !ready) wdh::conv_forget_weights(hW);  // (may not have been filled)
+      if (rc != WDH_OK && kept && !ready) drop_filters(filters);  // (may not have been filled)
       if (!kept) (void)wdh_free(hP);
       return rc;
     }
