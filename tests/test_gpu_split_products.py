@@ -291,6 +291,19 @@ def test_recorded_weights_outlive_another_size(ctx, split):
         ctx.graph_destroy(graph)
 
 
+@pytest.mark.parametrize("shift", [-120, -112, -100])
+def test_rows_of_tiny_elements(ctx, split, shift):
+    """Elements whose last part does not fit bfloat16 leave tiny sums, which are added up again, also against large partners."""
+    rng = np.random.default_rng(11)
+    a = (rng.uniform(1, 2, (256, 512)) * 2.0 ** shift).astype(np.float32)
+    b = (rng.uniform(1, 2, (512, 256)) * 2.0 ** 40).astype(np.float32)
+    split(3)
+    got = product(ctx, a, b, False)
+    assert ctx.last_plan()["tile"] == "128x128"
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    assert within(got, a @ b, a @ b, 512)
+
+
 def test_groups_that_fill_the_chip(ctx, split):
     """The projections of an attention block as one launch of 64x64 tiles; ragged rows and columns, one weight k-contiguous by shape."""
     rng = np.random.default_rng(9)

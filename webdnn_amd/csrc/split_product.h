@@ -24,8 +24,9 @@
 //
 // What the split cannot hold is done again with the fp32 instruction, a whole tile (or chunk) at a time:
 //   * an Inf or NaN operand leaves NaN in x - h and therefore in every sum it enters; so does a sum that overflows;
-//   * elements below 2^-110 lose bits of l below 2^-133.  Only a sum of such elements shows that, and it is tiny:
-//     a tile that holds a nonzero sum below 2^-100 is done again.
+//   * elements below 2^-110 lose bits of l below 2^-133.  Only a sum of such elements shows that, and it is tiny unless
+//     their partners are beyond 2^50: a tile that holds a nonzero sum below 2^-60 is done again.  (Terms around
+//     one do not cancel down to there: what they leave is zero or a rounding, 2^-24 of a term.)
 // Both show in the sums themselves, so the loop carries no test.
 #pragma once
 #include "contraction.h"
@@ -50,9 +51,9 @@ __device__ __forceinline__ SplitPair split_pair(float x0, float x1) {
 }
 
 // Whether a tile holds a sum that the split cannot vouch for, from the largest and the least (zeros aside) of the doubled
-// bits of its sums: not finite, or nonzero below 2^-100.
+// bits of its sums: not finite, or nonzero below 2^-60.
 __device__ __forceinline__ bool split_fails(unsigned most, unsigned least) {
-  return most >= 0xff000000u || least < ((127u - 100u) << 24) - 1u;
+  return most >= 0xff000000u || least < ((127u - 60u) << 24) - 1u;
 }
 
 // Workgroups a CU holds: the accumulators are two per result, so 128x128 tiles take 64 + 64 registers of
@@ -331,7 +332,7 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
   }
 
   // ---- the two sums meet; is there anything the split could not hold? ------------------------------------
-  // (bits of |sum| doubled: zero is fine, so is 2^-100 up to the largest float)
+  // (bits of |sum| doubled: zero is fine, so is 2^-60 up to the largest float)
   unsigned most = 0, least = 0xffffffffu;
 #pragma unroll
   for (int a = 0; a < MT; a++)
