@@ -1465,6 +1465,18 @@ def test_attention_one_launch_equals_the_four_node_chain(ctx, tq, tk, heads, d):
     assert_close_max(got, chain.get_data(), 1e-5, "attention vs unfused chain")
 
 
+@pytest.mark.parametrize("tk,d", [(1, 64), (255, 64), (256, 64), (257, 64), (512, 64), (513, 64), (512, 32), (513, 32), (40, 128), (256, 128), (257, 128)])
+def test_attention_at_the_key_counts_where_the_form_changes(ctx, tk, d):
+    """Every number of key blocks a wavefront may own, at both ends of its range, with a NaN in V behind the last key."""
+    rng = np.random.default_rng(tk + d)
+    q, k = rng.standard_normal((33, 3 * d)).astype(np.float32), rng.standard_normal((tk, 3 * d)).astype(np.float32)
+    v = np.full((tk + 1, 3 * d), np.nan, np.float32)
+    v[:tk] = rng.standard_normal((tk, 3 * d))
+    held = ctx.move_tensor(v)
+    got = H.attention(ctx, ctx.move_tensor(q), ctx.move_tensor(k), held.alias([tk, 3 * d]), 3, 1.0 / np.sqrt(d)).get_data()
+    assert_close_max(got, attention_chain_ref(q, k, v[:tk], 3, 1.0 / np.sqrt(d)), GEMM_TOL, "attention vs oracle chain")
+
+
 def test_attention_special_values_and_limits(ctx):
     """A +inf in V beside masked keys, a NaN score, and the shapes the entry point turns down."""
     rng = np.random.default_rng(5)

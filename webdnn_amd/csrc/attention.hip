@@ -47,14 +47,26 @@ struct AttParams {
 // ATT_WAVES wavefronts per workgroup: 16 for a head dimension of 32 (every phase is a chain of
 // dependent steps per wavefront; twice the wavefronts halve each chain), 8 where a wavefront's
 // registers hold less of K and V.
-template <int HD, int ATT_WAVES>
+//
+// Bound: latency -- a workgroup has a CU to itself and goes through its phases once.  So a wavefront asks for everything at
+// once, and for no more than its keys: PER_WAVE blocks of 32 keys (at most 32 * ATT_WAVES * PER_WAVE keys), not always the blocks of
+// 1024; V before the scores where the registers hold it beside K, else before the softmax.
+// (us, always 1024 keys' loads / these: 12 heads of 64, 200 tokens 12.6 / 11.0, 384 16.7 / 15.9, 600 26.4 / 24.1; 16 of 64, 1024 tokens
+// 80.8 / 67.6; 8 of 32, 100 keys 7.8 / 6.4, 300 11.3 / 9.4; 8 of 128, 128 keys 14.2 / 12.2.)
+template <int HD, int ATT_WAVES, int PER_WAVE>
 __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParams p) {
   static_assert(HD % 32 == 0 && HD >= 32 && HD <= 128, "head dimension");
-  static_assert(ATT_WAVES == 8 || ATT_WAVES == 16, "32 rows and 32 key blocks are dealt over the wavefronts");
+  static_assert(ATT_WAVES == 8 || ATT_WAVES == 16, "32 rows and the key blocks are dealt over the wavefronts");
+  static_assert(32 * ATT_WAVES * PER_WAVE <= ATT_MAX_KEYS, "keys");
   constexpr int HALF = HD / 2;   // head-dimension indices per half wavefront
   constexpr int NB = HD / 32;    // 32-column blocks of the output
+  constexpr int V_REGS = 16 * NB * PER_WAVE;
+  constexpr bool V_FIRST = V_REGS <= 64, V_HELD = V_REGS <= 128;
+  // Blocks beyond the keys are not asked for, except where most wavefronts have all of theirs anyway and the branches cost
+  // more (us, asked for / left out: 8 heads of 32, 850 keys 18.1 / 18.7; 8 of 128, 900 keys 61 / 80; but 12 of 64, 600 keys 33.0 / 24.6).
+  constexpr bool SKIP = HD == 64 || PER_WAVE == 1;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = SKIP ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int li = lane & 31, half = lane >> 5;
   const int b = blockIdx.x / p.row_blocks;
   const int row0 = (blockIdx.x - b * p.row_blocks) * ATT_ROWS;
@@ -63,27 +75,26 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
   const float *V = p.V + (long long)b * p.sVb;
   const int ncb = (p.tk + 31) >> 5;  // blocks of 32 keys
 
-  // At most 1024 keys are 32 blocks of 32: four (two) per wavefront.  Each phase issues the loads
-  // of all four before the first use, so a wavefront waits for memory once per phase.
-  constexpr int PER_WAVE = ATT_MAX_KEYS / 32 / ATT_WAVES;
-
-  // Every value of V this wavefront will need in step 3 is requested before step 1, so the
-  // loads travel while the scores are computed (64 registers per 32 columns of V).
-  float vb[NB == 1 ? PER_WAVE : 1][NB][16];
-  if constexpr (NB == 1) {
+  // Every value of V this wavefront will need in step 3 (up to 64 registers travel while the scores are computed, up to
+  // 128 during the softmax).
+  float vb[V_HELD ? PER_WAVE : 1][NB][16];
+  auto fetch_v = [&](int kc, int nb, float (&v)[16]) {
+    const int key0 = kc * 32 + 16 * half;
 #pragma unroll
-    for (int it = 0; it < PER_WAVE; it++) {
-      const int key0 = (wave + ATT_WAVES * it) * 32 + 16 * half;
-#pragma unroll
-      for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-        for (int s = 0; s < 16; s++) {
-          const int key = key0 + s;
-          const float t = V[(long long)(key < p.tk ? key : p.tk - 1) * p.sVj + nb * 32 + li];
-          vb[it][nb][s] = key < p.tk ? t : 0.0f;  // (P is 0 there; this keeps an inf or NaN of V out)
-        }
+    for (int s = 0; s < 16; s++) {
+      const int key = key0 + s;
+      const float t = V[(long long)(key < p.tk ? key : p.tk - 1) * p.sVj + nb * 32 + li];
+      v[s] = key < p.tk ? t : 0.0f;  // (P is 0 there; this keeps an inf or NaN of V out)
     }
-  }
+  };
+  auto fetch_held = [&]() {
+#pragma unroll
+    for (int it = 0; it < (V_HELD ? PER_WAVE : 1); it++)
+      if (!SKIP || wave + ATT_WAVES * it < ncb)
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) fetch_v(wave + ATT_WAVES * it, nb, vb[it][nb]);
+  };
+  if (V_FIRST) fetch_held();
 
   // ---- 1. scores -------------------------------------------------------------------
   {
@@ -98,6 +109,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
     f32x4 kb[PER_WAVE][HALF / 4];
 #pragma unroll
     for (int it = 0; it < PER_WAVE; it++) {
+      if (SKIP && wave + ATT_WAVES * it >= ncb) continue;
       const int key = (wave + ATT_WAVES * it) * 32 + li;
       const float *k = K + (long long)(key < p.tk ? key : p.tk - 1) * p.sKj + HALF * half;
 #pragma unroll
@@ -121,22 +133,24 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
       }
     }
   }
+  if (V_HELD && !V_FIRST) fetch_held();
   __syncthreads();
 
   // ---- 2. softmax over each row, in place (softmax.ts:34-57) ------------------------
   // The wavefront's four (two) rows are taken through every step together.
   {
     constexpr int RPW = ATT_ROWS / ATT_WAVES;
-    const int ncols = ncb * 32;  // a multiple of 4; at most 1024: four 16-byte pieces per lane
+    constexpr int PIECES = 32 * ATT_WAVES * PER_WAVE / 256;  // 16-byte pieces per lane
+    const int ncols = ncb * 32;  // a multiple of 4
     const float ninf = -INFINITY;
-    f32x4 v[RPW][4];
+    f32x4 v[RPW][PIECES];
     float mx[RPW], sum[RPW];
 #pragma unroll
     for (int j = 0; j < RPW; j++) {
       const float *srow = lds + (wave + ATT_WAVES * j) * p.pitch;
       mx[j] = ninf;
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
+      for (int i = 0; i < PIECES; i++) {
         const int c = 4 * lane + 256 * i;
         v[j][i] = c < ncols ? *reinterpret_cast<const f32x4 *>(srow + c) : f32x4{ninf, ninf, ninf, ninf};
 #pragma unroll
@@ -149,7 +163,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
     for (int j = 0; j < RPW; j++) {
       sum[j] = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < PIECES; i++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const float ex = 4 * lane + 256 * i + e < p.tk ? exp_f32(v[j][i][e] - mx[j]) : 0.0f;
@@ -164,7 +178,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
       float *srow = lds + (wave + ATT_WAVES * j) * p.pitch;
       const float inv = 1.0f / sum[j];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
+      for (int i = 0; i < PIECES; i++) {
         const int c = 4 * lane + 256 * i;
         if (c < ncols) {
           f32x4 t;
@@ -182,15 +196,18 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
 #pragma unroll
   for (int nb = 0; nb < NB; nb++)
     o[nb] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if constexpr (NB == 1) {
+  auto fetch_p = [&](int kc, f32x4 (&pa)[4]) {
+    const float *prow = lds + li * p.pitch + kc * 32 + 16 * half;
+#pragma unroll
+    for (int c = 0; c < 4; c++) pa[c] = *reinterpret_cast<const f32x4 *>(prow + 4 * c);
+  };
+  f32x4 pa[4];
+  if constexpr (V_HELD) {
 #pragma unroll
     for (int it = 0; it < PER_WAVE; it++) {
       const int kc = wave + ATT_WAVES * it;
       if (kc >= ncb) break;
-      const float *prow = lds + li * p.pitch + kc * 32 + 16 * half;
-      f32x4 pa[4];
-#pragma unroll
-      for (int c = 0; c < 4; c++) pa[c] = *reinterpret_cast<const f32x4 *>(prow + 4 * c);
+      fetch_p(kc, pa);
 #pragma unroll
       for (int nb = 0; nb < NB; nb++)
 #pragma unroll
@@ -199,20 +216,11 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
     }
   } else {
     for (int kc = wave; kc < ncb; kc += ATT_WAVES) {
-      const int key0 = kc * 32 + 16 * half;
-      const float *prow = lds + li * p.pitch + key0;
-      f32x4 pa[4];
-#pragma unroll
-      for (int c = 0; c < 4; c++) pa[c] = *reinterpret_cast<const f32x4 *>(prow + 4 * c);
+      fetch_p(kc, pa);
 #pragma unroll
       for (int nb = 0; nb < NB; nb++) {
         float vn[16];
-#pragma unroll
-        for (int s = 0; s < 16; s++) {
-          const int key = key0 + s;
-          const float t = V[(long long)(key < p.tk ? key : p.tk - 1) * p.sVj + nb * 32 + li];
-          vn[s] = key < p.tk ? t : 0.0f;
-        }
+        fetch_v(kc, nb, vn);
 #pragma unroll
         for (int s = 0; s < 16; s++)
           o[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(pa[s >> 2][s & 3], vn[s], o[nb], 0, 0, 0);
@@ -250,16 +258,33 @@ int lds_pitch(int tk) {
   return pitch;
 }
 
-template <int HD, int ATT_WAVES>
+template <int HD, int ATT_WAVES, int PER_WAVE>
 int launch_attention(const AttParams &p, int batch) {
   // the scores block, and later the wavefronts' partial outputs, whichever is larger
   size_t bytes = (size_t)ATT_ROWS * p.pitch * 4;
   const size_t partials = (size_t)ATT_WAVES * ATT_ROWS * (HD + 1) * 4;
   if (partials > bytes) bytes = partials;
-  hipLaunchKernelGGL((attention_rows_kernel<HD, ATT_WAVES>), dim3((unsigned)((long long)batch * p.row_blocks)),
+  hipLaunchKernelGGL((attention_rows_kernel<HD, ATT_WAVES, PER_WAVE>), dim3((unsigned)((long long)batch * p.row_blocks)),
                      dim3(64 * ATT_WAVES), bytes, wdh::stream(), p);
   WDH_LAUNCH_CHECK();
   return WDH_OK;
+}
+template <int HD>
+int launch_attention(const AttParams &p, int batch) {
+  // (64: sixteen wavefronts of one block each, 512 keys 18.8 us, eight of two 19.4; 200 keys 11.6 and 11.0)
+  if constexpr (HD == 32)
+    return p.tk > 512 ? launch_attention<HD, 16, 2>(p, batch) : launch_attention<HD, 16, 1>(p, batch);
+  else if constexpr (HD == 64)
+    return p.tk > 512   ? launch_attention<HD, 8, 4>(p, batch)
+           : p.tk > 256 ? launch_attention<HD, 16, 1>(p, batch) : launch_attention<HD, 8, 1>(p, batch);
+  else
+    return p.tk > 256 ? launch_attention<HD, 8, 4>(p, batch) : launch_attention<HD, 8, 1>(p, batch);
+}
+
+template <int HD, int ATT_WAVES, int PER_WAVE>
+hipError_t allow_lds() {
+  return hipFuncSetAttribute(reinterpret_cast<const void *>(attention_rows_kernel<HD, ATT_WAVES, PER_WAVE>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
 }
 
 }  // namespace
@@ -268,13 +293,9 @@ namespace wdh {
 // More than 64 KB of dynamic LDS has to be asked for once per kernel and device (called by
 // wdh_init with the device current, so that no launch -- captured ones included -- has to).
 int init_attention() {
-  const int limit = 160 * 1024;
-  WDH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_rows_kernel<32, 16>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, limit));
-  WDH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_rows_kernel<64, 8>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, limit));
-  WDH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(attention_rows_kernel<128, 8>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, limit));
+  for (hipError_t e : {allow_lds<32, 16, 2>(), allow_lds<32, 16, 1>(), allow_lds<64, 8, 4>(), allow_lds<64, 16, 1>(),
+                       allow_lds<64, 8, 1>(), allow_lds<128, 8, 4>(), allow_lds<128, 8, 1>()})
+    WDH_HIP_CHECK(e);
   return WDH_OK;
 }
 }  // namespace wdh
@@ -316,7 +337,7 @@ extern "C" int wdh_attention(wdh_buf hQ, wdh_buf hK, wdh_buf hV, wdh_buf hY, int
   p.tq = tq; p.tk = tk; p.pitch = lds_pitch(tk); p.row_blocks = (int)row_blocks;
   p.sQb = sQb; p.sQi = sQi; p.sKb = sKb; p.sKj = sKj; p.sVb = sVb; p.sVj = sVj; p.sYb = sYb; p.sYi = sYi;
   p.alpha = alpha;
-  if (d == 32) return launch_attention<32, 16>(p, batch);
-  if (d == 64) return launch_attention<64, 8>(p, batch);
-  return launch_attention<128, 8>(p, batch);
+  if (d == 32) return launch_attention<32>(p, batch);
+  if (d == 64) return launch_attention<64>(p, batch);
+  return launch_attention<128>(p, batch);
 }
