@@ -662,7 +662,8 @@ constexpr int STAGE_FLOATS = 32 * STAGE_LD;
 // rows 8*(r/4) + 4*half + r%4 for accumulator register r.  Chunk workgroups store raw
 // sums for splitk_reduce_kernel; whole tiles apply alpha, the C/bias term, the
 // residual and Relu and store to Y (NCHW for CONV).
-template <int BM, int BN, int WM, int WN, bool CONV>
+// LOOK: how far ahead the bias and the residual of a wide tile are requested (see there).
+template <int BM, int BN, int WM, int WN, bool CONV, int LOOK = (BM / (WM * 32)) * (BN / (WN * 32)) <= 2 ? 1 : 0>
 __device__ __forceinline__ void finish_tile(const Params &p,
                                             f32x16 (&acc)[BM / (WM * 32)][BN / (WN * 32)],
                                             bool whole, int lin, int chunk, int bz, int row0,
@@ -705,6 +706,81 @@ __device__ __forceinline__ void finish_tile(const Params &p,
     const rsrc_t rsrc_c = make_rsrc(p.C ? p.C : p.Y, p.C ? p.c_bytes : 0);
     const int lr = lane >> 3, lc = (lane & 7) * 4;  // row (of every eight) and first column
     const bool c_per_row = CONV || p.sC1 == 0;
+    // LOOK 2 (the main loop's other registers leave room): a block's bias and residual are requested before the block
+    // before it is stored.  Loads and stores of a wavefront come back in order, so that a load asked for behind a store waits for that
+    // store, and sixteen row groups of a 128x128 tile are as many round trips.
+    // (us, 128 images, 128x128 tiles: 128 -> 512 on 28x28 with a residual 191 -> 166, 256 -> 1024 on 14x14 110 -> 101, 64 -> 256 on
+    // 56x56 279 -> 209; the whole tile's requests up front are no faster.)
+    if constexpr (LOOK == 2) {
+      auto blocks = [&](auto with_r) {
+        constexpr bool RES = decltype(with_r)::value;
+        int voff_y[NT], voff_c[NT], ystride = 0, cstride = 1;
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+          const int col = col0 + wcol + nt * 32 + lc;
+          int ybase = col;
+          if (CONV) {
+            const unsigned ohw = (unsigned)(p.cv.oh * p.cv.ow);
+            const unsigned img = (unsigned)fdiv(col, p.cv.fd_ohw);
+            ybase = (int)((img * (unsigned)p.cv.cout_total + (unsigned)(bz * p.cv.cout_g)) * ohw +
+                          ((unsigned)col - img * ohw));
+            ystride = (int)ohw;
+            voff_c[nt] = (bz * p.cv.cout_g + lr) * 4;
+          } else {
+            ystride = (int)p.sY0;
+            voff_c[nt] = (int)((lr * p.sC0 + col * p.sC1) * 4);
+            cstride = (int)p.sC0;
+          }
+          voff_y[nt] = (ybase + lr * ystride) * 4;
+        }
+        f32x4 cv[2][4], rv[2][4];
+        auto request = [&](int b) {
+          const int nt = b / MT, rbase = __builtin_amdgcn_readfirstlane(row0 + wrow + b % MT * 32);
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            if (p.C) {
+              const int soff = (rbase + 8 * i) * cstride * 4;
+              if (c_per_row) {
+                const float c = buf_load(rsrc_c, voff_c[nt], soff);
+                cv[b & 1][i] = f32x4{c, c, c, c};
+              } else {
+                cv[b & 1][i] = buf_load4(rsrc_c, voff_c[nt], soff);
+              }
+            }
+            if constexpr (RES) rv[b & 1][i] = buf_load4(rsrc_r, voff_y[nt], (rbase + 8 * i) * ystride * 4);
+          }
+        };
+        request(0);
+#pragma unroll
+        for (int b = 0; b < MT * NT; b++) {
+          const int nt = b / MT, mt = b % MT;
+          const int rbase = __builtin_amdgcn_readfirstlane(row0 + wrow + mt * 32);
+          if (b + 1 < MT * NT) request(b + 1);
+          __builtin_amdgcn_wave_barrier();  // the previous block's reads come first
+#pragma unroll
+          for (int r = 0; r < 16; r++)
+            st[(8 * (r >> 2) + 4 * half + (r & 3)) * STAGE_LD + li] = acc[mt][nt][r];
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(&st[(lr + 8 * i) * STAGE_LD + lc]);
+            f32x4 y;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              float t = CONV ? v[e] : p.alpha * v[e];
+              if (p.C) t = CONV ? t + cv[b & 1][i][e] : __builtin_fmaf(cv[b & 1][i][e], p.beta, t);
+              if constexpr (RES) t = t + rv[b & 1][i][e];
+              if (p.epilogue == WDH_EPI_RELU) t = relu_js(t);
+              y[e] = t;
+            }
+            buf_store4(rsrc_y, y, voff_y[nt] + (rbase + 8 * i) * ystride * 4);  // (offset: see below)
+          }
+        }
+      };
+      if (p.R) blocks(std::true_type{});
+      else blocks(std::false_type{});
+      return;
+    }
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) {
       const int col = col0 + wcol + nt * 32 + lc;
@@ -730,7 +806,7 @@ __device__ __forceinline__ void finish_tile(const Params &p,
         // Tiles with one or two blocks per wavefront have registers to spare and request the
         // bias / residual values of all four row groups before the first is used; the
         // 64-accumulator tiles request them row group by row group (anything else spills).
-        constexpr bool AHEAD = MT * NT <= 2;
+        constexpr bool AHEAD = LOOK == 1;
         f32x4 cv[AHEAD ? 4 : 1], rv[AHEAD ? 4 : 1];
         auto request = [&](int i, int slot) {
           if (p.C) {

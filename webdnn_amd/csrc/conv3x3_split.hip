@@ -247,7 +247,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
           acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(ea[mt], eb[nt], acc[mt][nt], 0, 0, 0);
     }
   }
-  finish_tile<BM, BN, WM, WN, true>(p, acc, tw.whole, tw.lin, tw.chunk, 0, row0, col0,
+  finish_tile<BM, BN, WM, WN, true, 2>(p, acc, tw.whole, tw.lin, tw.chunk, 0, row0, col0,
                                     reinterpret_cast<float *>(xs) + wave * STAGE_FLOATS);
 }
 
