@@ -1472,8 +1472,10 @@ def test_attention_at_the_key_counts_where_the_form_changes(ctx, tk, d):
     q, k = rng.standard_normal((33, 3 * d)).astype(np.float32), rng.standard_normal((tk, 3 * d)).astype(np.float32)
     v = np.full((tk + 1, 3 * d), np.nan, np.float32)
     v[:tk] = rng.standard_normal((tk, 3 * d))
-    held = ctx.move_tensor(v)
-    got = H.attention(ctx, ctx.move_tensor(q), ctx.move_tensor(k), held.alias([tk, 3 * d]), 3, 1.0 / np.sqrt(d)).get_data()
+    tq, tk_, tv, y = ctx.move_tensor(q), ctx.move_tensor(k), ctx.move_tensor(v), ctx.empty_tensor([33, 3 * d])
+    strides = (d, 3 * d) * 4
+    capi.call("wdh_attention", tq.handle, tk_.handle, tv.handle, y.handle, 3, 33, tk, d, *strides, float(1.0 / np.sqrt(d)))
+    got = y.get_data()
     assert_close_max(got, attention_chain_ref(q, k, v[:tk], 3, 1.0 / np.sqrt(d)), GEMM_TOL, "attention vs oracle chain")
 
 
