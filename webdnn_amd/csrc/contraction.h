@@ -710,7 +710,8 @@ __device__ __forceinline__ void finish_tile(const Params &p,
     // before it is stored.  Loads and stores of a wavefront come back in order, so that a load asked for behind a store waits for that
     // store, and sixteen row groups of a 128x128 tile are as many round trips.
     // (us, 128 images, 128x128 tiles: 128 -> 512 on 28x28 with a residual 191 -> 166, 256 -> 1024 on 14x14 110 -> 101, 64 -> 256 on
-    // 56x56 279 -> 209; the whole tile's requests up front are no faster.)
+    // 56x56 279 -> 209; the whole tile's requests up front are no faster, nor is this for tiles of one or two blocks a
+    // wavefront: a 6-layer encoder 819, 810 with LOOK 1.)
     if constexpr (LOOK == 2) {
       auto blocks = [&](auto with_r) {
         constexpr bool RES = decltype(with_r)::value;

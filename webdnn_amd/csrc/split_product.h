@@ -417,7 +417,7 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
           acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(ea[mt], eb[nt], acc[mt][nt], 0, 0, 0);
     }
   }
-  finish_tile<BM, BN, WM, WN, CONV, 2>(p, acc, tw.whole, tw.lin, tw.chunk, bz, row0, col0,
+  finish_tile<BM, BN, WM, WN, CONV, (MT * NT > 2 ? 2 : 1)>(p, acc, tw.whole, tw.lin, tw.chunk, bz, row0, col0,
                                     reinterpret_cast<float *>(&lds[0][0]) + wave * STAGE_FLOATS);
 }
 
