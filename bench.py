@@ -53,6 +53,7 @@ if ROOT not in sys.path:
 import numpy as np  # noqa: E402
 
 METRIC = "fp32 Gemm/Conv GFLOP/s (% MFMA peak) + ResNet-50 b32 images/sec, 1 MI355X"
+# The fp32 matrix instruction's peak.  fp32 products made of six bf16 ones (csrc/split_product.h) may exceed it.
 PEAK_FP32_MFMA_TFLOPS = 157.3
 # HBM-side bytes of the ResNet-50 step per Conv / Gemm node (54 nodes; contraction kernels, reduce passes
 # and the transforms of the minimal-filtering convs): rocprofv3 --pmc FETCH_SIZE (x2.000) + WRITE_SIZE
@@ -522,7 +523,8 @@ def main():
         "roofline": {
             "bound": "mfma",
             "kernel": "contraction kernels (implicit-GEMM Conv: in-place 1x1, LDS-tile 3x3, F(2x2,3x3) minimal filtering "
-                      "for 3x3 from 128 channels on, gathered forms, stem; Gemm head), %d Conv/Gemm nodes per step; device "
+                      "for 3x3 from 256 channels on, gathered forms, stem; Gemm head; most as six bf16 products on operands split "
+                      "exactly, so that peak, the fp32 instruction's, is no limit), %d Conv/Gemm nodes per step; device "
                       "time = HIP events around each timed graph replay (whole step: transforms, MaxPool and "
                       "GlobalAveragePool included); achieved = direct-sum FLOPs (2MNK per node) / that time"
                       % resnet["contraction_launches"],
