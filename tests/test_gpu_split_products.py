@@ -291,17 +291,74 @@ def test_recorded_weights_outlive_another_size(ctx, split):
         ctx.graph_destroy(graph)
 
 
-@pytest.mark.parametrize("shift", [-120, -112, -100])
-def test_rows_of_tiny_elements(ctx, split, shift):
-    """Elements whose last part does not fit bfloat16 leave tiny sums, which are added up again, also against large partners."""
+# exponents of the tiny operand and of its partners: some bits lost, all lost, subnormal floats; results from 2^-128 to 2^-17
+TINY = [(-112, 40), (-118, 12), (-118, 100), (-126, 64), (-126, 100), (-135, 100), (-140, 12), (-140, 100)]
+
+
+def uniform(rng, shape, exponent):
+    return (rng.uniform(1, 2, shape) * 2.0 ** exponent).astype(np.float32)
+
+
+def sums_hold(got, want, magnitudes, k):
+    """As `within`, down to the least float there is."""
+    return (np.abs(got - want) <= (k + 8) * 2.0 ** -24 * magnitudes + k * 2.0 ** -149).all()
+
+
+@pytest.mark.parametrize("mode", [3, 6, 7, 8, 9])
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("tiny,partner", TINY)
+def test_tiny_elements(ctx, split, mode, transposed, tiny, partner):
+    """Elements that bfloat16 parts hold in part or not at all, as the left and as the right operand, nothing else in the tile."""
     rng = np.random.default_rng(11)
-    a = (rng.uniform(1, 2, (256, 512)) * 2.0 ** shift).astype(np.float32)
-    b = (rng.uniform(1, 2, (512, 256)) * 2.0 ** 40).astype(np.float32)
-    split(3)
+    a, b = uniform(rng, (256, 144), tiny), uniform(rng, (144, 256), partner)
+    split(mode)
+    ctx.set_option("gemm_wavesplit", 0)
+    try:
+        for l, r in ((a, b), (np.ascontiguousarray(b.T), np.ascontiguousarray(a.T))):
+            got = product(ctx, l, r, transposed)
+            assert ctx.last_plan()["tile"] == TILES[mode]
+            want = l.astype(np.float64) @ r.astype(np.float64)
+            assert sums_hold(got, want, want, 144)
+    finally:
+        ctx.set_option("gemm_wavesplit", 1)
+
+
+@pytest.mark.parametrize("mode", [3, 9])
+@pytest.mark.parametrize("chunks", [1, 3])
+@pytest.mark.parametrize("partner", [100, 30, -3])
+def test_tiny_elements_among_others(ctx, split, mode, chunks, partner):
+    """One of them in a row of ordinary elements: it counts where its partner lifts it, and every sum is far above 2^-60."""
+    rng = np.random.default_rng(12)
+    a, b = uniform(rng, (256, 192), -30), uniform(rng, (192, 256), -20)
+    for at in (0, 100, 191):   # (one in each chunk)
+        a[:, at], b[at] = uniform(rng, 256, -126), uniform(rng, 256, partner)
+    split(mode)
+    ctx.set_option("split_k", chunks)
     got = product(ctx, a, b, False)
-    assert ctx.last_plan()["tile"] == "128x128"
+    assert ctx.last_plan()["tile"] == TILES[mode] and ctx.last_plan()["split"] == chunks
     a, b = a.astype(np.float64), b.astype(np.float64)
-    assert within(got, a @ b, a @ b, 512)
+    assert sums_hold(got, a @ b, a @ b, 192)
+
+
+@pytest.mark.parametrize("mode", [3, 4])
+@pytest.mark.parametrize("kernel,stride", [(3, 1), (3, 2), (1, 1), (1, 2)])
+@pytest.mark.parametrize("tiny,partner", TINY)
+def test_tiny_elements_of_convs(ctx, split, mode, kernel, stride, tiny, partner):
+    """The same in the input and in the weights (which the 3x3 form lays out beforehand)."""
+    rng = np.random.default_rng(13)
+    split(mode)
+    ctx.set_option("conv3x3_winograd", 0)
+    for ex, ew in ((tiny, partner), (partner, tiny)):
+        x, w = uniform(rng, (2, 32, 12, 12), ex), uniform(rng, (128, 32, kernel, kernel), ew)
+        tw = ctx.move_tensor(w)
+        pad = kernel // 2
+        padded = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (pad, pad), (pad, pad)))
+        windows = np.lib.stride_tricks.sliding_window_view(padded, (kernel, kernel), (2, 3))[:, :, ::stride, ::stride]
+        want = np.einsum("ncyxij,ocij->noyx", windows, w.astype(np.float64))
+        for constant in (False, True, True):
+            got = H.conv(ctx, ctx.move_tensor(x), tw, pads=[pad] * 4, strides=[stride, stride], constant_weights=constant).get_data()
+            assert ctx.last_plan()["tile"] == TILES[mode]
+            assert sums_hold(got, want, want, 32 * kernel * kernel)
 
 
 def test_groups_that_fill_the_chip(ctx, split):

@@ -8,6 +8,7 @@
 // from its pixel's corner, neighbouring lanes side by side.  Rows and columns of padding are slots that are filled with zeros
 // (loads outside the descriptor).  The weights are laid out fragment by fragment beforehand (pack_kernel; kept per weight
 // buffer when the caller vouches for it), [32 rows][block, tap][h, m, l][lane][8 channels], and go from L2 straight into registers.
+// Behind them a word for each [32 rows][block, tap] says what the split has to know of its weights (WEIGHTS_*).
 #include <string.h>
 
 #include "split_product.h"
@@ -16,6 +17,8 @@ namespace wdhc {
 
 constexpr int CB = 16;          // channels per block
 constexpr int KGRAN = CB * 9;   // k per block
+constexpr unsigned WEIGHTS_LOSE = 1, WEIGHTS_LARGE = 2;  // some lose bits; some reach 2^30 (split_product.h)
+__host__ __device__ constexpr long long fragment_bytes(long long rows, long long steps) { return (rows + 31) / 32 * steps * 3072; }
 
 // One thread: one lane's eight channels of one (row block, channel block, tap).
 __global__ __launch_bounds__(256) void pack3x3_kernel(const float *__restrict__ W, u32x4 *__restrict__ P, int cout, int c) {
@@ -29,14 +32,21 @@ __global__ __launch_bounds__(256) void pack3x3_kernel(const float *__restrict__ 
   float w[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) w[j] = row < cout ? W[((long long)row * c + c0 + j) * 9 + tap] : 0.0f;
+  unsigned least = 0xffffffffu;
+  bool large = false;
+#pragma unroll
+  for (int j = 0; j < 8; j++) large |= reaches_partners(w[j]);
   u32x4 h, m, l;
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const SplitPair s = split_pair(w[2 * j], w[2 * j + 1]);
+    least = least_of(least, w[2 * j], w[2 * j + 1]);
     h[j] = s.h;
     m[j] = s.m;
     l[j] = s.l;
   }
+  const unsigned word = (__any(loses_bits(least)) ? WEIGHTS_LOSE : 0) | (__any(large) ? WEIGHTS_LARGE : 0);
+  if (lane == 0) reinterpret_cast<unsigned *>(reinterpret_cast<char *>(P) + fragment_bytes(cout, steps))[at] = word;
   u32x4 *const p = P + at * 192 + lane;
   p[0] = h;
   p[64] = m;
@@ -92,7 +102,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
   }
   const rsrc_t rsrc_x = make_rsrc(p.B, p.b_bytes);
   const int steps = p.k / CB;  // (block, tap) steps of a row block
-  const rsrc_t rsrc_a = make_rsrc(packed, (int)((long long)((p.m + 31) / 32) * steps * 3072));
+  const rsrc_t rsrc_a = make_rsrc(packed, (int)fragment_bytes(p.m, steps));
 
   // where a lane finds the corner of its pixels, and its row blocks' weights
   int corner[NT], voff_a[MT];
@@ -119,6 +129,19 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[a][b][r] = small[a][b][r] = 0.0f;
 
+  // what is known of the weights of this tile and chunk
+  auto weights_have = [&](unsigned what) {
+    const unsigned *const words = reinterpret_cast<const unsigned *>(reinterpret_cast<const char *>(packed) + fragment_bytes(p.m, steps));
+    const int count = (kend - kbeg) / CB;
+    unsigned w = 0;
+#pragma unroll
+    for (int i = 0; i < BM / 32; i++)
+      if (row0 + 32 * i < p.m)
+        for (int j = tid; j < count; j += THREADS) w |= words[(row0 / 32 + i) * steps + kbeg / CB + j];
+    return __any((w & what) != 0);
+  };
+  bool lost = false;  // whether this wavefront has met elements that lose bits
+
   float x[XU][8];
   auto fetch_x = [&](int k0) {  // the block of channels that begins at k0
     const int soff = k0 / 9 * plane_in * 4;
@@ -128,12 +151,14 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
       for (int j = 0; j < 8; j++) x[i][j] = buf_load(rsrc_x, voff_x[i], soff + j * plane_in * 4);
   };
   auto put_x = [&]() {
+    unsigned least = 0xffffffffu;
 #pragma unroll
     for (int i = 0; i < XU; i++) {
       u32x4 h, m, l;
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         const SplitPair s = split_pair(x[i][2 * j], x[i][2 * j + 1]);
+        least = least_of(least, x[i][2 * j], x[i][2 * j + 1]);
         h[j] = s.h;
         m[j] = s.m;
         l[j] = s.l;
@@ -144,6 +169,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
         *reinterpret_cast<u32x4 *>(xs + lds_x[i] + 2 * PLANE_X) = l;
       }
     }
+    lost |= __any(loses_bits(least));
   };
   struct Frags { bf16x8 a[MT][3], b[NT][3]; };
   auto fetch_a = [&](int step, Frags &f) {
@@ -171,6 +197,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
   Frags f[2];
   fetch_x(kbeg);
   fetch_a(kbeg / CB, f[0]);
+  lost = weights_have(WEIGHTS_LOSE);
   for (int k0 = kbeg; k0 < kend; k0 += KGRAN) {
     if (k0 != kbeg) __syncthreads();  // everybody has read the block before
     put_x();
@@ -197,7 +224,7 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
   }
 
   // the two sums meet; what the split could not hold is done again (split_product.h)
-  unsigned most = 0, least = 0xffffffffu;
+  SumRange sums = {0xffffffffu, 0};
 #pragma unroll
   for (int a = 0; a < MT; a++)
 #pragma unroll
@@ -205,11 +232,21 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         acc[a][b][r] += small[a][b][r];
-        const unsigned u = __float_as_uint(acc[a][b][r]) << 1;
-        most = u > most ? u : most;
-        least = u - 1u < least ? u - 1u : least;
+        add_sum(sums, acc[a][b][r]);
       }
-  if (__syncthreads_or(split_fails(most, least))) {
+  bool again = __syncthreads_or(not_finite(sums) || lost);
+  if (again && !__syncthreads_or(not_finite(sums) || small_sums(sums))) {
+    bool large = weights_have(WEIGHTS_LARGE);
+    for (int k0 = kbeg; k0 < kend; k0 += KGRAN) {
+      fetch_x(k0);
+#pragma unroll
+      for (int i = 0; i < XU; i++)
+#pragma unroll
+        for (int j = 0; j < 8; j++) large |= reaches_partners(x[i][j]);
+    }
+    again = __syncthreads_or(large);
+  }
+  if (again) {
 #pragma unroll
     for (int a = 0; a < MT; a++)
 #pragma unroll
@@ -251,7 +288,10 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
                                     reinterpret_cast<float *>(xs) + wave * STAGE_FLOATS);
 }
 
-size_t packed3x3_bytes(int cout, int c) { return (size_t)((cout + 31) / 32) * (c / CB) * 9 * 3072; }
+size_t packed3x3_bytes(int cout, int c) {
+  const long long steps = c / CB * 9;
+  return (size_t)(fragment_bytes(cout, steps) + ((cout + 31) / 32 * steps) * 4);
+}
 
 int pack3x3_launch(const float *W, void *P, int cout, int c) {
   const long long threads = (long long)((cout + 31) / 32) * (c / CB) * 9 * 64;

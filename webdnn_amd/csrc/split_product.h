@@ -14,9 +14,9 @@
 //
 // Bound: power.  A loop of nothing but these instructions runs at 1550 to 1800 TFLOP/s, which is 260 to 300 of fp32
 // products (the fp32 instruction's own limit is 157); at 4096^3 the matrix cores are busy 79 % of the cycles and the clock
-// falls to 1.5 GHz.  What a slab adds to the products is the split (11 vector instructions per pair of elements) and
-// LDS traffic (6 bytes an element), so an operand is split once, on its way from registers to LDS, not by every
-// wavefront that multiplies it.  The split and the LDS stores of the next slab are placed between the matrix
+// falls to 1.5 GHz.  What a slab adds to the products is the split (14 vector instructions per pair of elements, three of
+// them to look at it) and LDS traffic (6 bytes an element), so an operand is split once, on its way from registers to LDS,
+// not by every wavefront that multiplies it.  The split and the LDS stores of the next slab are placed between the matrix
 // instructions of this one (sched_group_barrier): 195 -> 209 TFLOP/s, because the wavefronts of a SIMD else meet the same phase
 // at the same time.  Measured at 4096^3 (TFLOP/s; fp32 instruction 146): 64x64 tiles 159, 64x128 and 128x64 181, 128x128 209,
 // 256x128 210 to 222.  Tried without gain: fragments of the next slab read ahead (204), loads two to eight slabs ahead (204), small
@@ -24,10 +24,13 @@
 //
 // What the split cannot hold is done again with the fp32 instruction, a whole tile (or chunk) at a time:
 //   * an Inf or NaN operand leaves NaN in x - h and therefore in every sum it enters; so does a sum that overflows;
-//   * elements below 2^-110 lose bits of l below 2^-133.  Only a sum of such elements shows that, and it is tiny unless
-//     their partners are beyond 2^50: a tile that holds a nonzero sum below 2^-60 is done again.  (Terms around
-//     one do not cancel down to there: what they leave is zero or a rounding, 2^-24 of a term.)
-// Both show in the sums themselves, so the loop carries no test.
+//   * bfloat16 ends at 2^-133 (parts and results below 2^-126 are kept, by the conversion and by the matrix instruction): an element
+//     below 2^-110 loses up to 2^-134, one below 2^-134 all of itself.  So every element is looked at where it is split (least_of).
+//     The sums cannot tell: large partners lift what is left of such an element to any size, and one that vanished leaves a
+//     zero.  A tile with such elements is done again unless all its sums are at least 2^-60 and no operand element reaches
+//     2^30: then K terms are off by at most K 2^-104, beyond the last bits of the sums.  (That keeps softmax rows and
+//     weights with a few vanishing elements on the fast path.  The look costs a net of two 4096^3 products and a narrow one
+//     1411 -> 1428 us, ResNet-50 of 128 images 6965 -> 7034.)
 #pragma once
 #include "contraction.h"
 
@@ -50,11 +53,27 @@ __device__ __forceinline__ SplitPair split_pair(float x0, float x1) {
   return SplitPair{h, m, nearest_pair(s0, s1)};
 }
 
-// Whether a tile holds a sum that the split cannot vouch for, from the largest and the least (zeros aside) of the doubled
-// bits of its sums: not finite, or nonzero below 2^-60.
-__device__ __forceinline__ bool split_fails(unsigned most, unsigned least) {
-  return most >= 0xff000000u || least < ((127u - 60u) << 24) - 1u;
+// The least nonzero magnitude of what was split, as doubled bits less one (a zero becomes the largest), and what it and the sums say.
+__device__ __forceinline__ unsigned least_of(unsigned least, float x0, float x1) {
+  const unsigned u0 = (__float_as_uint(x0) << 1) - 1u, u1 = (__float_as_uint(x1) << 1) - 1u;
+  const unsigned u = u0 < u1 ? u0 : u1;
+  return u < least ? u : least;
 }
+constexpr unsigned doubled_bits(int exponent) { return (unsigned)(127 + exponent) << 24; }
+__device__ __forceinline__ bool loses_bits(unsigned least) { return least < doubled_bits(-110) - 1u; }
+__device__ __forceinline__ bool reaches_partners(float x) { return (__float_as_uint(x) << 1) >= doubled_bits(30); }
+__device__ __forceinline__ bool reaches_partners(f32x4 v) {
+  return reaches_partners(v.x) | reaches_partners(v.y) | reaches_partners(v.z) | reaches_partners(v.w);
+}
+// The range of a tile's sums, as doubled bits.
+struct SumRange { unsigned least, most; };
+__device__ __forceinline__ void add_sum(SumRange &g, float x) {
+  const unsigned u = __float_as_uint(x) << 1;
+  g.most = u > g.most ? u : g.most;
+  g.least = u < g.least ? u : g.least;
+}
+__device__ __forceinline__ bool not_finite(const SumRange &g) { return g.most >= doubled_bits(128); }
+__device__ __forceinline__ bool small_sums(const SumRange &g) { return g.least < doubled_bits(-60); }
 
 // Workgroups a CU holds: the accumulators are two per result, so 128x128 tiles take 64 + 64 registers of
 // accumulators and two of them fit; 256x128 is the same wavefront with eight of them in one workgroup.
@@ -227,7 +246,9 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
       }
     }
   };
+  unsigned least = 0xffffffffu;  // of this thread's pieces
   auto put4 = [&](unsigned char *cell, int plane, f32x4 v) {
+    least = least_of(least_of(least, v.x, v.y), v.z, v.w);
     const SplitPair lo = split_pair(v.x, v.y), hi = split_pair(v.z, v.w);
     *reinterpret_cast<u32x2 *>(cell) = u32x2{lo.h, hi.h};
     *reinterpret_cast<u32x2 *>(cell + plane) = u32x2{lo.m, hi.m};
@@ -304,7 +325,7 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
     put(lds[cur ^ 1], now);
     // fragment reads, requests, then products with the split and the stores in between
     constexpr int PIECES = NA + (B_IS_KC ? NB : (IM2COL ? L / 4 : CPP));
-    constexpr int PRODUCTS = MT * NT * 6, VALU = PIECES * 22 + (IM2COL ? 2 * L : 0), STORES = PIECES * 3;
+    constexpr int PRODUCTS = MT * NT * 6, VALU = PIECES * 28 + (IM2COL ? 2 * L : 0), STORES = PIECES * 3;
     constexpr int LOADS = NA + (B_IS_KC ? NB : (IM2COL ? L : PIX_ANY ? 4 * CPP : 4));
     __builtin_amdgcn_sched_group_barrier(0x100, (MT + NT) * 3, 0);
     __builtin_amdgcn_sched_group_barrier(0x20, LOADS, 0);
@@ -332,20 +353,35 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
   }
 
   // ---- the two sums meet; is there anything the split could not hold? ------------------------------------
-  // (bits of |sum| doubled: zero is fine, so is 2^-60 up to the largest float)
-  unsigned most = 0, least = 0xffffffffu;
+  SumRange sums = {0xffffffffu, 0};
 #pragma unroll
-  for (int a = 0; a < MT; a++)
+  for (int b = 0; b < NT; b++)
 #pragma unroll
-    for (int b = 0; b < NT; b++)
+    for (int a = 0; a < MT; a++)
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         acc[a][b][r] += small[a][b][r];
-        const unsigned u = __float_as_uint(acc[a][b][r]) << 1;
-        most = u > most ? u : most;
-        least = u - 1u < least ? u - 1u : least;
+        add_sum(sums, acc[a][b][r]);
       }
-  const bool again = __syncthreads_or(split_fails(most, least));
+  bool again = __syncthreads_or(not_finite(sums) || loses_bits(least));
+  if (again && !__syncthreads_or(not_finite(sums) || small_sums(sums))) {
+    // (elements that lost bits, but every sum is large: what were their partners?)
+    bool large = false;
+    read_taps(kbeg);
+    for (int k0 = kbeg; k0 < kend; k0 += 2 * BK) {
+      Slab q[2];
+      fetch(k0, q[0], true);
+      fetch(k0 + BK, q[1], true);
+#pragma unroll
+      for (const Slab &s : q) {
+#pragma unroll
+        for (const f32x4 &v : s.a) large |= reaches_partners(v);
+#pragma unroll
+        for (const f32x4 &v : s.b) large |= reaches_partners(v);
+      }
+    }
+    again = __syncthreads_or(large);
+  }
   if (KG > 1 && !again) {
     // sums of the groups behind the first, in order; each through its own LDS
     float *const mine = reinterpret_cast<float *>(&lds[0][0]);
