@@ -361,6 +361,29 @@ def test_tiny_elements_of_convs(ctx, split, mode, kernel, stride, tiny, partner)
             assert sums_hold(got, want, want, 32 * kernel * kernel)
 
 
+@pytest.mark.parametrize("mode,form", [(1, 1), (3, 1), (6, 3)])
+def test_transformed_convs_do_not_see_what_the_pool_held(ctx, split, mode, form):
+    """60 (20) tiles in rows of 64 (32): what lies behind them is not another matrix's rest."""
+    rng = np.random.default_rng(14)
+    n, c, h, w = 5, 512, 6, 8
+    x = ctx.move_tensor(rng.standard_normal((n, c, h, w)).astype(np.float32))
+    wt = ctx.move_tensor((rng.standard_normal((c, c, 3, 3)) * 0.02).astype(np.float32))
+    split(mode)
+    ctx.set_option("conv3x3_winograd", form)
+    positions, pitch = (16, 64) if form == 1 else (36, 32)
+    elements = positions * c * pitch
+    out = []
+    for junk in (np.zeros(elements, np.float32), np.full(elements, np.nan, np.float32), np.full(elements, 5, np.int32)):
+        held = [ctx.move_tensor(junk) for _ in range(4)]
+        for t in held:
+            t.dispose()
+        y = H.conv(ctx, x, wt, pads=[1] * 4)
+        assert "transforms" in ctx.last_plan()["form"], ctx.last_plan()
+        out.append(y.get_data())
+        y.dispose()
+    assert (out[0] == out[1]).all() and (out[0] == out[2]).all()
+
+
 def test_groups_that_fill_the_chip(ctx, split):
     """The projections of an attention block as one launch of 64x64 tiles; ragged rows and columns, one weight k-contiguous by shape."""
     rng = np.random.default_rng(9)

@@ -65,11 +65,13 @@ __global__ __launch_bounds__(256) void wino_filter_kernel(const float *__restric
 }
 
 // V[xi][ci][t] = (Bt d B)[xi] for the 4x4 patch d of channel ci whose corner is input pixel
-// (2 ty - pt, 2 tx - pl) of the tile's image; pixels outside the image are 0.
-// grid (ceil(tiles / 256), c): consecutive threads take consecutive tiles of one channel.
+// (2 ty - pt, 2 tx - pl) of the tile's image; pixels outside the image are 0, and so are the columns from
+// the last tile to the row's end.
+// grid (ceil(pitch / 256), c): consecutive threads take consecutive tiles of one channel.
 __global__ __launch_bounds__(256) void wino_input_kernel(const float *__restrict__ X, float *__restrict__ V, WinoGeom g) {
   const int t = blockIdx.x * 256 + threadIdx.x, ci = blockIdx.y;
-  if (t >= g.tiles) return;
+  if (t >= g.pitch) return;
+  const bool tile = t < g.tiles;
   const int img = fdiv(t, g.fd_thw), r = t - img * (g.th * g.tw);
   const int ty = fdiv(r, g.fd_tw), tx = r - ty * g.tw;
   const int iy0 = 2 * ty - g.pt, ix0 = 2 * tx - g.pl;
@@ -78,7 +80,7 @@ __global__ __launch_bounds__(256) void wino_input_kernel(const float *__restrict
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int iy = iy0 + i;
-    const bool row_in = (unsigned)iy < (unsigned)g.h;
+    const bool row_in = tile && (unsigned)iy < (unsigned)g.h;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       const int ix = ix0 + j;
@@ -213,7 +215,8 @@ __global__ __launch_bounds__(256) void wino4_filter_kernel(const float *__restri
 
 __global__ __launch_bounds__(256) void wino4_input_kernel(const float *__restrict__ X, float *__restrict__ V, WinoGeom g) {
   const int t = blockIdx.x * 256 + threadIdx.x, ci = blockIdx.y;
-  if (t >= g.tiles) return;
+  if (t >= g.pitch) return;
+  const bool tile = t < g.tiles;
   const int img = fdiv(t, g.fd_thw), r = t - img * (g.th * g.tw);
   const int ty = fdiv(r, g.fd_tw), tx = r - ty * g.tw;
   const int iy0 = 4 * ty - g.pt, ix0 = 4 * tx - g.pl;
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(256) void wino4_input_kernel(const float *__restric
 #pragma unroll
   for (int j = 0; j < 6; j++) {
     const int ix = ix0 + j;
-    const bool col_in = (unsigned)ix < (unsigned)g.w;
+    const bool col_in = tile && (unsigned)ix < (unsigned)g.w;
     float d[6], o[6];
 #pragma unroll
     for (int i = 0; i < 6; i++) {
@@ -291,9 +294,9 @@ namespace wdh {
 
 // r: the output block size, 2 for F(2x2, 3x3) (16 positions) or 4 for F(4x4, 3x3) (36 positions)
 long long wino_tiles(int r, int n, int oh, int ow) { return (long long)n * ((oh + r - 1) / r) * ((ow + r - 1) / r); }
-// Row length of V and M: rows start on 64-byte boundaries whatever the tile count (the columns past the
-// last tile are never written by the input transform and never read by the output transform; what the
-// product makes of them stays in them, every column of a matrix product being independent of the others).
+// Row length of V and M: rows start on 64-byte boundaries whatever the tile count.  The columns past the
+// last tile are zeros in V and never read in M: the product on the bf16 matrix cores looks at whole tiles of
+// operands and sums, so what a pool block held before must not be among them.
 long long wino_pitch(long long tiles) { return (tiles + 15) / 16 * 16; }
 
 int wino_filter_launch(int r, const float *W, float *U, int cout, int c) {
@@ -318,7 +321,7 @@ static WinoGeom make_geom(int r, int n, int c, int h, int w, int cout, int oh, i
 
 int wino_input_launch(int r, const float *X, float *V, int n, int c, int h, int w, int oh, int ow, int pt, int pl) {
   const WinoGeom g = make_geom(r, n, c, h, w, 0, oh, ow, pt, pl);
-  const dim3 grid((unsigned)((g.tiles + 255) / 256), (unsigned)c);
+  const dim3 grid((unsigned)((g.pitch + 255) / 256), (unsigned)c);
   if (r == 2) hipLaunchKernelGGL(wino_input_kernel, grid, dim3(256), 0, stream(), X, V, g);
   else hipLaunchKernelGGL(wino4_input_kernel, grid, dim3(256), 0, stream(), X, V, g);
   WDH_LAUNCH_CHECK();
