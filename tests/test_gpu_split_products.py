@@ -3,6 +3,7 @@ instruction."""
 import numpy as np
 import pytest
 
+from webdnn_amd import capi
 from webdnn_amd import hostops as H
 
 pytestmark = pytest.mark.gpu
@@ -381,6 +382,30 @@ def test_transformed_convs_do_not_see_what_the_pool_held(ctx, split, mode, form)
         assert "transforms" in ctx.last_plan()["form"], ctx.last_plan()
         out.append(y.get_data())
         y.dispose()
+    assert (out[0] == out[1]).all() and (out[0] == out[2]).all()
+
+
+@pytest.mark.parametrize("mode", sorted(TILES))
+@pytest.mark.parametrize("n", [4, 70, 131, 132, 250])
+def test_columns_beside_a_matrix_stay_out(ctx, split, mode, n):
+    """B as the first columns of a wider buffer: what lies beside them changes no bit, also where a tile reads it."""
+    rng = np.random.default_rng(n)
+    m, k, ld = 96, 80, 264
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, ld)).astype(np.float32)
+    ta, y = ctx.move_tensor(a), ctx.empty_tensor([m, n])
+    split(mode)
+    ctx.set_option("gemm_wavesplit", 0)
+    out = []
+    try:
+        for beside in (0.0, np.nan, 1e-40):
+            b[:, n:] = beside
+            tb = ctx.move_tensor(b)
+            capi.call("wdh_gemm_ex", ta.handle, tb.handle, 0, y.handle, 1, m, n, k, 0, k, 1, 0, ld, 1, 0, 0, 1.0, 1.0, 0, 0, m * n, n)
+            out.append(y.get_data())
+    finally:
+        ctx.set_option("gemm_wavesplit", 1)
+    a, b = a.astype(np.float64), b[:, :n].astype(np.float64)
+    assert within(out[0], a @ b, np.abs(a) @ np.abs(b), k)
     assert (out[0] == out[1]).all() and (out[0] == out[2]).all()
 
 

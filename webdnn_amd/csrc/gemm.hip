@@ -706,8 +706,9 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
   }
   // A few rows against a transposed weight: a pass over the weight (gemm_rows.hip)
   if (useA_kc && useB_kc && gemm_rows_suits(batch, m, n, k, vec)) return launch_gemm_rows(p, batch, vec);
-  // Enough to multiply: the bf16 matrix cores (split_product.h)
-  if (useA_kc && split_legal(p, vec)) {
+  // Enough to multiply: the bf16 matrix cores (split_product.h; they read columns of B in pairs, and every element they
+  // read decides whether a tile is done again, so a pair must not reach into what lies beside the matrix)
+  if (useA_kc && split_legal(p, vec) && (useB_kc || n % 2 == 0)) {
     if (const SplitPlan s = split_gemm_plan(batch, m, n, k, useB_kc); s.tile >= 0) {
       auto launch = [&](const SplitPlan &q) { return launch_split_gemm(useB_kc, q, p, batch); };
       const int rc = wavesplit_suits(batch, m, n, k) ? launch(s) : run_split(s, launch);

@@ -191,7 +191,8 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
     padding(col, pf);
   } else {
 #pragma unroll
-    for (int i = 0; i < CPP; i++) voff_b[i] = (bkq * 4 * ldb + column(col0 + bcol + i)) * 4;
+    for (int i = 0; i < CPP; i++)  // (columns past a matrix may hold anything: they read as zeros)
+      voff_b[i] = CONV || col0 + bcol + i < p.n ? (bkq * 4 * ldb + column(col0 + bcol + i)) * 4 : BUF_OOB;
   }
   const int b_window = CONV ? p.b_bytes - (int)((long long)bz * p.cv.c_in_g * p.cv.h * p.cv.w * 4) : p.b_bytes;
   const rsrc_t rsrc_b = make_rsrc(B - bias, b_window);
@@ -355,14 +356,17 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
   // ---- the two sums meet; is there anything the split could not hold? ------------------------------------
   SumRange sums = {0xffffffffu, 0};
 #pragma unroll
-  for (int b = 0; b < NT; b++)
+  for (int b = 0; b < NT; b++) {
 #pragma unroll
     for (int a = 0; a < MT; a++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        acc[a][b][r] += small[a][b][r];
-        add_sum(sums, acc[a][b][r]);
-      }
+      for (int r = 0; r < 16; r++) acc[a][b][r] += small[a][b][r];
+    if (!CONV && !B_IS_KC && col0 + wcol + b * 32 + li >= p.n) continue;  // (zeros; elsewhere surplus columns repeat the last one)
+#pragma unroll
+    for (int a = 0; a < MT; a++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) add_sum(sums, acc[a][b][r]);
+  }
   bool again = __syncthreads_or(not_finite(sums) || loses_bits(least));
   if (again && !__syncthreads_or(not_finite(sums) || small_sums(sums))) {
     // (elements that lost bits, but every sum is large: what were their partners?)
