@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 from oracle import ref
+from webdnn_amd import capi
 from webdnn_amd import hostops as H
 
 pytestmark = pytest.mark.gpu
@@ -21,6 +22,22 @@ def test_gather_of_runs(ctx, inner, outer, axis, n):
     view.dispose()
     xi = rng.integers(-9, 9, x.shape).astype(np.int32)
     assert (H.gather(ctx, ctx.move_tensor(xi), ctx.move_tensor(idx), 1).get_data() == xi[:, idx]).all()
+
+
+# (a little under and at the limit; 3.2 GB of results)
+@pytest.mark.parametrize("runs", [(1 << 24) - 1, 1 << 24])
+def test_gather_of_more_runs_than_a_launch_has_workgroups(ctx, runs):
+    """2^24 workgroups of 256 threads are one too many for a launch."""
+    inner = 49
+    x = np.arange(3 * inner, dtype=np.float32).reshape(3, inner)
+    idx = (np.arange(runs) % 3).astype(np.int32)
+    y = H.gather(ctx, ctx.move_tensor(x), ctx.move_tensor(idx), 0)
+    part = np.empty((1000, inner), np.float32)
+    for first in (0, runs // 2, runs - 1000):
+        capi.call("wdh_read", y.handle, first * inner * 4, part.ctypes.data, part.nbytes)
+        assert (part == x[idx[first:first + 1000]]).all()
+    y.dispose()
+    capi.call("wdh_trim", 0)
 
 
 def test_gather_out_of_range_reads_the_first_run(ctx):

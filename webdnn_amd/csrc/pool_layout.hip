@@ -691,7 +691,8 @@ extern "C" int wdh_gather(wdh_buf hD, wdh_buf hI, wdh_buf hY, int64_t outer,
   const uintptr_t at = (uintptr_t)pd | (uintptr_t)py;
   const int unit = inner % 4 == 0 && (at & 15) == 0 ? 4 : inner % 2 == 0 && (at & 7) == 0 ? 2 : 1;
   const long long units = inner / unit, rows = (long long)outer * n_idx, chunks = (units + 1023) / 1024;
-  if (units >= 48 && rows <= 0x7fffffffLL / chunks && units <= 0x7fffffffLL) {
+  // (a launch has at most 2^32 - 1 threads in a direction; the kernel below steps through what is beyond)
+  if (units >= 48 && rows <= 0xffffffffLL / 256 / chunks && units <= 0x7fffffffLL) {
     const wdh::FastDiv fd_chunks = wdh::make_fastdiv(chunks), fd_idx = wdh::make_fastdiv(n_idx);
     const dim3 grid((unsigned)(rows * chunks)), block(256);
     const uint32_t *d = (const uint32_t *)pd;
