@@ -161,6 +161,24 @@ def test_convs(ctx, split, mode, shape):
     assert (np.isnan(out[0]) == np.isnan(out[mode])).all() and (np.isinf(out[0]) == np.isinf(out[mode])).all()
 
 
+@pytest.mark.parametrize("shape", CONVS)
+def test_convs_without_a_tile_of_that_size(ctx, split, shape):
+    """There are no 256x128 tiles for convs: asked for them, a conv takes the fp32 instruction."""
+    n, cin, h, w, cout, kernel, stride, pad, dil, group = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal((n, cin, h, w)).astype(np.float32)
+    wt = rng.standard_normal((cout, cin // group, kernel, kernel)).astype(np.float32)
+    ctx.set_option("conv3x3_winograd", 0)
+    run = lambda x, wt: H.conv(ctx, ctx.move_tensor(x), ctx.move_tensor(wt), None, [dil, dil], group, None, [pad] * 4, [stride, stride]).get_data()
+    split(0)
+    want, magnitudes = run(x, wt), run(np.abs(x), np.abs(wt))
+    split(7)
+    got = run(x, wt)
+    assert ctx.last_plan()["tile"] != TILES[7], ctx.last_plan()
+    k = cin // group * kernel * kernel
+    assert (np.abs(want.astype(np.float64) - got) <= 2 * (k + 8) * 2.0 ** -24 * magnitudes).all()
+
+
 def test_one_image_keeps_its_bits(ctx, split):
     """A single image stays with the fp32 instruction; the same image in a batch agrees with it as sums in another order do."""
     rng = np.random.default_rng(4)

@@ -1262,7 +1262,9 @@ direct_forms:
   if (small && vec && ntaps == 1 && pt == 0 && pl == 0 && pb == 0 && pr == 0) {
     p.m = cout_g; p.n = (int)npix; p.k = (int)kdim;
     p.fast = 1;
-    if (split_legal(p, true) && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS))) {
+    SplitPlan s = {-1, {}, 0.0};
+    if (split_legal(p, true) && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS))) s = plan_split(group, p.m, p.n, p.k, SPLIT_PIXELS);
+    if (s.tile >= 0) {
       p.sAb = (long long)cout_g * kdim; p.sA0 = kdim; p.sA1 = 1;
       p.sBb = (long long)c_in_g * plane; p.sB0 = plane; p.sB1 = 1;
       p.alpha = 1.0f; p.beta = 1.0f; p.epilogue = epilogue;
@@ -1277,8 +1279,7 @@ direct_forms:
       p.c_bytes = cout * 4;
       set_wide(p, true);
       g_last_form = WDH_FORM_CONV_GATHER32;  // (the form it stands in for)
-      return run_split(plan_split(group, p.m, p.n, p.k, SPLIT_PIXELS),
-                       [&](const SplitPlan &q) { return launch_split_conv(B_PIXELS_ANY, q, p, group); });
+      return run_split(s, [&](const SplitPlan &q) { return launch_split_conv(B_PIXELS_ANY, q, p, group); });
     }
   }
   auto it = g_ktabs.find(key);
