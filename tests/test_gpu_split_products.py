@@ -359,6 +359,59 @@ def test_tiny_elements_among_others(ctx, split, mode, chunks, partner):
     assert sums_hold(got, a @ b, a @ b, 192)
 
 
+# one slab, a ragged last one, an odd and an even number of slabs; edges in both directions; cut along K
+@pytest.mark.parametrize("mode", sorted(TILES))
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("m,n,k,chunks", [(64, 64, 16, 1), (65, 132, 44, 1), (129, 68, 64, 1), (257, 260, 76, 1), (100, 196, 244, 3)])
+def test_tiles_done_again(ctx, split, mode, transposed, m, n, k, chunks):
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32) * np.float32(2.0 ** -120), rng.standard_normal((k, n)).astype(np.float32) * np.float32(2.0 ** 120)
+    bias = rng.standard_normal(n).astype(np.float32)
+    split(mode)
+    ctx.set_option("gemm_wavesplit", 0)
+    ctx.set_option("split_k", chunks)
+    try:
+        got = product(ctx, a, b, transposed, bias)
+    finally:
+        ctx.set_option("gemm_wavesplit", 1)
+    assert ctx.last_plan()["tile"] == TILES[mode], ctx.last_plan()
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    assert within(got, a @ b + bias, np.abs(a) @ np.abs(b) + np.abs(bias), k)
+
+
+@pytest.mark.parametrize("kind", ["gemm", "rows", "taps", "pixels"])
+def test_tiles_done_again_cost_little_more_than_the_fp32_instruction(ctx, split, kind):
+    """A NaN that reaches every tile: both instructions one after the other, each at its own pace (with loads a
+    single element at a time it was 3.5 to 5.5 times)."""
+    rng = np.random.default_rng(15)
+    if kind == "gemm":
+        a, b = rng.standard_normal((2048, 2048)).astype(np.float32), rng.standard_normal((2048, 2048)).astype(np.float32)
+        a[:, 5] = np.nan
+        ta, tb = ctx.move_tensor(a), ctx.move_tensor(b)
+        run = lambda: H.gemm(ctx, ta, tb, trans_b=1)
+    else:
+        cin, cout, size, kernel, stride = {"rows": (128, 128, 28, 3, 1), "taps": (128, 128, 56, 3, 2), "pixels": (256, 512, 28, 1, 2)}[kind]
+        x, w = rng.standard_normal((32, cin, size, size)).astype(np.float32), rng.standard_normal((cout, cin, kernel, kernel)).astype(np.float32)
+        w[::8] = np.nan
+        tx, tw = ctx.move_tensor(x), ctx.move_tensor(w)
+        ctx.set_option("conv3x3_winograd", 0)
+        run = lambda: H.conv(ctx, tx, tw, pads=[kernel // 2] * 4, strides=[stride, stride], constant_weights=True)
+    best = {}
+    for value in (0, 1):
+        split(value)
+        run().dispose()
+        times = []
+        for _ in range(5):
+            ctx.event_record(0)
+            for _ in range(5):
+                run().dispose()
+            ctx.event_record(1)
+            ctx.sync()
+            times.append(ctx.event_elapsed_ms(0, 1))
+        best[value] = min(times)
+    assert best[1] <= 2.8 * best[0], best
+
+
 @pytest.mark.parametrize("mode", [3, 4])
 @pytest.mark.parametrize("kernel,stride", [(3, 1), (3, 2), (1, 1), (1, 2)])
 @pytest.mark.parametrize("tiny,partner", TINY)

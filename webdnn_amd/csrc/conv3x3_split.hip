@@ -253,36 +253,50 @@ __global__ __launch_bounds__(WM * WN * 64, BM * BN >= 128 * 128 ? 2 : PX <= 480 
       for (int b = 0; b < NT; b++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
-    int base[NT], iy0[NT], ix0[NT];
+    // The same rows through the same LDS, whole: [channel half][pixel][8 channels]; the weights as the caller has them.
+    const float *wt[MT];
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-      int P = col0 + wcol + nt * 32 + li;
-      P = P < (int)cv.npix ? P : (int)cv.npix - 1;
-      const int R = fdiv(P, cv.fd_ow), img = fdiv(R, cv.fd_oh);
-      iy0[nt] = R - img * cv.oh - cv.pt;
-      ix0[nt] = P - R * cv.ow - cv.pl;
-      base[nt] = img * cv.c_total * plane_in;
+    for (int mt = 0; mt < MT; mt++) {
+      const int r = row0 + wrow + mt * 32 + li;
+      wt[mt] = p.A + (long long)(r < p.m ? r : p.m - 1) * p.k + 72 * half;
     }
-    for (int k0 = kbeg; k0 < kend; k0 += 2) {
-      const int k = k0 + half, ci = k / 9, tap = k - ci * 9, ky = tap / 3, kx = tap - ky * 3;  // (k < kend: both are even)
-      float ea[MT], eb[NT];
+    fetch_x(kbeg);
+    for (int k0 = kbeg; k0 < kend; k0 += KGRAN) {
+      __syncthreads();  // everybody has read the block before
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++) {
-        const int r = row0 + wrow + mt * 32 + li;
-        ea[mt] = p.A[(long long)(r < p.m ? r : p.m - 1) * p.k + k];
+      for (int i = 0; i < XU; i++)
+        if (lds_x[i] >= 0) {
+          f32x4 *const cell = reinterpret_cast<f32x4 *>(xs + 2 * lds_x[i]);
+          cell[0] = f32x4{x[i][0], x[i][1], x[i][2], x[i][3]};
+          cell[1] = f32x4{x[i][4], x[i][5], x[i][6], x[i][7]};
+        }
+      __syncthreads();
+      if (k0 + KGRAN < kend) fetch_x(k0 + KGRAN);
+#pragma unroll 1
+      for (int tap = 0; tap < 9; tap++) {
+        const int shift = (tap / 3 * cv.pitch + tap % 3) * 32;
+        float ea[MT][8];
+        f32x4 eb[NT][2];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+          for (int j = 0; j < 8; j++) ea[mt][j] = wt[mt][k0 + j * 9 + tap];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+          const f32x4 *const cell = reinterpret_cast<const f32x4 *>(xs + 2 * corner[nt] + shift);
+          eb[nt][0] = cell[0];
+          eb[nt][1] = cell[1];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+#pragma unroll
+          for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++)
+              acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(ea[mt][j], eb[nt][j >> 2][j & 3], acc[mt][nt], 0, 0, 0);
       }
-#pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
-        const int iy = iy0[nt] + ky, ix = ix0[nt] + kx;
-        const bool in = iy >= 0 && iy < cv.h && ix >= 0 && ix < cv.w;
-        eb[nt] = in ? p.B[base[nt] + ci * plane_in + iy * cv.w + ix] : 0.0f;
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(ea[mt], eb[nt], acc[mt][nt], 0, 0, 0);
     }
+    __syncthreads();  // (the epilogue's staging is this LDS)
   }
   finish_tile<BM, BN, WM, WN, true, 2>(p, acc, tw.whole, tw.lin, tw.chunk, 0, row0, col0,
                                     reinterpret_cast<float *>(xs) + wave * STAGE_FLOATS);

@@ -119,7 +119,7 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
   const int klast = tw.whole ? p.k : (kfirst + p.kchunk < p.k ? kfirst + p.kchunk : p.k);
   const int kshare = KG == 1 ? klast - kfirst : ((klast - kfirst + BK - 1) / BK + KG - 1) / KG * BK;
   const int kbeg = kfirst + group * kshare;   // (a group may have less than the others, or nothing: zeros, then)
-  const int kend = KG == 1 || kbeg + kshare < klast ? kbeg + kshare : klast;
+  int kend = KG == 1 || kbeg + kshare < klast ? kbeg + kshare : klast;
   const float *const A = p.A + (long long)bz * p.sAb;
   const float *const B = CONV ? p.B + (long long)bz * p.cv.c_in_g * p.cv.h * p.cv.w : p.B + (long long)bz * p.sBb;
   const int lda = (int)p.sA0, ldb = (int)(B_IS_KC ? p.sB1 : p.sB0);
@@ -372,10 +372,11 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
     // (elements that lost bits, but every sum is large: what were their partners?)
     bool large = false;
     read_taps(kbeg);
-    for (int k0 = kbeg; k0 < kend; k0 += 2 * BK) {
-      Slab q[2];
-      fetch(k0, q[0], true);
-      fetch(k0 + BK, q[1], true);
+    constexpr int AHEAD = IM2COL ? 1 : 2;
+    for (int k0 = kbeg; k0 < kend; k0 += AHEAD * BK) {
+      Slab q[AHEAD];
+#pragma unroll
+      for (int i = 0; i < AHEAD; i++) fetch(k0 + i * BK, q[i], true);
 #pragma unroll
       for (const Slab &s : q) {
 #pragma unroll
@@ -412,50 +413,54 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
   }
   if (again) {
     if (group > 0) return;  // (the first group does the whole K again)
-    // Operands straight from memory, one element a lane and k; never the common case.
-    const float *pa[MT];
-    int cb[NT];
-    PixelFast pb[NT];
+    // The same slabs through the same LDS, whole: [row or column][16 k, 4 apart]; a lane multiplies eight neighbouring k.
+    // (us, fp32 instruction / a NaN in every row: 4096^3 940 / 1586, 4096x3072x768 146 / 273, 1024^3 36 / 44; with loads of
+    // single elements 4089, 605, 128.)
+    constexpr int LDW = BK + 4;
+    static_assert((BM + BN) * LDW * 4 <= BUF, "whole slabs");
+    auto put_whole = [&](float *buf, const Slab &s) {
+      float *const b = buf + BM * LDW;
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-      const int r = row0 + wrow + mt * 32 + li;
-      pa[mt] = A + (long long)(r < p.m ? r : p.m - 1) * lda;
-    }
+      for (int i = 0; i < NA; i++) *reinterpret_cast<f32x4 *>(buf + ((tid >> 2) + i * RPP) * LDW + kq * 4) = s.a[i];
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-      int c = col0 + wcol + nt * 32 + li;
-      if (IM2COL) padding(c, pb[nt]);
-      c = c < p.n ? c : p.n - 1;
-      cb[nt] = B_IS_KC ? c * ldb : column(c) - bias;
-    }
+      for (int i = 0; i < (B_IS_KC ? NB : (IM2COL ? L / 4 : CPP)); i++) {
+        const int col = B_IS_KC ? (tid >> 2) + i * RPP : (IM2COL ? tid % BN : bcol + i);
+        const int q = B_IS_KC ? kq : (IM2COL ? (kgroup0 >> 2) + i : bkq);
+        *reinterpret_cast<f32x4 *>(b + col * LDW + q * 4) = s.b[i];
+      }
+    };
 #pragma unroll
     for (int a = 0; a < MT; a++)
 #pragma unroll
       for (int b = 0; b < NT; b++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
-    for (int k0 = kfirst; k0 < klast; k0 += 2) {
-      const int k = k0 + half;
-      const bool in = k < klast;
-      float ea[MT], eb[NT];
+    kend = klast;  // (of group 0, which begins with the tile's first slab)
+    read_taps(kfirst);
+    fetch(kfirst, next, true);
+    for (int k0 = kfirst, cur = 0; k0 < klast; k0 += BK, cur ^= 1) {
+      float *const buf = reinterpret_cast<float *>(&lds[cur][0]);
+      put_whole(buf, next);
+      if (k0 + BK < klast) fetch(k0 + BK, next, true);
+      __syncthreads();
+      const float *const fa = buf + (wrow + li) * LDW + 8 * half, *const fb = buf + (BM + wcol + li) * LDW + 8 * half;
+      f32x4 a[MT][2], b[NT][2];
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++) ea[mt] = in ? pa[mt][k] : 0.0f;
+      for (int h = 0; h < 2; h++) {
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) {
-        if (IM2COL) {
-          const int2 e = p.cv.ktab[in ? k : kfirst];
-          const unsigned word = (BMODE == B_IM2COL64 && (e.y & 32)) ? pb[nt].pad_hi : pb[nt].pad_lo;
-          eb[nt] = in && !((word >> (e.y & 31)) & 1u) ? B[cb[nt] + (e.x >> 2)] : 0.0f;
-        } else {
-          eb[nt] = in ? B[B_IS_KC ? (long long)cb[nt] + k : (long long)k * ldb + cb[nt]] : 0.0f;
-        }
+        for (int mt = 0; mt < MT; mt++) a[mt][h] = *reinterpret_cast<const f32x4 *>(fa + mt * 32 * LDW + 4 * h);
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) b[nt][h] = *reinterpret_cast<const f32x4 *>(fb + nt * 32 * LDW + 4 * h);
       }
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++)
+      for (int e = 0; e < 8; e++)
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(ea[mt], eb[nt], acc[mt][nt], 0, 0, 0);
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+          for (int nt = 0; nt < NT; nt++)
+            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mt][e >> 2][e & 3], b[nt][e >> 2][e & 3], acc[mt][nt], 0, 0, 0);
     }
+    __syncthreads();  // (the epilogue's staging is this LDS)
   }
   finish_tile<BM, BN, WM, WN, CONV, (MT * NT > 2 ? 2 : 1)>(p, acc, tw.whole, tw.lin, tw.chunk, bz, row0, col0,
                                     reinterpret_cast<float *>(&lds[0][0]) + wave * STAGE_FLOATS);
