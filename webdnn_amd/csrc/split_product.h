@@ -41,7 +41,7 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 // Two elements -> their three parts, packed (the first in the lower sixteen bits).
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-struct SplitPair { unsigned h, m, l; };
+struct SplitPair { unsigned h, m, l; float r0, r1; };  // r: what l is the nearest value to
 __device__ __forceinline__ unsigned nearest_pair(float x0, float x1) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x0, x1}, bf16x2));
 }
@@ -50,7 +50,7 @@ __device__ __forceinline__ SplitPair split_pair(float x0, float x1) {
   const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xffff0000u);
   const unsigned m = nearest_pair(r0, r1);
   const float s0 = r0 - __uint_as_float(m << 16), s1 = r1 - __uint_as_float(m & 0xffff0000u);
-  return SplitPair{h, m, nearest_pair(s0, s1)};
+  return SplitPair{h, m, nearest_pair(s0, s1), s0, s1};
 }
 
 // The least nonzero magnitude of what was split, as doubled bits less one (a zero becomes the largest), and what it and the sums say.
@@ -61,6 +61,11 @@ __device__ __forceinline__ unsigned least_of(unsigned least, float x0, float x1)
 }
 constexpr unsigned doubled_bits(int exponent) { return (unsigned)(127 + exponent) << 24; }
 __device__ __forceinline__ bool loses_bits(unsigned least) { return least < doubled_bits(-110) - 1u; }
+// The same asked of a pair by itself: only what is left of small elements (below 2^-102) is subnormal and not zero.
+__device__ __forceinline__ bool may_lose_bits(const SplitPair &s) {
+  constexpr int SUBNORMAL = 0x90;  // (of either sign)
+  return __builtin_amdgcn_classf(s.r0, SUBNORMAL) | __builtin_amdgcn_classf(s.r1, SUBNORMAL);
+}
 __device__ __forceinline__ bool reaches_partners(float x) { return (__float_as_uint(x) << 1) >= doubled_bits(30); }
 __device__ __forceinline__ bool reaches_partners(f32x4 v) {
   return reaches_partners(v.x) | reaches_partners(v.y) | reaches_partners(v.z) | reaches_partners(v.w);
@@ -247,10 +252,16 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
       }
     }
   };
-  unsigned least = 0xffffffffu;  // of this thread's pieces
+  // Were there elements that lose bits?  The least of them takes three vector instructions a pair, each by itself two and two
+  // scalar ones, which wide tiles have the slots for (us, 4096^3 with 256x128 tiles 652 / 634, without either 638; 384x3072x768
+  // 26.6 / 27.5, 26.5).
+  constexpr bool BY_PAIR = BM * BN > 128 * 128;
+  unsigned least = 0xffffffffu;
+  bool lost = false;
   auto put4 = [&](unsigned char *cell, int plane, f32x4 v) {
-    least = least_of(least_of(least, v.x, v.y), v.z, v.w);
     const SplitPair lo = split_pair(v.x, v.y), hi = split_pair(v.z, v.w);
+    if (BY_PAIR) lost = lost | may_lose_bits(lo) | may_lose_bits(hi);
+    else least = least_of(least_of(least, v.x, v.y), v.z, v.w);
     *reinterpret_cast<u32x2 *>(cell) = u32x2{lo.h, hi.h};
     *reinterpret_cast<u32x2 *>(cell + plane) = u32x2{lo.m, hi.m};
     *reinterpret_cast<u32x2 *>(cell + 2 * plane) = u32x2{lo.l, hi.l};
@@ -326,7 +337,7 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
     put(lds[cur ^ 1], now);
     // fragment reads, requests, then products with the split and the stores in between
     constexpr int PIECES = NA + (B_IS_KC ? NB : (IM2COL ? L / 4 : CPP));
-    constexpr int PRODUCTS = MT * NT * 6, VALU = PIECES * 28 + (IM2COL ? 2 * L : 0), STORES = PIECES * 3;
+    constexpr int PRODUCTS = MT * NT * 6, VALU = PIECES * (BY_PAIR ? 26 : 28) + (IM2COL ? 2 * L : 0), STORES = PIECES * 3;
     constexpr int LOADS = NA + (B_IS_KC ? NB : (IM2COL ? L : PIX_ANY ? 4 * CPP : 4));
     __builtin_amdgcn_sched_group_barrier(0x100, (MT + NT) * 3, 0);
     __builtin_amdgcn_sched_group_barrier(0x20, LOADS, 0);
@@ -367,7 +378,7 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
 #pragma unroll
       for (int r = 0; r < 16; r++) add_sum(sums, acc[a][b][r]);
   }
-  bool again = __syncthreads_or(not_finite(sums) || loses_bits(least));
+  bool again = __syncthreads_or(not_finite(sums) || lost || loses_bits(least));
   if (again && !__syncthreads_or(not_finite(sums) || small_sums(sums))) {
     // (elements that lost bits, but every sum is large: what were their partners?)
     bool large = false;
