@@ -196,6 +196,7 @@ def test_one_image_keeps_its_bits(ctx, split):
 
 def test_a_geometry_first_met_while_recording(ctx, split):
     """The gathered form needs a tap table, which cannot be built then: the form that reads an LDS tile serves."""
+    split(2)
     rng = np.random.default_rng(6)
     x, wt = ctx.move_tensor(rng.standard_normal((2, 72, 20, 24)).astype(np.float32)), ctx.move_tensor(rng.standard_normal((64, 72, 3, 3)).astype(np.float32))
     ctx.sync()
@@ -212,6 +213,22 @@ def test_a_geometry_first_met_while_recording(ctx, split):
         assert np.abs(got - want.get_data()).max() <= 1e-5 * np.abs(got).max()
         want.dispose()
     ctx.graph_destroy(graph)
+
+
+@pytest.mark.parametrize("shape,pays", [((118, 192, 8, 8, 320, 3, 2), False), ((13, 264, 11, 47, 192, 3, 1), False),
+                                        ((64, 128, 28, 28, 256, 3, 2), True)])
+def test_gathered_taps_pay_where_128_channels_share_them(ctx, split, shape, pays):
+    """Where no tile of 128 channels is planned the fp32 instruction serves, bit for bit; elsewhere the other one is taken."""
+    n, cin, h, w, cout, kernel, stride = shape
+    rng = np.random.default_rng(sum(shape))
+    x = ctx.move_tensor(rng.standard_normal((n, cin, h, w)).astype(np.float32))
+    wt = ctx.move_tensor(rng.standard_normal((cout, cin, kernel, kernel)).astype(np.float32))
+    out, plans = [], []
+    for value in (0, 1):
+        split(value)
+        out.append(H.conv(ctx, x, wt, pads=[1] * 4, strides=[stride, stride]).get_data())
+        plans.append(ctx.last_plan())
+    assert (plans[0] == plans[1] and (out[0] == out[1]).all()) == (not pays), plans
 
 
 ROWS = [

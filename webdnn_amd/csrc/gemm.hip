@@ -451,11 +451,19 @@ static SplitPlan split_gemm_plan(int batch, int m, int n, int k, bool b_kc) {
 // Whether a conv of a batch does.  A single image stays with the fp32 instruction: its launches are short of tiles (ResNet-50's
 // 50 of them take 3 to 10 us each, mostly latency), and its results stay bit for bit what they were.  K below 96 leaves
 // nothing to gain from faster products (128 images 64 -> 256 on 56x56 173 us / 190, 16 images 32 -> 64 on 112x112 18.4 / 20).
-// Gathered taps cost vector instructions, which pay where whole tiles of output channels share them: 64 -> 64 on 56x56,
-// 32 images 73 / 66, 256 -> 256 on 28x28 stride 2 82 / 63; 108 -> 94 39 / 44, 400 -> 32 14.4 / 16.3.
+// Rows of channels that hardly fill their tiles leave nothing either (108 -> 94 39 / 44).
 static bool split_conv_suits(int images, int m, int k, SplitSource source) {
   if (images < 2 || k < 96) return false;
   return source == SPLIT_PIXELS || (m >= 64 && m * 10 >= (m + 63) / 64 * 64 * 9);
+}
+// Of those, a conv that gathers its taps.  Taps cost vector instructions, an element by itself, which pay where 128 output
+// channels share them.  (750 convs of kernels of 3 and 5, strides of 1 and 2, 5e8 operations and more, us against the fp32
+// instruction: tiles of 128 channels 0.861 and 0.918 times its, 7 of 202 slower by over 5 %; of 64 channels 1.04 and 1.07, 153 of
+// 329 -- 118 images 192 -> 320 of stride 2 on 8x8 36.4 / 47.8, 5 images 64 -> 320 of 5x5 and stride 2 on 57x98 88.8 / 113.8.
+// 3x3 convs of 8 (mod 16) channels, whose other form reads an LDS tile: 128x128 0.876, 64x64 1.061.)
+static bool taps_pay(int group, int m, long long npix, int k) {
+  const int tile = plan_split(group, m, (int)npix, k, SPLIT_TAPS).tile;
+  return tile == S128x128 || tile == S128x64;
 }
 // Whether the fp32 form of a conv that reads X in place would run as a stream of K slabs (64x64 tiles; see stream_width).
 static bool conv_streams(const Params &p, int group) {
@@ -1115,7 +1123,8 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   key.c_in_g = c_in_g; key.kh = kh; key.kw = kw; key.dh = dh; key.dw = dw;
   key.h = h; key.w = w; key.mode = mode;
   // (while a graph is being recorded the gathered forms serve only geometries whose tap table is there already)
-  const bool gather_split = mode != B_IM2COL_BIG && (!wdh::capturing() || g_ktabs.count(key)) && split_possible(n, cout_g, (int)kdim);
+  const bool gather_split = mode != B_IM2COL_BIG && (!wdh::capturing() || g_ktabs.count(key)) && split_possible(n, cout_g, (int)kdim) &&
+                            (g_split > 1 || taps_pay(group, cout_g, npix, (int)kdim));
   // 3x3, stride 1, no dilation, one group, many channels: minimal filtering -- filters and input patches
   // are transformed, the positions of the transform domain (16 for F(2x2, 3x3), 36 for F(4x4, 3x3)) are
   // one batched product M[xi] = U[xi] [cout, c] x V[xi] [c, tiles] with 4/9 or 1/4 of the direct form's
