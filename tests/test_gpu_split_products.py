@@ -231,6 +231,21 @@ def test_gathered_taps_pay_where_128_channels_share_them(ctx, split, shape, pays
     assert (plans[0] == plans[1] and (out[0] == out[1]).all()) == (not pays), plans
 
 
+@pytest.mark.parametrize("residual", [False, True])
+def test_a_short_k_with_a_residual_on_odd_planes(ctx, split, residual):
+    """Stays with the fp32 instruction where 128x128 tiles would serve, bit for bit."""
+    rng = np.random.default_rng(17)
+    x = ctx.move_tensor(rng.standard_normal((42, 96, 15, 77)).astype(np.float32))
+    wt = ctx.move_tensor(rng.standard_normal((512, 96, 1, 1)).astype(np.float32))
+    r = ctx.move_tensor(rng.standard_normal((42, 512, 15, 77)).astype(np.float32)) if residual else None
+    out = []
+    for value in (0, 1):
+        split(value)
+        out.append(H.conv(ctx, x, wt, residual=r).get_data())
+    assert (out[0] == out[1]).all() == residual
+    assert np.abs(out[0].astype(np.float64) - out[1]).max() <= 1e-5 * np.abs(out[0]).max()
+
+
 ROWS = [
     # n, c, h, w, cout, pads: ragged tiles and channels, tiles over several images, unequal and wide pads, wide rows
     (2, 16, 8, 9, 64, [1, 1, 1, 1]),

@@ -1123,7 +1123,7 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   key.c_in_g = c_in_g; key.kh = kh; key.kw = kw; key.dh = dh; key.dw = dw;
   key.h = h; key.w = w; key.mode = mode;
   // (while a graph is being recorded the gathered forms serve only geometries whose tap table is there already)
-  const bool gather_split = mode != B_IM2COL_BIG && (!wdh::capturing() || g_ktabs.count(key)) && split_possible(n, cout_g, (int)kdim) &&
+  bool gather_split = mode != B_IM2COL_BIG && (!wdh::capturing() || g_ktabs.count(key)) && split_possible(n, cout_g, (int)kdim) &&
                             (g_split > 1 || taps_pay(group, cout_g, npix, (int)kdim));
   // 3x3, stride 1, no dilation, one group, many channels: minimal filtering -- filters and input patches
   // are transformed, the positions of the transform domain (16 for F(2x2, 3x3), 36 for F(4x4, 3x3)) are
@@ -1273,6 +1273,13 @@ direct_forms:
     p.fast = 1;
     SplitPlan s = {-1, {}, 0.0};
     if (split_legal(p, true) && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS))) s = plan_split(group, p.m, p.n, p.k, SPLIT_PIXELS);
+    // (a short K hides little of an epilogue that takes a residual 4 bytes at a time, and two 128x128 tiles a CU overlap
+    // little: 42 images 96 -> 512 on 15x77 73.4 us with the fp32 instruction, 85.7 here; without a residual 68.1 / 58.5 (74
+    // images 96 -> 1024 on 17x19); K 128 in narrower tiles 18.9 / 17.0)
+    if (g_split == 1 && s.tile == S128x128 && p.k < 128 && p.R && (long long)oh * ow % 4 != 0) {
+      s.tile = -1;
+      gather_split = false;
+    }
     if (s.tile >= 0) {
       p.sAb = (long long)cout_g * kdim; p.sA0 = kdim; p.sA1 = 1;
       p.sBb = (long long)c_in_g * plane; p.sB0 = plane; p.sB1 = 1;
