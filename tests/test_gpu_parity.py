@@ -1479,6 +1479,24 @@ def test_attention_at_the_key_counts_where_the_form_changes(ctx, tk, d):
     assert_close_max(got, attention_chain_ref(q, k, v[:tk], 3, 1.0 / np.sqrt(d)), GEMM_TOL, "attention vs oracle chain")
 
 
+@pytest.mark.parametrize("batch", [(1 << 22) - 1, 1 << 22])
+def test_attention_of_more_row_blocks_than_wide_workgroups_fit_a_launch(ctx, batch):
+    """2^22 workgroups of 1024 threads are one too many for a launch (the rows of Q overlap; 1 GB of results)."""
+    rng = np.random.default_rng(6)
+    tk, d = 300, 64
+    q = rng.standard_normal(4 * batch + d).astype(np.float32)
+    k, v = rng.standard_normal((tk, d)).astype(np.float32), rng.standard_normal((tk, d)).astype(np.float32)
+    tq, tk_, tv, y = ctx.move_tensor(q), ctx.move_tensor(k), ctx.move_tensor(v), ctx.empty_tensor([batch, d])
+    capi.call("wdh_attention", tq.handle, tk_.handle, tv.handle, y.handle, batch, 1, tk, d, 4, d, 0, d, 0, d, d, d, 0.125)
+    part = np.empty((50, d), np.float32)
+    for first in (0, batch // 2, batch - 50):
+        capi.call("wdh_read", y.handle, first * d * 4, part.ctypes.data, part.nbytes)
+        rows = np.stack([q[4 * i:4 * i + d] for i in range(first, first + 50)])
+        assert_close_max(part, attention_chain_ref(rows, k, v, 1, 0.125), GEMM_TOL, "attention vs oracle chain")
+    y.dispose()
+    capi.call("wdh_trim", 0)
+
+
 def test_attention_special_values_and_limits(ctx):
     """A +inf in V beside masked keys, a NaN score, and the shapes the entry point turns down."""
     rng = np.random.default_rng(5)

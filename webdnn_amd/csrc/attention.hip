@@ -274,9 +274,10 @@ int launch_attention(const AttParams &p, int batch) {
   // (64: sixteen wavefronts of one block each, 512 keys 18.8 us, eight of two 19.4; 200 keys 11.6 and 11.0)
   if constexpr (HD == 32)
     return p.tk > 512 ? launch_attention<HD, 16, 2>(p, batch) : launch_attention<HD, 16, 1>(p, batch);
-  else if constexpr (HD == 64)
-    return p.tk > 512   ? launch_attention<HD, 8, 4>(p, batch)
-           : p.tk > 256 ? launch_attention<HD, 16, 1>(p, batch) : launch_attention<HD, 8, 1>(p, batch);
+  else if constexpr (HD == 64)  // (a launch has at most 2^32 - 1 threads in a direction: twice as many row blocks with eight wavefronts)
+    return p.tk <= 256 ? launch_attention<HD, 8, 1>(p, batch)
+           : p.tk <= 512 && (long long)batch * p.row_blocks <= 0xffffffffLL / 1024 ? launch_attention<HD, 16, 1>(p, batch)
+                                                                                    : launch_attention<HD, 8, 4>(p, batch);
   else
     return p.tk > 256 ? launch_attention<HD, 8, 4>(p, batch) : launch_attention<HD, 8, 1>(p, batch);
 }
