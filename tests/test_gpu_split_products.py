@@ -512,6 +512,21 @@ def test_columns_beside_a_matrix_stay_out(ctx, split, mode, n):
     assert (out[0] == out[1]).all() and (out[0] == out[2]).all()
 
 
+@pytest.mark.parametrize("mode", [m for m in sorted(TILES) if m != 7])
+def test_pixels_past_the_last_stay_in_their_channel(ctx, split, mode):
+    """A 1x1 conv's surplus columns repeat the last pixels: the next channel's first one, a NaN, changes no bit of their tile."""
+    rng = np.random.default_rng(18)
+    x, wt = rng.standard_normal((2, 128, 10, 10)).astype(np.float32), ctx.move_tensor(rng.standard_normal((128, 128, 1, 1)).astype(np.float32))
+    split(mode)
+    out = []
+    for value in (0.5, np.nan):
+        x[1, 5, 0, 0] = value
+        out.append(H.conv(ctx, ctx.move_tensor(x), wt).get_data())
+        assert ctx.last_plan()["tile"] == TILES[mode] and "in place" in ctx.last_plan()["form"], ctx.last_plan()
+    assert np.isnan(out[1][1, :, 0, 0]).all()
+    assert (out[0][1, :, 9, 2:] == out[1][1, :, 9, 2:]).all()  # (pixels 192 to 199 of 200)
+
+
 def test_groups_that_fill_the_chip(ctx, split):
     """The projections of an attention block as one launch of 64x64 tiles; ragged rows and columns, one weight k-contiguous by shape."""
     rng = np.random.default_rng(9)

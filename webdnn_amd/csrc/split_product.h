@@ -160,7 +160,9 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
   // receptive field's corner, plus `bias`)
   auto column = [&](int col) -> int {
     if (!CONV) return col;
-    const unsigned P = (unsigned)col < (unsigned)p.n ? (unsigned)col : (unsigned)p.n - 1u;
+    // (columns past the last repeat it, or the last pair where they are read in pairs)
+    constexpr unsigned LAST = BMODE == B_PIXELS ? CPP : 1;
+    const unsigned P = (unsigned)col < (unsigned)p.n ? (unsigned)col : (unsigned)p.n - LAST;
     const unsigned plane = (unsigned)(p.cv.h * p.cv.w), ohw = (unsigned)(p.cv.oh * p.cv.ow);
     const unsigned img = (unsigned)fdiv((int)P, p.cv.fd_ohw), q = P - img * ohw;
     const unsigned oy = (unsigned)fdiv((int)q, p.cv.fd_ow), ox = q - oy * (unsigned)p.cv.ow;
@@ -372,7 +374,7 @@ __device__ __forceinline__ void split_tile(const Params &p, int pid) {
     for (int a = 0; a < MT; a++)
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[a][b][r] += small[a][b][r];
-    if (!CONV && !B_IS_KC && col0 + wcol + b * 32 + li >= p.n) continue;  // (zeros; elsewhere surplus columns repeat the last one)
+    if (!CONV && !B_IS_KC && col0 + wcol + b * 32 + li >= p.n) continue;  // (zeros; elsewhere surplus columns repeat the last ones)
 #pragma unroll
     for (int a = 0; a < MT; a++)
 #pragma unroll
