@@ -231,6 +231,43 @@ def test_gathered_taps_pay_where_128_channels_share_them(ctx, split, shape, pays
     assert (plans[0] == plans[1] and (out[0] == out[1]).all()) == (not pays), plans
 
 
+# (us, the form that was taken before / the one that is)
+@pytest.mark.parametrize("shape,form", [((4, 512, 45, 63, 160), "F(2x2,3x3)"), ((2, 832, 63, 63, 192), "F(2x2,3x3)"),   # rows 141 / 100, 149 / 105
+                                        ((13, 336, 19, 91, 416), "F(2x2,3x3)"),                                        # gathered taps 447 / 293
+                                        ((32, 128, 28, 28, 128), "LDS tile"), ((32, 256, 14, 14, 256), "F(2x2,3x3)")])
+def test_3x3_convs_take_the_form_of_the_least_estimate(ctx, split, shape, form):
+    n, cin, h, w, cout = shape
+    rng = np.random.default_rng(sum(shape))
+    x = ctx.move_tensor(rng.standard_normal((n, cin, h, w)).astype(np.float32))
+    wt = ctx.move_tensor(rng.standard_normal((cout, cin, 3, 3)).astype(np.float32))
+    y = H.conv(ctx, x, wt, pads=[1] * 4)
+    assert form in ctx.last_plan()["form"], ctx.last_plan()
+    got = y.get_data()
+    ctx.set_option("conv3x3_winograd", 0)
+    split(0)
+    want = H.conv(ctx, x, wt, pads=[1] * 4).get_data()
+    assert np.abs(got.astype(np.float64) - want).max() <= 1e-5 * np.abs(want).max()
+
+
+def test_a_product_short_of_blocks_stays_with_the_fp32_instruction(ctx, split):
+    """223x2292x1272: 22.6 us in 64x64 tiles whose K four groups share, 17.6 in blocks of 32x32."""
+    a, b = ctx.move_tensor(np.ones((223, 1272), np.float32)), ctx.move_tensor(np.ones((1272, 2292), np.float32))
+    assert (H.gemm(ctx, a, b).get_data() == 1272).all()
+    assert ctx.last_plan()["tile"] == "32x32", ctx.last_plan()
+
+
+def test_gathered_taps_of_a_full_round_of_tiles_and_a_few(ctx, split):
+    """28 images 672 -> 544, stride 2, on 18x25: 256 of 260 128x64 tiles whole and four in 32 chunks each 263 us, 128x128 tiles 191."""
+    rng = np.random.default_rng(19)
+    x = ctx.move_tensor(rng.standard_normal((28, 672, 18, 25)).astype(np.float32))
+    wt = ctx.move_tensor(rng.standard_normal((544, 672, 3, 3)).astype(np.float32))
+    got = H.conv(ctx, x, wt, pads=[1] * 4, strides=[2, 2]).get_data()
+    assert ctx.last_plan()["tile"] == "128x128", ctx.last_plan()
+    split(0)
+    want = H.conv(ctx, x, wt, pads=[1] * 4, strides=[2, 2]).get_data()
+    assert np.abs(got.astype(np.float64) - want).max() <= 1e-5 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("residual", [False, True])
 def test_a_short_k_with_a_residual_on_odd_planes(ctx, split, residual):
     """Stays with the fp32 instruction where 128x128 tiles would serve, bit for bit."""
@@ -340,6 +377,19 @@ def test_recorded_weights_outlive_another_size(ctx, split):
             for t in junk + [z]:
                 t.dispose()
         ctx.graph_destroy(graph)
+
+
+@pytest.mark.parametrize("shift", [-120, -112, -100])
+def test_rows_of_tiny_elements(ctx, split, shift):
+    """Elements whose last part does not fit bfloat16 leave tiny sums, which are added up again, also against large partners."""
+    rng = np.random.default_rng(11)
+    a = (rng.uniform(1, 2, (256, 512)) * 2.0 ** shift).astype(np.float32)
+    b = (rng.uniform(1, 2, (512, 256)) * 2.0 ** 40).astype(np.float32)
+    split(3)
+    got = product(ctx, a, b, False)
+    assert ctx.last_plan()["tile"] == "128x128"
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    assert within(got, a @ b, a @ b, 512)
 
 
 # exponents of the tiny operand and of its partners: some bits lost, all lost, subnormal floats; results from 2^-128 to 2^-17

@@ -364,19 +364,22 @@ static bool tiles_beat_wavesplit(int batch, int m, int n, int k, bool b_kc, bool
 }
 
 // How a product on the bf16 matrix cores is laid out: the tile and the cut along K with the least estimated time.
-// The model (us): a CU works through its workgroups' slabs of 16 k at `slab` each, a workgroup alone on a CU at `solo`;
-// `fixed` is a launch with one empty workgroup a CU (prologue, epilogue); a cut adds the pass over the partial sums, which
-// are written and read once.  Fitted to 21 products of 33x4096x4096 to 4096x4096x4096 on every tile in 1 to 12 cuts and to
-// 40 convs (the form it picks takes at most 11 % longer than the best one).
+// The model (us): a CU works through its workgroups' slabs of 16 k at `slab` each, and no workgroup is faster than `solo` a
+// slab, its pace alone on a CU; `fixed` is a launch with one empty workgroup a CU (prologue, epilogue); a cut adds the pass over
+// the partial sums, which are written and read once.  Result and residual are the same for every tile and not in it.
+// Fitted to 250 products and 250 convs of each kind (1e8 to 3e10 multiplications, every tile, 1 to 16 cuts, recorded launches).
+// Of 195 others that it serves the form it picks takes 4 % longer than the best one measured in the mean, 12 % one in ten, 17 %
+// at most (K below 100 or a residual bounds the launch there); of 1120 it takes over 5 % longer than the fp32 instruction 13
+// (no product, 7 of 281 1x1 convs, 3 of 355 3x3 ones, 3 of 240 with gathered taps), 21 % at most.
 enum SplitSource { SPLIT_GEMM, SPLIT_PIXELS, SPLIT_TAPS, SPLIT_ROWS };  // where B comes from: a matrix, X in place, gathered taps, rows of X in LDS
 static SplitPlan search_split(int nz, int m, int n, int k, SplitSource source, bool large_tiles) {
   struct Model { int bm, bn; double slab, solo, fixed; };
   static const Model models[4][7] = {
-      {{128, 128, 0.63, 0.56, 9.5}, {64, 128, 0.37, 0.39, 6.5}, {128, 64, 0.37, 0.39, 6.5}, {64, 64, 0.21, 0.29, 5.2}, {256, 128, 1.20, 0.95, 10.0}, {64, 64, 0.21, 0.20, 5.7}, {64, 64, 0.25, 0.16, 6.2}},
+      {{128, 128, 0.63, 0.56, 9.5}, {64, 128, 0.37, 0.39, 6.5}, {128, 64, 0.37, 0.39, 6.5}, {64, 64, 0.21, 0.29, 5.2}, {256, 128, 1.20, 0.95, 10.0}, {64, 64, 0.22, 0.24, 6.0}, {64, 64, 0.23, 0.14, 10.7}},
       {{128, 128, 0.63, 0.60, 9.5}, {64, 128, 0.38, 0.42, 6.5}, {128, 64, 0.37, 0.42, 6.5}, {64, 64, 0.21, 0.36, 5.2}, {0, 0, 0, 0, 0}, {64, 64, 0.21, 0.22, 5.7}, {64, 64, 0.25, 0.18, 6.2}},
       // (gathered taps: two more vector instructions an element, and a slab's loads wait for its part of the tap table)
-      {{128, 128, 0.66, 0.80, 9.5}, {64, 128, 0.43, 0.60, 6.5}, {128, 64, 0.39, 0.50, 6.5}, {64, 64, 0.24, 0.36, 5.2}, {0, 0, 0, 0, 0}, {64, 64, 0.24, 0.25, 5.7}, {64, 64, 0.28, 0.20, 6.2}},
-      {{128, 128, 0.66, 0.90, 11.0}, {64, 128, 0.35, 0.40, 8.0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}}};
+      {{128, 128, 0.75, 1.11, 7.9}, {64, 128, 0.56, 0.89, 6.7}, {128, 64, 0.42, 0.67, 6.4}, {64, 64, 0.29, 0.52, 5.7}, {0, 0, 0, 0, 0}, {64, 64, 0.29, 0.37, 7.1}, {64, 64, 0.33, 0.29, 13.2}},
+      {{128, 128, 0.53, 0.66, 4.4}, {64, 128, 0.305, 0.46, 3.9}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}, {0, 0, 0, 0, 0}}};
   const long long cus = wdh::compute_units();
   const int unit = source == SPLIT_ROWS ? 9 : 1;  // a chunk is a whole number of these, in slabs
   const int slabs = (k + BK - 1) / BK;
@@ -398,8 +401,8 @@ static SplitPlan search_split(int nz, int m, int n, int k, SplitSource source, b
         if (part && (tail == 0 || tail == tiles)) continue;
         const long long whole = tiles - tail;
         const long long rounds = s == 1 ? (tiles + cus - 1) / cus : whole / cus, cut_rounds = (tail * s + cus - 1) / cus;
-        double us = mo.fixed + (rounds + cut_rounds == 1 ? (rounds ? slabs : per) * mo.solo
-                                                          : rounds * slabs * mo.slab + cut_rounds * per * mo.slab);
+        const double path = (rounds ? slabs : per) * mo.solo, shared = (double)(rounds * slabs + cut_rounds * per) * mo.slab;
+        double us = mo.fixed + (rounds + cut_rounds == 1 || shared < path ? path : shared);
         us += 0.3 * (mo.fixed - 3.5) * (double)(rounds + cut_rounds - 1);
         if (s > 1) us += 3.0 + 2.0 * (double)tail * s * mo.bm * mo.bn * 4.0 / 7.0e6;
         if (us < best.us) {
@@ -457,9 +460,9 @@ static bool split_conv_suits(int images, int m, int k, SplitSource source) {
   return source == SPLIT_PIXELS || (m >= 64 && m * 10 >= (m + 63) / 64 * 64 * 9);
 }
 // Of those, a conv that gathers its taps.  Taps cost vector instructions, an element by itself, which pay where 128 output
-// channels share them.  (750 convs of kernels of 3 and 5, strides of 1 and 2, 5e8 operations and more, us against the fp32
-// instruction: tiles of 128 channels 0.861 and 0.918 times its, 7 of 202 slower by over 5 %; of 64 channels 1.04 and 1.07, 153 of
-// 329 -- 118 images 192 -> 320 of stride 2 on 8x8 36.4 / 47.8, 5 images 64 -> 320 of 5x5 and stride 2 on 57x98 88.8 / 113.8.
+// channels share them.  (500 convs of 3x3 with stride 2 and of 5x5, us against the fp32 instruction: the 240 planned in tiles of 128
+// channels take 0.873 times its time, 3 of them over 5 % longer; of 64 channels 1.04 and 1.07, 153 of 329 of an earlier sweep --
+// 118 images 192 -> 320 of stride 2 on 8x8 36.4 / 47.8, 5 images 64 -> 320 of 5x5 and stride 2 on 57x98 88.8 / 113.8.
 // 3x3 convs of 8 (mod 16) channels, whose other form reads an LDS tile: 128x128 0.876, 64x64 1.061.)
 static bool taps_pay(int group, int m, long long npix, int k) {
   const int tile = plan_split(group, m, (int)npix, k, SPLIT_TAPS).tile;
@@ -768,7 +771,6 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
 }
 
 namespace {
-// Launches what wdh_linear_group queued: one launch per kernel variant and GROUP_MAX problems.
 // Problems queued for gemm_wavesplit_kernel that together fill the chip with 64x64 tiles, one a CU at most, whose K four
 // groups of wavefronts share (split_product.h): 32x32 blocks read every operand twice as often.  Three of 384x768x768 23.7 us as
 // blocks, 19.1 so; 512x512x512 17.3 / 14.5, 300x1024x1024 29.8 / 23.9, 256x768x768 19.0 / 17.5; 850x256x256 (8.2) and 200x768x768
@@ -790,6 +792,7 @@ bool group_splits(int variant) {
   return count > 1 && count <= GROUP_MAX && tiles <= cus &&
          6.2 + 0.16 * ((k + BK - 1) / BK) < 0.9 * (3.0 + 0.0065 * (double)((blocks + cus - 1) / cus) * k);
 }
+// Launches what wdh_linear_group queued: one launch per kernel variant and GROUP_MAX problems.
 int flush_group() {
   for (int variant = 0; variant < 4; variant++) {
     if (group_splits(variant)) {
@@ -1141,14 +1144,24 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   };
   const bool rows_split = rows_possible();
   bool wino_memory = true;  // there was room for the transform-domain tensors, if they were wanted
-  // Where the direct forms on the bf16 matrix cores are the faster ones after all: below 256 channels rows read straight from X
-  // do not pay for transforms (us, transforms / rows: 32 images 128 -> 128 on 28x28 61 / 52, 12 on 34x39 45 / 36, 5 on 24x32 21 / 18;
-  // small planes stay: 20 us either way), and transform-domain tensors that outgrow the 256 MB last-level cache
-  // cost more than the multiplications saved (128 images of it, V and M 206 MB each, 254 / 150).  From 256 channels on the
-  // multiplications count: 32 images 256 -> 256 on 14x14 46 / 61, 512 -> 512 on 7x7 47 / 61.
+  // Where the direct forms on the bf16 matrix cores are the faster ones after all.  Rows read straight from X do not pay for
+  // transforms, which move V and M, four times the input and four times the result, out and in again (at 5.2 and 4.1 TB/s); transforms
+  // save 5 multiplications in 9.  From 3500 pixels on both are estimated (their product by the model of plan_split); fewer
+  // stay with the transforms, whose launches are as short.  Of 134 convs of 128 channels and more none takes over 4 % longer than
+  // with the fp32 instruction.  (us, transforms / rows: 32 images 128 -> 128 on 28x28 61 / 52, 256 -> 256 on 14x14 46 / 61;
+  // 4 images 512 -> 160 on 45x63 100 / 141, 2 images 832 -> 192 on 63x63 105 / 149; 224 -> 992 on 8x8 12.3 / 14.8.)
+  // Transform-domain tensors that outgrow the 256 MB last-level cache cost more (128 images 128 -> 128 on 28x28, V and M 206 MB
+  // each, 254 / 150); there gathered taps are asked too, where rows are too wide for LDS (13 images 336 -> 416 on 19x91 293 / 447).
   auto direct_suits = [&]() {
     if (g_winograd != 1 || !(gather_split || rows_split)) return false;
-    return (rows_split && wino_min < 256 && npix >= 3500) || 64LL * (c + cout) * wdh::wino_tiles(2, n, oh, ow) > (256LL << 20);
+    const long long blocks = wdh::wino_tiles(2, n, oh, ow), pitch = wdh::wino_pitch(blocks);
+    const bool outgrown = 64LL * (c + cout) * blocks > (256LL << 20);
+    if (rows_split && outgrown) return true;
+    if (rows_split ? npix < 3500 : !outgrown) return false;
+    const double v = 4.0 * c * (16.0 * (double)pitch + (double)n * h * w), m = 4.0 * cout * (16.0 * (double)pitch + (double)npix * (p.R ? 2 : 1));
+    const SplitPlan product = plan_split(16, cout, (int)pitch, c, SPLIT_GEMM);
+    const SplitPlan direct = plan_split(1, cout, (int)npix, (int)kdim, rows_split ? SPLIT_ROWS : SPLIT_TAPS);
+    return direct.tile >= 0 && direct.us < 8.6 + 0.94 * product.us + 0.19e-6 * v + 0.245e-6 * m;
   };
   int wino_r = 0;
   if (g_winograd == 2) wino_r = 2;
