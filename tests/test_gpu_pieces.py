@@ -18,8 +18,6 @@ def test_gather_of_runs(ctx, inner, outer, axis, n):
     idx = rng.integers(-axis, axis, n).astype(np.int32)
     y = H.gather(ctx, ctx.move_tensor(x), ctx.move_tensor(idx), 1).get_data()
     assert (y == x[:, idx]).all()
-    view = ctx.move_tensor(np.concatenate([x.ravel(), x.ravel()[:8]]))  # (int32 as well)
-    view.dispose()
     xi = rng.integers(-9, 9, x.shape).astype(np.int32)
     assert (H.gather(ctx, ctx.move_tensor(xi), ctx.move_tensor(idx), 1).get_data() == xi[:, idx]).all()
 
@@ -57,7 +55,7 @@ def test_maxpool_bands(ctx, w, h, kernel, stride, pad):
     assert (got == ref.maxpool(x, [kernel] * 2, pads=[pad] * 4, strides=[stride] * 2)).all()
 
 
-# rows of 2 (mod 4) elements: pieces of two, tiles and flat runs; an operand by channel, by column, a scalar, and one that is misaligned by a row
+# rows of 2 (mod 4) elements: pieces of two, tiles and flat runs; an operand by channel, by column and a scalar
 @pytest.mark.parametrize("op", ["Add", "Sub", "Mul", "Div", "Pow"])
 @pytest.mark.parametrize("shape,other", [((2, 3, 5, 126), (3, 1, 1)), ((4, 6, 50), (50,)), ((7, 5, 30), (7, 1, 30)), ((3, 1026), (1,)), ((2, 3, 9, 14), (2, 1, 9, 1)),
                                          ((5, 3, 2), (3, 1)), ((4, 130), (4, 1))])

@@ -489,7 +489,8 @@ int wdh_free(wdh_buf h) {
 // The host's copies between the caller's memory and pinned memory, which bound a transfer once DMA and copy overlap (DMA
 // 55 GB/s).  From a megabyte on the stores go past the caches: a plain copy reads every line of its target first, and the
 // data is on its way elsewhere (12.6 MB into pinned memory 221 to 468 us / 166, out of it behind a DMA 374 to 492 / 278 to 314;
-// 512 KB 9 to 21 / 16 to 23).
+// 512 KB 9 to 21 / 16 to 23).  A download's reader finds its first pass colder and still has the result earlier: read and maximum of
+// a fresh array 101 / 91 us for 1 MiB, 127 / 132 for 1.75, 181 / 155 for 2, 300 / 255 for 4, 783 / 740 for 12.6 MB, 3498 / 3225 for 32 MiB.
 static void copy_through(void *to, const void *from, size_t bytes, size_t whole) {
 #if defined(__SSE2__) && !defined(__HIP_DEVICE_COMPILE__)
   if (whole >= (1u << 20)) {
