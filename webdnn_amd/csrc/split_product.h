@@ -12,9 +12,10 @@
 // instruction / this): K 64 14.5e-8 / 5.0e-8, 256 28.7e-8 / 8.9e-8, 1024 5.8e-7 / 1.9e-7, 4096 11.5e-7 / 4.0e-7; positive
 // operands 12.2e-8 / 5.2e-8 to 9.8e-7 / 3.5e-7, no drift to either side (below 1e-8).
 //
-// Bound: power.  A loop of nothing but these instructions runs at 1550 to 1800 TFLOP/s, which is 260 to 300 of fp32
-// products (the fp32 instruction's own limit is 157); at 4096^3 the matrix cores are busy 79 % of the cycles and the clock
-// falls to 1.5 GHz.  What a slab adds to the products is the split (14 vector instructions per pair of elements, three of
+// Bound: power, then instruction issue.  A loop of nothing but these instructions on normally distributed operands runs at 1720 to
+// 1770 TFLOP/s and 1.8 GHz (on zeros 2320 and 2.4), which is 290 of fp32 products (the fp32 instruction's own limit is 157); at
+// 4096^3 the clock is the same and the matrix cores are busy 70 % of the cycles (counters in
+// profiles/contraction_kernel_gemm4096_conv_c3.txt).  What a slab adds to the products is the split (14 vector instructions per pair of elements, three of
 // them to look at it) and LDS traffic (6 bytes an element), so an operand is split once, on its way from registers to LDS,
 // not by every wavefront that multiplies it.  The split and the LDS stores of the next slab are placed between the matrix
 // instructions of this one (sched_group_barrier): 195 -> 209 TFLOP/s, because the wavefronts of a SIMD else meet the same phase
