@@ -13,14 +13,14 @@ run is eager, the second records the run's kernels into a HIP graph, every timed
 graph (same kernels, same order, one launch) and reads the logits.  `value` = 32 * steps / total time.
 
 `roofline` is for the dominant kernels of that workload, the implicit-GEMM contraction kernels (the
-1x1 convs read X in place, the 3x3 stride-1 convs stage input rows in LDS or, from 128 channels on,
-run as F(2x2, 3x3) minimal filtering -- transforms around a batched product of the same kernel -- the
+1x1 convs read X in place, the 3x3 stride-1 convs stage input rows in LDS or, where an
+estimate says so, run as F(2x2, 3x3) minimal filtering -- transforms around a batched product -- the
 rest gather taps; all share one tile schedule and epilogue): their algorithmic FLOPs (2*M*N*K per
 Conv/Gemm node as the direct sum needs them, summed over the node list) over the device time of
 the timed steps, measured with one HIP event pair on the library's stream around each graph replay
-(the step's other kernels are inside that bracket, which makes the figure a lower bound).  Minimal
-filtering issues fewer multiplications than that numerator counts: `mfma_flops_issued_per_step` and
-`frac_issued` give what the matrix cores really execute per step and its share of the peak.
+(the step's other kernels are inside that bracket, which makes the figure a lower bound).  The peak
+is the fp32 matrix instruction's; it bounds neither minimal filtering, which issues fewer
+multiplications than that numerator counts, nor products made of six bf16 ones, so fractions may exceed 1.
 Inside `roofline`, so that one record holds everything the metric names:
   kernels        Gemm 4096^3 and the config-3 Conv as single-kernel figures (ms, GFLOP/s, fraction of the
                  fp32 MFMA peak), each timed as replays of a HIP graph that holds the launches back to back,
@@ -58,11 +58,11 @@ PEAK_FP32_MFMA_TFLOPS = 157.3
 # HBM-side bytes of the ResNet-50 step per Conv / Gemm node (54 nodes; contraction kernels, reduce passes
 # and the transforms of the minimal-filtering convs): rocprofv3 --pmc FETCH_SIZE (x2.000) + WRITE_SIZE
 # (x1.000), factors from a 256 MiB device copy; recorded in profiles/contraction_kernel_resnet50_b32.txt
-# (bench.py cannot read counters itself).  The transform-domain tensors of the 13 minimal-filtering convs
+# (bench.py cannot read counters itself).  The transform-domain tensors of the 9 minimal-filtering convs
 # (four times the conv's input and output, written once, read once or twice) and the partial sums of
 # tiles cut along K are in it; both live between consecutive launches and are counted in front of the
 # Infinity Cache.
-TRAFFIC_BYTES_PER_LAUNCH = 110.6e6  # (110.56 in the latest profile)
+TRAFFIC_BYTES_PER_LAUNCH = 93.5e6
 CLI = os.path.join(ROOT, "webdnn_amd", "js", "cli", "run_model.js")
 ORACLE_JS = os.path.join(ROOT, "oracle", "js", "cpuOperators.js")
 
@@ -132,7 +132,6 @@ def bench_resnet(steps, warmup, workdir):
         "two_in_flight_ms_per_step": pipe_resident_ms, "two_in_flight_host_input_ms_per_step": pipe_host_ms,
         "three_in_flight_ms_per_step": pipe3_resident_ms,
         "f4x4_device_ms": sum(f4["deviceMsPerRun"]) / len(f4["deviceMsPerRun"]),
-        "flops_saved": g.flops_saved,
         "batch": batch, "flops": g.flops, "nodes": timed["nodes"], "ms_per_step": total_ms / steps,
         "images_per_s": batch * steps / total_ms * 1e3, "contraction_ms": contraction_ms,
         "contraction_launches": launches, "device_ms": all_ms,
@@ -298,7 +297,7 @@ def bench_kernels(steps, warmup, calibrate_copy=False):
                 "ms_launched_one_by_one": round(eager, 4)}
 
     return {
-        "gemm_4096": entry("Gemm M=N=K=4096 + bias[4096], alpha=beta=1, U[-1,1] (north_star NS-4096)", gemm_flops, gemm_ms,
+        "gemm_4096": entry("Gemm M=N=K=4096 + bias[4096], alpha=beta=1, U[-1,1]", gemm_flops, gemm_ms,
                            gemm_eager),
         "conv_c3": entry("Conv 3x3 X[32,64,56,56] W[64,64,3,3] pad 1 + bias + Relu fused (config 3)", conv_flops, conv_ms,
                          conv_eager),
@@ -523,7 +522,7 @@ def main():
         "roofline": {
             "bound": "mfma",
             "kernel": "contraction kernels (implicit-GEMM Conv: in-place 1x1, LDS-tile 3x3, F(2x2,3x3) minimal filtering "
-                      "for 3x3 from 256 channels on, gathered forms, stem; Gemm head; most as six bf16 products on operands split "
+                      "for 3x3 of 256 and 512 channels, gathered forms, stem; Gemm head; most as six bf16 products on operands split "
                       "exactly, so that peak, the fp32 instruction's, is no limit), %d Conv/Gemm nodes per step; device "
                       "time = HIP events around each timed graph replay (whole step: transforms, MaxPool and "
                       "GlobalAveragePool included); achieved = direct-sum FLOPs (2MNK per node) / that time"
@@ -534,13 +533,9 @@ def main():
             "frac": round(achieved / PEAK_FP32_MFMA_TFLOPS, 4),
             "traffic": TRAFFIC_BYTES_PER_LAUNCH,
             "traffic_note": "bytes per Conv/Gemm node from rocprofv3 FETCH_SIZE+WRITE_SIZE, see profiles/; algorithmic "
-                            "64.1e6; the excess is the transform-domain tensors of the 13 F(2x2,3x3) convs (36.6e6 per "
+                            "64.1e6; the excess is the transform-domain tensors of the 9 F(2x2,3x3) convs (18.7e6 per "
                             "node), which pass between consecutive launches through the Infinity Cache",
             "flops_per_step": resnet["flops"],
-            # what the matrix cores execute: minimal filtering replaces 36 multiplications per 2x2 block by 16
-            "mfma_flops_issued_per_step": resnet["flops"] - resnet["flops_saved"],
-            "frac_issued": round((resnet["flops"] - resnet["flops_saved"]) / resnet["graph_device_ms"] / 1e9
-                                 / PEAK_FP32_MFMA_TFLOPS, 4),
             "avg_launch_ms": round(resnet["graph_device_ms"] / resnet["contraction_launches"], 5),
             "step_device_ms": round(resnet["graph_device_ms"], 4),
             # the two single-kernel figures the metric names (graph replays of back-to-back launches)
