@@ -268,19 +268,38 @@ def test_gathered_taps_of_a_full_round_of_tiles_and_a_few(ctx, split):
     assert np.abs(got.astype(np.float64) - want).max() <= 1e-5 * np.abs(want).max()
 
 
-@pytest.mark.parametrize("residual", [False, True])
-def test_a_short_k_with_a_residual_on_odd_planes(ctx, split, residual):
-    """Stays with the fp32 instruction where 128x128 tiles would serve, bit for bit."""
+@pytest.mark.parametrize("shape,residual,small", [((42, 96, 15, 77, 512, 1), True, True), ((42, 96, 15, 77, 512, 1), False, True), ((8, 192, 28, 28, 512, 2), True, True),
+                                                  ((64, 128, 28, 28, 512, 1), True, True), ((64, 128, 28, 28, 512, 1), False, True), ((64, 208, 28, 28, 512, 1), True, False),
+                                                  ((88, 128, 28, 28, 512, 1), True, False)])
+def test_1x1_convs_of_a_short_k_take_small_tiles(ctx, split, shape, residual, small):
+    """In place, a pixel at a time and with stride 2; what bounds them is the results and the residual."""
+    n, cin, h, w, cout, stride = shape
     rng = np.random.default_rng(17)
-    x = ctx.move_tensor(rng.standard_normal((42, 96, 15, 77)).astype(np.float32))
-    wt = ctx.move_tensor(rng.standard_normal((512, 96, 1, 1)).astype(np.float32))
-    r = ctx.move_tensor(rng.standard_normal((42, 512, 15, 77)).astype(np.float32)) if residual else None
+    x = ctx.move_tensor(rng.standard_normal((n, cin, h, w)).astype(np.float32))
+    wt = ctx.move_tensor(rng.standard_normal((cout, cin, 1, 1)).astype(np.float32))
+    r = ctx.move_tensor(rng.standard_normal((n, cout, h // stride, w // stride)).astype(np.float32)) if residual else None
     out = []
     for value in (0, 1):
         split(value)
-        out.append(H.conv(ctx, x, wt, residual=r).get_data())
-    assert (out[0] == out[1]).all() == residual
+        out.append(H.conv(ctx, x, wt, residual=r, strides=[stride, stride]).get_data())
+    assert (ctx.last_plan()["tile"] == "64x64") == small, ctx.last_plan()
+    assert not (out[0] == out[1]).all()
     assert np.abs(out[0].astype(np.float64) - out[1]).max() <= 1e-5 * np.abs(out[0]).max()
+
+
+@pytest.mark.parametrize("n,cin,h,w,cout,kernel,stride", [(42, 96, 15, 77, 128, 1, 1), (5, 128, 28, 28, 512, 1, 1), (3, 160, 14, 14, 320, 1, 1), (2, 256, 23, 31, 96, 1, 2),
+                                                          (4, 512, 45, 63, 160, 3, 1), (12, 128, 34, 39, 128, 3, 1), (6, 128, 30, 30, 128, 3, 2)])
+def test_a_residual_does_not_decide_the_form(ctx, n, cin, h, w, cout, kernel, stride):
+    """Conv with bias, residual and Relu in one launch has the bits of the three nodes."""
+    rng = np.random.default_rng(n + cin + h)
+    pads = [kernel // 2] * 4
+    x, wt = rng.standard_normal((n, cin, h, w)).astype(np.float32), rng.standard_normal((cout, cin, kernel, kernel)).astype(np.float32)
+    x, wt, b = ctx.move_tensor(x), ctx.move_tensor(wt), ctx.move_tensor(rng.standard_normal(cout).astype(np.float32))
+    y = H.conv(ctx, x, wt, b, pads=pads, strides=[stride, stride])
+    r = ctx.move_tensor(rng.standard_normal(y.dims).astype(np.float32))
+    want = H.unary(ctx, "Relu", H.binary(ctx, "Add", y, r)).get_data()
+    got = H.conv(ctx, x, wt, b, pads=pads, strides=[stride, stride], residual=r, epilogue="relu").get_data()
+    assert (got == want).all()
 
 
 ROWS = [

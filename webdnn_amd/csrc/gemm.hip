@@ -372,7 +372,8 @@ static bool tiles_beat_wavesplit(int batch, int m, int n, int k, bool b_kc, bool
 // at most (K below 100 or a residual bounds the launch there); of 1120 it takes over 5 % longer than the fp32 instruction 13
 // (no product, 7 of 281 1x1 convs, 3 of 355 3x3 ones, 3 of 240 with gathered taps), 21 % at most.
 enum SplitSource { SPLIT_GEMM, SPLIT_PIXELS, SPLIT_TAPS, SPLIT_ROWS };  // where B comes from: a matrix, X in place, gathered taps, rows of X in LDS
-static SplitPlan search_split(int nz, int m, int n, int k, SplitSource source, bool large_tiles) {
+enum SplitSizes { SIZES_ANY, SIZES_LARGE, SIZES_SMALL };  // SIZES_LARGE: no 64x64 tiles; SIZES_SMALL: those whose K is not shared, only
+static SplitPlan search_split(int nz, int m, int n, int k, SplitSource source, SplitSizes sizes) {
   struct Model { int bm, bn; double slab, solo, fixed; };
   static const Model models[4][7] = {
       {{128, 128, 0.63, 0.56, 9.5}, {64, 128, 0.37, 0.39, 6.5}, {128, 64, 0.37, 0.39, 6.5}, {64, 64, 0.21, 0.29, 5.2}, {256, 128, 1.20, 0.95, 10.0}, {64, 64, 0.22, 0.24, 6.0}, {64, 64, 0.23, 0.14, 10.7}},
@@ -386,7 +387,8 @@ static SplitPlan search_split(int nz, int m, int n, int k, SplitSource source, b
   SplitPlan best = {-1, {}, 1e30};
   for (int t = 0; t <= S64x64K4; t++) {
     const Model &mo = models[source][t];
-    if (mo.bm == 0 || (large_tiles && mo.bm * mo.bn == 64 * 64) || (g_split >= 3 && t != g_split - 3)) continue;
+    if (mo.bm == 0 || (sizes == SIZES_LARGE && mo.bm * mo.bn == 64 * 64) || (sizes == SIZES_SMALL && t != S64x64) ||
+        (g_split >= 3 && t != g_split - 3)) continue;
     const long long tiles = (long long)((m + mo.bm - 1) / mo.bm) * ((n + mo.bn - 1) / mo.bn) * nz;
     const int most = g_forced_split >= 1 && slabs > 0 ? (g_forced_split < slabs ? g_forced_split : slabs)
                                          : slabs / 4 < 32 ? slabs / 4 : 32;  // at least 64 elements of K per chunk
@@ -416,17 +418,28 @@ static SplitPlan search_split(int nz, int m, int n, int k, SplitSource source, b
   return best;
 }
 // (the search takes a few microseconds on the host, so the plans of the last sizes are kept)
-static SplitPlan plan_split(int nz, int m, int n, int k, SplitSource source, bool large_tiles = false) {
-  struct Kept { int cus, nz, m, n, k, source, large_tiles; SplitPlan plan; };
+static SplitPlan plan_split(int nz, int m, int n, int k, SplitSource source, SplitSizes sizes = SIZES_ANY) {
+  struct Kept { int cus, nz, m, n, k, source, sizes; SplitPlan plan; };
   static thread_local Kept kept[256] = {};
-  if (g_split != 1 || g_forced_split >= 1) return search_split(nz, m, n, k, source, large_tiles);
+  if (g_split != 1 || g_forced_split >= 1) return search_split(nz, m, n, k, source, sizes);
   const int cus = wdh::compute_units();
   unsigned h = (unsigned)nz;
-  for (int v : {m, n, k, (int)source, (int)large_tiles}) h = (h ^ (unsigned)v) * 0x9e3779b1u;
+  for (int v : {m, n, k, (int)source, (int)sizes}) h = (h ^ (unsigned)v) * 0x9e3779b1u;
   Kept &e = kept[h >> 24];
-  if (e.cus != cus || e.nz != nz || e.m != m || e.n != n || e.k != k || e.source != (int)source || e.large_tiles != (int)large_tiles)
-    e = {cus, nz, m, n, k, (int)source, (int)large_tiles, search_split(nz, m, n, k, source, large_tiles)};
+  if (e.cus != cus || e.nz != nz || e.m != m || e.n != n || e.k != k || e.source != (int)source || e.sizes != (int)sizes)
+    e = {cus, nz, m, n, k, (int)source, (int)sizes, search_split(nz, m, n, k, source, sizes)};
   return e.plan;
+}
+// A 1x1 conv.  With a short K the results and the residual bound it, and tiles of which a CU holds more overlap their epilogues
+// better.  (Of 300 convs of 96 to 160 channels with a residual 97 took over 5 % longer than with the fp32 instruction as the model
+// plans them, 42 % at most, and 2 % in the mean; in 64x64 tiles 21, 17 % at most, and 6 % less in the mean.  96 -> 96 on 54x54 with 92
+// images 97.8 us, 139 / 101.  Without a residual there is nothing in it either way, nor with one from 200 channels on; whether there is
+// one must not decide, because a result does not depend on what is fused to it.)  Rounds of whole 128-row tiles keep theirs: between the convs of a network, with the clock that it leaves, 128 -> 512 on 28x28 and the two convs
+// behind it take 384 us for 128 images, 390 with 64x64 tiles (396 with the fp32 instruction); 64 images 206 / 205 (208), 32 119 / 114 (113).
+static SplitPlan plan_pixels(int group, const Params &p) {
+  const bool rounds = p.m % 128 == 0 && (long long)p.cv.oh * p.cv.ow % 4 == 0 && (long long)(p.m / 128) * ((p.n + 127) / 128) * group >= 8LL * wdh::compute_units();
+  const bool small = p.k <= 160 && !rounds;
+  return plan_split(group, p.m, p.n, p.k, SPLIT_PIXELS, small && g_split < 3 ? SIZES_SMALL : SIZES_ANY);
 }
 // Whether a Gemm / MatMul that may go to them does, and how.
 // Where gemm_wavesplit_kernel could serve, whose time is its blocks' rounds over the CUs: long products that go to cut
@@ -446,7 +459,7 @@ static SplitPlan split_gemm_plan(int batch, int m, int n, int k, bool b_kc) {
     }
     const long long blocks32 = (long long)((m + 31) / 32) * ((n + 31) / 32) * batch, cus = wdh::compute_units();
     // (below the lengths that tiles_beat_wavesplit looks at the tile is free)
-    const SplitPlan s = plan_split(batch, m, n, k, SPLIT_GEMM, k >= 2000);
+    const SplitPlan s = plan_split(batch, m, n, k, SPLIT_GEMM, k >= 2000 ? SIZES_LARGE : SIZES_ANY);
     return s.us < 0.85 * (3.0 + 0.0078 * (double)((blocks32 + cus - 1) / cus) * k) ? s : none;
   }
   return (double)batch * m * n * k >= 1e8 ? plan_split(batch, m, n, k, SPLIT_GEMM) : none;
@@ -1115,7 +1128,7 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
     // (what the plan schedules as a stream of K slabs stays one)
     g_last_form = in_place_s2 ? B_PIXELS_S2 : B_PIXELS;
     if (split_legal(p, true) && !(g_split == 1 && conv_streams(p, group)))
-      if (const SplitPlan s = plan_split(group, p.m, p.n, p.k, SPLIT_PIXELS);
+      if (const SplitPlan s = plan_pixels(group, p);
           s.tile >= 0 && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS)))
         return run_split(s, [&](const SplitPlan &q) { return launch_split_conv(in_place_s2 ? B_PIXELS_ANY : B_PIXELS, q, p, group); });
     return launch_conv_pixels(p, group, true, in_place_s2);
@@ -1126,7 +1139,7 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   key.c_in_g = c_in_g; key.kh = kh; key.kw = kw; key.dh = dh; key.dw = dw;
   key.h = h; key.w = w; key.mode = mode;
   // (while a graph is being recorded the gathered forms serve only geometries whose tap table is there already)
-  bool gather_split = mode != B_IM2COL_BIG && (!wdh::capturing() || g_ktabs.count(key)) && split_possible(n, cout_g, (int)kdim) &&
+  const bool gather_split = mode != B_IM2COL_BIG && (!wdh::capturing() || g_ktabs.count(key)) && split_possible(n, cout_g, (int)kdim) &&
                             (g_split > 1 || taps_pay(group, cout_g, npix, (int)kdim));
   // 3x3, stride 1, no dilation, one group, many channels: minimal filtering -- filters and input patches
   // are transformed, the positions of the transform domain (16 for F(2x2, 3x3), 36 for F(4x4, 3x3)) are
@@ -1158,7 +1171,7 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
     const bool outgrown = 64LL * (c + cout) * blocks > (256LL << 20);
     if (rows_split && outgrown) return true;
     if (rows_split ? npix < 3500 : !outgrown) return false;
-    const double v = 4.0 * c * (16.0 * (double)pitch + (double)n * h * w), m = 4.0 * cout * (16.0 * (double)pitch + (double)npix * (p.R ? 2 : 1));
+    const double v = 4.0 * c * (16.0 * (double)pitch + (double)n * h * w), m = 4.0 * cout * (16.0 * (double)pitch + (double)npix);
     const SplitPlan product = plan_split(16, cout, (int)pitch, c, SPLIT_GEMM);
     const SplitPlan direct = plan_split(1, cout, (int)npix, (int)kdim, rows_split ? SPLIT_ROWS : SPLIT_TAPS);
     return direct.tile >= 0 && direct.us < 8.6 + 0.94 * product.us + 0.19e-6 * v + 0.245e-6 * m;
@@ -1283,16 +1296,10 @@ direct_forms:
   // any other unpadded 1x1 conv of a batch: each pixel of X is read where it lies, whatever the strides and the plane
   if (small && vec && ntaps == 1 && pt == 0 && pl == 0 && pb == 0 && pr == 0) {
     p.m = cout_g; p.n = (int)npix; p.k = (int)kdim;
+    p.cv.oh = oh; p.cv.ow = ow;
     p.fast = 1;
     SplitPlan s = {-1, {}, 0.0};
-    if (split_legal(p, true) && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS))) s = plan_split(group, p.m, p.n, p.k, SPLIT_PIXELS);
-    // (a short K hides little of an epilogue that takes a residual 4 bytes at a time, and two 128x128 tiles a CU overlap
-    // little: 42 images 96 -> 512 on 15x77 73.4 us with the fp32 instruction, 85.7 here; without a residual 68.1 / 58.5 (74
-    // images 96 -> 1024 on 17x19); K 128 in narrower tiles 18.9 / 17.0)
-    if (g_split == 1 && s.tile == S128x128 && p.k < 128 && p.R && (long long)oh * ow % 4 != 0) {
-      s.tile = -1;
-      gather_split = false;
-    }
+    if (split_legal(p, true) && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS))) s = plan_pixels(group, p);
     if (s.tile >= 0) {
       p.sAb = (long long)cout_g * kdim; p.sA0 = kdim; p.sA1 = 1;
       p.sBb = (long long)c_in_g * plane; p.sB0 = plane; p.sB1 = 1;
