@@ -465,8 +465,10 @@ static SplitPlan split_gemm_plan(int batch, int m, int n, int k, bool b_kc) {
   return (double)batch * m * n * k >= 1e8 ? plan_split(batch, m, n, k, SPLIT_GEMM) : none;
 }
 // Whether a conv of a batch does.  A single image stays with the fp32 instruction: its launches are short of tiles (ResNet-50's
-// 50 of them take 3 to 10 us each, mostly latency), and its results stay bit for bit what they were.  K below 96 leaves
-// nothing to gain from faster products (128 images 64 -> 256 on 56x56 173 us / 190, 16 images 32 -> 64 on 112x112 18.4 / 20).
+// 50 of them take 3 to 10 us each, mostly latency), and its results stay bit for bit what they were.  (Of larger images many would
+// gain: 350 convs of 10 to 200 us 0.91 of the fp32 instruction's time in the mean, 0.58 to 1.20.)  K below 96 leaves nothing to gain
+// from faster products (1x1 convs of K 64 1.00 of its time, 1.03 with a residual, 80 0.97 and 1.02, 96 0.94 and 0.99; 128 images
+// 64 -> 256 on 56x56 173 us / 190).
 // Rows of channels that hardly fill their tiles leave nothing either (108 -> 94 39 / 44).
 static bool split_conv_suits(int images, int m, int k, SplitSource source) {
   if (images < 2 || k < 96) return false;
@@ -1146,8 +1148,8 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   // one batched product M[xi] = U[xi] [cout, c] x V[xi] [c, tiles] with 4/9 or 1/4 of the direct form's
   // multiplications, and the products are transformed back under the epilogue (winograd.hip).
   // g_winograd: 0 never; 1 = F(2x2, 3x3) from 128 channels on (F(4x4, 3x3) from g_winograd4_channels on, when
-  // that is set: faster from 64 channels on, but its rounding errors are about ten times the direct form's,
-  // which a 50-layer network's logits show); 2 / 3 = F(2x2, 3x3) / F(4x4, 3x3) wherever legal.
+  // that is set: one image is faster so from 64 channels on, 32 images of ResNet-50 are not (2.29 ms for 2.21), and its rounding
+  // errors are about ten times the direct form's, which a 50-layer network's logits show); 2 / 3 = F(2x2, 3x3) / F(4x4, 3x3) wherever legal.
   const int wino_min = c < cout ? c : cout;
   auto rows_possible = [&]() {
     if (!(g_halo && kh == 3 && kw == 3 && sh == 1 && sw == 1 && dh == 1 && dw == 1 && group == 1 && c % 16 == 0)) return false;
