@@ -113,7 +113,7 @@ int wdh_device_info(char *name, int name_cap, int *compute_units,
  *                       instruction's; tiles with an Inf, a NaN or elements too small for three parts, nonzero below
  *                       2^-110, are computed again with the fp32 one where that can show), 0 = the fp32 one
  *                       everywhere, 2 = the bf16 ones wherever they are legal;
- *                       3..9 = that, with 128x128, 64x128, 128x64, 64x64, 256x128 tiles, or 64x64 ones whose K two or
+ *                       3..9 = that, with 128x128, 64x128, 128x64, 64x64, 256x128 (products only) tiles, or 64x64 ones whose K two or
  *                       four groups of wavefronts share (tuning and test hooks).
  *                       "stream_k" 2, and "contraction_tile" or "split_k" beside 1, keep the fp32 instruction.
  *   "wide_stores"       1 (default) = whole result tiles whose rows are 16-byte aligned

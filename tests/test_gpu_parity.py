@@ -2,7 +2,7 @@
 
 Criteria: bit-exact for indexing / layout / selection ops and for
 fp32 Add/Sub/Mul/Div/Relu; max|diff| <= 1e-4 * max|ref| for Gemm / MatMul / Conv.  Softmax and
-LayerNormalization, for which north_star names no figure, use 1e-6 and 1e-5 of max|ref| (the
+LayerNormalization use 1e-6 and 1e-5 of max|ref| (the
 oracle evaluates exp in double and rounds once; the kernel evaluates it in fp32).
 """
 import ctypes

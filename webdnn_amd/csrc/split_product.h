@@ -30,8 +30,8 @@
 //     The sums cannot tell: large partners lift what is left of such an element to any size, and one that vanished leaves a
 //     zero.  A tile with such elements is done again unless all its sums are at least 2^-60 and no operand element reaches
 //     2^30: then K terms are off by at most K 2^-104, beyond the last bits of the sums.  (That keeps softmax rows and
-//     weights with a few vanishing elements on the fast path.  The look costs a net of two 4096^3 products and a narrow one
-//     1411 -> 1428 us, ResNet-50 of 128 images 6965 -> 7034.)
+//     weights with a few vanishing elements on the fast path.  The look costs ResNet-50 of 128 images 6986 -> 7045 us, products in
+//     256x128 tiles nothing (see BY_PAIR).)
 #pragma once
 #include "contraction.h"
 
