@@ -9,9 +9,9 @@
 // Only the order of the additions inside the two products and the row sum differs.
 //
 // A workgroup of eight or sixteen wavefronts owns 32 query rows of one head:
-//   1. scores: each wavefront takes 32-key column blocks in turn
-//      (v_mfma_f32_32x32x2_f32 over the head dimension) and writes alpha * S to LDS,
-//      the whole 32 x keys block (keys <= 1024: 129 KB of the CU's 160 KB);
+//   1. scores: Q and 32-key blocks of K go through LDS, each wavefront takes its blocks in turn
+//      (v_mfma_f32_32x32x2_f32 over the head dimension) and, when all are done with K, writes
+//      alpha * S to LDS, the whole 32 x keys block (keys <= 1024: 129 KB of the CU's 160 KB);
 //   2. softmax: four (two) rows per wavefront, in place in LDS;
 //   3. output: the keys are cut across the wavefronts in blocks of 32, each wavefront
 //      accumulates its share of P V on the matrix cores, and the partial 32 x HD
@@ -50,11 +50,18 @@ struct AttParams {
 //
 // Bound: latency -- a workgroup has a CU to itself and goes through its phases once.  So a wavefront asks for everything at
 // once, and for no more than its keys: PER_WAVE blocks of 32 keys (at most 32 * ATT_WAVES * PER_WAVE keys), not always the blocks of
-// 1024; V before the scores where the registers hold it beside K, else before the softmax.
+// 1024; V under the scores where the registers hold it beside them, else before the softmax.
 // (us, always 1024 keys' loads / these: 12 heads of 64, 200 tokens 12.6 / 11.0, 384 16.7 / 15.9, 600 26.4 / 24.1; 16 of 64, 1024 tokens
 // 80.8 / 67.6; 8 of 32, 100 keys 7.8 / 6.4, 300 11.3 / 9.4; 8 of 128, 128 keys 14.2 / 12.2.)
+// And for whole rows: K and Q, whose rows the matrix instruction wants one to a lane, pass through LDS.  Loaded by the lanes that
+// multiply them they are 16 bytes from 64 places, and a line is fetched again for each of its eight pieces.  (us, lane by lane / rows
+// through LDS, same bits: 12 heads of 64, 200 tokens 11.6 / 10.7, 384 16.9 / 14.8, 600 26.1 / 22.7; 128 of 64, 384 105.7 / 88.6; 16 of 64, 1024
+// 71.4 / 62.5; 8 of 32, 100 keys 6.9 / 6.8, 850 19.7 / 18.7; 128 of 32, 300 41.2 / 40.3; 8 of 128, 128 keys 12.7 / 11.8, 900 64.6 / 56.7.  Lane by
+// lane with everything requested at once is slower than one piece after the other: 384 tokens 19.1.)  Of V a lane wants a column: its
+// loads are whole rows as they are; they are asked for when the wavefront's first keys are in LDS and waited for where they multiply.
+// Heads of 32 with one block a wavefront are held to 64 registers, so that two workgroups share a CU (512 heads, 100 keys 46.3 / 35.5).
 template <int HD, int ATT_WAVES, int PER_WAVE>
-__global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParams p) {
+__global__ __launch_bounds__(64 * ATT_WAVES, HD == 32 && PER_WAVE == 1 ? 8 : ATT_WAVES / 4) void attention_rows_kernel(AttParams p) {
   static_assert(HD % 32 == 0 && HD >= 32 && HD <= 128, "head dimension");
   static_assert(ATT_WAVES == 8 || ATT_WAVES == 16, "32 rows and the key blocks are dealt over the wavefronts");
   static_assert(32 * ATT_WAVES * PER_WAVE <= ATT_MAX_KEYS, "keys");
@@ -66,7 +73,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
   // more (us, asked for / left out: 8 heads of 32, 850 keys 18.1 / 18.7; 8 of 128, 900 keys 61 / 80; but 12 of 64, 600 keys 33.0 / 24.6).
   constexpr bool SKIP = HD == 64 || PER_WAVE == 1;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = SKIP ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, half = lane >> 5;
   const int b = blockIdx.x / p.row_blocks;
   const int row0 = (blockIdx.x - b * p.row_blocks) * ATT_ROWS;
@@ -75,7 +82,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
   const float *V = p.V + (long long)b * p.sVb;
   const int ncb = (p.tk + 31) >> 5;  // blocks of 32 keys
 
-  // Every value of V this wavefront will need in step 3 (up to 64 registers travel while the scores are computed, up to
+  // Every value of V this wavefront will need in step 3 (up to 64 registers travel while the scores are multiplied, up to
   // 128 during the softmax).
   float vb[V_HELD ? PER_WAVE : 1][NB][16];
   auto fetch_v = [&](int kc, int nb, float (&v)[16]) {
@@ -83,53 +90,85 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
 #pragma unroll
     for (int s = 0; s < 16; s++) {
       const int key = key0 + s;
-      const float t = V[(long long)(key < p.tk ? key : p.tk - 1) * p.sVj + nb * 32 + li];
-      v[s] = key < p.tk ? t : 0.0f;  // (P is 0 there; this keeps an inf or NaN of V out)
+      v[s] = V[(long long)(key < p.tk ? key : p.tk - 1) * p.sVj + nb * 32 + li];
     }
   };
+  // What keys past the end read is put to 0 where V is used, not where it is asked for: a wavefront would wait for it there.
+  // (P is 0 there; this keeps an inf or NaN of V out.)
+  auto only_keys = [&](int kc, float (&v)[16]) {
+    if (kc * 32 + 32 <= p.tk) return;
+    const int key0 = kc * 32 + 16 * half;
+#pragma unroll
+    for (int s = 0; s < 16; s++) v[s] = key0 + s < p.tk ? v[s] : 0.0f;
+  };
+  auto has = [&](int it) { return wave + ATT_WAVES * it < ncb; };
   auto fetch_held = [&]() {
 #pragma unroll
     for (int it = 0; it < (V_HELD ? PER_WAVE : 1); it++)
-      if (!SKIP || wave + ATT_WAVES * it < ncb)
+      if (!SKIP || has(it))
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) fetch_v(wave + ATT_WAVES * it, nb, vb[it][nb]);
   };
-  if (V_FIRST) fetch_held();
 
   // ---- 1. scores -------------------------------------------------------------------
   {
-    float qa[HALF];
-    const int qrow = row0 + li < p.tq ? row0 + li : p.tq - 1;  // rows past the end are never stored
-    const float *q = Q + (long long)qrow * p.sQi + HALF * half;
+    // Q of the workgroup, then a block of keys for each wavefront: [row][HD + 4 floats]
+    constexpr int LP = HD + 4, PPR = HD / 4, KL = 32 * PPR / 64, QL = (32 * PPR + 64 * ATT_WAVES - 1) / (64 * ATT_WAVES);
+    constexpr int AHEAD = PER_WAVE < 2 ? PER_WAVE : 2;
+    float *const qs = lds, *const ks = lds + (1 + wave) * (32 * LP);
+    f32x4 qr[QL], kr[AHEAD][KL];
+    const int r0 = lane / PPR, c0 = lane % PPR * 4;
 #pragma unroll
-    for (int c = 0; c < HALF / 4; c++) {
-      const f32x4 t = *reinterpret_cast<const f32x4 *>(q + 4 * c);
-      qa[4 * c] = t.x; qa[4 * c + 1] = t.y; qa[4 * c + 2] = t.z; qa[4 * c + 3] = t.w;
+    for (int i = 0; i < QL; i++) {
+      const int at = tid + i * 64 * ATT_WAVES, row = row0 + at / PPR;
+      qr[i] = *reinterpret_cast<const f32x4 *>(Q + (long long)(row < p.tq ? row : p.tq - 1) * p.sQi + at % PPR * 4);  // (rows past the end are never stored)
     }
-    f32x4 kb[PER_WAVE][HALF / 4];
+    auto fetch_k = [&](int it) {
+#pragma unroll
+      for (int i = 0; i < KL; i++) {
+        const int key = (wave + ATT_WAVES * it) * 32 + i * (64 / PPR) + r0;
+        kr[it % AHEAD][i] = *reinterpret_cast<const f32x4 *>(K + (long long)(key < p.tk ? key : p.tk - 1) * p.sKj + c0);
+      }
+    };
+#pragma unroll
+    for (int it = 0; it < AHEAD; it++)
+      if (has(it)) fetch_k(it);
+#pragma unroll
+    for (int i = 0; i < QL; i++) {
+      const int at = tid + i * 64 * ATT_WAVES;
+      if (32 * PPR % (64 * ATT_WAVES) == 0 || at < 32 * PPR) *reinterpret_cast<f32x4 *>(qs + at / PPR * LP + at % PPR * 4) = qr[i];
+    }
+    __syncthreads();
+    f32x16 acc[PER_WAVE];
 #pragma unroll
     for (int it = 0; it < PER_WAVE; it++) {
-      if (SKIP && wave + ATT_WAVES * it >= ncb) continue;
+      if (!has(it)) break;
+#pragma unroll
+      for (int i = 0; i < KL; i++) *reinterpret_cast<f32x4 *>(ks + (i * (64 / PPR) + r0) * LP + c0) = kr[it % AHEAD][i];
+      if (it + AHEAD < PER_WAVE && has(it + AHEAD)) fetch_k(it + AHEAD);
+      if (V_FIRST && it == 0) fetch_held();
+      __builtin_amdgcn_wave_barrier();
+      acc[it] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < HALF / 4; c++) {
+        const f32x4 q = *reinterpret_cast<const f32x4 *>(qs + li * LP + HALF * half + 4 * c);
+        const f32x4 k = *reinterpret_cast<const f32x4 *>(ks + li * LP + HALF * half + 4 * c);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[it] = __builtin_amdgcn_mfma_f32_32x32x2f32(q[e], k[e], acc[it], 0, 0, 0);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();  // the scores go where Q and the keys were
+#pragma unroll
+    for (int it = 0; it < PER_WAVE; it++) {
+      if (!has(it)) break;
       const int key = (wave + ATT_WAVES * it) * 32 + li;
-      const float *k = K + (long long)(key < p.tk ? key : p.tk - 1) * p.sKj + HALF * half;
-#pragma unroll
-      for (int c = 0; c < HALF / 4; c++) kb[it][c] = *reinterpret_cast<const f32x4 *>(k + 4 * c);
-    }
-#pragma unroll
-    for (int it = 0; it < PER_WAVE; it++) {
-      const int cb = wave + ATT_WAVES * it;
-      if (cb >= ncb) break;
-      const int key = cb * 32 + li;
       const bool key_ok = key < p.tk;
-      f32x16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < HALF; s++)
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(qa[s], kb[it][s >> 2][s & 3], acc, 0, 0, 0);
       // lane holds column li, rows 8*(r/4) + 4*half + r%4; keys past the end count as -inf
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         const int row = 8 * (r >> 2) + 4 * half + (r & 3);
-        lds[row * p.pitch + key] = key_ok ? p.alpha * acc[r] : -INFINITY;
+        lds[row * p.pitch + key] = key_ok ? p.alpha * acc[it][r] : -INFINITY;
       }
     }
   }
@@ -209,6 +248,8 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
       if (kc >= ncb) break;
       fetch_p(kc, pa);
 #pragma unroll
+      for (int nb = 0; nb < NB; nb++) only_keys(kc, vb[it][nb]);
+#pragma unroll
       for (int nb = 0; nb < NB; nb++)
 #pragma unroll
         for (int s = 0; s < 16; s++)
@@ -221,6 +262,7 @@ __global__ __launch_bounds__(64 * ATT_WAVES) void attention_rows_kernel(AttParam
       for (int nb = 0; nb < NB; nb++) {
         float vn[16];
         fetch_v(kc, nb, vn);
+        only_keys(kc, vn);
 #pragma unroll
         for (int s = 0; s < 16; s++)
           o[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(pa[s >> 2][s & 3], vn[s], o[nb], 0, 0, 0);
@@ -260,8 +302,11 @@ int lds_pitch(int tk) {
 
 template <int HD, int ATT_WAVES, int PER_WAVE>
 int launch_attention(const AttParams &p, int batch) {
-  // the scores block, and later the wavefronts' partial outputs, whichever is larger
+  // Q and a block of keys a wavefront, then the scores block, and later the wavefronts' partial outputs, whichever is larger
   size_t bytes = (size_t)ATT_ROWS * p.pitch * 4;
+  const size_t blocks = (size_t)(p.tk + 31) / 32, rows = (size_t)(1 + (blocks < ATT_WAVES ? blocks : ATT_WAVES)) * 32 * (HD + 4) * 4;
+  static_assert((1 + ATT_WAVES) * 32 * (HD + 4) * 4 <= 160 * 1024, "LDS");
+  if (rows > bytes) bytes = rows;
   const size_t partials = (size_t)ATT_WAVES * ATT_ROWS * (HD + 1) * 4;
   if (partials > bytes) bytes = partials;
   hipLaunchKernelGGL((attention_rows_kernel<HD, ATT_WAVES, PER_WAVE>), dim3((unsigned)((long long)batch * p.row_blocks)),
