@@ -14,9 +14,9 @@
 // the LDS traffic and the vector instructions of a version with both operands in LDS (4096^3, us: 522 so, 395 packed; and with every strip
 // read by one wavefront instead of two, 32 rows x 128 columns each: 427 with packing for 455).
 //
-// Bound: nothing by itself.  The matrix cores are busy half of the time, the rest goes into vector instructions (two an element every 64 k,
-// three an element for the split), LDS reads and waits for L2, and into a start and an end of 9 to 12 us, part of it code that
-// arrives line by line.  A loop of nothing but the instruction makes 1830 TFLOP/s (32x32x16: 1640, bf16 16x16x32 1960), 610 of
+// Bound: no unit by itself.  The matrix cores are busy 0.62 of the time at 4096^3, 0.4 in 1x1 convs, the rest goes into vector
+// instructions (two an element every 64 k, three an element for the split), LDS reads and waits for L2, and into a start and an end of 9 to
+// 12 us, part of it code that arrives line by line; launched in a row, power joins in (415 us, the seventh 468).  A loop of nothing but the instruction makes 1830 TFLOP/s (32x32x16: 1640, bf16 16x16x32 1960), 610 of
 // products; 4096^3 349 without the packing (bfloat16 parts 212), 1024 -> 256 on 14x14 with 128 images 195 (142), 128 -> 128 3x3
 // on 28x28 222 (197).  Tried without gain: 64x64 a wavefront, groups of 32 columns, totals added a group later without reads ahead, LDS planes
 // 16 to 64 bytes apart, two buffers of rows for 3x3 convs of 640 pixels.
