@@ -569,9 +569,9 @@ static HalfPlan half_gemm_plan(int m, int n, int k, bool b_kc) {
   if (other.tile < 0 || s.us + pack > 0.85 * other.us || !half_is_as_precise(s, split_chain(other, k), HALF_GEMM)) s.tile = -1;
   return s;
 }
-// Whether the f16 matrix cores may serve a product at all.
+// Whether the f16 matrix cores may serve a product at all.  (An empty K has no blocks to plan, and nothing to multiply.)
 static bool half_legal(const Params &p) {
-  if (!g_half || g_split != 1 || g_fp32_hint || g_stream == 2 || !p.fast || p.k % 8 != 0 || g_static_scratch || g_group.collecting) return false;
+  if (!g_half || g_split != 1 || g_fp32_hint || g_stream == 2 || !p.fast || p.k < 8 || p.k % 8 != 0 || g_static_scratch || g_group.collecting) return false;
   return g_half > 1 || (g_forced_tile < 0 && g_forced_split < 0);
 }
 template <typename Launch>
