@@ -116,7 +116,9 @@ __global__ __launch_bounds__(WP * WQ * KG * 64, 2) void conv3x3_half_kernel(Para
   auto fetch_strips = [&](int k0, int pi, Strips &s) {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      const int soff = (strip0 + i) * stripsize + (k0 / KGRAN * 5 + 2 * pi) * STEP_BYTES;
+      // (past the last strip, or the last block: some other one again, as in half_product.h)
+      const int strip = strip0 + i < w.strips ? strip0 + i : w.strips - 1, block = k0 < p.k ? k0 / KGRAN : 0;
+      const int soff = strip * stripsize + (block * 5 + 2 * pi) * STEP_BYTES;
 #pragma unroll
       for (int t = 0; t < (pi < 2 ? 2 : 1); t++) {
         s.h[i][t] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc_p, lane * 16, soff + t * STEP_BYTES, 0));

@@ -283,7 +283,10 @@ __global__ __launch_bounds__(WP * KG * 64, 2) void half_kernel(Params p, HalfOpe
   auto fetch_strips = [&](int k0, Strips &s) {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      const int soff = (strip0 + i) * stripsize + k0 / HSTEP * STEP_BYTES;  // (strips past the last: outside the descriptor, zeros)
+      // (past the last strip, or the last step: some other one again, whose sums are never stored.  A scalar offset is no part of what
+      // a descriptor is checked for, so it stays within the block.)
+      const int strip = strip0 + i < w.strips ? strip0 + i : w.strips - 1, step = k0 / HSTEP < w.steps ? k0 / HSTEP : 0;
+      const int soff = strip * stripsize + step * STEP_BYTES;
 #pragma unroll
       for (int t = 0; t < 2; t++) {
         s.h[i][t] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc_p, lane * 16, soff + t * STEP_BYTES, 0));
