@@ -1,4 +1,5 @@
-"""What products and convolutions owe without any tolerance: the sum over nothing."""
+"""What products and convolutions owe without any tolerance, whichever form they take: the sum over nothing; a sum of one term; images
+and channels scaled by powers of two; the same results whether or not weights are vouched for."""
 import numpy as np
 import pytest
 
@@ -24,3 +25,48 @@ def test_an_empty_inner_dimension_leaves_the_other_terms(ctx, m, n, ta, tb):
     x = ctx.move_tensor(np.zeros((3, m, 0), np.float32))   # a batch, which may share its right operand
     assert (H.matmul(ctx, x, tb_, tc).get_data() == c).all()
     assert (H.matmul(ctx, x, ctx.move_tensor(np.zeros((3, 0, n), np.float32))).get_data() == 0).all()
+
+
+EXPONENTS = [0, -13, -20, -24, -28, -32, -40]
+CONVS = [  # n, c, h, w, cout, kernel, stride: enough sums of 500 to 4000 terms for the forms that large convs take
+    (64, 96, 28, 28, 96, 3, 1), (64, 128, 28, 28, 128, 3, 1), (128, 256, 14, 14, 256, 3, 1), (16, 256, 28, 28, 256, 3, 1), (9, 96, 31, 29, 100, 3, 1)]
+
+
+def convolve(ctx, x, w, stride, constant=True):
+    pads = [w.shape[2] // 2] * 4
+    tx, tw = ctx.move_tensor(x), ctx.move_tensor(w)
+    y = H.conv(ctx, tx, tw, pads=pads, strides=[stride, stride], constant_weights=constant)
+    out = y.get_data()
+    for t in (tx, tw, y):
+        t.dispose()
+    return out
+
+
+@pytest.mark.parametrize("shape", CONVS)
+def test_images_and_channels_of_other_magnitudes_are_the_same_sums(ctx, shape):
+    n, c, h, w, cout, kernel, stride = shape
+    rng = np.random.default_rng(sum(shape))
+    x, wt = rng.standard_normal((n, c, h, w)).astype(np.float32), (rng.standard_normal((cout, c, kernel, kernel)) * 0.03).astype(np.float32)
+    x[::3] = np.float32(1.2345678)
+    want = convolve(ctx, x, wt, stride)
+    ex, ew = (2.0 ** rng.choice(EXPONENTS, (count, 1, 1, 1)).astype(np.float32) for count in (n, cout))
+    assert (convolve(ctx, x * ex, wt, stride) == want * ex).all()
+    assert (convolve(ctx, x, wt * ew, stride) == want * ew[:, 0]).all()
+
+
+@pytest.mark.parametrize("shape", CONVS)
+def test_weights_that_are_vouched_for_change_no_bits(ctx, shape):
+    n, c, h, w, cout, kernel, stride = shape
+    rng = np.random.default_rng(sum(shape))
+    x, wt = rng.standard_normal((n, c, h, w)).astype(np.float32), (rng.standard_normal((cout, c, kernel, kernel)) * 0.03).astype(np.float32)
+    assert (convolve(ctx, x, wt, stride, True) == convolve(ctx, x, wt, stride, False)).all()
+
+
+@pytest.mark.parametrize("shape", [s for s in CONVS if s[5] == 1 or s[1] < 128])  # (minimal filtering adds inputs before it multiplies them)
+def test_a_conv_of_one_tap_moves_channels(ctx, shape):
+    n, c, h, w, cout, kernel, stride = shape
+    rng = np.random.default_rng(sum(shape))
+    x, wt = rng.standard_normal((n, c, h, w)).astype(np.float32), np.zeros((cout, c, kernel, kernel), np.float32)
+    pick = rng.integers(0, c, cout)
+    wt[np.arange(cout), pick, kernel // 2, kernel // 2] = 1
+    assert (convolve(ctx, x, wt, stride) == x[:, pick, ::stride, ::stride]).all()

@@ -1342,28 +1342,6 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
     const SplitPlan direct = plan_split(1, cout, (int)npix, (int)kdim, rows_split ? SPLIT_ROWS : SPLIT_TAPS);
     return direct.tile >= 0 && direct.us < transformed_us();
   };
-  // the f16 matrix cores, for weights that are kept (conv3x3_half.hip)
-  if ((flags & WDH_CONV_CONSTANT_WEIGHTS) && n >= 2 && (g_half > 1 || (g_winograd <= 1 && !g_winograd4_channels)) && rows_fit()) {
-    p.k = (int)kdim;
-    p.fast = 1;
-    const HalfOperand w3 = half_rows3x3(cout, c);
-    HalfPlan s = half_legal(p) && half_bytes(w3) < (1LL << 30) ? plan_half(cout, (int)npix, (int)kdim, HALF_3X3) : HalfPlan{-1, {}, 0.0, 0};
-    if (g_half == 1 && s.tile >= 0) {
-      const SplitPlan rows = plan_split(1, cout, (int)npix, (int)kdim, SPLIT_ROWS);
-      // (transforms, where they would serve, go on doing so while V and M stay below 100 MiB together, also where rows would be faster,
-      // because callers count on the form: 16 images 256 -> 256 on 28x28 80.5 us, 63 in rows; 32 on 14x14 45.6 / 46.9)
-      const bool by_transforms = g_winograd == 1 && wino_min >= 128 && !direct_suits();
-      const bool small_domain = 64LL * (c + cout) * wdh::wino_tiles(2, n, oh, ow) <= (100LL << 20);
-      if (by_transforms ? small_domain || s.us > 1.05 * transformed_us()
-                        : s.us > 1.05 * rows.us || !half_is_as_precise(s, split_chain(rows, (int)kdim), HALF_3X3)) s.tile = -1;
-    }
-    if (s.tile >= 0) {
-      rows_params();
-      if (int rc = WDH_OK; with_packed(FilterKey{hW, 3, cout, c}, w3, true, [&](const HalfOperand &o) { return half_pack3x3(p.A, o, cout, c); },
-                                       [&](const HalfOperand &o) { return run_half(s, [&](const HalfPlan &q) { return launch_conv3x3_half(p, q, o); }); }, &rc))
-        return rc;
-    }
-  }
   int wino_r = 0;
   if (g_winograd == 2) wino_r = 2;
   else if (g_winograd == 3) wino_r = 4;
