@@ -29,6 +29,7 @@ def test_an_empty_inner_dimension_leaves_the_other_terms(ctx, m, n, ta, tb):
 
 EXPONENTS = [0, -13, -20, -24, -28, -32, -40]
 CONVS = [  # n, c, h, w, cout, kernel, stride: enough sums of 500 to 4000 terms for the forms that large convs take
+    (32, 1024, 14, 14, 256, 1, 1), (60, 512, 12, 12, 128, 1, 1), (4, 512, 34, 36, 256, 1, 1), (64, 1024, 13, 15, 520, 1, 1), (16, 1024, 28, 28, 512, 1, 2),
     (64, 96, 28, 28, 96, 3, 1), (64, 128, 28, 28, 128, 3, 1), (128, 256, 14, 14, 256, 3, 1), (16, 256, 28, 28, 256, 3, 1), (9, 96, 31, 29, 100, 3, 1)]
 
 

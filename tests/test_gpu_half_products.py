@@ -8,7 +8,6 @@ from webdnn_amd import hostops as H
 pytestmark = pytest.mark.gpu
 
 TILES = {2: "128x256", 3: "128x128", 4: "64x128", 5: "64x128"}   # of products: columns are packed
-CONV_TILES = {2: "256x128", 3: "128x128", 4: "128x64", 5: "128x64"}
 
 
 @pytest.fixture
@@ -160,72 +159,3 @@ def test_a_batch_that_shares_its_weight_has_the_bits_of_one_tall_product(ctx, ha
     assert ctx.last_plan() == tall
     half(0)
     assert not (H.matmul(ctx, x, w).get_data() == plain.get_data()).all()   # (it is one for the f16 instruction)
-
-
-CONVS = [  # n, cin, h, w, cout, stride: whole planes, odd ones, strides, ragged K, rows and pixels
-    (3, 64, 8, 10, 70, 1), (2, 72, 7, 7, 64, 1), (5, 136, 9, 11, 130, 2), (2, 320, 12, 12, 260, 2), (2, 40, 5, 26, 16, 3), (9, 200, 4, 4, 300, 1)]
-
-
-def conv64(x, w, stride, pad, bias=None):
-    x, w = x.astype(np.float64), w.astype(np.float64)
-    k = w.shape[2]
-    windows = np.lib.stride_tricks.sliding_window_view(np.pad(x, ((0, 0), (0, 0), (pad[0], pad[2]), (pad[1], pad[3]))), (k, k), (2, 3))[:, :, ::stride, ::stride]
-    y = np.einsum("ncyxij,ocij->noyx", windows, w, optimize=True)
-    return y if bias is None else y + bias.reshape(1, -1, 1, 1)
-
-
-@pytest.mark.parametrize("mode,chunks", [(2, 1), (3, 1), (4, 1), (4, 2), (5, 1), (5, 2)])
-@pytest.mark.parametrize("shape", CONVS)
-def test_1x1_convs(ctx, half, mode, chunks, shape):
-    n, cin, h, w, cout, stride = shape
-    rng = np.random.default_rng(sum(shape))
-    x, wt = rng.standard_normal((n, cin, h, w)).astype(np.float32), rng.standard_normal((cout, cin, 1, 1)).astype(np.float32)
-    bias = rng.standard_normal(cout).astype(np.float32)
-    half(mode, chunks)
-    tx, tw, tb = (ctx.move_tensor(v) for v in (x, wt, bias))
-    run = lambda: H.conv(ctx, tx, tw, tb, strides=[stride, stride], epilogue="relu", constant_weights=True)
-    magnitudes = conv64(np.abs(x), np.abs(wt), stride, [0] * 4, np.abs(bias))
-    for _ in range(2):
-        y = run()
-        assert ctx.last_plan()["tile"] == CONV_TILES[mode] and ctx.last_plan()["split"] == min(chunks, (cin + 63) // 64), ctx.last_plan()
-        assert within(y.get_data(), np.maximum(conv64(x, wt, stride, [0] * 4, bias), 0), magnitudes, cin)
-    wt *= rng.choice([1e-12, 3, 1e9], (cout, 1, 1, 1)).astype(np.float32)  # (what was packed goes with the weights; rows of any scale)
-    tw.set_data(wt)
-    magnitudes = conv64(np.abs(x), np.abs(wt), stride, [0] * 4, np.abs(bias))
-    assert within(run().get_data(), np.maximum(conv64(x, wt, stride, [0] * 4, bias), 0), magnitudes, cin)
-    x[0, 1, h // 2, w // 2], x[n - 1, cin - 1, 0, 0] = np.inf, 1e30
-    tx.set_data(x)
-    out = {}
-    for value in (0, mode):
-        half(value, chunks)
-        out[value] = run().get_data()
-    assert (np.isnan(out[0]) == np.isnan(out[mode])).all() and (np.isinf(out[0]) == np.isinf(out[mode])).all()
-
-
-@pytest.mark.parametrize("shape,kernel", [((32, 1024, 14, 14, 256), 1)])
-def test_recorded_runs_read_what_was_packed(ctx, half, shape, kernel):
-    """Planned, packed before and while a graph is recorded, replayed between eager runs."""
-    n, c, h, w, cout = shape
-    rng = np.random.default_rng(5)
-    x, wt = ctx.move_tensor(rng.standard_normal((n, c, h, w)).astype(np.float32)), ctx.move_tensor((rng.standard_normal((cout, c, kernel, kernel)) * 0.02).astype(np.float32))
-    run = lambda: H.conv(ctx, x, wt, pads=[kernel // 2] * 4, constant_weights=True)
-    half(0)
-    other = run().get_data()
-    half(1)
-    want = []
-    for warm in (False, True):
-        if warm:
-            want.append(run().get_data())
-        ctx.sync()
-        ctx.graph_begin()
-        y = run()
-        graph = ctx.graph_end()
-        for _ in range(3):
-            ctx.graph_launch(graph)
-            want.append(y.get_data())
-            z = run()
-            want.append(z.get_data())
-            z.dispose()
-        ctx.graph_destroy(graph)
-    assert all((v == want[0]).all() for v in want)
-    assert not (want[0] == other).all() and np.abs(want[0].astype(np.float64) - other).max() <= 1e-5 * np.abs(other).max()

@@ -1032,42 +1032,6 @@ void drop_filters(const FilterKey &key) {
   (void)wdh_free(u);
 }
 
-// Runs `launch` on what `pack` makes of weights: kept from call to call (constant), or for this call only.  False: there was no room
-// for it; otherwise *rc says how it went.
-template <typename Pack, typename Launch>
-bool with_packed(const FilterKey &key, HalfOperand w, bool constant, Pack pack, Launch launch, int *rc) {
-  bool ready = false;
-  const size_t bytes = (size_t)half_bytes(w);
-  wdh_buf packed = constant ? kept_filters(key, bytes, &ready) : 0;
-  const bool kept = packed != 0;
-  if (!packed) packed = wdh_alloc(bytes);
-  if (!packed) {
-    wdh::clear_error();  // (nothing failed for the caller: the other forms need none)
-    return false;
-  }
-  w.packed = (unsigned char *)wdh::resolve(packed, nullptr);
-  *rc = ready ? WDH_OK : pack(w);
-  if (*rc == WDH_OK) *rc = launch(w);
-  if (*rc != WDH_OK && kept && !ready) drop_filters(key);  // (may not have been filled)
-  if (!kept) (void)wdh_free(packed);  // (back to the pool at once: whoever gets it next is ordered behind these kernels)
-  return true;
-}
-// A 1x1 conv on the f16 matrix cores, if it is one for them.
-bool half_conv1x1(Params &p, wdh_buf hW, int images, int group, int flags, int *rc) {
-  if (!(flags & WDH_CONV_CONSTANT_WEIGHTS) || group != 1 || images < 2 || !half_legal(p)) return false;
-  const HalfPlan s = plan_half(p.m, p.n, p.k, HALF_PIXELS);
-  if (s.tile < 0) return false;
-  if (g_half == 1) {
-    // (what would run as a stream of K slabs does so on the fp32 instruction, whose chains have no such limit)
-    const SplitPlan other = plan_pixels(1, p);
-    if (s.us > 1.05 * other.us || !(conv_streams(p, 1) || half_is_as_precise(s, split_chain(other, p.k), HALF_PIXELS))) return false;
-  }
-  const HalfOperand w = half_rows(p.m, p.k, true);
-  return half_bytes(w) < (1LL << 30) &&
-         with_packed(FilterKey{hW, 1, p.m, p.k}, w, true, [&](const HalfOperand &o) { return half_pack(p.A, o, p.m, p.k, p.sA0, 1); },
-                     [&](const HalfOperand &o) { return run_half(s, [&](const HalfPlan &q) { return launch_half_conv(q, p, o); }); }, rc);
-}
-
 }  // namespace
 
 namespace wdh {
@@ -1273,7 +1237,6 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
     p.c_bytes = cout * 4;
     set_wide(p, true);
     g_last_form = in_place_s2 ? B_PIXELS_S2 : B_PIXELS;
-    if (int rc = WDH_OK; half_conv1x1(p, hW, n, group, flags, &rc)) return rc;
     // (what the plan schedules as a stream of K slabs stays one)
     if (split_legal(p, true) && !(g_split == 1 && conv_streams(p, group)))
       if (const SplitPlan s = plan_pixels(group, p);
@@ -1467,7 +1430,6 @@ direct_forms:
     p.c_bytes = cout * 4;
     set_wide(p, true);
     g_last_form = WDH_FORM_CONV_GATHER32;  // (the form it stands in for)
-    if (int rc = WDH_OK; half_conv1x1(p, hW, n, group, flags, &rc)) return rc;
     SplitPlan s = {-1, {}, 0.0};
     if (split_legal(p, true) && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS))) s = plan_pixels(group, p);
     if (s.tile >= 0) return run_split(s, [&](const SplitPlan &q) { return launch_split_conv(B_PIXELS_ANY, q, p, group); });
