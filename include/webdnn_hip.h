@@ -116,13 +116,6 @@ int wdh_device_info(char *name, int name_cap, int *compute_units,
  *                       3..9 = that, with 128x128, 64x128, 128x64, 64x64, 256x128 (products only) tiles, or 64x64 ones whose K two or
  *                       four groups of wavefronts share (tuning and test hooks).
  *                       "stream_k" 2, and "contraction_tile" or "split_k" beside 1, keep the fp32 instruction.
- *   "half_products"     of those, which go to the f16 instruction instead, in three products of operands held in two f16 parts
- *                       (23 bits) and one packed beforehand: 1 (default) = large products, and convolutions with
- *                       WDH_CONV_CONSTANT_WEIGHTS, where that is faster and no less precise; tiles with an Inf, a NaN or elements
- *                       that two parts cannot hold are computed again with the fp32 instruction where that can show; 0 = none;
- *                       2..5 = wherever legal, with tiles of 256x128, 128x128 or 128x64, or 128x64 whose K two groups of
- *                       wavefronts share (3x3: 128x128, 64x128, 64x128 shared), "split_k" chunks (tuning and test hooks).
- *                       "split_products" other than 1 leaves it out.
  *   "wide_stores"       1 (default) = whole result tiles whose rows are 16-byte aligned
  *                       (Conv: output planes of a multiple of four pixels; Gemm: row and
  *                       batch strides of Y that are multiples of four) are turned through

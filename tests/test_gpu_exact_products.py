@@ -1,5 +1,5 @@
-"""What products and convolutions owe without any tolerance, whichever form they take: the sum over nothing; a sum of one term; images
-and channels scaled by powers of two; the same results whether or not weights are vouched for."""
+"""What products and convolutions owe without any tolerance, whichever form they take: the sum over nothing; a sum of one term; rows,
+columns and images scaled by powers of two; the same results whether or not weights are vouched for."""
 import numpy as np
 import pytest
 
@@ -27,8 +27,52 @@ def test_an_empty_inner_dimension_leaves_the_other_terms(ctx, m, n, ta, tb):
     assert (H.matmul(ctx, x, ctx.move_tensor(np.zeros((3, 0, n), np.float32))).get_data() == 0).all()
 
 
+# products and convs with sums of 500 to 4000 terms, enough of them for the forms that large ones take
+PRODUCTS = [(2866, 1016, 3336), (3807, 2004, 2736), (4096, 4096, 1024)]
 EXPONENTS = [0, -13, -20, -24, -28, -32, -40]
-CONVS = [  # n, c, h, w, cout, kernel, stride: enough sums of 500 to 4000 terms for the forms that large convs take
+
+
+def operands(m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), (rng.standard_normal((k, n)) * 0.03).astype(np.float32)
+    a[::7] = np.float32(1.2345678)   # (rows of one value among them, and columns)
+    b[:, ::5] = np.float32(0.87654321)
+    return rng, a, b
+
+
+def multiply(ctx, a, b, transposed):
+    y = H.gemm(ctx, ctx.move_tensor(a), ctx.move_tensor(np.ascontiguousarray(b.T) if transposed else b), trans_b=int(transposed))
+    out = y.get_data()
+    y.dispose()
+    return out
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("m,n,k", PRODUCTS)
+def test_rows_and_columns_of_other_magnitudes_are_the_same_sums(ctx, m, n, k, transposed):
+    """A power of two changes no rounding, whatever lies in the rows and columns beside it."""
+    rng, a, b = operands(m, n, k)
+    want = multiply(ctx, a, b, transposed)
+    ea, eb = (2.0 ** rng.choice(EXPONENTS, count).astype(np.float32) for count in (m, n))
+    assert (multiply(ctx, a * ea[:, None], b, transposed) == want * ea[:, None]).all()
+    assert (multiply(ctx, a, b * eb, transposed) == want * eb).all()
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("m,n,k", PRODUCTS)
+def test_a_sum_of_one_term_is_that_product(ctx, m, n, k, transposed):
+    rng, a, b = operands(m, n, k)
+    few = np.zeros_like(b)
+    pick = rng.permutation(max(n, k))[:n] % k
+    few[pick, np.arange(n)] = np.float32(0.5)
+    assert (multiply(ctx, a, few, transposed) == a[:, pick] * np.float32(0.5)).all()
+    few = np.zeros_like(a)
+    pick = rng.integers(0, k, m)
+    few[np.arange(m), pick] = np.float32(-2)
+    assert (multiply(ctx, few, b, transposed) == b[pick] * np.float32(-2)).all()
+
+
+CONVS = [  # n, c, h, w, cout, kernel, stride
     (32, 1024, 14, 14, 256, 1, 1), (60, 512, 12, 12, 128, 1, 1), (4, 512, 34, 36, 256, 1, 1), (64, 1024, 13, 15, 520, 1, 1), (16, 1024, 28, 28, 512, 1, 2),
     (64, 96, 28, 28, 96, 3, 1), (64, 128, 28, 28, 128, 3, 1), (128, 256, 14, 14, 256, 3, 1), (16, 256, 28, 28, 256, 3, 1), (9, 96, 31, 29, 100, 3, 1)]
 

@@ -18,7 +18,7 @@ ADDON_SRC = os.path.join(ROOT, "webdnn_amd", "napi", "addon.c")
 ADDON = os.path.join(LIBDIR, "webdnn_hip.node")
 
 HIP_SOURCES = ["runtime.hip", "gemm.hip", "contraction_gemm_akc.hip", "contraction_gemm_amc.hip", "contraction_conv_gather.hip",
-               "contraction_conv_pixels.hip", "contraction_conv3x3.hip", "split_gemm.hip", "split_conv.hip", "conv3x3_split.hip", "half_pack.hip", "half_gemm.hip", "conv_patch.hip", "winograd.hip", "depthwise.hip", "gemm_rows.hip", "elementwise.hip", "reduce.hip", "attention.hip", "pool_layout.hip"]
+               "contraction_conv_pixels.hip", "contraction_conv3x3.hip", "split_gemm.hip", "split_conv.hip", "conv3x3_split.hip", "conv_patch.hip", "winograd.hip", "depthwise.hip", "gemm_rows.hip", "elementwise.hip", "reduce.hip", "attention.hip", "pool_layout.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

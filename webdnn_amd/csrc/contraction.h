@@ -2037,34 +2037,5 @@ bool conv3x3_split_fits(ConvGeom &cv, int bn, int images, int pr);
 size_t packed3x3_bytes(int cout, int c);
 int pack3x3_launch(const float *W, void *P, int cout, int c);
 int launch_conv3x3_split(Params &p, const SplitPlan &s, const void *packed);
-// The same on the f16 matrix cores, one operand packed beforehand (half_product.h); k % 8 == 0.
-constexpr int HK = 64;            // k per block: plans cut K into whole blocks
-constexpr int HSTEP = 32;         // k per matrix instruction
-constexpr int STEP_BYTES = 2048;  // of a strip's 32 k: h of 64 lanes, then l
-constexpr int PACK_CHUNK = 8;     // steps that a workgroup of half_pack_kernel lays out, where it has not the whole K
-// The operand whose rows come packed: strips of 16 rows, [strip][32 k][h, l][lane][8]; row lane % 16, k 8 * (lane / 16) on.
-// Behind them the exponent that each row is scaled by, and for each strip and chunk how many elements lie below 2^FULL_EXPONENT.
-struct HalfOperand {
-  unsigned char *packed;
-  int strips, steps, chunks;  // of a 1x1 conv or a product steps are even; chunks: 1, or of PACK_CHUNK steps
-};
-__host__ __device__ constexpr long long half_fragment_bytes(long long strips, long long steps) { return strips * steps * STEP_BYTES; }
-constexpr long long half_bytes(const HalfOperand &w) { return half_fragment_bytes(w.strips, w.steps) + (long long)w.strips * (16 + w.chunks) * 4; }
-constexpr HalfOperand half_operand(int rows, int steps, bool whole) { return {nullptr, (rows + 15) / 16, steps, whole ? 1 : (steps + PACK_CHUNK - 1) / PACK_CHUNK}; }
-constexpr HalfOperand half_rows(int rows, int k, bool whole) { return half_operand(rows, (k + HK - 1) / HK * (HK / HSTEP), whole); }
-constexpr HalfOperand half_rows3x3(int cout, int c) { return half_operand(cout, c / 16 * 5, true); }  // (sixteen channels of two taps a step)
-enum HalfTile { H256x128 = 0, H128x128 = 1, H128x64 = 2, H128x64K2 = 3 };  // packed rows x columns; two groups share K
-enum Half3x3Tile { H3_128 = 0, H3_64 = 1, H3_64K2 = 2 };                   // output channels x 128 pixels
-struct HalfPlan {
-  int tile;       // HalfTile or Half3x3Tile, or -1: not a product for them
-  WorkPlan work;
-  double us;      // estimate
-  int chain;      // the longest chain of sums, in k
-};
-int half_pack(const float *W, const HalfOperand &out, int rows, int k, long long sr, long long sk);  // half_pack.hip
-int half_pack3x3(const float *W, const HalfOperand &out, int cout, int c);                           // half_pack.hip
-int launch_half_gemm(const HalfPlan &s, Params &p, const HalfOperand &w);                            // half_gemm.hip: B is packed
-int launch_half_conv(const HalfPlan &s, Params &p, const HalfOperand &w);                            // half_conv.hip: the weights are
-int launch_conv3x3_half(Params &p, const HalfPlan &s, const HalfOperand &w);                         // conv3x3_half.hip
 
 }  // namespace wdhc

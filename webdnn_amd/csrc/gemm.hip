@@ -142,7 +142,6 @@ int g_pixels_s2 = 1;      // 0: 1x1 convs with a column stride of 2 gather their
 int g_winograd4_channels = 0;  // when not 0: "conv3x3_winograd" 1 takes F(4x4, 3x3) from this many input and output channels on
 int g_winograd = 1;       // 3x3 stride-1 convs by minimal filtering: 0 never, 1 = F(2x2, 3x3) where it wins, 2 / 3 = F(2x2, 3x3) / F(4x4, 3x3) wherever legal
 int g_split = 1;          // products on the bf16 matrix cores (split_product.h): 0 never, 1 where they are faster, 2 wherever legal, 3 + t: that with tile t
-int g_half = 1;           // of those, on the f16 matrix cores (half_product.h): 0 never, 1 where they are faster, 2 + t: wherever legal with tile t
 int g_wide_stores = 1;    // 0: whole tiles store one element per lane and instruction
 int g_stream = 1;         // launches scheduled as streams of K slabs: 0 never, 1 where the plan below gains, 2 wherever legal
 int g_stream_wgs = 4;     // workgroups per CU of a stream launch (at most what the kernel's resources allow)
@@ -499,89 +498,6 @@ static int run_split(SplitPlan s, Launch launch) {
   s.work = {s.work.full + s.work.tail, 0, 1, 0};
   return launch(s);
 }
-// How a product on the f16 matrix cores is laid out (half_product.h, conv3x3_half.hip): as search_split, in blocks of 64 k (144 of a 3x3
-// conv).  np rows are packed, nq columns are the other operand's.  Fitted to 270 products, 250 convs of 1x1 and of 3x3 (0.5 to 30
-// GFLOP, every tile, 1, 2 and 4 cuts): 7 to 15 % off a single launch, and the form it picks takes 2 to 5 % longer than the best one.
-enum HalfKind { HALF_GEMM, HALF_PIXELS, HALF_3X3 };
-static HalfPlan search_half(int np, int nq, int k, HalfKind kind) {
-  struct Model { int bp, bq, groups; double block, solo, fixed, extra, sums; };
-  static const Model models[3][4] = {
-      {{256, 128, 1, 2.38, 2.28, 14.2, 3.5, 0.9}, {128, 128, 1, 1.42, 2.11, 15.5, 4.2, 0.3}, {128, 64, 1, 0.80, 1.21, 12.4, 2.0, 0.2}, {128, 64, 2, 0.73, 0.80, 14.2, 5.4, 0.2}},
-      {{256, 128, 1, 2.62, 2.56, 11.7, 7.1, 0.8}, {128, 128, 1, 1.63, 2.17, 12.0, 3.9, 0.6}, {128, 64, 1, 0.86, 1.12, 9.2, 3.0, 0.3}, {128, 64, 2, 0.92, 0.89, 11.3, 6.5, 0.2}},
-      {{128, 128, 1, 3.10, 2.91, 9.3, 4.4, 0.9}, {64, 128, 1, 1.67, 2.04, 9.7, 2.7, 0.7}, {64, 128, 2, 1.66, 1.65, 13.2, 8.1, 0.8}, {0, 0, 0, 0, 0, 0, 0, 0}}};
-  const long long cus = wdh::compute_units();
-  const int unit = kind == HALF_3X3 ? 144 : HK, blocks = (k + unit - 1) / unit;
-  HalfPlan best = {-1, {}, 1e30, 0};
-  for (int t = 0; t < 4; t++) {
-    const Model &mo = models[kind][t];
-    if (mo.bp == 0 || (g_half >= 2 && t != g_half - 2)) continue;
-    const long long tiles = (long long)((np + mo.bp - 1) / mo.bp) * ((nq + mo.bq - 1) / mo.bq);
-    const int most = g_half >= 2 ? (g_forced_split > 1 ? (g_forced_split < blocks ? g_forced_split : blocks) : 1) : k / 256 < 8 ? k / 256 : 8;
-    for (int s = g_half >= 2 ? most : 1; s == 1 || s <= most; s++) {
-      const int per = (blocks + s - 1) / s, chunks = (blocks + per - 1) / per;
-      if (chunks != s && g_half < 2) continue;
-      // the whole launch cut s ways, or only the tiles beyond the last full round
-      for (int part = 0; part < (chunks > 1 && g_half < 2 ? 2 : 1); part++) {
-        const long long tail = chunks == 1 ? 0 : part ? tiles % cus : tiles;
-        if (part && (tail == 0 || tail == tiles)) continue;
-        const long long whole = tiles - tail;
-        const long long rounds = chunks == 1 ? (tiles + cus - 1) / cus : whole / cus, cut_rounds = (tail * chunks + cus - 1) / cus;
-        const double path = (rounds ? blocks : per) * mo.solo, shared = (double)(rounds * blocks + cut_rounds * per) * mo.block;
-        double us = mo.fixed + (rounds + cut_rounds == 1 || shared < path ? path : shared) + mo.extra * (double)(rounds + cut_rounds - 1);
-        if (chunks > 1) us += 3.0 + mo.sums * (double)tail * chunks * mo.bp * mo.bq * 8.0 / 7.0e6;
-        if (us < best.us) best = {t, {whole, tail, chunks, per * unit}, us, (whole > 0 ? blocks : per) * unit / mo.groups};
-      }
-    }
-  }
-  return best;
-}
-static HalfPlan plan_half(int np, int nq, int k, HalfKind kind) {
-  struct Kept { int cus, np, nq, k, kind; HalfPlan plan; };
-  static thread_local Kept kept[256] = {};
-  if (g_half != 1) return search_half(np, nq, k, kind);
-  const int cus = wdh::compute_units();
-  unsigned h = (unsigned)np;
-  for (int v : {nq, k, (int)kind}) h = (h ^ (unsigned)v) * 0x9e3779b1u;
-  Kept &e = kept[h >> 24];
-  if (e.cus != cus || e.np != np || e.nq != nq || e.k != k || e.kind != (int)kind) e = {cus, np, nq, k, (int)kind, search_half(np, nq, k, kind)};
-  return e.plan;
-}
-// How long the longest chain of sums of a product in bfloat16 parts is, in k.
-static int split_chain(const SplitPlan &s, int k) {
-  return (s.work.full > 0 || s.work.tail == 0 ? k : s.work.kchunk) / (s.tile == S64x64K2 ? 2 : s.tile == S64x64K4 ? 4 : 1);
-}
-// Two parts hold 23 bits and leave out the smallest product, so a sum on the f16 matrix cores starts at 1.0e-7 (2-norm against 64 bits) and
-// grows by 5.1e-18 k in square, 6e-18 k for a 3x3 conv, because every 64 k leave the accumulator; one in bfloat16 parts starts at nothing
-// and grows by 2.0e-17 k (images after a Relu; 3.2e-17 on normal operands).  They meet at 700 k, and nearer than that the others are
-// kept.  (1e-7, that / this: 1x1 K 512 0.99 / 1.13, 1024 1.45 / 1.24, in eight chunks 0.71 / 1.24; fp32 instruction 2.3; 3x3 64 channels
-// 1.03 / 1.21, 128 1.51 / 1.32; by transforms 128 1.32 / 1.32, 256 1.60 / 1.58, 512 2.07 / 1.95; 4096^3 3.96 / 1.77.)
-static bool half_is_as_precise(const HalfPlan &s, int chain, HalfKind kind) {
-  return kind == HALF_3X3 ? 1.10e-14 + 6.0e-18 * s.chain <= 2.0e-17 * chain : 1.02e-14 + 5.1e-18 * s.chain <= 2.0e-17 * chain;
-}
-// A Gemm / MatMul, whose right operand is packed on every call: another launch, and for a caller that runs node by node another block of
-// memory, which the gain has to be worth ([4096, 768] x 3072 103 us / 90, [4096, 3072] x 768 122 / 107, and the feed-forward block around
-// them, from the host, 1016 / 1016; 4096^3 660 / 420, 3807x2004x2736 255 / 173, 2866x1016x3336 138 / 114; 1182x3132x2416 114 / 98 stays).
-static HalfPlan half_gemm_plan(int m, int n, int k, bool b_kc) {
-  HalfPlan s = plan_half(n, m, k, HALF_GEMM);
-  if (g_half != 1 || s.tile < 0) return s;
-  const SplitPlan other = split_gemm_plan(1, m, n, k, b_kc);
-  const double pack = b_kc ? 4.0 + 8.0 * n * k / 2.0e6 : 6.0 + 8.0 * n * k / 1.2e6;
-  if (other.tile < 0 || s.us + pack > 0.85 * other.us || !half_is_as_precise(s, split_chain(other, k), HALF_GEMM)) s.tile = -1;
-  return s;
-}
-// Whether the f16 matrix cores may serve a product at all.  (An empty K has no blocks to plan, and nothing to multiply.)
-static bool half_legal(const Params &p) {
-  if (!g_half || g_split != 1 || g_fp32_hint || g_stream == 2 || !p.fast || p.k < 8 || p.k % 8 != 0 || g_static_scratch || g_group.collecting) return false;
-  return g_half > 1 || (g_forced_tile < 0 && g_forced_split < 0);
-}
-template <typename Launch>
-static int run_half(HalfPlan s, Launch launch) {
-  const int rc = launch(s);
-  if (rc != WDH_ENOMEM || s.work.tail == 0) return rc;
-  wdh::clear_error();  // (nothing failed for the caller)
-  s.work = {s.work.full + s.work.tail, 0, 1, 0};
-  return launch(s);
-}
 // Whether the bf16 matrix cores may serve a product at all.
 static bool split_legal(const Params &p, bool vec) {
   if (!g_split || g_fp32_hint || g_stream == 2 || !p.fast || !vec || p.k % 4 != 0 || p.k < BK || g_static_scratch) return false;
@@ -619,11 +535,6 @@ extern "C" int wdh_set_option(const char *name, int value) {
     if (value != 0 && value != 1)
       return fail(WDH_EINVAL, "wdh_set_option: wide_stores %d (use 0 or 1)", value);
     g_wide_stores = value;
-    return WDH_OK;
-  }
-  if (strcmp(name, "half_products") == 0) {
-    if (value < 0 || value > 2 + H128x64K2) return fail(WDH_EINVAL, "wdh_set_option: half_products %d (use 0..%d)", value, 2 + H128x64K2);
-    g_half = value;
     return WDH_OK;
   }
   if (strcmp(name, "split_products") == 0) {
@@ -823,26 +734,6 @@ extern "C" int wdh_gemm_ex(wdh_buf hA, wdh_buf hB, wdh_buf hC, wdh_buf hY,
   if (useA_kc && useB_kc && gemm_rows_suits(batch, m, n, k, vec)) return launch_gemm_rows(p, batch, vec);
   // Enough to multiply: the bf16 matrix cores (split_product.h; they read columns of B in pairs, and every element they
   // read decides whether a tile is done again, so a pair must not reach into what lies beside the matrix)
-  // (a batch that shares B and lies row behind row is one tall product, so that a residual, with which callers leave the batch as it
-  // is, does not decide the form)
-  const bool tall = batch > 1 && sBb == 0 && sAb == (int64_t)m * p.sA0 && sYb == (int64_t)m * sY0 && (!p.C || sC0 == 0);
-  if ((batch == 1 || tall) && useA_kc && vec && half_legal(p) && (long long)batch * m < 0x7fffffffLL &&
-      span(1, 0, (long long)batch * m, p.sA0, k, 1) * 4 < 0x7fffffffLL - 4096) {
-    Params q = p;
-    q.m = batch * m;
-    q.a_bytes = (int)(span(1, 0, q.m, p.sA0, k, 1) * 4);
-    HalfOperand w = half_rows(n, k, false);
-    if (const HalfPlan s = half_gemm_plan(q.m, n, k, useB_kc); s.tile >= 0 && half_bytes(w) < (1LL << 30)) {
-      if (const wdh_buf packed = wdh_alloc((size_t)half_bytes(w))) {
-        w.packed = (unsigned char *)wdh::resolve(packed, nullptr);
-        int rc = half_pack(q.B, w, n, k, q.sB1, q.sB0);
-        if (rc == WDH_OK) rc = run_half(s, [&](const HalfPlan &h) { return launch_half_gemm(h, q, w); });
-        (void)wdh_free(packed);
-        return rc;
-      }
-      wdh::clear_error();  // (no room for them: the other forms need none)
-    }
-  }
   if (useA_kc && split_legal(p, vec) && (useB_kc || n % 2 == 0)) {
     if (const SplitPlan s = split_gemm_plan(batch, m, n, k, useB_kc); s.tile >= 0) {
       auto launch = [&](const SplitPlan &q) { return launch_split_gemm(useB_kc, q, p, batch); };
@@ -1008,7 +899,7 @@ std::map<KtabKey, KtabVal> g_ktabs;
 // go, because recorded graphs read it.
 struct FilterKey {
   wdh_buf weights;
-  int form, cout, c;  // form: 2 or 4 = transformed for that output patch, 0 = in bfloat16 parts (conv3x3_split.hip), 1 and 3 = in f16 parts of a 1x1 or 3x3 conv (half_pack.hip)
+  int form, cout, c;  // form: 2 or 4 = transformed for that output patch, 0 = in parts (conv3x3_split.hip)
   bool operator<(const FilterKey &o) const {
     return std::tie(weights, form, cout, c) < std::tie(o.weights, o.form, o.cout, o.c);
   }
@@ -1236,8 +1127,8 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
     p.y_bytes = g_descriptors && out_bytes < 0x7fffffffULL ? (int)out_bytes : 0;
     p.c_bytes = cout * 4;
     set_wide(p, true);
-    g_last_form = in_place_s2 ? B_PIXELS_S2 : B_PIXELS;
     // (what the plan schedules as a stream of K slabs stays one)
+    g_last_form = in_place_s2 ? B_PIXELS_S2 : B_PIXELS;
     if (split_legal(p, true) && !(g_split == 1 && conv_streams(p, group)))
       if (const SplitPlan s = plan_pixels(group, p);
           s.tile >= 0 && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS)))
@@ -1260,26 +1151,11 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   // that is set: one image is faster so from 64 channels on, 32 images of ResNet-50 are not (2.29 ms for 2.21), and its rounding
   // errors are about ten times the direct form's, which a 50-layer network's logits show); 2 / 3 = F(2x2, 3x3) / F(4x4, 3x3) wherever legal.
   const int wino_min = c < cout ? c : cout;
-  auto rows_fit = [&]() {
-    if (!(g_halo && small && kh == 3 && kw == 3 && sh == 1 && sw == 1 && dh == 1 && dw == 1 && group == 1 && c % 16 == 0)) return false;
+  auto rows_possible = [&]() {
+    if (!(g_halo && kh == 3 && kw == 3 && sh == 1 && sw == 1 && dh == 1 && dw == 1 && group == 1 && c % 16 == 0)) return false;
+    if (!split_possible(n, cout, (int)kdim) || packed3x3_bytes(cout, c) >= 0x7fffffffULL || g_split > 4) return false;
     p.cv.h = h; p.cv.w = w; p.cv.oh = oh; p.cv.ow = ow; p.cv.pt = pt; p.cv.pl = pl;
     return conv3x3_split_fits(p.cv, 128, n, pr);
-  };
-  auto rows_possible = [&]() {
-    return split_possible(n, cout, (int)kdim) && packed3x3_bytes(cout, c) < 0x7fffffffULL && g_split <= 4 && rows_fit();
-  };
-  auto rows_params = [&]() {
-    p.m = cout_g; p.n = (int)npix; p.k = (int)kdim;
-    p.sAb = 0; p.sA0 = kdim; p.sA1 = 1;
-    p.alpha = 1.0f; p.beta = 1.0f; p.epilogue = epilogue;
-    p.cv.c_in_g = c; p.cv.sh = p.cv.sw = p.cv.dh = p.cv.dw = 1; p.cv.kh = p.cv.kw = 3;
-    p.cv.c_total = c; p.cv.cout_total = cout; p.cv.cout_g = cout;
-    p.cv.ntaps = 9; p.cv.npix = npix;
-    p.fast = 1;
-    p.b_bytes = (int)((long long)n * c * h * w * 4);
-    p.y_bytes = g_descriptors && out_bytes < 0x7fffffffULL ? (int)out_bytes : 0;
-    p.c_bytes = cout * 4;
-    set_wide(p, true);
   };
   const bool rows_split = rows_possible();
   bool wino_memory = true;  // there was room for the transform-domain tensors, if they were wanted
@@ -1291,19 +1167,16 @@ extern "C" int wdh_conv2d_ex(wdh_buf hX, wdh_buf hW, wdh_buf hBias, wdh_buf hY,
   // 4 images 512 -> 160 on 45x63 100 / 141, 2 images 832 -> 192 on 63x63 105 / 149; 224 -> 992 on 8x8 12.3 / 14.8.)
   // Transform-domain tensors that outgrow the 256 MB last-level cache cost more (128 images 128 -> 128 on 28x28, V and M 206 MB
   // each, 254 / 150); there gathered taps are asked too, where rows are too wide for LDS (13 images 336 -> 416 on 19x91 293 / 447).
-  auto transformed_us = [&]() {
-    const long long pitch = wdh::wino_pitch(wdh::wino_tiles(2, n, oh, ow));
-    const double v = 4.0 * c * (16.0 * (double)pitch + (double)n * h * w), m = 4.0 * cout * (16.0 * (double)pitch + (double)npix);
-    return 8.6 + 0.94 * plan_split(16, cout, (int)pitch, c, SPLIT_GEMM).us + 0.19e-6 * v + 0.245e-6 * m;
-  };
   auto direct_suits = [&]() {
     if (g_winograd != 1 || !(gather_split || rows_split)) return false;
-    const long long blocks = wdh::wino_tiles(2, n, oh, ow);
+    const long long blocks = wdh::wino_tiles(2, n, oh, ow), pitch = wdh::wino_pitch(blocks);
     const bool outgrown = 64LL * (c + cout) * blocks > (256LL << 20);
     if (rows_split && outgrown) return true;
     if (rows_split ? npix < 3500 : !outgrown) return false;
+    const double v = 4.0 * c * (16.0 * (double)pitch + (double)n * h * w), m = 4.0 * cout * (16.0 * (double)pitch + (double)npix);
+    const SplitPlan product = plan_split(16, cout, (int)pitch, c, SPLIT_GEMM);
     const SplitPlan direct = plan_split(1, cout, (int)npix, (int)kdim, rows_split ? SPLIT_ROWS : SPLIT_TAPS);
-    return direct.tile >= 0 && direct.us < transformed_us();
+    return direct.tile >= 0 && direct.us < 8.6 + 0.94 * product.us + 0.19e-6 * v + 0.245e-6 * m;
   };
   int wino_r = 0;
   if (g_winograd == 2) wino_r = 2;
@@ -1372,7 +1245,17 @@ direct_forms:
     const bool kept = hP != 0;
     if (!hP) hP = wdh_alloc(packed3x3_bytes(cout, c));
     if (hP) {
-      rows_params();
+      p.m = cout_g; p.n = (int)npix; p.k = (int)kdim;
+      p.sAb = 0; p.sA0 = kdim; p.sA1 = 1;
+      p.alpha = 1.0f; p.beta = 1.0f; p.epilogue = epilogue;
+      p.cv.c_in_g = c; p.cv.sh = p.cv.sw = p.cv.dh = p.cv.dw = 1; p.cv.kh = p.cv.kw = 3;
+      p.cv.c_total = c; p.cv.cout_total = cout; p.cv.cout_g = cout;
+      p.cv.ntaps = 9; p.cv.npix = npix;
+      p.fast = 1;
+      p.b_bytes = (int)((long long)n * c * h * w * 4);
+      p.y_bytes = g_descriptors && out_bytes < 0x7fffffffULL ? (int)out_bytes : 0;
+      p.c_bytes = cout * 4;
+      set_wide(p, true);
       void *const packed = wdh::resolve(hP, nullptr);
       int rc = ready ? WDH_OK : pack3x3_launch(p.A, packed, cout, c);
       if (rc == WDH_OK)
@@ -1415,24 +1298,27 @@ direct_forms:
   // any other unpadded 1x1 conv of a batch: each pixel of X is read where it lies, whatever the strides and the plane
   if (small && vec && ntaps == 1 && pt == 0 && pl == 0 && pb == 0 && pr == 0) {
     p.m = cout_g; p.n = (int)npix; p.k = (int)kdim;
-    p.sAb = (long long)cout_g * kdim; p.sA0 = kdim; p.sA1 = 1;
-    p.sBb = (long long)c_in_g * plane; p.sB0 = plane; p.sB1 = 1;
-    p.alpha = 1.0f; p.beta = 1.0f; p.epilogue = epilogue;
-    p.cv.c_in_g = c_in_g; p.cv.h = h; p.cv.w = w; p.cv.oh = oh; p.cv.ow = ow;
-    p.cv.sh = sh; p.cv.sw = sw;
-    p.cv.kh = p.cv.kw = p.cv.dh = p.cv.dw = 1;
-    p.cv.c_total = c; p.cv.cout_total = cout; p.cv.cout_g = cout_g;
-    p.cv.ntaps = 1; p.cv.npix = npix;
+    p.cv.oh = oh; p.cv.ow = ow;
     p.fast = 1;
-    p.a_bytes = (int)w_bytes;
-    p.b_bytes = (int)x_bytes;
-    p.y_bytes = g_descriptors && out_bytes < 0x7fffffffULL ? (int)out_bytes : 0;
-    p.c_bytes = cout * 4;
-    set_wide(p, true);
-    g_last_form = WDH_FORM_CONV_GATHER32;  // (the form it stands in for)
     SplitPlan s = {-1, {}, 0.0};
     if (split_legal(p, true) && (g_split > 1 || split_conv_suits(n, p.m, p.k, SPLIT_PIXELS))) s = plan_pixels(group, p);
-    if (s.tile >= 0) return run_split(s, [&](const SplitPlan &q) { return launch_split_conv(B_PIXELS_ANY, q, p, group); });
+    if (s.tile >= 0) {
+      p.sAb = (long long)cout_g * kdim; p.sA0 = kdim; p.sA1 = 1;
+      p.sBb = (long long)c_in_g * plane; p.sB0 = plane; p.sB1 = 1;
+      p.alpha = 1.0f; p.beta = 1.0f; p.epilogue = epilogue;
+      p.cv.c_in_g = c_in_g; p.cv.h = h; p.cv.w = w; p.cv.oh = oh; p.cv.ow = ow;
+      p.cv.sh = sh; p.cv.sw = sw;
+      p.cv.kh = p.cv.kw = p.cv.dh = p.cv.dw = 1;
+      p.cv.c_total = c; p.cv.cout_total = cout; p.cv.cout_g = cout_g;
+      p.cv.ntaps = 1; p.cv.npix = npix;
+      p.a_bytes = (int)w_bytes;
+      p.b_bytes = (int)x_bytes;
+      p.y_bytes = g_descriptors && out_bytes < 0x7fffffffULL ? (int)out_bytes : 0;
+      p.c_bytes = cout * 4;
+      set_wide(p, true);
+      g_last_form = WDH_FORM_CONV_GATHER32;  // (the form it stands in for)
+      return run_split(s, [&](const SplitPlan &q) { return launch_split_conv(B_PIXELS_ANY, q, p, group); });
+    }
   }
   auto it = g_ktabs.find(key);
   if (it == g_ktabs.end()) {
