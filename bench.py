@@ -20,7 +20,7 @@ Conv/Gemm node as the direct sum needs them, summed over the node list) over the
 the timed steps, measured with one HIP event pair on the library's stream around each graph replay
 (the step's other kernels are inside that bracket, which makes the figure a lower bound).  The peak
 is the fp32 matrix instruction's; it bounds neither minimal filtering, which issues fewer
-multiplications than that numerator counts, nor products made of six bf16 or three f16 ones, so fractions may exceed 1.
+multiplications than that numerator counts, nor products made of six bf16 ones, so fractions may exceed 1.
 Inside `roofline`, so that one record holds everything the metric names:
   kernels        Gemm 4096^3 and the config-3 Conv as single-kernel figures (ms, GFLOP/s, fraction of the
                  fp32 MFMA peak), each timed as replays of a HIP graph that holds the launches back to back,
@@ -53,8 +53,7 @@ if ROOT not in sys.path:
 import numpy as np  # noqa: E402
 
 METRIC = "fp32 Gemm/Conv GFLOP/s (% MFMA peak) + ResNet-50 b32 images/sec, 1 MI355X"
-# The fp32 matrix instruction's peak.  fp32 products made of six bf16 ones (csrc/split_product.h) or
-# three f16 ones (csrc/half_product.h) may exceed it.
+# The fp32 matrix instruction's peak.  fp32 products made of six bf16 ones (csrc/split_product.h) may exceed it.
 PEAK_FP32_MFMA_TFLOPS = 157.3
 # HBM-side bytes of the ResNet-50 step per Conv / Gemm node (54 nodes; contraction kernels, reduce passes
 # and the transforms of the minimal-filtering convs): rocprofv3 --pmc FETCH_SIZE (x2.000) + WRITE_SIZE
@@ -524,7 +523,7 @@ def main():
             "bound": "mfma",
             "kernel": "contraction kernels (implicit-GEMM Conv: in-place 1x1, LDS-tile 3x3, F(2x2,3x3) minimal filtering "
                       "for 3x3 of 256 and 512 channels, gathered forms, stem; Gemm head; most as six bf16 products on operands split "
-                      "exactly or three f16 ones, so that peak, the fp32 instruction's, is no limit), %d Conv/Gemm nodes per step; device "
+                      "exactly, so that peak, the fp32 instruction's, is no limit), %d Conv/Gemm nodes per step; device "
                       "time = HIP events around each timed graph replay (whole step: transforms, MaxPool and "
                       "GlobalAveragePool included); achieved = direct-sum FLOPs (2MNK per node) / that time"
                       % resnet["contraction_launches"],
